@@ -132,7 +132,7 @@ int hplai_getrf_nopiv_f32(hplai_ctx ctx, int n, float *A, int64_t lda, int *info
     CTX_CHECK(ctx);
     HPLAI_CHECK(n >= 0 && n <= 1024, "getrf_nopiv: n=%d outside [0,1024]", n);
     HPLAI_CHECK(A != nullptr && lda >= n, "getrf_nopiv: A NULL or lda < n");
-    return launch_getrf(n, A, lda, info_dev, as_stream(stream));
+    return launch_getrf(n, A, lda, info_dev, nullptr, as_stream(stream));
 }
 
 int hplai_trsm_lpanel_f32(hplai_ctx ctx, int64_t m, int b, const float *Ukk, int64_t ldu, float *L,

@@ -167,32 +167,23 @@ __device__ __forceinline__ void tile_max_reduce(float *amax, int64_t tile, float
 
 namespace hplai {
 
-// In-place inverse of a lower-triangular 32 x 32 matrix held in LDS
-// (M[r * 33 + c], non-zero diagonal) by recursive doubling:
-//   [A 0; C B]^-1 = [A^-1 0; -B^-1 C A^-1, B^-1]
-// with block sizes 1, 2, 4, 8, 16.  T is a 32 x 33 LDS scratch.  Every thread
-// of the workgroup must call it (it contains barriers).
-__device__ inline void lower_inv32(float *M, float *T, int tid, int nthr)
+// Packed inverses of the triangles of a b x b block in 32 x 32 blocks of 1024
+// floats, nb = ceil(b / 32), entries past b those of the identity:
+//   Linv block (I, J): [lane 16 + kk] = Linv(32 I + lane % 32, 32 J + 2 kk + lane / 32),
+//   the left operand of v_mfma_f32_32x32x2_f32 (for U := Linv A);
+//   Uinv block (I, J): [lane 16 + kk] = Uinv(32 I + 2 kk + lane / 32, 32 J + lane % 32),
+//   the right operand (for L := A Uinv).
+// Blocks above the diagonal of Linv and below the diagonal of Uinv are never
+// written or read.
+template <typename T>
+__device__ __forceinline__ T *tri_block_l(T *tri, int nb, int I, int J)
 {
-    for (int i = tid; i < 32; i += nthr) M[i * 33 + i] = 1.0f / M[i * 33 + i];
-    __syncthreads();
-    for (int s = 1; s < 32; s *= 2) {
-        const int np = 16 / s, per = s * s;
-        for (int e = tid; e < np * per; e += nthr) {      // T = C A^-1
-            const int p = e / per, ij = e % per, i = ij / s, j = ij % s, base = p * 2 * s;
-            float acc = 0.0f;
-            for (int k = j; k < s; ++k) acc = fmaf(M[(base + s + i) * 33 + base + k], M[(base + k) * 33 + base + j], acc);
-            T[(base + s + i) * 33 + base + j] = acc;
-        }
-        __syncthreads();
-        for (int e = tid; e < np * per; e += nthr) {      // C = -B^-1 T
-            const int p = e / per, ij = e % per, i = ij / s, j = ij % s, base = p * 2 * s;
-            float acc = 0.0f;
-            for (int k = 0; k <= i; ++k) acc = fmaf(M[(base + s + i) * 33 + base + s + k], T[(base + s + k) * 33 + base + j], acc);
-            M[(base + s + i) * 33 + base + j] = -acc;
-        }
-        __syncthreads();
-    }
+    return tri + (static_cast<int64_t>(I) * nb + J) * 1024;
+}
+template <typename T>
+__device__ __forceinline__ T *tri_block_u(T *tri, int nb, int I, int J)
+{
+    return tri + (static_cast<int64_t>(nb) * nb + static_cast<int64_t>(J) * nb + I) * 1024;
 }
 
 }  // namespace hplai

@@ -1,0 +1,855 @@
+// getrf.hip — LU of a diagonal block (n <= 1024) and the inverses of its
+// triangles, spread over the device.
+//
+// Replaces getrf_nopiv (getrf_nopiv.hpp:124-160).  The block is walked in
+// sub-blocks of 128 columns; per sub-block three kinds of work, all FP32 on
+// v_mfma_f32_32x32x2_f32:
+//   lu_update_kernel  workgroup 0 takes the 128 x 128 diagonal sub-block: its
+//                     update with the sub-block before it, its LU and the
+//                     inverses of both triangles, all in LDS; the other
+//                     workgroups update the rest of the trailing matrix;
+//   lu_strip_kernel   L21 := A21 U11^-1 and U12 := L11^-1 A12 as products
+//                     with those inverses, 32 rows or columns per workgroup.
+// Then tri_merge_kernel joins the inverses of neighbouring sub-blocks (128 ->
+// 256 -> 512 -> 1024):
+//   [A 0; C B]^-1 = [A^-1 0; -B^-1 C A^-1, B^-1].
+//
+// What bounds it: the chain of 32 x 32 LUs, inverses and strips (17k clocks a
+// link, one or two waves working) and, between sub-blocks, a launch and the
+// 128^3 update of the next diagonal sub-block.  One workgroup for the whole
+// 512 block spent half its time on trailing updates through a single CU's
+// path to the L2, and the inverses were two more kernels after it: 511 + 73
+// us, now 200 us and about 25 us for the joins (b = 512, alone); b = 60: 94 ->
+// 15 us; n = 1000: 645 us with v_readlane steps, 427 us as here.
+#include <type_traits>
+#include <utility>
+
+#include "device_common.hpp"
+#include "internal.hpp"
+
+namespace hplai {
+
+typedef float floatx16g_t __attribute__((ext_vector_type(16)));
+
+constexpr int kLuNB = 128;            // columns per sub-block
+constexpr int kLuThreads = 512;
+constexpr int kLuS = kLuNB + 1;       // LDS column stride: odd, so that walks along rows and columns both spread
+constexpr int kMergeMax = 512;        // largest half joined by tri_merge_kernel
+
+__device__ __forceinline__ floatx16g_t zero16()
+{
+    floatx16g_t z;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) z[e] = 0.0f;
+    return z;
+}
+
+// LDS stores of the wave's lanes before, seen by its other lanes after
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// acc[4 q + r] of a 32 x 32 MFMA result is row 8 q + 4 (lane / 32) + r, column lane % 32
+__device__ __forceinline__ int acc_row(int e, int lh) { return 8 * (e >> 2) + 4 * lh + (e & 3); }
+
+struct LuLds {
+    float S[kLuNB * kLuS];            // the sub-block, S[c * kLuS + r]
+    float V[kLuNB * kLuS];            // its inverses: Linv below the diagonal (unit diagonal implied), Uinv on and above
+    float Li[32 * 33], Ui[32 * 33];   // inverses of the current 32 x 32 triangles, row-major
+};
+
+// entry (i, j) of a unit-lower / an upper triangle whose block also holds the other one
+__device__ __forceinline__ float lower_entry(float v, int i, int j) { return i > j ? v : (i == j ? 1.0f : 0.0f); }
+__device__ __forceinline__ float upper_entry(float v, int i, int j) { return i <= j ? v : 0.0f; }
+
+// acc += A B of one 32 x 32 x 32 product from its operand registers.  The
+// operands are loaded before: left to itself the compiler waits for each load
+// right before its product.
+__device__ __forceinline__ floatx16g_t mfma16(const float (&av)[16], const float (&bv)[16], floatx16g_t acc)
+{
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[kk], bv[kk], acc, 0, 0, 0);
+    return acc;
+}
+
+// The 32 x 32 steps run in one wave, lane = 16 g + r: r is a row of 16 and g
+// splits the columns four ways.  A pivot row then reaches the other rows of
+// its 16 lanes as a DPP row broadcast inside the multiply-add; with one row
+// per lane and v_readlane the same steps took 2.2 (LU) and 4 times (inverse)
+// as long, one scalar broadcast per element.
+// (written out: the compiler does not fold the broadcast into v_fmac_f32.  A
+// DPP operand must not be one of the last two instructions' results, so each
+// sequence waits two slots first and reads nothing that it has written.)
+template <int K>
+__device__ __forceinline__ float bcast16(float v)   // lane K of every 16
+{
+    float o;
+    asm("s_nop 1\n\tv_mov_b32_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "=v"(o) : "v"(v), "n"(K));
+    return o;
+}
+#define HPLAI_FMAC16(D, B, M) "\n\tv_fmac_f32_dpp " D ", " B ", " M " row_newbcast:%[k] row_mask:0xf bank_mask:0xf"
+// p += mp * q and then q += mq * q, with q's lane K of every 16 for the last q
+template <int K>
+__device__ __forceinline__ void fmac16_2(float &p, float mp, float &q, float mq)
+{
+    asm("s_nop 1" HPLAI_FMAC16("%0", "%1", "%2") HPLAI_FMAC16("%1", "%1", "%3")
+        : "+&v"(p), "+&v"(q)
+        : "v"(mp), "v"(mq), [k] "n"(K));
+}
+template <int K>
+__device__ __forceinline__ void fmac16_2x4(float &p0, float &p1, float &p2, float &p3, float mp, float &q0, float &q1,
+                                           float &q2, float &q3, float mq)
+{
+    asm("s_nop 1" HPLAI_FMAC16("%0", "%4", "%8") HPLAI_FMAC16("%1", "%5", "%8") HPLAI_FMAC16("%2", "%6", "%8")
+            HPLAI_FMAC16("%3", "%7", "%8") HPLAI_FMAC16("%4", "%4", "%9") HPLAI_FMAC16("%5", "%5", "%9")
+                HPLAI_FMAC16("%6", "%6", "%9") HPLAI_FMAC16("%7", "%7", "%9")
+        : "+&v"(p0), "+&v"(p1), "+&v"(p2), "+&v"(p3), "+&v"(q0), "+&v"(q1), "+&v"(q2), "+&v"(q3)
+        : "v"(mp), "v"(mq), [k] "n"(K));
+}
+// q += m * q's lane K of every 16
+template <int K>
+__device__ __forceinline__ void fmac16_1(float &q, float m)
+{
+    asm("s_nop 1" HPLAI_FMAC16("%0", "%0", "%1") : "+&v"(q) : "v"(m), [k] "n"(K));
+}
+template <int K>
+__device__ __forceinline__ void fmac16_1x4(float &q0, float &q1, float &q2, float &q3, float m)
+{
+    asm("s_nop 1" HPLAI_FMAC16("%0", "%0", "%4") HPLAI_FMAC16("%1", "%1", "%4") HPLAI_FMAC16("%2", "%2", "%4")
+            HPLAI_FMAC16("%3", "%3", "%4")
+        : "+&v"(q0), "+&v"(q1), "+&v"(q2), "+&v"(q3)
+        : "v"(m), [k] "n"(K));
+}
+// columns J .. N - 1 of p and q (fmac16_2) or of q alone
+template <int K, int J, int N>
+__device__ __forceinline__ void fmac16_cols(float *p, float mp, float *q, float mq)
+{
+    if constexpr (J + 4 <= N) {
+        fmac16_2x4<K>(p[J], p[J + 1], p[J + 2], p[J + 3], mp, q[J], q[J + 1], q[J + 2], q[J + 3], mq);
+        fmac16_cols<K, J + 4, N>(p, mp, q, mq);
+    } else if constexpr (J < N) {
+        fmac16_2<K>(p[J], mp, q[J], mq);
+        fmac16_cols<K, J + 1, N>(p, mp, q, mq);
+    }
+}
+template <int K, int J, int N>
+__device__ __forceinline__ void fmac16_cols(float *q, float m)
+{
+    if constexpr (J + 4 <= N) {
+        fmac16_1x4<K>(q[J], q[J + 1], q[J + 2], q[J + 3], m);
+        fmac16_cols<K, J + 4, N>(q, m);
+    } else if constexpr (J < N) {
+        fmac16_1<K>(q[J], m);
+        fmac16_cols<K, J + 1, N>(q, m);
+    }
+}
+
+template <int... I, typename F>
+__device__ __forceinline__ void unrolled(std::integer_sequence<int, I...>, F &&f)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void unrolled(F &&f)
+{
+    unrolled(std::make_integer_sequence<int, N>{}, f);
+}
+
+// Reciprocal of a pivot: v_rcp_f32 and one Newton step (half the instructions
+// of the IEEE division) for magnitudes where that cannot over- or underflow;
+// EXACT divides.
+template <bool EXACT>
+__device__ __forceinline__ float pivot_rcp(float p)
+{
+    if (EXACT) return 1.0f / p;
+    const float r = __builtin_amdgcn_rcpf(p);
+    return fmaf(fmaf(-p, r, 1.0f), r, r);
+}
+
+// LU of the 32 x 32 block at (c0, c0) of S in place.  Every group of 16 lanes
+// holds all 16 columns of the current panel (Pt: rows 0..15, Pb: rows 16..31)
+// and a quarter of the columns right of it.  Returns the pivot of lane
+// (row) lane % 32; without EXACT the block is not written when a pivot's
+// magnitude is outside [2^-100, 2^100].
+template <bool EXACT>
+__device__ __forceinline__ float lu32_run(float *S, int c0, int lane)
+{
+    const int r = lane & 15, g = lane >> 4;
+    float *B = S + c0 * kLuS + c0;
+    float Pt[16], Pb[16], Rt[4], Rb[4];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+        Pt[c] = B[c * kLuS + r];
+        Pb[c] = B[c * kLuS + 16 + r];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        Rt[u] = B[(16 + 4 * u + g) * kLuS + r];
+        Rb[u] = B[(16 + 4 * u + g) * kLuS + 16 + r];
+    }
+    unrolled<16>([&](auto kc) {
+        constexpr int k = kc;
+        const float inv = pivot_rcp<EXACT>(bcast16<k>(Pt[k]));
+        const float lt = r > k ? Pt[k] * inv : 0.0f, lb = Pb[k] * inv;
+        Pt[k] = r > k ? lt : Pt[k];
+        Pb[k] = lb;
+        fmac16_cols<k, k + 1, 16>(Pb, -lb, Pt, -lt);
+        fmac16_cols<k, 0, 4>(Rb, -lb, Rt, -lt);
+    });
+    // the second panel, rows 16..31 of columns 16..31, to every group
+    float Q[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c)
+        Q[c] = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (16 * (c & 3) + r), __float_as_int(Rb[c >> 2])));
+    unrolled<16>([&](auto kc) {
+        constexpr int k = kc;
+        const float inv = pivot_rcp<EXACT>(bcast16<k>(Q[k]));
+        const float l = r > k ? Q[k] * inv : 0.0f;
+        Q[k] = r > k ? l : Q[k];
+        fmac16_cols<k, k + 1, 16>(Q, -l);
+    });
+    // pivot of row lane % 32 (groups 0, 2: the first panel's, 1, 3: the second's)
+    float piv = 1.0f;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) piv = r == c ? ((g & 1) ? Q[c] : Pt[c]) : piv;
+    if (!EXACT) {
+        const float m = fabsf(piv);
+        if (__any(!(m >= 0x1p-100f && m <= 0x1p100f))) return piv;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) B[(16 + 4 * u + g) * kLuS + r] = Rt[u];
+#pragma unroll
+    for (int c = 0; c < 16; ++c)
+        if (g == c >> 2) {
+            B[c * kLuS + r] = Pt[c];
+            B[c * kLuS + 16 + r] = Pb[c];
+            B[(16 + c) * kLuS + 16 + r] = Q[c];
+        }
+    return piv;
+}
+
+// returns 1 + the first zero or non-finite pivot, or 0
+__device__ __forceinline__ int lu32(float *S, int c0, int lane)
+{
+    float piv = lu32_run<false>(S, c0, lane);
+    const float m = fabsf(piv);
+    if (__any(!(m >= 0x1p-100f && m <= 0x1p100f))) piv = lu32_run<true>(S, c0, lane);
+    const uint32_t z = static_cast<uint32_t>(__ballot(!(piv != 0.0f && isfinite(piv))));
+    return __ffs(z);
+}
+
+// Inverse of the unit-lower (UP = false) or upper triangle of the 32 x 32
+// block at (c0, c0) of S by Gauss-Jordan, one wave: the triangle's rows are in
+// every group, the inverse's columns 4 u + g in group g.  U = D V with V unit
+// upper, so Uinv = Vinv D^-1.  To M (row-major, stride 33, when given) and V.
+template <bool UP>
+__device__ __forceinline__ void invert32(const float *S, float *V, int c0, int lane, float *M)
+{
+    const int r = lane & 15, g = lane >> 4;
+    const float *B = S + c0 * kLuS + c0;
+    float Tt[32], Tb[32];   // rows r and 16 + r of the triangle, negated
+#pragma unroll
+    for (int c = 0; c < 32; ++c) {
+        if (UP || c < 16) Tt[c] = -B[c * kLuS + r];
+        if (!UP || c >= 16) Tb[c] = -B[c * kLuS + 16 + r];
+    }
+    float Xt[8], Xb[8];     // columns 4 u + g
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        Xt[u] = 4 * u + g == r ? 1.0f : 0.0f;
+        Xb[u] = 4 * u + g == 16 + r ? 1.0f : 0.0f;
+    }
+    if constexpr (!UP) {
+        unrolled<16>([&](auto cc) {
+            constexpr int c = cc;
+            fmac16_cols<c, 0, c / 4 + 1>(Xb, Tb[c], Xt, r > c ? Tt[c] : 0.0f);
+        });
+        unrolled<16>([&](auto cc) {
+            constexpr int c = cc;
+            fmac16_cols<c, 0, 4 + c / 4 + 1>(Xb, r > c ? Tb[16 + c] : 0.0f);
+        });
+    } else {
+        float dt = -1.0f, db = -1.0f;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            dt = r == c ? Tt[c] : dt;
+            db = r == c ? Tb[16 + c] : db;
+        }
+        dt = -1.0f / dt;
+        db = -1.0f / db;
+        unrolled<16>([&](auto cc) {
+            constexpr int c = 15 - cc;
+            fmac16_cols<c, 4 + c / 4, 8>(Xt, Tt[16 + c] * dt, Xb, r < c ? Tb[16 + c] * db : 0.0f);
+        });
+        unrolled<16>([&](auto cc) {
+            constexpr int c = 15 - cc;
+            fmac16_cols<c, c / 4, 8>(Xt, r < c ? Tt[c] * dt : 0.0f);
+        });
+        // column j times 1 / d_j
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int src = 4 * ((4 * u + g) & 15);
+            const float d = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(u < 4 ? dt : db)));
+            Xt[u] *= d;
+            Xb[u] *= d;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int j = 4 * u + g;
+        if (M != nullptr) {
+            M[r * 33 + j] = Xt[u];
+            M[(16 + r) * 33 + j] = Xb[u];
+        }
+        if (UP ? r <= j : r > j) V[(c0 + j) * kLuS + c0 + r] = Xt[u];
+        if (UP ? 16 + r <= j : 16 + r > j) V[(c0 + j) * kLuS + c0 + 16 + r] = Xb[u];
+    }
+}
+
+// Row q of Linv and column q of Uinv of the sub-block, 32 x 32 block by block:
+//   Linv(q, b) = -Linv(q, q) T,   T  = sum_{b <= K < q} L(q, K) Linv(K, b)
+//   Uinv(b, q) = -T' Uinv(q, q),  T' = sum_{b <= K < q} Uinv(b, K) U(K, q)
+// T needs only what was final before step q, so it is formed while one wave
+// factors the 32 x 32 block q; it stays in the wave's accumulators, whose rows
+// set the order of the second product's K (acc_row).  The U side works on
+// transposes so that T' is a right operand too.
+template <bool UP>
+__device__ __forceinline__ floatx16g_t inverse_row_product(const float *S, const float *V, int q, int b, int lane)
+{
+    const int l32 = lane & 31, lh = lane >> 5;
+    floatx16g_t acc = zero16();
+    for (int K = b; K < q; ++K) {
+        float av[16], bv[16];
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk) {
+            const int k = 2 * kk + lh;
+            av[kk] = UP ? S[(32 * q + l32) * kLuS + 32 * K + k] : S[(32 * K + k) * kLuS + 32 * q + l32];
+            bv[kk] = UP ? V[(32 * K + k) * kLuS + 32 * b + l32] : V[(32 * b + l32) * kLuS + 32 * K + k];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (K == b)   // the triangle's own block
+#pragma unroll
+            for (int kk = 0; kk < 16; ++kk) {
+                const int k = 2 * kk + lh;
+                bv[kk] = UP ? upper_entry(bv[kk], l32, k) : lower_entry(bv[kk], k, l32);
+            }
+        acc = mfma16(av, bv, acc);
+    }
+    return acc;
+}
+
+template <bool UP>
+__device__ __forceinline__ void inverse_row_finish(float *V, int q, int b, int lane, const floatx16g_t &T)
+{
+    const int l32 = lane & 31, lh = lane >> 5;
+    float av[16], bv[16];
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk) {
+        const int k = acc_row(kk, lh);
+        av[kk] = UP ? V[(32 * q + l32) * kLuS + 32 * q + k] : V[(32 * q + k) * kLuS + 32 * q + l32];
+        bv[kk] = T[kk];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk) {
+        const int k = acc_row(kk, lh);
+        av[kk] = UP ? upper_entry(av[kk], k, l32) : lower_entry(av[kk], l32, k);
+    }
+    const floatx16g_t acc = mfma16(av, bv, zero16());
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        if (UP)
+            V[(32 * q + acc_row(e, lh)) * kLuS + 32 * b + l32] = -acc[e];
+        else
+            V[(32 * b + l32) * kLuS + 32 * q + acc_row(e, lh)] = -acc[e];
+    }
+}
+
+// One wave: block t of row q of Linv (t <= q) or column q of Uinv (t - q - 1)
+// into the packed arrays, 16 consecutive floats per MFMA lane.  sides: 1
+// Linv, 2 Uinv, 3 both.
+__device__ __forceinline__ void write_inverse_row(const float *V, float *tri, int nb, int q0, int q, int t, int sides,
+                                                  int lane)
+{
+    const int l32 = lane & 31, lh = lane >> 5;
+    const bool up = t > q;
+    if (tri == nullptr || t >= 2 * (q + 1) || !(sides & (up ? 2 : 1))) return;
+    const int b = up ? t - q - 1 : t;
+    float v[16];
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk)
+        v[kk] = *(up ? &V[(32 * q + l32) * kLuS + 32 * b + 2 * kk + lh] : &V[(32 * b + 2 * kk + lh) * kLuS + 32 * q + l32]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (b == q)
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk)
+            v[kk] = up ? upper_entry(v[kk], 2 * kk + lh, l32) : lower_entry(v[kk], l32, 2 * kk + lh);
+    float4 *o = reinterpret_cast<float4 *>(up ? tri_block_u(tri, nb, q0 + b, q0 + q)
+                                              : tri_block_l(tri, nb, q0 + q, q0 + b)) + lane * 4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = float4{v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]};
+}
+
+// Sub-block k0 of the n x n block A.  FACTOR: the update with sub-block
+// k0 - 128 (when there is one), LU, inverses; workgroups 1.. update the rest
+// of the trailing matrix.  Without FACTOR: A is already factored and
+// workgroup q inverts the triangles of sub-block q.
+template <bool FACTOR>
+__global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, float *__restrict__ A, int64_t lda,
+                                                               float *__restrict__ tri, int sides,
+                                                               int *__restrict__ info)
+{
+    __shared__ LuLds sm;
+    float *S = sm.S, *V = sm.V;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, lh = lane >> 5;
+    const int nb = (n + 31) / 32;
+    if (!FACTOR) k0 = static_cast<int>(blockIdx.x) * kLuNB;
+    const int p0 = k0 - kLuNB;
+    float *Ak = A + static_cast<int64_t>(k0) * lda + k0;
+
+    if (FACTOR && blockIdx.x > 0) {
+        // ---- a 128 x 64 tile of the trailing matrix, one 32 x 32 block per wave ----
+        const int rest = n - k0, ct = (rest + 63) / 64;
+        // tiles in row-major order without the two of the diagonal sub-block
+        const int two = ct < 2 ? ct : 2;
+        const int t = static_cast<int>(blockIdx.x) - 1 + two;
+        const int r0 = (t / ct) * 128 + (wave & 3) * 32, c0 = (t % ct) * 64, cw = c0 + (wave >> 2) * 32;
+        // U12 (128 x 64) through LDS: its MFMA operand walks along columns
+        {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                const int c = (tid >> 7) + 4 * u, k = tid & 127;
+                v[u] = A[static_cast<int64_t>(k0 + min(c0 + c, rest - 1)) * lda + p0 + k];
+            }
+#pragma unroll
+            for (int u = 0; u < 16; ++u) S[((tid >> 7) + 4 * u) * kLuS + (tid & 127)] = v[u];
+        }
+        __syncthreads();
+        if (r0 >= rest || cw >= rest) return;
+        const float *lp = A + static_cast<int64_t>(p0 + lh) * lda + k0 + min(r0 + l32, rest - 1);
+        float cv[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            cv[e] = Ak[static_cast<int64_t>(min(cw + l32, rest - 1)) * lda + min(r0 + acc_row(e, lh), rest - 1)];
+        floatx16g_t acc = zero16();
+        float av[64];
+#pragma unroll
+        for (int kk = 0; kk < 64; ++kk) av[kk] = lp[static_cast<int64_t>(2 * kk) * lda];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            float bv[16];
+#pragma unroll
+            for (int kk = 0; kk < 16; ++kk) bv[kk] = S[(cw - c0 + l32) * kLuS + 32 * h + 2 * kk + lh];
+#pragma unroll
+            for (int kk = 0; kk < 16; ++kk)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[16 * h + kk], bv[kk], acc, 0, 0, 0);
+        }
+        if (cw + l32 < rest) {
+            float *cp = Ak + static_cast<int64_t>(cw + l32) * lda + r0;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int r = acc_row(e, lh);
+                if (r0 + r < rest) cp[r] = cv[e] - acc[e];
+            }
+        }
+        return;
+    }
+
+    // ---- the diagonal sub-block, padded to 128 with the identity ----
+    const int w = n - k0 < kLuNB ? n - k0 : kLuNB;
+    const int steps = (w + 31) / 32, q0 = k0 / 32;
+    const bool pre = FACTOR && k0 > 0;   // the update with the sub-block before: U12 of it goes to V
+    {
+        const int r = tid & 127;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            float v[16], u[16];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int c = (tid >> 7) + 4 * (16 * h + e);
+                v[e] = Ak[static_cast<int64_t>(min(c, w - 1)) * lda + min(r, w - 1)];
+                if (pre) u[e] = A[static_cast<int64_t>(k0 + min(c, w - 1)) * lda + p0 + r];
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int c = (tid >> 7) + 4 * (16 * h + e);
+                S[c * kLuS + r] = (r < w && c < w) ? v[e] : (r == c ? 1.0f : 0.0f);
+                if (pre) V[c * kLuS + r] = u[e];
+            }
+        }
+    }
+    __syncthreads();
+    if (!FACTOR) {
+        // waves 2 q, 2 q + 1 invert the triangles of 32-block q
+        if (wave & 1)
+            invert32<true>(S, V, 32 * (wave >> 1), lane, nullptr);
+        else
+            invert32<false>(S, V, 32 * (wave >> 1), lane, nullptr);
+        __syncthreads();
+        for (int q = 0; q < steps; ++q) {
+            if (wave < 2 * q) {
+                const int b = wave >> 1;
+                if (wave & 1)
+                    inverse_row_finish<true>(V, q, b, lane, inverse_row_product<true>(S, V, q, b, lane));
+                else
+                    inverse_row_finish<false>(V, q, b, lane, inverse_row_product<false>(S, V, q, b, lane));
+            }
+            __syncthreads();
+            write_inverse_row(V, tri, nb, q0, q, wave, sides, lane);
+        }
+        return;
+    }
+
+    // blocks (rb, cb .. cb + nc - 1) of S take L21 U12 of the sub-block before (K = 128)
+    auto pre_update = [&](int ln, int rb, int cb, int nc) {
+        const int l32 = ln & 31, lh = ln >> 5;
+        const float *lp = A + static_cast<int64_t>(p0 + lh) * lda + k0 + min(32 * rb + l32, w - 1);
+        float av[4][16];
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+#pragma unroll
+            for (int kk = 0; kk < 16; ++kk) av[h][kk] = lp[static_cast<int64_t>(32 * h + 2 * kk) * lda];
+        for (int y = 0; y < nc; ++y, ++cb) {
+            floatx16g_t acc = zero16();
+            float bv[2][16];
+            auto read = [&](int h) {
+#pragma unroll
+                for (int kk = 0; kk < 16; ++kk) bv[h & 1][kk] = V[(32 * cb + l32) * kLuS + 32 * h + 2 * kk + lh];
+            };
+            read(0);
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                if (h < 3) read(h + 1);
+                acc = mfma16(av[h], bv[h & 1], acc);
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int r = 32 * rb + acc_row(e, lh), c = 32 * cb + l32;
+                if (r < w && c < w) S[c * kLuS + r] -= acc[e];
+            }
+        }
+    };
+    // 32 x 32 block (r0, cc) of S takes the strips of the 32 columns at c0
+    auto update = [&](int ln, int c0, int r0, int cc) {
+        const int l32 = ln & 31, lh = ln >> 5;
+        floatx16g_t acc = zero16();
+        float av[16], bv[16];
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk) {
+            const int k = 2 * kk + lh;
+            av[kk] = S[(c0 + k) * kLuS + r0 + l32];
+            bv[kk] = S[(cc + l32) * kLuS + c0 + k];
+        }
+        acc = mfma16(av, bv, acc);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) S[(cc + l32) * kLuS + r0 + acc_row(e, lh)] -= acc[e];
+    };
+    int bad = 0;
+    for (int q = 0; q < steps; ++q) {
+        const int c0 = 32 * q, t = 7 - wave;   // t: this wave's block of the inverses' row q
+        // a lane number of the iteration's own: addresses and masks hoisted out
+        // of this loop fill the register file
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        floatx16g_t T = zero16();
+        // wave 0: the next diagonal block's update, then its LU; the other
+        // waves meanwhile update the rest, write out the inverses' row q - 1
+        // and form the products of row q
+        if (wave == 0) {
+            if (q > 0) {
+                update(ln, c0 - 32, c0, c0);
+                wave_lds_sync();
+            } else if (pre) {
+                pre_update(ln, 0, 0, 1);
+                wave_lds_sync();
+            }
+            const int z = lu32(S, c0, ln);
+            if (bad == 0 && z != 0) bad = k0 + c0 + z;
+        } else if (q > 0) {
+            const int R = steps - q;
+            for (int i = wave; i < R * R; i += kLuThreads / 64 - 1) update(ln, c0 - 32, c0 + 32 * (i % R), c0 + 32 * (i / R));
+            write_inverse_row(V, tri, nb, q0, q - 1, wave - 1, sides, ln);
+            if (tri != nullptr && t < 2 * q)
+                T = t & 1 ? inverse_row_product<true>(S, V, q, t >> 1, ln) : inverse_row_product<false>(S, V, q, t >> 1, ln);
+        } else if (pre) {
+            // row block wave % 4: columns 0, 1 or 2, 3; wave 4 also wave 0's second
+            const int cb = wave < 4 ? 0 : wave == 4 ? 1 : 2, ce = wave < 4 ? 2 : 4;
+            if ((wave & 3) < steps) pre_update(ln, wave & 3, cb, (ce < steps ? ce : steps) - cb);
+        }
+        __syncthreads();
+        if (wave == 0) {
+            invert32<false>(S, V, c0, ln, sm.Li);
+        } else if (wave == 1) {
+            invert32<true>(S, V, c0, ln, sm.Ui);
+        } else if (q + 1 == steps) {   // all of S is final: factors back to A
+#pragma unroll 4
+            for (int c = (wave - 2) >> 1; c < w; c += 3) {
+                const int r = 64 * (wave & 1) + ln;
+                if (r < w) Ak[static_cast<int64_t>(c) * lda + r] = S[c * kLuS + r];
+            }
+        }
+        __syncthreads();
+        // L21 := A21 U11^-1 and U12 := L11^-1 A12, one 32 x 32 block per wave
+        const int R = steps - 1 - q;
+        if (wave < 2 * R) {
+            const bool up = wave >= R;
+            const int o = c0 + 32 * (1 + (up ? wave - R : wave)), l32 = ln & 31, lh = ln >> 5;
+            float av[16], bv[16];
+            if (up) {
+#pragma unroll
+                for (int kk = 0; kk < 16; ++kk) {
+                    av[kk] = sm.Li[l32 * 33 + 2 * kk + lh];
+                    bv[kk] = S[(o + l32) * kLuS + c0 + 2 * kk + lh];
+                }
+            } else {
+#pragma unroll
+                for (int kk = 0; kk < 16; ++kk) {
+                    av[kk] = S[(c0 + 2 * kk + lh) * kLuS + o + l32];
+                    bv[kk] = sm.Ui[(2 * kk + lh) * 33 + l32];
+                }
+            }
+            floatx16g_t acc = zero16();
+            acc = mfma16(av, bv, acc);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int r = acc_row(e, lh);
+                if (up)
+                    S[(o + l32) * kLuS + c0 + r] = acc[e];
+                else
+                    S[(c0 + l32) * kLuS + o + r] = acc[e];
+            }
+        }
+        if (tri != nullptr && t < 2 * q) {
+            if (t & 1)
+                inverse_row_finish<true>(V, q, t >> 1, ln, T);
+            else
+                inverse_row_finish<false>(V, q, t >> 1, ln, T);
+        }
+        __syncthreads();
+    }
+    write_inverse_row(V, tri, nb, q0, steps - 1, wave, sides, lane);
+    if (tid == 0 && info != nullptr && (k0 == 0 || (bad != 0 && *info == 0))) *info = bad;
+}
+
+// L21 := A21 Uinv and U12 := Linv A12 for the rows and columns past the
+// sub-block at p0 (128 wide).  A workgroup owns 32 rows of L21 (blockIdx.x <
+// strips) or 32 columns of U12; wave j computes its 32-wide block j.
+__global__ __launch_bounds__(256) void lu_strip_kernel(int n, int p0, float *__restrict__ A, int64_t lda,
+                                                       const float *__restrict__ tri, int strips)
+{
+    __shared__ float X[kLuNB * 33];
+    const int tid = threadIdx.x, lane = tid & 63, J = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, lh = lane >> 5;
+    const int nb = (n + 31) / 32, q0 = p0 / 32, k1 = p0 + kLuNB;
+    const bool up = static_cast<int>(blockIdx.x) >= strips;
+    const int o = k1 + 32 * (static_cast<int>(blockIdx.x) - (up ? strips : 0));   // first row / column
+    const int cnt = n - o < 32 ? n - o : 32;
+    {
+        float v[16];
+        if (up) {
+            // X[k * 33 + c]: row p0 + k, column o + c
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+                v[u] = A[static_cast<int64_t>(o + min((tid >> 7) + 2 * u, cnt - 1)) * lda + p0 + (tid & 127)];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) X[(tid & 127) * 33 + (tid >> 7) + 2 * u] = v[u];
+        } else {
+            // X[k * 33 + r]: column p0 + k, row o + r
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+                v[u] = A[static_cast<int64_t>(p0 + (tid >> 5) + 8 * u) * lda + o + min(tid & 31, cnt - 1)];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) X[((tid >> 5) + 8 * u) * 33 + (tid & 31)] = v[u];
+        }
+    }
+    __syncthreads();
+    floatx16g_t acc = zero16();
+    for (int K = 0; K <= J; ++K) {
+        const float *blk = up ? tri_block_l(tri, nb, q0 + J, q0 + K) : tri_block_u(tri, nb, q0 + K, q0 + J);
+        const float4 *b4 = reinterpret_cast<const float4 *>(blk) + lane * 4;
+        const float4 t0 = b4[0], t1 = b4[1], t2 = b4[2], t3 = b4[3];
+        const float iv[16] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w,
+                              t2.x, t2.y, t2.z, t2.w, t3.x, t3.y, t3.z, t3.w};
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk) {
+            const float x = X[(32 * K + 2 * kk + lh) * 33 + l32];
+            acc = up ? __builtin_amdgcn_mfma_f32_32x32x2f32(iv[kk], x, acc, 0, 0, 0)
+                     : __builtin_amdgcn_mfma_f32_32x32x2f32(x, iv[kk], acc, 0, 0, 0);
+        }
+    }
+    if (up) {
+        if (l32 < cnt) {
+            float *cp = A + static_cast<int64_t>(o + l32) * lda + p0 + 32 * J;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) cp[acc_row(e, lh)] = acc[e];
+        }
+    } else {
+        float *cp = A + static_cast<int64_t>(p0 + 32 * J + l32) * lda + o;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            if (acc_row(e, lh) < cnt) cp[acc_row(e, lh)] = acc[e];
+    }
+}
+
+// Joins the inverses of the halves [I0, I0 + H) and [I0 + H, I1) (32-blocks)
+// of every pair.  blockIdx.x: a 32-column strip J; blockIdx.y + side0: 0 the
+// L side (J in the first half), 1 the U side (J in the second):
+//   T(I, J) = sum_K L(I, K) Linv(K, J),   Linv(I, J) = -sum_K Linv(I, K) T(K, J)
+//   T(I, J) = sum_K U(I, K) Uinv(K, J),   Uinv(I, J) = -sum_K Uinv(I, K) T(K, J)
+__global__ __launch_bounds__(kLuThreads) void tri_merge_kernel(int n, int H, const float *__restrict__ A, int64_t lda,
+                                                               float *__restrict__ tri, int side0)
+{
+    __shared__ float T[kMergeMax * 33];   // T[row * 33 + c], rows from the half's first
+    __shared__ float W[kMergeMax * 33];   // the strip of the L side's first factor, Linv(:, J)
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, lh = lane >> 5;
+    const int nb = (n + 31) / 32;
+    const bool up = static_cast<int>(blockIdx.y) + side0 != 0;
+    const int I0 = static_cast<int>(blockIdx.x) / H * 2 * H;
+    const int I1 = I0 + 2 * H < nb ? I0 + 2 * H : nb;
+    const int J = I0 + (up ? H : 0) + static_cast<int>(blockIdx.x) % H;
+    if (I0 + H >= I1 || J >= I1) return;
+    const int R0 = up ? I0 : I0 + H, R1 = up ? I0 + H : I1;   // output rows
+    if (!up) {
+        for (int K = J; K < I0 + H; ++K)
+            for (int e = tid; e < 1024; e += kLuThreads) {
+                const int ln = e >> 4, kk = e & 15;   // lane ln holds row ln % 32, column 2 kk + ln / 32
+                W[((K - I0) * 32 + (ln & 31)) * 33 + 2 * kk + (ln >> 5)] = tri_block_l(tri, nb, K, J)[e];
+            }
+        __syncthreads();
+    }
+    for (int I = R0 + wave; I < R1; I += kLuThreads / 64) {
+        floatx16g_t acc = zero16();
+        const int row = 32 * I + l32;
+        const int K0 = up ? I0 + H : J, K1 = up ? J + 1 : I0 + H;
+        for (int K = K0; K < K1; ++K) {
+            float av[16], bv[16];
+#pragma unroll
+            for (int kk = 0; kk < 16; ++kk) {
+                const int col = 32 * K + 2 * kk + lh;
+                const float v = A[static_cast<int64_t>(min(col, n - 1)) * lda + min(row, n - 1)];
+                av[kk] = (row < n && col < n) ? v : 0.0f;
+            }
+            if (up) {
+                const float4 *b4 = reinterpret_cast<const float4 *>(tri_block_u(tri, nb, K, J)) + lane * 4;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float4 q = b4[e];
+                    bv[4 * e] = q.x;
+                    bv[4 * e + 1] = q.y;
+                    bv[4 * e + 2] = q.z;
+                    bv[4 * e + 3] = q.w;
+                }
+            } else {
+#pragma unroll
+                for (int kk = 0; kk < 16; ++kk) bv[kk] = W[((K - I0) * 32 + 2 * kk + lh) * 33 + l32];
+            }
+            acc = mfma16(av, bv, acc);
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) T[((I - R0) * 32 + acc_row(e, lh)) * 33 + l32] = acc[e];
+    }
+    __syncthreads();
+    // rows with the most products first: I from the end (L) or from the start (U)
+    for (int p = wave; p < R1 - R0; p += kLuThreads / 64) {
+        const int I = up ? R0 + p : R1 - 1 - p;
+        floatx16g_t acc = zero16();
+        const int K0 = up ? I : R0, K1 = up ? R1 : I + 1;
+        for (int K = K0; K < K1; ++K) {
+            float av[16], bv[16];
+            if (up) {
+                // Uinv(I, K) as the left operand (row l32, k = 2 kk + lh) out of the right-operand order
+                const float *blk = tri_block_u(tri, nb, I, K) + 512 * (l32 & 1) + (l32 >> 1);
+#pragma unroll
+                for (int kk = 0; kk < 16; ++kk) av[kk] = blk[(2 * kk + lh) * 16];
+            } else {
+                const float4 *a4 = reinterpret_cast<const float4 *>(tri_block_l(tri, nb, I, K)) + lane * 4;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float4 q = a4[e];
+                    av[4 * e] = q.x;
+                    av[4 * e + 1] = q.y;
+                    av[4 * e + 2] = q.z;
+                    av[4 * e + 3] = q.w;
+                }
+            }
+#pragma unroll
+            for (int kk = 0; kk < 16; ++kk) bv[kk] = T[((K - R0) * 32 + 2 * kk + lh) * 33 + l32];
+            acc = mfma16(av, bv, acc);
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int rho = acc_row(e, lh);
+            if (up)
+                tri_block_u(tri, nb, I, J)[(l32 + 32 * (rho & 1)) * 16 + (rho >> 1)] = -acc[e];
+            else
+                tri_block_l(tri, nb, I, J)[(rho + 32 * (l32 & 1)) * 16 + (l32 >> 1)] = -acc[e];
+        }
+    }
+}
+
+int64_t tri_floats(int b)
+{
+    const int64_t nb = ceil_div(b, 32);
+    return 2 * nb * nb * 1024;
+}
+
+static int merge_inverses(int n, const float *A, int64_t lda, float *tri, int sides, hipStream_t s)
+{
+    const int nb = static_cast<int>(ceil_div(n, 32));
+    for (int H = kLuNB / 32; H < nb; H *= 2) {
+        const unsigned strips = static_cast<unsigned>(ceil_div(nb, 2 * H)) * H;
+        hipLaunchKernelGGL(tri_merge_kernel, dim3(strips, sides == 3 ? 2 : 1), dim3(kLuThreads), 0, s, n, H, A, lda,
+                           tri, sides == 2 ? 1 : 0);
+        HPLAI_HIP(hipGetLastError());
+    }
+    return HPLAI_OK;
+}
+
+// Without tri only the sub-blocks' own inverses are needed, and only past one
+// sub-block; they live in a stream-ordered temporary.
+int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, hipStream_t s)
+{
+    if (n <= 0) return HPLAI_OK;
+    float *tmp = nullptr;
+    if (tri == nullptr && n > kLuNB)
+        HPLAI_HIP(hipMallocAsync(reinterpret_cast<void **>(&tmp), sizeof(float) * tri_floats(n), s));
+    float *t = tri != nullptr ? tri : tmp;
+    auto body = [&]() -> int {
+        for (int k = 0; k < n; k += kLuNB) {
+            const int rest = n - k;
+            const int rt = (rest + 127) / 128, ct = (rest + 63) / 64;
+            const int tiles = k == 0 ? 0 : rt * ct - (ct < 2 ? ct : 2);
+            // the last sub-block's inverses serve only a caller who asked for them
+            hipLaunchKernelGGL((lu_update_kernel<true>), dim3(static_cast<unsigned>(1 + tiles)), dim3(kLuThreads), 0, s,
+                               n, k, A, lda, tri == nullptr && rest <= kLuNB ? nullptr : t, 3, info);
+            HPLAI_HIP(hipGetLastError());
+            if (rest > kLuNB) {
+                const int strips = (rest - kLuNB + 31) / 32;
+                hipLaunchKernelGGL(lu_strip_kernel, dim3(static_cast<unsigned>(2 * strips)), dim3(256), 0, s, n, k, A,
+                                   lda, t, strips);
+                HPLAI_HIP(hipGetLastError());
+            }
+        }
+        return tri != nullptr ? merge_inverses(n, A, lda, tri, 3, s) : HPLAI_OK;
+    };
+    const int rc = body();
+    if (tmp != nullptr) HPLAI_HIP(hipFreeAsync(tmp, s));
+    return rc;
+}
+
+int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, hipStream_t s)
+{
+    if (b <= 0) return HPLAI_OK;
+    hipLaunchKernelGGL((lu_update_kernel<false>), dim3(static_cast<unsigned>(ceil_div(b, kLuNB))), dim3(kLuThreads), 0,
+                       s, b, 0, const_cast<float *>(LU), lda, tri, sides, nullptr);
+    HPLAI_HIP(hipGetLastError());
+    return merge_inverses(b, LU, lda, tri, sides, s);
+}
+
+}  // namespace hplai

@@ -66,16 +66,17 @@ int launch_higham_norm(int64_t n, double alpha, double beta, double *ones, doubl
                        double *out, hipStream_t s);
 int launch_gen_rhs(int64_t n, uint64_t seed, int64_t i0, int64_t cnt, double *b, hipStream_t s);
 
-int launch_getrf(int n, float *A, int64_t lda, int *info, hipStream_t s);
-// Diagonal-block sub-inverses used by the strip TRSMs: for each 32 x 32
-// diagonal sub-block of a factored b x b block, Linv then Uinv (row-major).
-int64_t diag_inv_floats(int b);
-int launch_diag_inv(int b, const float *LU, int64_t lda, float *inv, hipStream_t s);
-// inv: the factored diagonal block's sub-inverses, or NULL (computed on the fly)
+// LU of an n x n block (n <= 1024) in place.  tri (may be NULL): receives the
+// full inverses of its triangles, packed (device_common.hpp), tri_floats(n).
+int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, hipStream_t s);
+int64_t tri_floats(int b);
+// the same inverses of a block that is already factored; sides: 1 L, 2 U, 3 both
+int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, hipStream_t s);
+// tri: the packed inverses of the factored diagonal block, or NULL (computed on the fly)
 int launch_trsm_l(int64_t m, int b, const float *U, int64_t ldu, float *L, int64_t ldl,
-                  float *amax, int tb, const float *inv, hipStream_t s);
+                  float *amax, int tb, const float *tri, hipStream_t s);
 int launch_trsm_u(int b, int64_t n, const float *Lkk, int64_t ldl, float *U, int64_t ldu,
-                  float *amax, int tb, const float *inv, hipStream_t s);
+                  float *amax, int tb, const float *tri, hipStream_t s);
 // amax: per-tile maxima of |src| (nullable for FMT_F16 → exponents 0).
 // packed: dst in the panel-packed layout (packed_off), rows a multiple of 256 from its base.
 int launch_quantize(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds,
@@ -113,7 +114,6 @@ int noalloc_setup(int device, void **out);
 // triangular solves with the FP32 factors of LU, FP64 vectors; nrhs columns
 // of x with stride ldx
 bool tri_inverse_ok(int b);
-int64_t tri_inverse_offset(int b);
 int launch_tri_trsv(bool upper, int b, const float *tri, const double *xin, double *xout, hipStream_t s);
 int launch_trsv_lower_inv(int64_t n, int bs, const float *LU, int64_t lda, double *x, const float *inv,
                           int64_t inv_stride, double *xsc, hipStream_t s);

@@ -232,8 +232,7 @@ static void launch_gemv(bool trans, int64_t m, int w, const float *P, int64_t ld
 }
 
 // The same block solves with the diagonal blocks applied through the inverses
-// the LU stored (tri_inv_kernel layout, one set per block at inv + q
-// inv_stride + tri_inverse_offset(bs)): x_q := Tinv_q r_q into the scratch
+// the LU stored (packed, one set per block at inv + q inv_stride): x_q := Tinv_q r_q into the scratch
 // segment xsc (bs doubles), then the update of the other rows from xsc, whose
 // workgroup 0 also moves x_q into x.  One right-hand side; n % bs == 0 and
 // tri_inverse_ok(bs).
@@ -241,9 +240,8 @@ int launch_trsv_lower_inv(int64_t n, int bs, const float *LU, int64_t lda, doubl
                           int64_t inv_stride, double *xsc, hipStream_t s)
 {
     HPLAI_CHECK(tri_inverse_ok(bs) && n % bs == 0, "trsv: no stored inverses for bs=%d", bs);
-    const int64_t off = tri_inverse_offset(bs);
     for (int64_t kb = 0; kb < n; kb += bs) {
-        int rc = launch_tri_trsv(false, bs, inv + (kb / bs) * inv_stride + off, x + kb, xsc, s);
+        int rc = launch_tri_trsv(false, bs, inv + (kb / bs) * inv_stride, x + kb, xsc, s);
         if (rc) return rc;
         const int64_t m = n - kb - bs;
         if (m > 0) {
@@ -260,9 +258,8 @@ int launch_trsv_upper_inv(int64_t n, int bs, const float *LU, int64_t lda, doubl
                           int64_t inv_stride, double *xsc, hipStream_t s)
 {
     HPLAI_CHECK(tri_inverse_ok(bs) && n % bs == 0, "trsv: no stored inverses for bs=%d", bs);
-    const int64_t off = tri_inverse_offset(bs);
     for (int64_t kb = n - bs; kb >= 0; kb -= bs) {
-        int rc = launch_tri_trsv(true, bs, inv + (kb / bs) * inv_stride + off, x + kb, xsc, s);
+        int rc = launch_tri_trsv(true, bs, inv + (kb / bs) * inv_stride, x + kb, xsc, s);
         if (rc) return rc;
         if (kb > 0) {
             launch_gemv(false, kb, bs, LU + kb * lda, lda, xsc, x, 0, 1, s, x + kb);

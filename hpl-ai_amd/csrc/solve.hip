@@ -48,7 +48,7 @@ struct Buffers {
     float *amaxL[2] = {nullptr, nullptr}, *amaxU[2] = {nullptr, nullptr};
     int *info = nullptr;
     double *chk = nullptr;
-    float *inv = nullptr;   // diagonal sub-block inverses, one set per diagonal block
+    float *inv = nullptr;   // packed inverses of the diagonal blocks' triangles, one set per block
     double *tsc = nullptr;  // one block of the IR's triangular solves (scratch)
     uint16_t *P = nullptr;  // FP16 trailing storage (n x n, leading dimension n)
     uint16_t *Q = nullptr;  // its back buffer (n x n), when on
@@ -305,7 +305,7 @@ struct LU {
     {
         return tiled() ? B->amaxU[buf] + t * ntiles + col / b : nullptr;
     }
-    const float *dinv(int64_t c) const { return B->inv + (c / b) * diag_inv_floats(b); }
+    float *dinv(int64_t c) const { return B->inv + (c / b) * tri_floats(b); }
 
     // cls: kTrailing, an outer step's update of blocks that have not joined a
     // panel yet (to the FP16 trailing storage when it is on); kBulk, the rows
@@ -414,12 +414,9 @@ struct LU {
             if (rc == HPLAI_OK) rc = lazy_init(c, c, rb0 - c, b, s);
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_DIAG_LU, 2.0 / 3.0 * bd * bd * bd, s, [&] {
-                    int r = launch_getrf(b, a(c, c), lda, B->info + c / b, s);
                     // the inverses also serve the IR's block solves, so the
                     // last diagonal block gets them too
-                    if (r == HPLAI_OK && b <= 512)
-                        r = launch_diag_inv(b, a(c, c), lda, const_cast<float *>(dinv(c)), s);
-                    return r;
+                    return launch_getrf(b, a(c, c), lda, B->info + c / b, dinv(c), s);
                 });
             if (rc) break;
             // bulk: L := A U^-1 and quantization of the rows below
@@ -428,7 +425,7 @@ struct LU {
                 HPLAI_HIP(hipStreamWaitEvent(q, ev_inv, 0));
                 rc = timed(HPLAI_PHASE_TRSM_L, static_cast<double>(mb) * bd * bd, q, [&] {
                     return launch_trsm_l(mb, b, a(c, c), lda, a(rb0, c), lda, aml(buf, t, rb0), b,
-                                         b <= 512 ? dinv(c) : nullptr, q);
+                                         dinv(c), q);
                 });
                 if (rc == HPLAI_OK)
                     rc = timed(HPLAI_PHASE_CONV_L, static_cast<double>(mb) * bd, q, [&] {
@@ -442,7 +439,7 @@ struct LU {
             if (mrow <= 0) continue;
             rc = timed(HPLAI_PHASE_TRSM_L, static_cast<double>(mrow) * bd * bd, s, [&] {
                 return launch_trsm_l(mrow, b, a(c, c), lda, a(c + b, c), lda, aml(buf, t, c + b), b,
-                                     b <= 512 ? dinv(c) : nullptr, s);
+                                     dinv(c), s);
             });
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_CONV_L, static_cast<double>(mrow) * bd, s, [&] {
@@ -457,7 +454,7 @@ struct LU {
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_TRSM_R, static_cast<double>(ncols) * bd * bd, s, [&] {
                     return launch_trsm_u(b, ncols, a(c, c), lda, a(c, c + b), lda, amu(buf, t, c + b), b,
-                                         b <= 512 ? dinv(c) : nullptr, s);
+                                         dinv(c), s);
                 });
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_CONV_R, static_cast<double>(ncols) * bd, s, [&] {
@@ -495,7 +492,7 @@ struct LU {
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_TRSM_R, static_cast<double>(ncols) * bd * bd, s, [&] {
                     return launch_trsm_u(b, ncols, a(c, c), lda, a(c, col0), lda, amu(buf, t, col0), b,
-                                         b <= 512 ? dinv(c) : nullptr, s);
+                                         dinv(c), s);
                 });
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_CONV_R, static_cast<double>(ncols) * bd, s, [&] {
@@ -628,7 +625,7 @@ int alloc_lu_buffers(const LU &lu, Buffers &B, hipStream_t s)
     const int64_t nt = lu.ntiles;
     int rc = alloc(reinterpret_cast<void **>(&B.info), sizeof(int) * nt, "hipMalloc info");
     if (rc == HPLAI_OK)
-        rc = alloc(reinterpret_cast<void **>(&B.inv), sizeof(float) * diag_inv_floats(lu.b) * nt, "hipMalloc inv");
+        rc = alloc(reinterpret_cast<void **>(&B.inv), sizeof(float) * tri_floats(lu.b) * nt, "hipMalloc inv");
     for (int i = 0; i < 2 && rc == HPLAI_OK; ++i) {
         const size_t qbytes = static_cast<size_t>(lu.n) * lu.ldq * lu.es;
         rc = alloc(&B.Lq[i], qbytes, "hipMalloc Lq");
@@ -932,7 +929,7 @@ int hplai_solve(hplai_ctx ctx, const hplai_params *p, hplai_result *res)
                 rc = lu.timed(HPLAI_PHASE_IR_TRSV, 2.0 * dn2, s, [&] {
                     // diagonal blocks through the inverses the LU stored, where it stored them
                     if (tri_inverse_ok(b)) {
-                        const int64_t st = diag_inv_floats(b);
+                        const int64_t st = tri_floats(b);
                         int r = launch_trsv_lower_inv(n, b, B.A, lu.lda, B.r, B.inv, st, B.tsc, s);
                         if (r == HPLAI_OK) r = launch_trsv_upper_inv(n, b, B.A, lu.lda, B.r, B.inv, st, B.tsc, s);
                         return r;

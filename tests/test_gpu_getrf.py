@@ -1,0 +1,109 @@
+"""Diagonal-block LU (128-column sub-blocks on several workgroups) and the
+panel TRSMs at the sizes where its tiling can go wrong: one row, the edges of
+the 32 x 32 steps and of the 128-column sub-blocks, orders that are no
+multiple of either, the largest, and a leading dimension that leaves the
+columns unaligned.  Against the oracle with the relative 2e-5 of the existing
+getrf and TRSM tests (FP32 with another order of the sums)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+SEED = 42
+
+
+def _dev(a):
+    import torch
+    return torch.from_numpy(a).cuda()
+
+
+def _factored(oracle, b, n):
+    D = oracle.gen_block(n, 0, 0, b, b, SEED)
+    ref = D.copy()
+    oracle.lib().orc_getrf_nopiv_f32(b, oracle._ptr(ref), b)
+    return D, ref
+
+
+@pytest.mark.parametrize("b", [1, 31, 33, 97, 127, 129, 160, 257, 384, 500, 513, 777, 1000])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_getrf_tiles(ctx, oracle, b, pad):
+    import torch
+    D, ref = _factored(oracle, b, 4 * b + 4)
+    buf = np.full((b, b + pad), 7.0, dtype=np.float32)      # buf[col, row]
+    buf[:, :b] = D
+    g = _dev(buf)
+    info = torch.full((1,), 5, dtype=torch.int32, device="cuda")
+    ctx.getrf(b, g, b + pad, info)
+    got = g.cpu().numpy()
+    assert int(info.cpu()[0]) == 0
+    assert np.all(got[:, b:] == 7.0)
+    assert np.max(np.abs(got[:, :b] - ref)) / np.max(np.abs(ref)) < 2e-5
+
+
+@pytest.mark.parametrize("b,z", [(96, 95), (300, 0), (300, 130), (512, 511), (1000, 900)])
+@pytest.mark.parametrize("bad", [0.0, np.inf])
+def test_getrf_first_bad_pivot_of_any_sub_block(ctx, b, z, bad):
+    import torch
+    A = np.eye(b, dtype=np.float32)
+    A[z, z] = bad
+    if z + 40 < b:
+        A[z + 40, z + 40] = 0.0                              # a later one is not reported
+    info = torch.zeros(1, dtype=torch.int32, device="cuda")
+    ctx.getrf(b, _dev(A), b, info)
+    assert int(info.cpu()[0]) == z + 1
+
+
+@pytest.mark.parametrize("scale", [2.0 ** 104, 2.0 ** -109])
+def test_getrf_pivots_past_the_fast_reciprocal(ctx, oracle, scale):
+    """A scaled by a power of two s: L stays, U scales with it.  Pivots are
+    about 2^7 s, so both s leave the range of the Newton reciprocal
+    (2^-100 .. 2^100), while every quantity formed on the way stays a normal
+    FP32 number: the smallest inverse entry about 2^-15 / s, the smallest
+    update term 2^-10 s.  The runs differ in how each pivot's reciprocal is
+    rounded, one FP32 ulp (1.2e-7) of every l and of the updates built on it:
+    2e-6 allows sixteen of them."""
+    b = 160
+    D, _ = _factored(oracle, b, 4 * b)
+    g, s = _dev(D), _dev((D * np.float32(scale)).astype(np.float32))
+    ctx.getrf(b, g, b)
+    ctx.getrf(b, s, b)
+    ref, got = g.cpu().numpy(), s.cpu().numpy()
+    lower = np.tril(np.ones((b, b), dtype=bool), -1).T       # [col, row] with row > col
+    want = np.where(lower, ref, ref * np.float32(scale))
+    assert np.max(np.abs(got - want)[lower]) / np.max(np.abs(want[lower])) < 2e-6
+    assert np.max(np.abs(got - want)[~lower]) / np.max(np.abs(want[~lower])) < 2e-6
+
+
+@pytest.mark.parametrize("b", [1, 33, 100, 257, 513, 777, 1000, 1024])
+@pytest.mark.parametrize("m", [1, 45])
+def test_trsm_tiles(ctx, oracle, b, m):
+    n = m + b
+    _, ref = _factored(oracle, b, n + 4)
+    L = oracle.gen_block(n + 4, b, 0, m, b, SEED)
+    U = oracle.gen_block(n + 4, 0, b, b, m, SEED)
+    gF, gL, gU = _dev(ref), _dev(L), _dev(U)
+    ctx.trsm_lpanel(m, b, gF, b, gL, m)
+    ctx.trsm_upanel(b, m, gF, b, gU, b)
+    oracle.lib().orc_trsm_runn_f32(m, b, oracle._ptr(ref), b, oracle._ptr(L), m)
+    oracle.lib().orc_trsm_llnu_f32(b, m, oracle._ptr(ref), b, oracle._ptr(U), b)
+    assert np.max(np.abs(gL.cpu().numpy() - L)) / np.max(np.abs(L)) < 2e-5
+    assert np.max(np.abs(gU.cpu().numpy() - U)) / np.max(np.abs(U)) < 2e-5
+
+
+def test_getrf_captured(ctx, oracle):
+    """Captured on the caller's stream and replayed, with eager work between."""
+    import torch
+    b = 320
+    D, _ = _factored(oracle, b, 4 * b)
+    src = _dev(D)
+    want = src.clone()
+    ctx.getrf(b, want, b)
+    buf = torch.empty_like(src)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        buf.copy_(src)
+        ctx.getrf(b, buf, b)
+    for _ in range(3):
+        buf.fill_(3.0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(buf, want)
