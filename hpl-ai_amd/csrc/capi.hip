@@ -164,21 +164,24 @@ int hplai_quantize(hplai_ctx ctx, int fmt, int side, int64_t m, int64_t k, int t
                 "quantize: bad shape/pointers");
     HPLAI_CHECK(lds >= (side == 0 ? m : k), "quantize: lds too small");
     if (m == 0 || k == 0) return HPLAI_OK;
-    float *amax = nullptr;
+    hipStream_t s = as_stream(stream);
     if (fmt != HPLAI_FMT_F16) {
         HPLAI_CHECK(exps != nullptr && tb > 0, "quantize: exps and tb required for tile formats");
+        if (tile_amax_splits(m, k, tb) == 1) {
+            const int rc = launch_tile_amax(fmt, side, m, k, tb, src, lds, nullptr, exps, s);
+            return rc ? rc : launch_quantize(fmt, side, m, k, tb, src, lds, dst, ldd, nullptr, exps, s);
+        }
+        float *amax = nullptr;
         const int64_t ntiles = ceil_div(m, tb);
-        hipStream_t s = as_stream(stream);
         HPLAI_HIP(hipMallocAsync(reinterpret_cast<void **>(&amax), sizeof(float) * ntiles, s));
         int rc = launch_fill_f32(amax, ntiles, 0.0f, s);
-        if (rc == HPLAI_OK) rc = launch_tile_amax(side, m, k, tb, src, lds, amax, s);
+        if (rc == HPLAI_OK) rc = launch_tile_amax(fmt, side, m, k, tb, src, lds, amax, exps, s);
         if (rc == HPLAI_OK)
             rc = launch_quantize(fmt, side, m, k, tb, src, lds, dst, ldd, amax, exps, s);
         HPLAI_HIP(hipFreeAsync(amax, s));
         return rc;
     }
-    return launch_quantize(fmt, side, m, k, tb > 0 ? tb : 1, src, lds, dst, ldd, nullptr, nullptr,
-                           as_stream(stream));
+    return launch_quantize(fmt, side, m, k, tb > 0 ? tb : 1, src, lds, dst, ldd, nullptr, nullptr, s);
 }
 
 int hplai_schur_update(hplai_ctx ctx, int fmt, int64_t m, int64_t n, int nslices, int kslice,

@@ -77,13 +77,17 @@ int launch_trsm_l(int64_t m, int b, const float *U, int64_t ldu, float *L, int64
                   float *amax, int tb, const float *tri, hipStream_t s);
 int launch_trsm_u(int b, int64_t n, const float *Lkk, int64_t ldl, float *U, int64_t ldu,
                   float *amax, int tb, const float *tri, hipStream_t s);
-// amax: per-tile maxima of |src| (nullable for FMT_F16 → exponents 0).
+// amax: per-tile maxima of |src|; NULL: the exponents are in exps (FMT_F16: 0).
 // packed: dst in the panel-packed layout (packed_off), rows a multiple of 256 from its base.
 int launch_quantize(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds,
                     void *dst, int64_t ldd, const float *amax, int32_t *exps, hipStream_t s,
                     bool packed = false);
-int launch_tile_amax(int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds,
-                     float *amax, hipStream_t s);
+// Exponents of a panel's tiles for launch_quantize without amax: written to
+// exps when one workgroup serves a tile (tile_amax_splits 1, amax NULL), else
+// the maxima to amax (zeroed by the caller).
+int tile_amax_splits(int64_t m, int64_t k, int tb);
+int launch_tile_amax(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds, float *amax,
+                     int32_t *exps, hipStream_t s);
 int launch_fill_f32(float *p, int64_t cnt, float v, hipStream_t s);
 // packed: Lq and Uq in the panel-packed layout (packed_off) from their bases.
 int launch_schur(int fmt, int64_t m, int64_t n, int nslices, int kslice, const void *Lq,
