@@ -58,15 +58,30 @@ __device__ __forceinline__ uint64_t lcg_jump(uint64_t x, uint64_t idx)
     return x;
 }
 
+// lcg_jump(x, base + t) for a wave-uniform base (scalar arithmetic) and a
+// lane's t < 2^BITS.
+template <int BITS>
+__device__ __forceinline__ uint64_t lcg_jump_lanes(uint64_t x, uint64_t base, uint32_t t)
+{
+    x = lcg_jump(x, base);
+#pragma unroll
+    for (int k = 0; k < BITS; ++k)
+        if ((t >> k) & 1) x = kLcg.p[k].a * x + kLcg.p[k].c;
+    return x;
+}
+
 // Initial state x1 = a*seed + c (RandStat::initialize, hpl_rand.hpp:38-43).
 __host__ __device__ inline uint64_t lcg_init(uint64_t seed) { return kLcgA * seed + kLcgC; }
 
 // Value map (hpl_rand.hpp:50-52): (int64)x * 0x1.fffffffffffffP-65 in [-0.5, 0.5).
-// int64 -> double is correctly rounded (one rounding in the final add of the
-// hi/lo split) and the product is an IEEE multiply.
+// int64 -> double is correctly rounded (the halves convert exactly; one
+// rounding in the multiply-add that joins them) and the product is an IEEE
+// multiply.
 __device__ __forceinline__ double lcg_value(uint64_t s)
 {
-    return __dmul_rn(static_cast<double>(static_cast<int64_t>(s)), 0x1.fffffffffffffP-65);
+    const double v = fma(static_cast<double>(static_cast<int32_t>(s >> 32)), 0x1p32,
+                         static_cast<double>(static_cast<uint32_t>(s)));
+    return __dmul_rn(v, 0x1.fffffffffffffP-65);
 }
 
 // ---------------------------------------------------------------------------

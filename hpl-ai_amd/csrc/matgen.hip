@@ -5,6 +5,8 @@
 // steps from the seed, mapped to [-0.5, 0.5).  Rows are consecutive states,
 // columns jump by (a,c)^n.  The diagonal entry is sum_{j != i} |a_ij|,
 // accumulated in FP64 with j ascending, exactly as calc_diag does.
+#include <type_traits>
+
 #include "device_common.hpp"
 #include "internal.hpp"
 
@@ -52,44 +54,72 @@ __global__ __launch_bounds__(kGenRows) void gen_matrix_kernel(
     }
 }
 
-// calc_diag (hpl_rand.hpp:108-123): one thread per row; the FP64 sum runs
-// j = 0..n-1 in order.  Four interleaved LCG chains (stride 4 columns) break
-// the 64-bit multiply dependency; the additions stay strictly sequential.
-__global__ __launch_bounds__(256) void gen_diag_kernel(int64_t n, uint64_t x1, int64_t i0,
-                                                       int64_t cnt, LcgCoeff jn, LcgCoeff jn4,
-                                                       double *__restrict__ d)
+// calc_diag (hpl_rand.hpp:108-123): the FP64 sum of a row runs j = 0..n-1 in
+// order, so the additions of a row are one chain.  A workgroup takes 64 rows:
+// wave 0 adds, one row per lane, while the other seven waves generate the next
+// kDiagCols columns into LDS (generating costs about eight times the add).
+// With a thread per row doing both, a matrix of 10^4 rows gave the device 157
+// waves: 382 us at n = 10007, now 99 us; 2.48 -> 1.80 ms at n = 61440 (VALU
+// bound there, 75 clocks an element).
+constexpr int kDiagPer = 8;                  // columns per generating wave and chunk
+constexpr int kDiagCols = 7 * kDiagPer;
+
+__global__ __launch_bounds__(512) void gen_diag_kernel(int64_t n, uint64_t x1, int64_t i0, int64_t cnt, LcgCoeff jn,
+                                                       LcgCoeff jn2, LcgCoeff jchunk, double *__restrict__ d)
 {
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= cnt) return;
-    const int64_t i = i0 + t;
-    uint64_t s0 = lcg_jump(x1, static_cast<uint64_t>(i));
-    uint64_t s1 = jn.a * s0 + jn.c;
-    uint64_t s2 = jn.a * s1 + jn.c;
-    uint64_t s3 = jn.a * s2 + jn.c;
-    double sum = 0.0;
-    int64_t j = 0;
-    for (; j + 3 < n; j += 4) {
-        double v0 = fabs(lcg_value(s0));
-        double v1 = fabs(lcg_value(s1));
-        double v2 = fabs(lcg_value(s2));
-        double v3 = fabs(lcg_value(s3));
-        // adding +0.0 leaves a non-negative sum unchanged, so the skipped
-        // diagonal term costs no branch
-        sum = __dadd_rn(sum, j + 0 == i ? 0.0 : v0);
-        sum = __dadd_rn(sum, j + 1 == i ? 0.0 : v1);
-        sum = __dadd_rn(sum, j + 2 == i ? 0.0 : v2);
-        sum = __dadd_rn(sum, j + 3 == i ? 0.0 : v3);
-        s0 = jn4.a * s0 + jn4.c;
-        s1 = jn4.a * s1 + jn4.c;
-        s2 = jn4.a * s2 + jn4.c;
-        s3 = jn4.a * s3 + jn4.c;
+    __shared__ double buf[2][kDiagCols][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * 64 + lane;
+    const int64_t i = i0 + (t < cnt ? t : cnt - 1);
+    const int64_t chunks = (n + kDiagCols - 1) / kDiagCols;
+    if (wave == 0) {
+        double sum = 0.0;
+        for (int64_t p = 0; p < chunks; ++p) {
+            __syncthreads();
+            const double *col = &buf[p & 1][0][lane];
+#pragma unroll
+            for (int c0 = 0; c0 < kDiagCols; c0 += 14) {
+                double v[14];
+#pragma unroll
+                for (int c = 0; c < 14; ++c) v[c] = col[64 * (c0 + c)];
+#pragma unroll
+                for (int c = 0; c < 14; ++c) sum = __dadd_rn(sum, fabs(v[c]));
+            }
+        }
+        if (t < cnt) d[t] = sum;
+    } else {
+        int64_t j = (wave - 1) * kDiagPer;
+        const int64_t b0 = i0 + static_cast<int64_t>(blockIdx.x) * 64;   // the workgroup's first row
+        // states of columns j and j + 1
+        uint64_t s0 = lcg_jump_lanes<6>(x1, static_cast<uint64_t>(b0) + static_cast<uint64_t>(n) * static_cast<uint64_t>(j),
+                                        static_cast<uint32_t>(i - b0));
+        uint64_t s1 = jn.a * s0 + jn.c;
+        for (int64_t p = 0; p < chunks; ++p) {
+            double *col = &buf[p & 1][(wave - 1) * kDiagPer][lane];
+            // adding +0.0 leaves a non-negative sum unchanged: the diagonal
+            // and the columns past the last are stored as zeros
+            auto columns = [&](auto mask) {
+#pragma unroll
+                for (int c = 0; c < kDiagPer; c += 2) {
+                    double v0 = lcg_value(s0), v1 = lcg_value(s1);
+                    if (decltype(mask)::value && (j + c == i || j + c >= n)) v0 = 0.0;
+                    if (decltype(mask)::value && (j + c + 1 == i || j + c + 1 >= n)) v1 = 0.0;
+                    col[64 * c] = v0;
+                    col[64 * (c + 1)] = v1;
+                    s0 = jn2.a * s0 + jn2.c;
+                    s1 = jn2.a * s1 + jn2.c;
+                }
+            };
+            if (j + kDiagPer <= n && (j + kDiagPer <= b0 || j >= b0 + 64))
+                columns(std::false_type{});
+            else
+                columns(std::true_type{});
+            s0 = jchunk.a * s0 + jchunk.c;   // past the other waves' columns
+            s1 = jchunk.a * s1 + jchunk.c;
+            j += kDiagCols;
+            __syncthreads();
+        }
     }
-    for (; j < n; ++j) {
-        double v0 = fabs(lcg_value(s0));
-        sum = __dadd_rn(sum, j == i ? 0.0 : v0);
-        s0 = jn.a * s0 + jn.c;
-    }
-    d[t] = sum;
 }
 
 // pcolvgen (matgen.hpp:193-207): b_i = value of state 1 + i + n*n.
@@ -162,9 +192,11 @@ int launch_gen_diag(int64_t n, uint64_t seed, int64_t i0, int64_t cnt, double *d
 {
     if (cnt <= 0) return HPLAI_OK;
     const LcgCoeff jn = lcg_pow_host(static_cast<uint64_t>(n));
-    const LcgCoeff jn4 = lcg_mul(lcg_mul(jn, jn), lcg_mul(jn, jn));
-    hipLaunchKernelGGL(gen_diag_kernel, dim3(static_cast<unsigned>(ceil_div(cnt, 256))), dim3(256),
-                       0, s, n, lcg_init(seed), i0, cnt, jn, jn4, d);
+    const LcgCoeff jn2 = lcg_mul(jn, jn);
+    LcgCoeff jchunk{1, 0};
+    for (int c = 0; c < kDiagCols - kDiagPer; c += 2) jchunk = lcg_mul(jn2, jchunk);
+    hipLaunchKernelGGL(gen_diag_kernel, dim3(static_cast<unsigned>(ceil_div(cnt, 64))), dim3(512), 0, s, n,
+                       lcg_init(seed), i0, cnt, jn, jn2, jchunk, d);
     HPLAI_HIP(hipGetLastError());
     return HPLAI_OK;
 }
