@@ -2,6 +2,8 @@
 // residual GEMV (A regenerated from the LCG), the blocked triangular solves
 // with FP32 factors and FP64 vectors, norms, vector updates and the factor
 // checksum.
+#include <type_traits>
+
 #include "device_common.hpp"
 #include "internal.hpp"
 #include "trsv_block.hpp"
@@ -11,69 +13,78 @@ namespace hplai {
 // ---------------------------------------------------------------------------
 // otf_gemv (panel_gemv.hpp:57-83, otf_gemv.cpp:5-131).
 // Pass 1: partial[c][i] = sum_{j in chunk c, j != i} (double)(int64)state_ij * x_j
-// (raw integers, like otf_gemv_kernel; the 2^-64-style scale is applied once).
+// (raw integers, like otf_gemv_kernel; the 2^-64-style scale is applied once;
+// one 64-bit integer's halves are summed apart).
 // Pass 2: y_i += alpha * (scale * sum_c partial[c][i] + d_i x_i), chunks in order.
 // ---------------------------------------------------------------------------
 constexpr int kGemvRows = 256;
 constexpr int kGemvChunk = 2048;
 
-__global__ __launch_bounds__(kGemvRows) void otf_gemv_partial_kernel(
-    int64_t n, uint64_t x1, int64_t row_blocks, LcgCoeff jn, LcgCoeff jn2,
-    const double *__restrict__ x, double *__restrict__ partial)
+// Columns per workgroup: as many as leave the device about eight workgroups
+// per CU, since a workgroup pays for its jump into the stream, 64 at least.
+// (2048 for every n left n = 1134 five workgroups: 22 us.)  The partial sums
+// stay under 32 MiB up to n = 92160 either way.
+static int otf_gemv_chunk(int64_t n)
 {
-    __shared__ double xs[kGemvChunk];
-    const int64_t rb = blockIdx.x % row_blocks;
-    const int64_t cb = blockIdx.x / row_blocks;
-    const int64_t j0 = cb * kGemvChunk;
-    const int64_t j1 = j0 + kGemvChunk < n ? j0 + kGemvChunk : n;
-    {
-        double v[kGemvChunk / kGemvRows];   // all loads in flight together
-#pragma unroll
-        for (int u = 0; u < kGemvChunk / kGemvRows; ++u) v[u] = x[min(j0 + u * kGemvRows + threadIdx.x, j1 - 1)];
-#pragma unroll
-        for (int u = 0; u < kGemvChunk / kGemvRows; ++u) xs[u * kGemvRows + threadIdx.x] = v[u];
-    }
-    __syncthreads();
-    const int64_t i = rb * kGemvRows + threadIdx.x;
-    if (i >= n) return;
-    uint64_t s0 = lcg_jump(x1, static_cast<uint64_t>(i) + static_cast<uint64_t>(n) * static_cast<uint64_t>(j0));
+    int chunk = kGemvChunk;
+    while (chunk > 64 && ceil_div(n, kGemvRows) * ceil_div(n, chunk) < 2048) chunk /= 2;
+    return chunk;
+}
+
+// What bounds it: VALU issue.  An element is one 64-bit LCG step (a 32 x 32 ->
+// 64 multiply-add and two 32-bit multiplies), the conversion of its two halves
+// and an FMA for each half into a sum of its own (one more rounding step per
+// element than converting the 64-bit integer first, without its shift and add,
+// and no less exact: the high sum is scaled and joined once).  x is uniform
+// over the wave and read through the scalar cache.
+__global__ __launch_bounds__(kGemvRows) void otf_gemv_partial_kernel(
+    int64_t n, uint64_t x1, int chunk, int row_blocks, LcgCoeff jn, LcgCoeff jn2, const double *__restrict__ x,
+    double *__restrict__ partial)
+{
+    const int rb = static_cast<int>(blockIdx.x) % row_blocks;
+    const int cb = static_cast<int>(blockIdx.x) / row_blocks;
+    const int64_t r0 = static_cast<int64_t>(rb) * kGemvRows, j0 = static_cast<int64_t>(cb) * chunk;
+    const int len = static_cast<int>(j0 + chunk < n ? chunk : n - j0);
+    const int64_t i = r0 + threadIdx.x;
+    uint64_t s0 = lcg_jump_lanes<8>(x1, static_cast<uint64_t>(r0) + static_cast<uint64_t>(n) * static_cast<uint64_t>(j0),
+                                    threadIdx.x);
     uint64_t s1 = jn.a * s0 + jn.c;
-    double acc0 = 0.0, acc1 = 0.0;
-    const int64_t len = j1 - j0;
-    const int64_t idiag = i - j0;   // local column of the diagonal, if in this chunk
-    int64_t t = 0;
-    // pairs (t, t + 1) with no diagonal element up to te; the one pair that
-    // holds the diagonal (when it is in this chunk) is masked on its own
-    auto pairs = [&](int64_t te) {
-        for (; t + 1 < te; t += 2) {
-            const double a0 = static_cast<double>(static_cast<int64_t>(s0));
-            const double a1 = static_cast<double>(static_cast<int64_t>(s1));
-            acc0 = fma(a0, xs[t], acc0);
-            acc1 = fma(a1, xs[t + 1], acc1);
-            s0 = jn2.a * s0 + jn2.c;
-            s1 = jn2.a * s1 + jn2.c;
+    const double *xc = x + j0;
+    double h0 = 0.0, l0 = 0.0, h1 = 0.0, l1 = 0.0;
+    auto add = [](uint64_t s, double xv, double &h, double &l) {
+        h = fma(static_cast<double>(static_cast<int32_t>(s >> 32)), xv, h);
+        l = fma(static_cast<double>(static_cast<uint32_t>(s)), xv, l);
+    };
+    int t = 0;
+    const int idiag = static_cast<int>(i - j0);   // in [0, len) when the diagonal is in this chunk
+    // columns t .. te - 1 (te - t a multiple of 8 but for the last range); with
+    // MASK the diagonal element counts as zero
+    auto range = [&](auto mask, int te) {
+        constexpr bool MASK = decltype(mask)::value;
+        for (; t + 8 <= te; t += 8) {
+#pragma unroll
+            for (int u = 0; u < 8; u += 2) {
+                add(MASK && t + u == idiag ? 0 : s0, xc[t + u], h0, l0);
+                add(MASK && t + u + 1 == idiag ? 0 : s1, xc[t + u + 1], h1, l1);
+                s0 = jn2.a * s0 + jn2.c;
+                s1 = jn2.a * s1 + jn2.c;
+            }
+        }
+        for (; t < te; ++t) {
+            add(MASK && t == idiag ? 0 : s0, xc[t], h0, l0);
+            const uint64_t next = jn2.a * s0 + jn2.c;
+            s0 = s1;
+            s1 = next;
         }
     };
-    const int64_t pd = (idiag >= 0 && idiag < len) ? (idiag & ~static_cast<int64_t>(1)) : len;
-    pairs(pd);
-    if (t == pd && t + 1 < len) {
-        double a0 = static_cast<double>(static_cast<int64_t>(s0));
-        double a1 = static_cast<double>(static_cast<int64_t>(s1));
-        a0 = (t == idiag) ? 0.0 : a0;
-        a1 = (t + 1 == idiag) ? 0.0 : a1;
-        acc0 = fma(a0, xs[t], acc0);
-        acc1 = fma(a1, xs[t + 1], acc1);
-        s0 = jn2.a * s0 + jn2.c;
-        s1 = jn2.a * s1 + jn2.c;
-        t += 2;
+    // the row block's own columns, where the diagonal is
+    const int64_t d0 = r0 - j0, d1 = d0 + kGemvRows;
+    if (d1 > 0 && d0 < len) {
+        if (d0 > 0) range(std::false_type{}, static_cast<int>(d0));
+        range(std::true_type{}, static_cast<int>(d1 < len ? d1 : len));
     }
-    pairs(len);
-    if (t < len) {
-        double a0 = static_cast<double>(static_cast<int64_t>(s0));
-        a0 = (t == idiag) ? 0.0 : a0;
-        acc0 = fma(a0, xs[t], acc0);
-    }
-    partial[cb * n + i] = acc0 + acc1;
+    range(std::false_type{}, len);
+    if (i < n) partial[static_cast<int64_t>(cb) * n + i] = fma(h0 + h1, 0x1p32, l0 + l1);
 }
 
 __global__ void otf_gemv_reduce_kernel(int64_t n, int64_t nchunks, double alpha,
@@ -88,18 +99,19 @@ __global__ void otf_gemv_reduce_kernel(int64_t n, int64_t nchunks, double alpha,
     y[i] = fma(alpha, ax, y[i]);
 }
 
-int64_t otf_gemv_work_doubles(int64_t n) { return ceil_div(n, kGemvChunk) * n; }
+int64_t otf_gemv_work_doubles(int64_t n) { return ceil_div(n, otf_gemv_chunk(n)) * n; }
 
 int launch_otf_gemv(int64_t n, uint64_t seed, const double *d, double alpha, const double *x,
                     double *y, double *work, hipStream_t s)
 {
     if (n <= 0) return HPLAI_OK;
+    const int chunk = otf_gemv_chunk(n);
     const int64_t row_blocks = ceil_div(n, kGemvRows);
-    const int64_t nchunks = ceil_div(n, kGemvChunk);
+    const int64_t nchunks = ceil_div(n, chunk);
     const LcgCoeff jn = lcg_pow_host(static_cast<uint64_t>(n));
     const LcgCoeff jn2 = lcg_mul(jn, jn);
     hipLaunchKernelGGL(otf_gemv_partial_kernel, dim3(static_cast<unsigned>(row_blocks * nchunks)),
-                       dim3(kGemvRows), 0, s, n, lcg_init(seed), row_blocks, jn, jn2, x, work);
+                       dim3(kGemvRows), 0, s, n, lcg_init(seed), chunk, static_cast<int>(row_blocks), jn, jn2, x, work);
     HPLAI_HIP(hipGetLastError());
     hipLaunchKernelGGL(otf_gemv_reduce_kernel, dim3(static_cast<unsigned>(ceil_div(n, 256))),
                        dim3(256), 0, s, n, nchunks, alpha, d, x, work, y);
