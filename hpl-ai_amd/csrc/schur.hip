@@ -71,65 +71,53 @@ __device__ __forceinline__ void store_c_nt(float *p, const float4 &c)
     __builtin_nontemporal_store(v, reinterpret_cast<floatx4_t *>(p));
 }
 
-// C -= acc for JB accumulator blocks side by side (columns col0 + 32 j ..),
-// rows row0 .. row0 + 31.  acc[j][4 q + r] is row 8 q + 4 lgrp + r, column
-// lrow of block j.  With VEC_C every lane loads its 4 JB float4 first
-// (addresses outside C are redirected to C itself and the values dropped),
-// so the loads are in flight together; a row group cut by M (M % 4 != 0)
-// takes a scalar path.
-template <int JB, bool VEC_C>
-__device__ __forceinline__ void epilogue_block_row(float *__restrict__ C, int64_t ldc, int64_t M, int64_t N,
-                                                   int64_t row0, int64_t col0, int lrow, int lgrp,
-                                                   const floatx16_t (&acc)[JB])
+// C -= acc for a wave's 32 IB x 32 JB part of a tile at (row0, col0), any
+// edges and any alignment of C.  acc[i][j][4 q + r] is row 8 q + 4 lgrp + r,
+// column lrow of block (i, j).  The MFMA layout gives each lane 4 rows of one
+// column, so a direct access touches 32 columns with 32 bytes each; through
+// the LDS scratch T (32 columns x kEpiAnyS(IB) floats, private to the wave)
+// every instruction covers 64 consecutive rows of one column.  (A column-major
+// C with an odd leading dimension, 4001 x 3003 x 60: the kernel 89 -> 31 us.)
+constexpr int kEpiAnyS(int IB) { return 32 * IB + 1; }   // odd: both walks spread over the banks
+
+template <int IB, int JB>
+__device__ __forceinline__ void epilogue_any(float *__restrict__ C, int64_t ldc, int64_t M, int64_t N, int64_t row0,
+                                             int64_t col0, int lane, float *T, const floatx16_t (&acc)[IB][JB])
 {
-    if constexpr (VEC_C) {
-        float4 cv[JB][4];
+    constexpr int S = kEpiAnyS(IB);
+    const int lrow = lane & 31, lgrp = lane >> 5;
 #pragma unroll
-        for (int j = 0; j < JB; ++j)
+    for (int j = 0; j < JB; ++j) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int64_t gc = col0 + j * 32 + lrow, gr = row0 + 8 * q + 4 * lgrp;
-                const bool full = gc < N && gr + 3 < M;
-                cv[j][q] = load_c_nt(full ? C + gc * ldc + gr : C);
-            }
+        for (int i = 0; i < IB; ++i)
 #pragma unroll
-        for (int j = 0; j < JB; ++j)
+            for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int64_t gc = col0 + j * 32 + lrow, gr = row0 + 8 * q + 4 * lgrp;
-                if (gc < N && gr + 3 < M) {
-                    float4 c4 = cv[j][q];
-                    c4.x -= acc[j][4 * q + 0];
-                    c4.y -= acc[j][4 * q + 1];
-                    c4.z -= acc[j][4 * q + 2];
-                    c4.w -= acc[j][4 * q + 3];
-                    store_c_nt(C + gc * ldc + gr, c4);
-                } else if (gc < N) {
+                for (int r = 0; r < 4; ++r) T[lrow * S + i * 32 + 8 * q + 4 * lgrp + r] = acc[i][j][4 * q + r];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (gr + r < M) C[gc * ldc + gr + r] -= acc[j][4 * q + r];
+        for (int h = 0; h < IB / 2; ++h) {
+            const int64_t gr = row0 + 64 * h + lane;
+            float *cp = C + (col0 + j * 32) * ldc + gr;
+            const int64_t left = N - (col0 + j * 32);
+            const int nc = left < 32 ? static_cast<int>(left) : 32;   // may be negative: nothing to do
+            if (gr < M) {
+#pragma unroll
+                for (int c0 = 0; c0 < 32; c0 += 16) {
+                    float v[16];
+#pragma unroll
+                    for (int c = 0; c < 16; ++c)
+                        if (c0 + c < nc) v[c] = cp[(c0 + c) * ldc];
+#pragma unroll
+                    for (int c = 0; c < 16; ++c)
+                        if (c0 + c < nc) cp[(c0 + c) * ldc] = v[c] - T[(c0 + c) * S + 64 * h + lane];
                 }
-            }
-    } else {
-#pragma unroll
-        for (int j = 0; j < JB; ++j) {
-            const int64_t gc = col0 + j * 32 + lrow;
-            if (gc >= N) continue;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int64_t gr = row0 + 8 * q + 4 * lgrp;
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (gr + r < M) C[gc * ldc + gr + r] -= acc[j][4 * q + r];
             }
         }
     }
 }
 
-// The same for a block row inside C (whole tile, 16-byte aligned C): the
-// MFMA layout gives each lane 4 rows of one column, so a direct float4 access
-// touches 32 columns per instruction with 32 bytes each; transposed through
-// the LDS scratch T (32 JB columns x 36 floats, private to the wave), 8 lanes
+// The same for a block row inside C (whole tile, 16-byte aligned C) with
+// float4 accesses: transposed through the LDS scratch T (32 JB columns x 36 floats, private to the wave), 8 lanes
 // cover one column's 128 bytes and each instruction 8 whole columns.
 constexpr int kEpiTS = 36;   // LDS column stride in floats (16-byte aligned)
 
@@ -208,10 +196,10 @@ __device__ __forceinline__ void epilogue_block_row_lds_h(uint16_t *__restrict__ 
     }
 }
 
-// EPI: 0 = element-wise C access (unaligned C), 1 = float4 per accumulator
-// row block with ragged edges, 2 = whole tiles only (M, N multiples of the
-// tile), C transposed through LDS (epilogue_block_row_lds), 3 = as 2 with an
-// FP16 C scaled by cscale (epilogue_block_row_lds_h).
+// EPI: 0 = any C (epilogue_any), 2 = whole tiles only (M, N multiples of the
+// tile) of a 16-byte aligned C, transposed through LDS
+// (epilogue_block_row_lds), 3 = as 2 with an FP16 C scaled by cscale
+// (epilogue_block_row_lds_h).
 template <int FMT, int BM, int BN, int EPI, bool PACKED>
 __global__ __launch_bounds__(kThreads) void schur_kernel(
     int64_t M, int64_t N, int nslices, int kslice, const uint8_t *__restrict__ Lq, int64_t ldl_b,
@@ -415,10 +403,10 @@ __global__ __launch_bounds__(kThreads) void schur_kernel(
                                            acc[i]);
         }
     } else {
-#pragma unroll
-        for (int i = 0; i < IB; ++i)
-            epilogue_block_row<JB, EPI == 1>(C, ldc, M, N, m0 + wm * (BM / 2) + i * 32, n0 + wn * (BN / 2), lrow,
-                                             lgrp, acc[i]);
+        static_assert(4 * 32 * kEpiAnyS(IB) * 4 <= 2 * BM * kLdsRow, "epilogue scratch fits the A stages");
+        __syncthreads();   // every wave is done with the operand stages
+        epilogue_any<IB, JB>(C, ldc, M, N, m0 + wm * (BM / 2), n0 + wn * (BN / 2), lane,
+                             reinterpret_cast<float *>(&As[0][0]) + wave * 32 * kEpiAnyS(IB), acc);
     }
 }
 
@@ -443,9 +431,7 @@ constexpr int kDmaLoadsPerStage = 2 * kDmaTile * kDmaStageBytes / (kThreads * 16
 // updates take the 128 x 128 kernel)
 constexpr int kDmaMaxSlices = 2048;
 
-// EPI: 0 = element-wise C access (unaligned C), 1 = float4 per accumulator
-// row block with ragged edges, 2 = whole tiles only (M, N multiples of 256),
-// C transposed through LDS for coalesced access.
+// EPI as in schur_kernel.
 template <int FMT, int EPI, bool PACKED>
 __global__ __launch_bounds__(kThreads) void schur_dma_kernel(
     int64_t M, int64_t N, int nslices, int kslice, const uint8_t *__restrict__ Lq, int64_t ldl_b,
@@ -685,14 +671,13 @@ __global__ __launch_bounds__(kThreads) void schur_dma_kernel(
                                           acc[i]);
         }
     } else {
-        // one accumulator row block (16 float4 per lane) at a time with all its
-        // loads in flight together; ragged edges element by element
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            epilogue_block_row<4, EPI == 1>(C, ldc, M, N, m0 + wm * (BM / 2) + i * 32, n0 + wn * (BN / 2), lrow,
-                                            lgrp, acc[i]);
+        __syncthreads();   // every wave is done with the operand stages
+        epilogue_any<4, 4>(C, ldc, M, N, m0 + wm * (BM / 2), n0 + wn * (BN / 2), lane,
+                           reinterpret_cast<float *>(S) + wave * 32 * kEpiAnyS(4), acc);
     }
 }
+
+static bool aligned_c(const void *C, int64_t ldc) { return reinterpret_cast<uintptr_t>(C) % 16 == 0 && ldc % 4 == 0; }
 
 // c16: C is the FP16 trailing storage (whole tiles, 8-byte aligned), C := fp16(C - cscale * L U)
 template <int FMT, bool PACKED>
@@ -708,21 +693,16 @@ static int schur_dma_launch(int64_t m, int64_t n, int nslices, int kslice, const
                   (long long)tiles_n);
         return HPLAI_EINVAL;
     }
-    const bool vec = (reinterpret_cast<uintptr_t>(C) % 16 == 0) && (ldc % 4 == 0);
     const dim3 grid(static_cast<unsigned>(tiles_m * tiles_n));
     const uint8_t *L8 = static_cast<const uint8_t *>(Lq);
     const uint8_t *U8 = static_cast<const uint8_t *>(Uq);
-    const bool whole = vec && m % kDmaTile == 0 && n % kDmaTile == 0;
+    const bool whole = aligned_c(C, ldc) && m % kDmaTile == 0 && n % kDmaTile == 0;
     if (c16)
         hipLaunchKernelGGL((schur_dma_kernel<FMT, 3, PACKED>), grid, dim3(kThreads), 0, s, m, n, nslices, kslice,
                            L8, ldl * F::es, eL, ldel, U8, ldu * F::es, eU, ldeu, tb, C, ldc,
                            static_cast<int>(tiles_m), static_cast<int>(tiles_n), cscale);
     else if (whole)
         hipLaunchKernelGGL((schur_dma_kernel<FMT, 2, PACKED>), grid, dim3(kThreads), 0, s, m, n, nslices, kslice,
-                           L8, ldl * F::es, eL, ldel, U8, ldu * F::es, eU, ldeu, tb, C, ldc,
-                           static_cast<int>(tiles_m), static_cast<int>(tiles_n), 1.0f);
-    else if (vec)
-        hipLaunchKernelGGL((schur_dma_kernel<FMT, 1, PACKED>), grid, dim3(kThreads), 0, s, m, n, nslices, kslice,
                            L8, ldl * F::es, eL, ldel, U8, ldu * F::es, eU, ldeu, tb, C, ldc,
                            static_cast<int>(tiles_m), static_cast<int>(tiles_n), 1.0f);
     else
@@ -746,21 +726,16 @@ static int schur_launch(int64_t m, int64_t n, int nslices, int kslice, const voi
                   (long long)tiles_n);
         return HPLAI_EINVAL;
     }
-    const bool vec = (reinterpret_cast<uintptr_t>(C) % 16 == 0) && (ldc % 4 == 0);
     const dim3 grid(static_cast<unsigned>(tiles_m * tiles_n));
     const uint8_t *L8 = static_cast<const uint8_t *>(Lq);
     const uint8_t *U8 = static_cast<const uint8_t *>(Uq);
-    const bool whole = vec && m % BM == 0 && n % BN == 0;
+    const bool whole = aligned_c(C, ldc) && m % BM == 0 && n % BN == 0;
     if (c16)
         hipLaunchKernelGGL((schur_kernel<FMT, BM, BN, 3, PACKED>), grid, dim3(kThreads), 0, s, m, n, nslices,
                            kslice, L8, ldl * F::es, eL, ldel, U8, ldu * F::es, eU, ldeu, tb, C, ldc,
                            static_cast<int>(tiles_m), static_cast<int>(tiles_n), cscale);
     else if (whole)
         hipLaunchKernelGGL((schur_kernel<FMT, BM, BN, 2, PACKED>), grid, dim3(kThreads), 0, s, m, n, nslices,
-                           kslice, L8, ldl * F::es, eL, ldel, U8, ldu * F::es, eU, ldeu, tb, C, ldc,
-                           static_cast<int>(tiles_m), static_cast<int>(tiles_n), 1.0f);
-    else if (vec)
-        hipLaunchKernelGGL((schur_kernel<FMT, BM, BN, 1, PACKED>), grid, dim3(kThreads), 0, s, m, n, nslices,
                            kslice, L8, ldl * F::es, eL, ldel, U8, ldu * F::es, eU, ldeu, tb, C, ldc,
                            static_cast<int>(tiles_m), static_cast<int>(tiles_n), 1.0f);
     else
