@@ -674,7 +674,9 @@ int hplai_batch_create(hplai_ctx ctx, int count, const int32_t *n, const int32_t
     b->out.resize(count);
     int rc = HPLAI_OK;
     auto alloc = [&](void **p, size_t bytes) {
-        if (rc == HPLAI_OK && hipMalloc(p, bytes) != hipSuccess) rc = hip_fail(hipGetLastError(), "hplai_batch_create: hipMalloc");
+        if (rc != HPLAI_OK) return;
+        const hipError_t e = device_malloc(ctx->device, p, bytes);
+        if (e != hipSuccess) rc = hip_fail(e, "hplai_batch_create: hipMalloc");
     };
     alloc(reinterpret_cast<void **>(&b->d_sys), sizeof(BatchSys) * count);
     alloc(reinterpret_cast<void **>(&b->d_order), sizeof(int32_t) * count);

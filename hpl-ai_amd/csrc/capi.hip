@@ -67,6 +67,11 @@ int hplai_create(int device, hplai_ctx *out)
         return hip_fail(e, "hipGetDeviceProperties");
     }
     c->num_cu = prop.multiProcessorCount;
+    if (block_cache_open(device, prop.totalGlobalMem) != HPLAI_OK) {
+        delete c;
+        return HPLAI_EINVAL;
+    }
+    c->cache_open = true;
     e = hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->bulk, hipStreamNonBlocking);
     for (int i = 0; e == hipSuccess && i < 8; ++i)
@@ -90,6 +95,8 @@ int hplai_destroy(hplai_ctx ctx)
     if (ctx == nullptr) return HPLAI_OK;
     (void)hipSetDevice(ctx->device);
     hplai_release(ctx);
+    ctx->pool.clear(ctx->device);
+    if (ctx->cache_open) block_cache_close(ctx->device);
     for (int i = 0; i < 8; ++i)
         if (ctx->ev[i]) (void)hipEventDestroy(ctx->ev[i]);
     if (ctx->side) (void)hipStreamDestroy(ctx->side);
@@ -132,7 +139,10 @@ int hplai_getrf_nopiv_f32(hplai_ctx ctx, int n, float *A, int64_t lda, int *info
     CTX_CHECK(ctx);
     HPLAI_CHECK(n >= 0 && n <= 1024, "getrf_nopiv: n=%d outside [0,1024]", n);
     HPLAI_CHECK(A != nullptr && lda >= n, "getrf_nopiv: A NULL or lda < n");
-    return launch_getrf(n, A, lda, info_dev, nullptr, as_stream(stream));
+    hipStream_t s = as_stream(stream);
+    ScratchLease tri(ctx, s, sizeof(float) * getrf_scratch_floats(n));
+    if (tri.rc) return tri.rc;
+    return launch_getrf(n, A, lda, info_dev, tri.as<float>(), false, s);
 }
 
 int hplai_trsm_lpanel_f32(hplai_ctx ctx, int64_t m, int b, const float *Ukk, int64_t ldu, float *L,
@@ -141,7 +151,12 @@ int hplai_trsm_lpanel_f32(hplai_ctx ctx, int64_t m, int b, const float *Ukk, int
     CTX_CHECK(ctx);
     HPLAI_CHECK(m >= 0 && b >= 0 && b <= 1024, "trsm_lpanel: bad shape");
     HPLAI_CHECK(Ukk != nullptr && L != nullptr && ldu >= b && ldl >= m, "trsm_lpanel: bad pointers/ld");
-    return launch_trsm_l(m, b, Ukk, ldu, L, ldl, nullptr, 1, nullptr, as_stream(stream));
+    if (m == 0 || b == 0) return HPLAI_OK;
+    hipStream_t s = as_stream(stream);
+    ScratchLease tri(ctx, s, sizeof(float) * tri_floats(b));
+    if (tri.rc) return tri.rc;
+    const int rc = launch_tri_inverse(b, Ukk, ldu, tri.as<float>(), 2, s);
+    return rc ? rc : launch_trsm_l(m, b, tri.as<float>(), L, ldl, nullptr, 1, s);
 }
 
 int hplai_trsm_upanel_f32(hplai_ctx ctx, int b, int64_t n, const float *Lkk, int64_t ldl, float *U,
@@ -150,7 +165,12 @@ int hplai_trsm_upanel_f32(hplai_ctx ctx, int b, int64_t n, const float *Lkk, int
     CTX_CHECK(ctx);
     HPLAI_CHECK(n >= 0 && b >= 0 && b <= 1024, "trsm_upanel: bad shape");
     HPLAI_CHECK(Lkk != nullptr && U != nullptr && ldl >= b && ldu >= b, "trsm_upanel: bad pointers/ld");
-    return launch_trsm_u(b, n, Lkk, ldl, U, ldu, nullptr, 1, nullptr, as_stream(stream));
+    if (n == 0 || b == 0) return HPLAI_OK;
+    hipStream_t s = as_stream(stream);
+    ScratchLease tri(ctx, s, sizeof(float) * tri_floats(b));
+    if (tri.rc) return tri.rc;
+    const int rc = launch_tri_inverse(b, Lkk, ldl, tri.as<float>(), 1, s);
+    return rc ? rc : launch_trsm_u(b, n, tri.as<float>(), U, ldu, nullptr, 1, s);
 }
 
 int hplai_quantize(hplai_ctx ctx, int fmt, int side, int64_t m, int64_t k, int tb, const float *src,
@@ -171,14 +191,13 @@ int hplai_quantize(hplai_ctx ctx, int fmt, int side, int64_t m, int64_t k, int t
             const int rc = launch_tile_amax(fmt, side, m, k, tb, src, lds, nullptr, exps, s);
             return rc ? rc : launch_quantize(fmt, side, m, k, tb, src, lds, dst, ldd, nullptr, exps, s);
         }
-        float *amax = nullptr;
         const int64_t ntiles = ceil_div(m, tb);
-        HPLAI_HIP(hipMallocAsync(reinterpret_cast<void **>(&amax), sizeof(float) * ntiles, s));
-        int rc = launch_fill_f32(amax, ntiles, 0.0f, s);
-        if (rc == HPLAI_OK) rc = launch_tile_amax(fmt, side, m, k, tb, src, lds, amax, exps, s);
+        ScratchLease amax(ctx, s, sizeof(float) * ntiles);
+        if (amax.rc) return amax.rc;
+        int rc = launch_fill_f32(amax.as<float>(), ntiles, 0.0f, s);
+        if (rc == HPLAI_OK) rc = launch_tile_amax(fmt, side, m, k, tb, src, lds, amax.as<float>(), exps, s);
         if (rc == HPLAI_OK)
-            rc = launch_quantize(fmt, side, m, k, tb, src, lds, dst, ldd, amax, exps, s);
-        HPLAI_HIP(hipFreeAsync(amax, s));
+            rc = launch_quantize(fmt, side, m, k, tb, src, lds, dst, ldd, amax.as<float>(), exps, s);
         return rc;
     }
     return launch_quantize(fmt, side, m, k, tb > 0 ? tb : 1, src, lds, dst, ldd, nullptr, nullptr, s);
@@ -207,12 +226,9 @@ int hplai_gemmschur_f16(hplai_ctx ctx, int64_t n, int64_t m, int64_t k, const ui
     HPLAI_CHECK(lda >= n && ldb >= k && ldc >= n, "gemmschur: need lda >= n, ldb >= k, ldc >= n");
     HPLAI_CHECK(k <= (int64_t(1) << 24), "gemmschur: k=%lld too large", (long long)k);
     hipStream_t s = as_stream(stream);
-    void *scratch = nullptr;
-    HPLAI_HIP(hipMallocAsync(&scratch, static_cast<size_t>(gemmschur_scratch_bytes(n, m, k)), s));
-    const int rc = launch_gemmschur_f16(n, m, k, a, lda, b, ldb, c, ldc, static_cast<uint16_t *>(scratch),
-                                        ctx->num_cu, s);
-    HPLAI_HIP(hipFreeAsync(scratch, s));
-    return rc;
+    ScratchLease scratch(ctx, s, static_cast<size_t>(gemmschur_scratch_bytes(n, m, k)));
+    if (scratch.rc) return scratch.rc;
+    return launch_gemmschur_f16(n, m, k, a, lda, b, ldb, c, ldc, scratch.as<uint16_t>(), ctx->num_cu, s);
 }
 
 int hplai_schur_update_f16c(hplai_ctx ctx, int fmt, int64_t m, int64_t n, int nslices, int kslice,
@@ -233,11 +249,9 @@ int hplai_otf_gemv_f64(hplai_ctx ctx, int64_t n, uint64_t seed, const double *d,
     CTX_CHECK(ctx);
     HPLAI_CHECK(n > 0 && d != nullptr && x != nullptr && y != nullptr, "otf_gemv: bad args");
     hipStream_t s = as_stream(stream);
-    double *work = nullptr;
-    HPLAI_HIP(hipMallocAsync(reinterpret_cast<void **>(&work), sizeof(double) * otf_gemv_work_doubles(n), s));
-    int rc = launch_otf_gemv(n, seed, d, alpha, x, y, work, s);
-    HPLAI_HIP(hipFreeAsync(work, s));
-    return rc;
+    ScratchLease work(ctx, s, sizeof(double) * otf_gemv_work_doubles(n));
+    if (work.rc) return work.rc;
+    return launch_otf_gemv(n, seed, d, alpha, x, y, work.as<double>(), s);
 }
 
 int hplai_trsv_lower_f32(hplai_ctx ctx, int64_t n, int bs, const float *LU, int64_t lda, double *x,

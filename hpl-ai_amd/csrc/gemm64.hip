@@ -189,13 +189,8 @@ extern "C" int hplai_gemm_f64(hplai_ctx ctx, int transa, int transb, int64_t m, 
     }
     hipStream_t s = as_stream(stream);
     const int splits = gemm64_splits(m, n, k, ctx->num_cu);
-    double *W = nullptr;
-    if (splits > 1)
-        HPLAI_HIP(hipMallocAsync(reinterpret_cast<void **>(&W), sizeof(double) * splits * m * n, s));
-    const int rc = launch_gemm64(transa != 0, transb != 0, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, W, splits, s);
-    if (W != nullptr) {
-        const hipError_t e = hipFreeAsync(W, s);
-        if (rc == HPLAI_OK && e != hipSuccess) return hip_fail(e, "hipFreeAsync");
-    }
-    return rc;
+    ScratchLease w(ctx, s, splits > 1 ? sizeof(double) * splits * m * n : 0);
+    if (w.rc) return w.rc;
+    return launch_gemm64(transa != 0, transb != 0, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, w.as<double>(), splits,
+                         s);
 }

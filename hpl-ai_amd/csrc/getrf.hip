@@ -811,36 +811,27 @@ static int merge_inverses(int n, const float *A, int64_t lda, float *tri, int si
     return HPLAI_OK;
 }
 
-// Without tri only the sub-blocks' own inverses are needed, and only past one
-// sub-block; they live in a stream-ordered temporary.
-int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, hipStream_t s)
+int64_t getrf_scratch_floats(int n) { return n > kLuNB ? tri_floats(n) : 0; }
+
+int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, bool full, hipStream_t s)
 {
     if (n <= 0) return HPLAI_OK;
-    float *tmp = nullptr;
-    if (tri == nullptr && n > kLuNB)
-        HPLAI_HIP(hipMallocAsync(reinterpret_cast<void **>(&tmp), sizeof(float) * tri_floats(n), s));
-    float *t = tri != nullptr ? tri : tmp;
-    auto body = [&]() -> int {
-        for (int k = 0; k < n; k += kLuNB) {
-            const int rest = n - k;
-            const int rt = (rest + 127) / 128, ct = (rest + 63) / 64;
-            const int tiles = k == 0 ? 0 : rt * ct - (ct < 2 ? ct : 2);
-            // the last sub-block's inverses serve only a caller who asked for them
-            hipLaunchKernelGGL((lu_update_kernel<true>), dim3(static_cast<unsigned>(1 + tiles)), dim3(kLuThreads), 0, s,
-                               n, k, A, lda, tri == nullptr && rest <= kLuNB ? nullptr : t, 3, info);
+    for (int k = 0; k < n; k += kLuNB) {
+        const int rest = n - k;
+        const int rt = (rest + 127) / 128, ct = (rest + 63) / 64;
+        const int tiles = k == 0 ? 0 : rt * ct - (ct < 2 ? ct : 2);
+        // the last sub-block's inverses serve only a caller who asked for them
+        hipLaunchKernelGGL((lu_update_kernel<true>), dim3(static_cast<unsigned>(1 + tiles)), dim3(kLuThreads), 0, s,
+                           n, k, A, lda, !full && rest <= kLuNB ? nullptr : tri, 3, info);
+        HPLAI_HIP(hipGetLastError());
+        if (rest > kLuNB) {
+            const int strips = (rest - kLuNB + 31) / 32;
+            hipLaunchKernelGGL(lu_strip_kernel, dim3(static_cast<unsigned>(2 * strips)), dim3(256), 0, s, n, k, A,
+                               lda, tri, strips);
             HPLAI_HIP(hipGetLastError());
-            if (rest > kLuNB) {
-                const int strips = (rest - kLuNB + 31) / 32;
-                hipLaunchKernelGGL(lu_strip_kernel, dim3(static_cast<unsigned>(2 * strips)), dim3(256), 0, s, n, k, A,
-                                   lda, t, strips);
-                HPLAI_HIP(hipGetLastError());
-            }
         }
-        return tri != nullptr ? merge_inverses(n, A, lda, tri, 3, s) : HPLAI_OK;
-    };
-    const int rc = body();
-    if (tmp != nullptr) HPLAI_HIP(hipFreeAsync(tmp, s));
-    return rc;
+    }
+    return full ? merge_inverses(n, A, lda, tri, 3, s) : HPLAI_OK;
 }
 
 int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, hipStream_t s)

@@ -335,10 +335,8 @@ int hplai_higham_gemv_f64(hplai_ctx ctx, int64_t n, double alpha, double beta, d
     HPLAI_CHECK(ctx != nullptr, "higham_gemv: NULL context");
     HPLAI_HIP(hipSetDevice(ctx->device));
     HPLAI_CHECK(n > 0 && x != nullptr && y != nullptr, "higham_gemv: bad arguments");
-    double *work = nullptr;
     const hipStream_t s = as_stream(stream);
-    HPLAI_HIP(hipMallocAsync(reinterpret_cast<void **>(&work), sizeof(double) * higham_gemv_work_doubles(n), s));
-    int rc = launch_higham_gemv(n, alpha, beta, scale, x, y, work, s);
-    HPLAI_HIP(hipFreeAsync(work, s));
-    return rc;
+    ScratchLease work(ctx, s, sizeof(double) * higham_gemv_work_doubles(n));
+    if (work.rc) return work.rc;
+    return launch_higham_gemv(n, alpha, beta, scale, x, y, work.as<double>(), s);
 }

@@ -2,9 +2,30 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <mutex>
 #include <string>
 
 #include "../../include/hplai.h"
+
+namespace hplai {
+// temporaries of the asynchronous entry points, one buffer per stream (memory.hip)
+struct StreamScratch {
+    struct Entry {
+        hipStream_t stream;
+        void *p;
+        hipEvent_t done;   // end of the last use
+        size_t bytes;
+    };
+    static constexpr int kMax = 32;
+    std::mutex mu;
+    Entry entries[kMax];
+    int count = 0;
+    size_t total = 0;
+    void drop(int device, Entry *e);
+    void clear(int device);
+};
+}  // namespace hplai
 
 struct hplai_ctx_s {
     int device = 0;
@@ -16,6 +37,9 @@ struct hplai_ctx_s {
     float *A = nullptr;
     int64_t n = 0, lda = 0;
     double *x = nullptr;
+    size_t A_bytes = 0, x_bytes = 0;   // block_free's sizes of the two
+    bool cache_open = false;
+    hplai::StreamScratch pool;
     // device address of this device's scratch array (hplai_otf_gemv_f64_noalloc)
     void *scratch = nullptr;
 };
@@ -38,6 +62,36 @@ int hip_fail(hipError_t e, const char *what);
             return HPLAI_EINVAL;                                     \
         }                                                            \
     } while (0)
+
+// ---- device memory (memory.hip) ----
+int block_cache_open(int device, size_t device_bytes);
+void block_cache_close(int device);
+hipError_t device_malloc(int device, void **p, size_t bytes);
+hipError_t block_alloc(int device, void **p, size_t *bytes);
+void block_free(int device, void *p, size_t bytes);
+
+// `bytes` of scratch for one call's kernels on `stream`, from construction to
+// the end of the scope that enqueues them.
+class ScratchLease {
+public:
+    ScratchLease(hplai_ctx ctx, hipStream_t stream, size_t bytes);
+    ~ScratchLease();
+    ScratchLease(const ScratchLease &) = delete;
+    ScratchLease &operator=(const ScratchLease &) = delete;
+    template <typename T>
+    T *as() const
+    {
+        return static_cast<T *>(ptr);
+    }
+    void *ptr = nullptr;
+    int rc = HPLAI_OK;
+
+private:
+    hipStream_t stream_;
+    std::unique_lock<std::mutex> lock_;
+    hipEvent_t done_ = nullptr;
+    bool async_ = false;
+};
 
 inline hipStream_t as_stream(void *s) { return static_cast<hipStream_t>(s); }
 __host__ __device__ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -66,17 +120,17 @@ int launch_higham_norm(int64_t n, double alpha, double beta, double *ones, doubl
                        double *out, hipStream_t s);
 int launch_gen_rhs(int64_t n, uint64_t seed, int64_t i0, int64_t cnt, double *b, hipStream_t s);
 
-// LU of an n x n block (n <= 1024) in place.  tri (may be NULL): receives the
-// full inverses of its triangles, packed (device_common.hpp), tri_floats(n).
-int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, hipStream_t s);
+// LU of an n x n block (n <= 1024) in place.  tri: tri_floats(n), packed
+// (device_common.hpp): the full inverses of the triangles (FULL), or scratch
+// (may be NULL up to getrf_scratch_floats(n) == 0).
+int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, bool full, hipStream_t s);
+int64_t getrf_scratch_floats(int n);
 int64_t tri_floats(int b);
 // the same inverses of a block that is already factored; sides: 1 L, 2 U, 3 both
 int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, hipStream_t s);
-// tri: the packed inverses of the factored diagonal block, or NULL (computed on the fly)
-int launch_trsm_l(int64_t m, int b, const float *U, int64_t ldu, float *L, int64_t ldl,
-                  float *amax, int tb, const float *tri, hipStream_t s);
-int launch_trsm_u(int b, int64_t n, const float *Lkk, int64_t ldl, float *U, int64_t ldu,
-                  float *amax, int tb, const float *tri, hipStream_t s);
+// tri: the packed inverses of the factored diagonal block
+int launch_trsm_l(int64_t m, int b, const float *tri, float *L, int64_t ldl, float *amax, int tb, hipStream_t s);
+int launch_trsm_u(int b, int64_t n, const float *tri, float *U, int64_t ldu, float *amax, int tb, hipStream_t s);
 // amax: per-tile maxima of |src|; NULL: the exponents are in exps (FMT_F16: 0).
 // packed: dst in the panel-packed layout (packed_off), rows a multiple of 256 from its base.
 int launch_quantize(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds,
@@ -134,6 +188,7 @@ int launch_trsv_lower_t(int64_t n, int bs, const float *LU, int64_t lda, double 
 int launch_norm_inf(int64_t n, const double *x, double *out, hipStream_t s);
 int launch_vec_div(int64_t n, const double *num, const double *den, double *out, hipStream_t s);
 int launch_vec_add(int64_t n, const double *x, double *y, hipStream_t s);
-int launch_checksum(int64_t n, const float *LU, int64_t lda, double *out3, hipStream_t s);
+// cols: 3 n doubles of scratch
+int launch_checksum(int64_t n, const float *LU, int64_t lda, double *cols, double *out3, hipStream_t s);
 
 }  // namespace hplai

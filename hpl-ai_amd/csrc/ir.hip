@@ -466,15 +466,12 @@ __global__ __launch_bounds__(1024) void checksum_final_kernel(int64_t n, const d
     }
 }
 
-int launch_checksum(int64_t n, const float *LU, int64_t lda, double *out3, hipStream_t s)
+int launch_checksum(int64_t n, const float *LU, int64_t lda, double *cols, double *out3, hipStream_t s)
 {
-    double *cols = nullptr;
-    HPLAI_HIP(hipMallocAsync(reinterpret_cast<void **>(&cols), sizeof(double) * 3 * n, s));
     hipLaunchKernelGGL(checksum_col_kernel, dim3(static_cast<unsigned>(n)), dim3(256), 0, s, n, LU, lda,
                        cols);
     hipLaunchKernelGGL(checksum_final_kernel, dim3(1), dim3(1024), 0, s, n, cols, out3);
     HPLAI_HIP(hipGetLastError());
-    HPLAI_HIP(hipFreeAsync(cols, s));
     return HPLAI_OK;
 }
 

@@ -2,8 +2,10 @@
 // memory (code under HIP graph capture, tight serving loops, harnesses that
 // forbid hipMalloc).
 //
-// hplai_otf_gemv_f64 takes its n * ceil(n / 2048) FP64 partial sums from a
-// hipMallocAsync per call.  hplai_otf_gemv_f64_noalloc runs the same two
+// hplai_otf_gemv_f64 takes its FP64 partial sums (at most n * ceil(n / 2048)
+// past n = 92160, under 32 MiB below) from the context's scratch buffer of the
+// stream, which a first or a captured call allocates.
+// hplai_otf_gemv_f64_noalloc runs the same two
 // kernels (otf_gemv_partial_kernel, otf_gemv_reduce_kernel) with the partial
 // sums in `scratch`, a file-scope device array of kNoAllocScratchBytes that
 // every device the library runs on holds until the process ends.  The

@@ -40,7 +40,17 @@ using namespace hplai;
 
 namespace {
 
+// Every buffer comes from and goes back to the device's block cache.
 struct Buffers {
+    explicit Buffers(int dev) : device(dev) {}
+    int device;
+    struct Owned {
+        void *p;
+        size_t bytes;
+    };
+    Owned owned[40];   // one per member below and to spare
+    int count = 0;
+
     float *A = nullptr;
     double *d = nullptr, *rhs = nullptr, *x = nullptr, *r = nullptr, *work = nullptr, *norms = nullptr;
     void *Lq[2] = {nullptr, nullptr}, *Uq[2] = {nullptr, nullptr};
@@ -52,37 +62,33 @@ struct Buffers {
     double *tsc = nullptr;  // one block of the IR's triangular solves (scratch)
     uint16_t *P = nullptr;  // FP16 trailing storage (n x n, leading dimension n)
     uint16_t *Q = nullptr;  // its back buffer (n x n), when on
-};
 
-void free_buffers(Buffers &B, bool keep_factors)
-{
-    auto f = [](void *p) {
-        if (p) (void)hipFree(p);
-    };
-    if (!keep_factors) {
-        f(B.A);
-        f(B.x);
+    template <typename T>
+    int alloc(T *&p, size_t bytes, const char *what)
+    {
+        void *v = nullptr;
+        const hipError_t e = block_alloc(device, &v, &bytes);
+        if (e != hipSuccess) return hip_fail(e, what);
+        p = static_cast<T *>(v);
+        owned[count++] = Owned{v, bytes};
+        return HPLAI_OK;
     }
-    f(B.d);
-    f(B.rhs);
-    f(B.r);
-    f(B.tsc);
-    f(B.work);
-    f(B.norms);
-    f(B.info);
-    f(B.chk);
-    f(B.inv);
-    f(B.P);
-    f(B.Q);
-    for (int i = 0; i < 2; ++i) {
-        f(B.Lq[i]);
-        f(B.Uq[i]);
-        f(B.eL[i]);
-        f(B.eU[i]);
-        f(B.amaxL[i]);
-        f(B.amaxU[i]);
+    // the caller keeps p: returns its size
+    size_t keep(const void *p)
+    {
+        for (int k = 0; k < count; ++k)
+            if (owned[k].p == p) {
+                owned[k].p = nullptr;
+                return owned[k].bytes;
+            }
+        return 0;
     }
-}
+    ~Buffers()
+    {
+        (void)hipDeviceSynchronize();   // blocks are cached idle
+        for (int k = 0; k < count; ++k) block_free(device, owned[k].p, owned[k].bytes);
+    }
+};
 
 double now_s()
 {
@@ -416,7 +422,7 @@ struct LU {
                 rc = timed(HPLAI_PHASE_DIAG_LU, 2.0 / 3.0 * bd * bd * bd, s, [&] {
                     // the inverses also serve the IR's block solves, so the
                     // last diagonal block gets them too
-                    return launch_getrf(b, a(c, c), lda, B->info + c / b, dinv(c), s);
+                    return launch_getrf(b, a(c, c), lda, B->info + c / b, dinv(c), true, s);
                 });
             if (rc) break;
             // bulk: L := A U^-1 and quantization of the rows below
@@ -424,8 +430,7 @@ struct LU {
                 HPLAI_HIP(hipEventRecord(ev_inv, s));
                 HPLAI_HIP(hipStreamWaitEvent(q, ev_inv, 0));
                 rc = timed(HPLAI_PHASE_TRSM_L, static_cast<double>(mb) * bd * bd, q, [&] {
-                    return launch_trsm_l(mb, b, a(c, c), lda, a(rb0, c), lda, aml(buf, t, rb0), b,
-                                         dinv(c), q);
+                    return launch_trsm_l(mb, b, dinv(c), a(rb0, c), lda, aml(buf, t, rb0), b, q);
                 });
                 if (rc == HPLAI_OK)
                     rc = timed(HPLAI_PHASE_CONV_L, static_cast<double>(mb) * bd, q, [&] {
@@ -438,8 +443,7 @@ struct LU {
             const int64_t mrow = rb0 - c - b;
             if (mrow <= 0) continue;
             rc = timed(HPLAI_PHASE_TRSM_L, static_cast<double>(mrow) * bd * bd, s, [&] {
-                return launch_trsm_l(mrow, b, a(c, c), lda, a(c + b, c), lda, aml(buf, t, c + b), b,
-                                     dinv(c), s);
+                return launch_trsm_l(mrow, b, dinv(c), a(c + b, c), lda, aml(buf, t, c + b), b, s);
             });
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_CONV_L, static_cast<double>(mrow) * bd, s, [&] {
@@ -453,8 +457,7 @@ struct LU {
             if (rc == HPLAI_OK) rc = lazy_init(c, c + b, b, ncols, s);
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_TRSM_R, static_cast<double>(ncols) * bd * bd, s, [&] {
-                    return launch_trsm_u(b, ncols, a(c, c), lda, a(c, c + b), lda, amu(buf, t, c + b), b,
-                                         dinv(c), s);
+                    return launch_trsm_u(b, ncols, dinv(c), a(c, c + b), lda, amu(buf, t, c + b), b, s);
                 });
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_CONV_R, static_cast<double>(ncols) * bd, s, [&] {
@@ -491,8 +494,7 @@ struct LU {
             if (rc == HPLAI_OK) rc = lazy_init(c, col0, b, ncols, s);   // block row right of the outer panel
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_TRSM_R, static_cast<double>(ncols) * bd * bd, s, [&] {
-                    return launch_trsm_u(b, ncols, a(c, c), lda, a(c, col0), lda, amu(buf, t, col0), b,
-                                         dinv(c), s);
+                    return launch_trsm_u(b, ncols, dinv(c), a(c, col0), lda, amu(buf, t, col0), b, s);
                 });
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_CONV_R, static_cast<double>(ncols) * bd, s, [&] {
@@ -614,30 +616,27 @@ void init_lu(LU &lu, hplai_ctx ctx, int64_t n, int64_t lda, int b, int fmt, int 
 }
 
 // Allocates the LU's working buffers: quantized panel double buffers, tile
-// exponents and maxima, diagonal inverses, pivot flags.  On failure the
-// buffers allocated so far stay in B for free_buffers.
+// exponents and maxima, diagonal inverses, pivot flags.
 int alloc_lu_buffers(const LU &lu, Buffers &B, hipStream_t s)
 {
-    auto alloc = [](void **p, size_t bytes, const char *what) {
-        const hipError_t e = hipMalloc(p, bytes);
-        return e == hipSuccess ? HPLAI_OK : hip_fail(e, what);
-    };
     const int64_t nt = lu.ntiles;
-    int rc = alloc(reinterpret_cast<void **>(&B.info), sizeof(int) * nt, "hipMalloc info");
-    if (rc == HPLAI_OK)
-        rc = alloc(reinterpret_cast<void **>(&B.inv), sizeof(float) * tri_floats(lu.b) * nt, "hipMalloc inv");
+    int rc = B.alloc(B.info, sizeof(int) * nt, "hipMalloc info");
+    if (rc == HPLAI_OK) rc = B.alloc(B.inv, sizeof(float) * tri_floats(lu.b) * nt, "hipMalloc inv");
     for (int i = 0; i < 2 && rc == HPLAI_OK; ++i) {
         const size_t qbytes = static_cast<size_t>(lu.n) * lu.ldq * lu.es;
-        rc = alloc(&B.Lq[i], qbytes, "hipMalloc Lq");
-        if (rc == HPLAI_OK) rc = alloc(&B.Uq[i], qbytes, "hipMalloc Uq");
-        if (rc == HPLAI_OK && hipMemsetAsync(B.Lq[i], 0, qbytes, s) != hipSuccess) rc = HPLAI_EHIP;
-        if (rc == HPLAI_OK && hipMemsetAsync(B.Uq[i], 0, qbytes, s) != hipSuccess) rc = HPLAI_EHIP;
+        rc = B.alloc(B.Lq[i], qbytes, "hipMalloc Lq");
+        if (rc == HPLAI_OK) rc = B.alloc(B.Uq[i], qbytes, "hipMalloc Uq");
+        // the quantizers write b of a slice's kpad values, the updates read all
+        if (lu.kpad != lu.b) {
+            if (rc == HPLAI_OK && hipMemsetAsync(B.Lq[i], 0, qbytes, s) != hipSuccess) rc = HPLAI_EHIP;
+            if (rc == HPLAI_OK && hipMemsetAsync(B.Uq[i], 0, qbytes, s) != hipSuccess) rc = HPLAI_EHIP;
+        }
         if (rc == HPLAI_OK && lu.fmt != HPLAI_FMT_F16) {
             const size_t cnt = static_cast<size_t>(lu.outer) * nt;
-            rc = alloc(reinterpret_cast<void **>(&B.eL[i]), sizeof(int32_t) * cnt, "hipMalloc eL");
-            if (rc == HPLAI_OK) rc = alloc(reinterpret_cast<void **>(&B.eU[i]), sizeof(int32_t) * cnt, "hipMalloc eU");
-            if (rc == HPLAI_OK) rc = alloc(reinterpret_cast<void **>(&B.amaxL[i]), sizeof(float) * cnt, "hipMalloc amaxL");
-            if (rc == HPLAI_OK) rc = alloc(reinterpret_cast<void **>(&B.amaxU[i]), sizeof(float) * cnt, "hipMalloc amaxU");
+            rc = B.alloc(B.eL[i], sizeof(int32_t) * cnt, "hipMalloc eL");
+            if (rc == HPLAI_OK) rc = B.alloc(B.eU[i], sizeof(int32_t) * cnt, "hipMalloc eU");
+            if (rc == HPLAI_OK) rc = B.alloc(B.amaxL[i], sizeof(float) * cnt, "hipMalloc amaxL");
+            if (rc == HPLAI_OK) rc = B.alloc(B.amaxU[i], sizeof(float) * cnt, "hipMalloc amaxU");
         }
     }
     if (rc == HPLAI_OK && hipMemsetAsync(B.info, 0, sizeof(int) * nt, s) != hipSuccess) rc = HPLAI_EHIP;
@@ -682,16 +681,14 @@ int hplai_factor_f32(hplai_ctx ctx, int64_t n, int b, int fmt, int outer, int lo
     if (rc) return rc;
     HPLAI_HIP(hipSetDevice(ctx->device));
     LU lu;
-    Buffers B;
+    Buffers B(ctx->device);
     GemmTimer timer;
     init_lu(lu, ctx, n, lda, b, fmt, outer > 0 ? outer : 1, false, 0, &B, &timer);
-    B.A = A;   // the caller's matrix: not freed below
+    B.A = A;   // the caller's matrix
     rc = alloc_lu_buffers(lu, B, nullptr);
     if (rc == HPLAI_OK) rc = lu.run(lookahead);
     if (hipDeviceSynchronize() != hipSuccess && rc == HPLAI_OK) rc = hip_fail(hipGetLastError(), "hplai_factor_f32");
     if (rc == HPLAI_OK) rc = check_pivots(lu, B, "hplai_factor_f32");
-    B.A = nullptr;
-    free_buffers(B, false);
     return rc;
 }
 
@@ -721,8 +718,8 @@ int hplai_release(hplai_ctx ctx)
 {
     if (ctx == nullptr) return HPLAI_OK;
     (void)hipSetDevice(ctx->device);
-    if (ctx->A) (void)hipFree(ctx->A);
-    if (ctx->x) (void)hipFree(ctx->x);
+    block_free(ctx->device, ctx->A, ctx->A_bytes);
+    block_free(ctx->device, ctx->x, ctx->x_bytes);
     ctx->A = nullptr;
     ctx->x = nullptr;
     ctx->n = ctx->lda = 0;
@@ -778,7 +775,7 @@ int hplai_solve(hplai_ctx ctx, const hplai_params *p, hplai_result *res)
     hplai_release(ctx);
 
     LU lu;
-    Buffers B;
+    Buffers B(ctx->device);
     GemmTimer timer;
     timer.on = p->profile != 0;
     init_lu(lu, ctx, n, (n + 63) / 64 * 64, b, fmt, outer, p->lazy != 0, p->seed, &B, &timer);
@@ -822,36 +819,26 @@ int hplai_solve(hplai_ctx ctx, const hplai_params *p, hplai_result *res)
     lu.epochs = &epochs;
     hipStream_t s = nullptr;
 
-#define ALLOC(ptr, bytes)                                                             \
-    do {                                                                              \
-        hipError_t _e = hipMalloc(reinterpret_cast<void **>(&(ptr)), (bytes));        \
-        if (_e != hipSuccess) {                                                       \
-            rc = hip_fail(_e, "hplai_solve: hipMalloc " #ptr);                        \
-            free_buffers(B, false);                                                   \
-            return rc;                                                                \
-        }                                                                             \
-    } while (0)
-    ALLOC(B.A, sizeof(float) * lu.lda * n);
-    ALLOC(B.d, sizeof(double) * n);
-    ALLOC(B.rhs, sizeof(double) * n);
-    ALLOC(B.x, sizeof(double) * n);
-    ALLOC(B.r, sizeof(double) * n);
-    ALLOC(B.tsc, sizeof(double) * b);
-    ALLOC(B.work, sizeof(double) * std::max(otf_gemv_work_doubles(n), higham_gemv_work_doubles(n)));
-    ALLOC(B.norms, sizeof(double) * 4);
-    ALLOC(B.chk, sizeof(double) * 3);
-    if (lu.trail16) ALLOC(B.P, sizeof(uint16_t) * n * n);
-    if (lu.bback) ALLOC(B.Q, sizeof(uint16_t) * n * n);
-#undef ALLOC
-    rc = alloc_lu_buffers(lu, B, s);
-    if (rc) {
-        free_buffers(B, false);
-        return rc;
-    }
+    auto alloc = [&](auto &p, size_t bytes, const char *what) {
+        if (rc == HPLAI_OK) rc = B.alloc(p, bytes, what);
+    };
+    alloc(B.A, sizeof(float) * lu.lda * n, "hplai_solve: hipMalloc A");
+    alloc(B.d, sizeof(double) * n, "hplai_solve: hipMalloc d");
+    alloc(B.rhs, sizeof(double) * n, "hplai_solve: hipMalloc rhs");
+    alloc(B.x, sizeof(double) * n, "hplai_solve: hipMalloc x");
+    alloc(B.r, sizeof(double) * n, "hplai_solve: hipMalloc r");
+    alloc(B.tsc, sizeof(double) * b, "hplai_solve: hipMalloc tsc");
+    alloc(B.work, sizeof(double) * std::max(3 * n, std::max(otf_gemv_work_doubles(n), higham_gemv_work_doubles(n))),
+          "hplai_solve: hipMalloc work");
+    alloc(B.norms, sizeof(double) * 4, "hplai_solve: hipMalloc norms");
+    alloc(B.chk, sizeof(double) * 3, "hplai_solve: hipMalloc chk");
+    if (lu.trail16) alloc(B.P, sizeof(uint16_t) * n * n, "hplai_solve: hipMalloc P");
+    if (lu.bback) alloc(B.Q, sizeof(uint16_t) * n * n, "hplai_solve: hipMalloc Q");
+    if (rc == HPLAI_OK) rc = alloc_lu_buffers(lu, B, s);
+    if (rc) return rc;
 
     // Everything after the allocations runs in one body whose every exit
-    // (HPLAI_HIP returns from it) comes back here, so the buffers are freed
-    // on every error path.
+    // (HPLAI_HIP returns from it) comes back here.
     bool converged = false;
     int steps = 0;
     auto body = [&]() -> int {
@@ -960,7 +947,7 @@ int hplai_solve(hplai_ctx ctx, const hplai_params *p, hplai_result *res)
             res->harness = -1.0;
         }
         if (rc == HPLAI_OK) {
-            rc = launch_checksum(n, B.A, lu.lda, B.chk, s);
+            rc = launch_checksum(n, B.A, lu.lda, B.work, B.chk, s);
             if (rc == HPLAI_OK)
                 HPLAI_HIP(hipMemcpy(res->checksum, B.chk, sizeof(double) * 3, hipMemcpyDeviceToHost));
         }
@@ -968,14 +955,14 @@ int hplai_solve(hplai_ctx ctx, const hplai_params *p, hplai_result *res)
     };
     rc = body();
 
-    const bool keep = p->keep_factors != 0 && rc == HPLAI_OK;
-    if (keep) {
+    if (p->keep_factors != 0 && rc == HPLAI_OK) {
         ctx->A = B.A;
         ctx->x = B.x;
+        ctx->A_bytes = B.keep(B.A);
+        ctx->x_bytes = B.keep(B.x);
         ctx->n = n;
         ctx->lda = lu.lda;
     }
-    free_buffers(B, keep);
     if (rc == HPLAI_OK && !converged) {
         set_error("hplai_solve: harness >= 16 after %d IR steps", steps);
         rc = HPLAI_ENOCONV;

@@ -338,51 +338,32 @@ static int tri_variant(int b, const float *P, int64_t ld)
     return b > 512 ? 2 : (b % 64 == 0 && aligned16(P, ld)) ? 0 : 1;
 }
 
-// The inverse of the triangle when the caller did not bring it (sides as in launch_tri_inverse)
-template <typename F>
-static int with_inverse(int b, const float *LU, int64_t ld, const float *tri, int sides, hipStream_t s, F &&f)
-{
-    if (tri != nullptr) return f(tri);
-    float *tmp = nullptr;
-    HPLAI_HIP(hipMallocAsync(reinterpret_cast<void **>(&tmp), sizeof(float) * tri_floats(b), s));
-    int rc = launch_tri_inverse(b, LU, ld, tmp, sides, s);
-    if (rc == HPLAI_OK) rc = f(tmp);
-    HPLAI_HIP(hipFreeAsync(tmp, s));
-    return rc;
-}
-
-int launch_trsm_l(int64_t m, int b, const float *U, int64_t ldu, float *L, int64_t ldl, float *amax, int tb,
-                  const float *tri, hipStream_t s)
+int launch_trsm_l(int64_t m, int b, const float *tri, float *L, int64_t ldl, float *amax, int tb, hipStream_t s)
 {
     if (m <= 0 || b <= 0) return HPLAI_OK;
     HPLAI_CHECK(amax == nullptr || tb % kStrip == 0, "trsm: tile %d not a multiple of %d", tb, kStrip);
-    return with_inverse(b, U, ldu, tri, 2, s, [&](const float *t) {
-        const dim3 g(static_cast<unsigned>(ceil_div(m, kStrip))), th(kTriThreads);
-        switch (tri_variant(b, L, ldl)) {
-        case 0: hipLaunchKernelGGL((trsm_l_tri_kernel<512, true>), g, th, 0, s, m, b, t, L, ldl, amax, tb); break;
-        case 1: hipLaunchKernelGGL((trsm_l_tri_kernel<512, false>), g, th, 0, s, m, b, t, L, ldl, amax, tb); break;
-        default: hipLaunchKernelGGL((trsm_l_tri_kernel<1024, false>), g, th, 0, s, m, b, t, L, ldl, amax, tb); break;
-        }
-        HPLAI_HIP(hipGetLastError());
-        return static_cast<int>(HPLAI_OK);
-    });
+    const dim3 g(static_cast<unsigned>(ceil_div(m, kStrip))), th(kTriThreads);
+    switch (tri_variant(b, L, ldl)) {
+    case 0: hipLaunchKernelGGL((trsm_l_tri_kernel<512, true>), g, th, 0, s, m, b, tri, L, ldl, amax, tb); break;
+    case 1: hipLaunchKernelGGL((trsm_l_tri_kernel<512, false>), g, th, 0, s, m, b, tri, L, ldl, amax, tb); break;
+    default: hipLaunchKernelGGL((trsm_l_tri_kernel<1024, false>), g, th, 0, s, m, b, tri, L, ldl, amax, tb); break;
+    }
+    HPLAI_HIP(hipGetLastError());
+    return HPLAI_OK;
 }
 
-int launch_trsm_u(int b, int64_t n, const float *Lkk, int64_t ldl, float *U, int64_t ldu, float *amax, int tb,
-                  const float *tri, hipStream_t s)
+int launch_trsm_u(int b, int64_t n, const float *tri, float *U, int64_t ldu, float *amax, int tb, hipStream_t s)
 {
     if (n <= 0 || b <= 0) return HPLAI_OK;
     HPLAI_CHECK(amax == nullptr || tb % kStrip == 0, "trsm: tile %d not a multiple of %d", tb, kStrip);
-    return with_inverse(b, Lkk, ldl, tri, 1, s, [&](const float *t) {
-        const dim3 g(static_cast<unsigned>(ceil_div(n, kStrip))), th(kTriThreads);
-        switch (tri_variant(b, U, ldu)) {
-        case 0: hipLaunchKernelGGL((trsm_u_tri_kernel<512, true>), g, th, 0, s, b, n, t, U, ldu, amax, tb); break;
-        case 1: hipLaunchKernelGGL((trsm_u_tri_kernel<512, false>), g, th, 0, s, b, n, t, U, ldu, amax, tb); break;
-        default: hipLaunchKernelGGL((trsm_u_tri_kernel<1024, false>), g, th, 0, s, b, n, t, U, ldu, amax, tb); break;
-        }
-        HPLAI_HIP(hipGetLastError());
-        return static_cast<int>(HPLAI_OK);
-    });
+    const dim3 g(static_cast<unsigned>(ceil_div(n, kStrip))), th(kTriThreads);
+    switch (tri_variant(b, U, ldu)) {
+    case 0: hipLaunchKernelGGL((trsm_u_tri_kernel<512, true>), g, th, 0, s, b, n, tri, U, ldu, amax, tb); break;
+    case 1: hipLaunchKernelGGL((trsm_u_tri_kernel<512, false>), g, th, 0, s, b, n, tri, U, ldu, amax, tb); break;
+    default: hipLaunchKernelGGL((trsm_u_tri_kernel<1024, false>), g, th, 0, s, b, n, tri, U, ldu, amax, tb); break;
+    }
+    HPLAI_HIP(hipGetLastError());
+    return HPLAI_OK;
 }
 
 }  // namespace hplai

@@ -110,8 +110,9 @@ int hplai_schur_update(hplai_ctx ctx, int fmt, int64_t m, int64_t n, int nslices
  * panel_trf.hpp:182-207), B = the U panel of convert_right_panels (column j at
  * b + j*ldb, panel_trf.hpp:208-233), binary16 bits; FP32 accumulation, C FP32
  * (device).  Any k >= 0 (the reference's C1 has k = b = 60).  The operands are
- * staged K-contiguous in a stream-ordered scratch allocation (hipMallocAsync,
- * (n + m) * roundup(k, 64) * 2 bytes) freed on the same stream. */
+ * staged K-contiguous in scratch memory ((n + m) * roundup(k, 64) * 2 bytes):
+ * the context's buffer for the stream, or a stream-ordered allocation past
+ * 256 MiB and under capture. */
 int hplai_gemmschur_f16(hplai_ctx ctx, int64_t n, int64_t m, int64_t k, const uint16_t *a, int64_t lda,
                         const uint16_t *b, int64_t ldb, float *c, int64_t ldc, void *stream);
 /* Replaces the FP16-C overload gemmschur(fp16 a, fp16 b, fp16 c) (schur_updator.hpp:24-27,
@@ -361,7 +362,13 @@ int hplai_solution_factors(hplai_ctx ctx, float *lu_host, int64_t ldh);
  * reference counterpart (the reference's factors stay in its panels). */
 int hplai_solution_block(hplai_ctx ctx, int64_t i0, int64_t j0, int64_t m, int64_t k, float *host,
                          int64_t ldh);
-int hplai_release(hplai_ctx ctx);   /* free buffers kept by keep_factors */
+/* Drop the factors and the solution kept by keep_factors.  Their memory, like
+ * the other buffers of hplai_solve and hplai_factor_f32, goes to a cache from
+ * which the next solve on the device allocates: at most a sixth of the
+ * device's memory, shared by the process's contexts, given back when the last
+ * context on the device is destroyed and when an allocation of this library
+ * would fail. */
+int hplai_release(hplai_ctx ctx);
 
 #ifdef __cplusplus
 }

@@ -1,0 +1,104 @@
+"""Memory that outlives a call: one scratch buffer per stream and context, and
+the cache of the solve's buffers.  What is checked is what can go wrong:
+calls on two streams at once, a buffer that has to grow under work in flight,
+captured calls replayed beside eager ones, factors kept across a later
+factorization, the bound of what stays allocated."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+SEED = 42
+
+
+def _residual_case(ctx, n, seed):
+    import torch
+    d = torch.empty(n, dtype=torch.float64, device="cuda")
+    ctx.gen_diag(n, seed, 0, n, d)
+    x = torch.from_numpy(np.random.default_rng(seed).standard_normal(n)).cuda()
+    y = torch.zeros(n, dtype=torch.float64, device="cuda")
+    ctx.otf_gemv(n, seed, d, 1.0, x, y)
+    torch.cuda.synchronize()
+    return d, x, y
+
+
+def test_two_streams_do_not_share_scratch(ctx):
+    import torch
+    sizes = [(3000, 1), (2000, 2)]
+    cases = [(n, s) + _residual_case(ctx, n, s) for n, s in sizes]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    outs = [[], []]
+    for _ in range(20):
+        for k, (n, s, d, x, _) in enumerate(cases):
+            with torch.cuda.stream(streams[k]):
+                y = torch.zeros(n, dtype=torch.float64, device="cuda")
+                ctx.otf_gemv(n, s, d, 1.0, x, y)
+                outs[k].append(y)
+    torch.cuda.synchronize()
+    for k, case in enumerate(cases):
+        for y in outs[k]:
+            assert torch.equal(y, case[4])
+
+
+def test_scratch_grows_under_work_in_flight(ctx):
+    import torch
+    cases = [(n, 7) + _residual_case(ctx, n, 7) for n in (500, 3000, 9000, 20000)]
+    st = torch.cuda.Stream()
+    outs = []
+    with torch.cuda.stream(st):
+        for n, s, d, x, _ in cases:
+            y = torch.zeros(n, dtype=torch.float64, device="cuda")
+            ctx.otf_gemv(n, s, d, 1.0, x, y)
+            outs.append(y)
+    torch.cuda.synchronize()
+    for y, case in zip(outs, cases):
+        assert torch.equal(y, case[4])
+
+
+def test_captured_calls_have_scratch_of_their_own(ctx):
+    import torch
+    n = 3000
+    d, x, want = _residual_case(ctx, n, 3)
+    d2, x2, want2 = _residual_case(ctx, n, 4)
+    y, y2 = torch.empty_like(want), torch.empty_like(want)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y.zero_()
+        ctx.otf_gemv(n, 3, d, 1.0, x, y)
+    for _ in range(4):
+        y.fill_(9.0)
+        g.replay()
+        y2.zero_()
+        ctx.otf_gemv(n, 4, d2, 1.0, x2, y2)
+        torch.cuda.synchronize()
+        assert torch.equal(y, want) and torch.equal(y2, want2)
+
+
+def test_kept_factors_survive_a_factorization(ctx):
+    import torch
+    n, b = 2048, 512
+    ctx.solve(n, b, fmt="e4m3", keep_factors=True)
+    lu = ctx.solution_factors(n)
+    x = ctx.solution_x(n)
+    A = torch.from_numpy(np.random.default_rng(1).uniform(-0.5, 0.5, (n, n)).astype(np.float32)).cuda()
+    A.diagonal().fill_(n)
+    ctx.factor(n, b, A, n, fmt="e4m3")
+    assert np.array_equal(ctx.solution_factors(n), lu)
+    assert np.array_equal(ctx.solution_x(n), x)
+    ctx.release()
+    import hplai
+    with pytest.raises(hplai.HplaiError):
+        ctx.solution_x(n)
+
+
+def test_what_stays_allocated_is_bounded(ctx):
+    """A sixth of the device at most is kept between solves, whatever ran."""
+    import torch
+    torch.cuda.empty_cache()
+    total = torch.cuda.mem_get_info()[1]
+    for n, fmt in ((65536, "f16"), (98304, "e4m3"), (32768, "e4m3")):
+        free0 = torch.cuda.mem_get_info()[0]
+        r = ctx.solve(n, 512, fmt=fmt, outer=16)
+        assert r["converged"]
+        ctx.release()
+        assert torch.cuda.mem_get_info()[0] >= min(free0, total) - total // 6 - (1 << 30)
+    assert total - torch.cuda.mem_get_info()[0] <= total // 6 + (8 << 30)
