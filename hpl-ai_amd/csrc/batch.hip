@@ -30,7 +30,6 @@
 
 #include "device_common.hpp"
 #include "internal.hpp"
-#include "trsv_block.hpp"
 
 namespace hplai {
 
@@ -296,11 +295,42 @@ __device__ __noinline__ int batch_lu(int n, int lda, float *A, uint8_t *lds)
     return info;
 }
 
-// The triangular solve of trsv_block (trsv_block.hpp) for the nr <= 4
-// right-hand sides of a system at once (columns x + rr bs): every strip of
-// the triangle is loaded once for all of them, and each right-hand side
-// takes exactly trsv_block's operations in its order.  xs: 4 x 32 doubles
-// of LDS.
+__device__ __forceinline__ double readlane_f64(double v, int lane)
+{
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+    return __hiloint2double(hi, lo);
+}
+
+// strip loader: dst[k][c] = element (row t + 256 k, column col0 + c) of the
+// triangle, clamped in-bounds
+template <int RPT>
+__device__ __forceinline__ void trsv_load_strip(const float *__restrict__ M, int64_t lda, int bs,
+                                                int col0, int tid, float (&dst)[RPT][32])
+{
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+        const int r = min(tid + 256 * k, bs - 1);
+#pragma unroll
+        for (int c = 0; c < 32; ++c) {
+            const int64_t col = min(col0 + c, bs - 1);
+            dst[k][c] = M[col * lda + r];
+        }
+    }
+}
+
+// Solves T x = x in place for the bs x bs triangle T (lower or upper, unit or
+// not; bs <= 256 RPT) and the nr <= 4 right-hand sides of a system at once
+// (columns x + rr bs), the diagonal-block step of panel_trsvL / panel_trsvU
+// (panel_trsv.hpp:310-758).  Thread t owns rows t + 256 k and keeps their x in
+// registers.  The triangle is walked in 32-column strips, each loaded once for
+// all right-hand sides and, where registers allow, a strip ahead.  The 32 x 32
+// diagonal sub-block is solved by the half-wave that owns its rows: x_c is
+// broadcast with v_readlane and the other lanes subtract l_ic x_c; the strip's
+// final x goes through LDS to the threads owning the rows further on.
+// Non-unit diagonals are applied as a multiply by 1 / t_cc computed before the
+// dependent chain (one rounding different from a division).  xs: 4 x 32
+// doubles of LDS.
 template <int RPT, bool UPPER, bool UNIT>
 __device__ __noinline__ void batch_trsv_multi(int bs, int lda, const float *__restrict__ T,
                                               double *__restrict__ x, int nr, double *xs)
@@ -317,13 +347,13 @@ __device__ __noinline__ void batch_trsv_multi(int bs, int lda, const float *__re
     const int nsb = (bs + 31) / 32;
     constexpr bool PF = RPT <= 2;
     float cur[RPT][32], nxt[PF ? RPT : 1][32];
-    trsv_load_strip<RPT, false>(T, lda, bs, (UPPER ? nsb - 1 : 0) * 32, tid, cur);
+    trsv_load_strip<RPT>(T, lda, bs, (UPPER ? nsb - 1 : 0) * 32, tid, cur);
     for (int step = 0; step < nsb; ++step) {
         const int q = UPPER ? nsb - 1 - step : step;
         const int sb = q * 32;
         const int w = bs - sb < 32 ? bs - sb : 32;
         if constexpr (PF)
-            if (step + 1 < nsb) trsv_load_strip<RPT, false>(T, lda, bs, (UPPER ? q - 1 : q + 1) * 32, tid, nxt);
+            if (step + 1 < nsb) trsv_load_strip<RPT>(T, lda, bs, (UPPER ? q - 1 : q + 1) * 32, tid, nxt);
         const int kq = sb / 256, owner = (sb % 256) / 64, half = ((sb % 256) / 32) & 1;
         if (wave == owner) {
             const int i = lane - 32 * half;
@@ -395,7 +425,7 @@ __device__ __noinline__ void batch_trsv_multi(int bs, int lda, const float *__re
 #pragma unroll
                     for (int c = 0; c < 32; ++c) cur[k][c] = nxt[k][c];
             } else {
-                trsv_load_strip<RPT, false>(T, lda, bs, (UPPER ? q - 1 : q + 1) * 32, tid, cur);
+                trsv_load_strip<RPT>(T, lda, bs, (UPPER ? q - 1 : q + 1) * 32, tid, cur);
             }
         }
     }

@@ -260,7 +260,11 @@ int hplai_trsv_lower_f32(hplai_ctx ctx, int64_t n, int bs, const float *LU, int6
     CTX_CHECK(ctx);
     HPLAI_CHECK(n >= 0 && bs > 0 && bs <= 1024 && LU != nullptr && x != nullptr && lda >= n,
                 "trsv_lower: bad args");
-    return launch_trsv_lower(n, bs, LU, lda, x, as_stream(stream));
+    if (n == 0) return HPLAI_OK;
+    hipStream_t s = as_stream(stream);
+    ScratchLease work(ctx, s, sizeof(double) * tri_solve_work_doubles(n, 1));
+    if (work.rc) return work.rc;
+    return launch_tri_solve(false, n, LU, lda, x, n, 1, work.as<double>(), s);
 }
 
 int hplai_trsv_upper_f32(hplai_ctx ctx, int64_t n, int bs, const float *LU, int64_t lda, double *x,
@@ -269,7 +273,11 @@ int hplai_trsv_upper_f32(hplai_ctx ctx, int64_t n, int bs, const float *LU, int6
     CTX_CHECK(ctx);
     HPLAI_CHECK(n >= 0 && bs > 0 && bs <= 1024 && LU != nullptr && x != nullptr && lda >= n,
                 "trsv_upper: bad args");
-    return launch_trsv_upper(n, bs, LU, lda, x, as_stream(stream));
+    if (n == 0) return HPLAI_OK;
+    hipStream_t s = as_stream(stream);
+    ScratchLease work(ctx, s, sizeof(double) * tri_solve_work_doubles(n, 1));
+    if (work.rc) return work.rc;
+    return launch_tri_solve(true, n, LU, lda, x, n, 1, work.as<double>(), s);
 }
 
 int hplai_norm_inf_f64(hplai_ctx ctx, int64_t n, const double *x, double *out_dev, void *stream)

@@ -169,22 +169,20 @@ int launch_otf_gemv(int64_t n, uint64_t seed, const double *d, double alpha, con
 int64_t otf_gemv_work_doubles(int64_t n);
 // address of the no-allocation scratch array on `device` (current), looked up once per device
 int noalloc_setup(int device, void **out);
-// triangular solves with the FP32 factors of LU, FP64 vectors; nrhs columns
-// of x with stride ldx
+// X := L^-1 X or U^-1 X, and X := (L U)^-1 X or (L U)^-T X, with the triangles
+// of LU; X FP64, nrhs columns with stride ldx (trisolve.hip)
+int64_t tri_solve_work_doubles(int64_t n, int nrhs);
+int launch_tri_solve(bool upper, int64_t n, const float *LU, int64_t lda, double *X, int64_t ldx, int nrhs,
+                     double *work, hipStream_t s);
+int launch_lu_solve(bool trans, int64_t n, const float *LU, int64_t lda, double *X, int64_t ldx, int nrhs,
+                    double *work, hipStream_t s);
+// one column, diagonal blocks through stored inverses (FP32 entries)
 bool tri_inverse_ok(int b);
 int launch_tri_trsv(bool upper, int b, const float *tri, const double *xin, double *xout, hipStream_t s);
 int launch_trsv_lower_inv(int64_t n, int bs, const float *LU, int64_t lda, double *x, const float *inv,
                           int64_t inv_stride, double *xsc, hipStream_t s);
 int launch_trsv_upper_inv(int64_t n, int bs, const float *LU, int64_t lda, double *x, const float *inv,
                           int64_t inv_stride, double *xsc, hipStream_t s);
-int launch_trsv_lower(int64_t n, int bs, const float *LU, int64_t lda, double *x, hipStream_t s,
-                      int nrhs = 1, int64_t ldx = 0);   // x := L^-1 x
-int launch_trsv_upper(int64_t n, int bs, const float *LU, int64_t lda, double *x, hipStream_t s,
-                      int nrhs = 1, int64_t ldx = 0);   // x := U^-1 x
-int launch_trsv_upper_t(int64_t n, int bs, const float *LU, int64_t lda, double *x, hipStream_t s,
-                        int nrhs = 1, int64_t ldx = 0);   // x := U^-T x
-int launch_trsv_lower_t(int64_t n, int bs, const float *LU, int64_t lda, double *x, hipStream_t s,
-                        int nrhs = 1, int64_t ldx = 0);   // x := L^-T x
 int launch_norm_inf(int64_t n, const double *x, double *out, hipStream_t s);
 int launch_vec_div(int64_t n, const double *num, const double *den, double *out, hipStream_t s);
 int launch_vec_add(int64_t n, const double *x, double *y, hipStream_t s);

@@ -6,7 +6,6 @@
 
 #include "device_common.hpp"
 #include "internal.hpp"
-#include "trsv_block.hpp"
 
 namespace hplai {
 
@@ -120,56 +119,27 @@ int launch_otf_gemv(int64_t n, uint64_t seed, const double *d, double alpha, con
 }
 
 // ---------------------------------------------------------------------------
-// Triangular solves (panel_trsvL / panel_trsvU, panel_trsv.hpp:310-758, with
-// tttrsvL/U, 115-153, and ttgemv, 10-45): FP32 factor entries widened to FP64.
-// Per block of bs rows: (1) one workgroup solves the diagonal block
-// (trsv_block, trsv_block.hpp), (2) a GEMV updates the rest of the vector
-// with the block's column panel.
+// The solve's own triangular solves (panel_trsvL / panel_trsvU,
+// panel_trsv.hpp:310-758; trisolve.hip has the general ones): one right-hand
+// side, diagonal blocks through the inverses the LU stored.
 // ---------------------------------------------------------------------------
-constexpr int kTrsvMax = 1024;
-
-// Right-hand side blockIdx.y at x + y * ldx.
-template <int RPT, bool UPPER, bool UNIT, bool TRANS>
-__global__ __launch_bounds__(256) void trsv_diag_kernel(int bs, const float *__restrict__ T, int64_t lda,
-                                                        double *__restrict__ x, int64_t ldx)
-{
-    __shared__ double xs[32];
-    trsv_block<RPT, UPPER, UNIT, TRANS>(bs, T, lda, x + static_cast<int64_t>(blockIdx.y) * ldx, xs);
-}
-
-template <bool UPPER, bool UNIT, bool TRANS>
-static void launch_trsv_diag(int w, const float *T, int64_t lda, double *x, int64_t ldx, int nrhs,
-                             hipStream_t s)
-{
-    const dim3 grid(1, static_cast<unsigned>(nrhs));
-    if (w <= 256)
-        hipLaunchKernelGGL((trsv_diag_kernel<1, UPPER, UNIT, TRANS>), grid, dim3(256), 0, s, w, T, lda, x, ldx);
-    else if (w <= 512)
-        hipLaunchKernelGGL((trsv_diag_kernel<2, UPPER, UNIT, TRANS>), grid, dim3(256), 0, s, w, T, lda, x, ldx);
-    else
-        hipLaunchKernelGGL((trsv_diag_kernel<4, UPPER, UNIT, TRANS>), grid, dim3(256), 0, s, w, T, lda, x, ldx);
-}
+constexpr int kTrsvMax = 512;
 
 // y(0:m) -= P(m x w) * xb(0:w), P column-major (ttgemv, panel_trsv.hpp:10-45).
 // Workgroup = 64 rows x 4 column groups; the 4 partial sums of a row are added
-// in a fixed order through LDS.  Right-hand side blockIdx.y at offset y * ldx.
+// in a fixed order through LDS.  Workgroup 0 also stores xb into xcopy(0:w):
+// the solved segment goes from its scratch copy to x while the update runs.
 constexpr int kGemvRowsT = 64;
 
-// With xcopy != nullptr (one right-hand side), workgroup 0 also stores xb
-// into xcopy(0:w): the solved segment goes from its scratch copy to x while
-// the update runs.
 __global__ __launch_bounds__(256) void trsv_gemv_kernel(int64_t m, int w, const float *__restrict__ P,
                                                         int64_t lda, const double *__restrict__ xb,
-                                                        double *__restrict__ y, int64_t ldx,
-                                                        double *__restrict__ xcopy)
+                                                        double *__restrict__ y, double *__restrict__ xcopy)
 {
     __shared__ double xs[kTrsvMax];
     __shared__ double part[4][kGemvRowsT];
-    xb += static_cast<int64_t>(blockIdx.y) * ldx;
-    y += static_cast<int64_t>(blockIdx.y) * ldx;
     for (int c = threadIdx.x; c < w; c += 256) {
         xs[c] = xb[c];
-        if (xcopy != nullptr && blockIdx.x == 0) xcopy[c] = xb[c];
+        if (blockIdx.x == 0) xcopy[c] = xb[c];
     }
     __syncthreads();
     const int lr = threadIdx.x % kGemvRowsT, g = threadIdx.x / kGemvRowsT;
@@ -196,55 +166,15 @@ __global__ __launch_bounds__(256) void trsv_gemv_kernel(int64_t m, int w, const 
     if (g == 0 && r < m) y[r] -= ((part[0][lr] + part[1][lr]) + part[2][lr]) + part[3][lr];
 }
 
-// Transposed panel: y(r) -= sum_c P[r*lda + c] * xb(c), r < m, c < w — each
-// row is contiguous; one wave per row at a time, lanes split the columns and
-// the partial sums are combined by a fixed shuffle tree.
-constexpr int kGemvTRows = 16;
-
-__global__ __launch_bounds__(256) void trsv_gemv_t_kernel(int64_t m, int w, const float *__restrict__ P,
-                                                          int64_t lda, const double *__restrict__ xb,
-                                                          double *__restrict__ y, int64_t ldx)
+static void launch_gemv(int64_t m, int w, const float *P, int64_t lda, const double *xb, double *y, double *xcopy,
+                        hipStream_t s)
 {
-    __shared__ double xs[kTrsvMax];
-    xb += static_cast<int64_t>(blockIdx.y) * ldx;
-    y += static_cast<int64_t>(blockIdx.y) * ldx;
-    for (int c = threadIdx.x; c < w; c += 256) xs[c] = xb[c];
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int rr = wave; rr < kGemvTRows; rr += 4) {
-        const int64_t r = static_cast<int64_t>(blockIdx.x) * kGemvTRows + rr;
-        if (r >= m) break;
-        const float *pr = P + r * lda;
-        double acc = 0.0;
-        // columns lane, lane + 64, ... in that order; 8 loads issued together
-        int c = lane;
-        for (; c + 64 * 7 < w; c += 64 * 8) {
-            float v[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) v[q] = pr[c + 64 * q];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) acc = fma(static_cast<double>(v[q]), xs[c + 64 * q], acc);
-        }
-        for (; c < w; c += 64) acc = fma(static_cast<double>(pr[c]), xs[c], acc);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-        if (lane == 0) y[r] -= acc;
-    }
+    hipLaunchKernelGGL(trsv_gemv_kernel, dim3(static_cast<unsigned>(ceil_div(m, kGemvRowsT))), dim3(256), 0, s, m, w,
+                       P, lda, xb, y, xcopy);
 }
 
-static void launch_gemv(bool trans, int64_t m, int w, const float *P, int64_t lda, const double *xb, double *y,
-                        int64_t ldx, int nrhs, hipStream_t s, double *xcopy = nullptr)
-{
-    if (trans)
-        hipLaunchKernelGGL(trsv_gemv_t_kernel, dim3(static_cast<unsigned>(ceil_div(m, kGemvTRows)), nrhs),
-                           dim3(256), 0, s, m, w, P, lda, xb, y, ldx);
-    else
-        hipLaunchKernelGGL(trsv_gemv_kernel, dim3(static_cast<unsigned>(ceil_div(m, kGemvRowsT)), nrhs),
-                           dim3(256), 0, s, m, w, P, lda, xb, y, ldx, xcopy);
-}
-
-// The same block solves with the diagonal blocks applied through the inverses
-// the LU stored (packed, one set per block at inv + q inv_stride): x_q := Tinv_q r_q into the scratch
+// The block solves with the diagonal blocks applied through the inverses the
+// LU stored (packed, one set per block at inv + q inv_stride): x_q := Tinv_q r_q into the scratch
 // segment xsc (bs doubles), then the update of the other rows from xsc, whose
 // workgroup 0 also moves x_q into x.  One right-hand side; n % bs == 0 and
 // tri_inverse_ok(bs).
@@ -257,7 +187,7 @@ int launch_trsv_lower_inv(int64_t n, int bs, const float *LU, int64_t lda, doubl
         if (rc) return rc;
         const int64_t m = n - kb - bs;
         if (m > 0) {
-            launch_gemv(false, m, bs, LU + kb * lda + kb + bs, lda, xsc, x + kb + bs, 0, 1, s, x + kb);
+            launch_gemv(m, bs, LU + kb * lda + kb + bs, lda, xsc, x + kb + bs, x + kb, s);
             HPLAI_HIP(hipGetLastError());
         } else {
             HPLAI_HIP(hipMemcpyAsync(x + kb, xsc, sizeof(double) * bs, hipMemcpyDeviceToDevice, s));
@@ -274,86 +204,10 @@ int launch_trsv_upper_inv(int64_t n, int bs, const float *LU, int64_t lda, doubl
         int rc = launch_tri_trsv(true, bs, inv + (kb / bs) * inv_stride, x + kb, xsc, s);
         if (rc) return rc;
         if (kb > 0) {
-            launch_gemv(false, kb, bs, LU + kb * lda, lda, xsc, x, 0, 1, s, x + kb);
+            launch_gemv(kb, bs, LU + kb * lda, lda, xsc, x, x + kb, s);
             HPLAI_HIP(hipGetLastError());
         } else {
             HPLAI_HIP(hipMemcpyAsync(x + kb, xsc, sizeof(double) * bs, hipMemcpyDeviceToDevice, s));
-        }
-    }
-    return HPLAI_OK;
-}
-
-// x := L^-1 x (unit lower L of LU), nrhs columns of x with stride ldx
-int launch_trsv_lower(int64_t n, int bs, const float *LU, int64_t lda, double *x, hipStream_t s, int nrhs,
-                      int64_t ldx)
-{
-    for (int64_t kb = 0; kb < n; kb += bs) {
-        const int w = n - kb < bs ? static_cast<int>(n - kb) : bs;
-        const float *Lkk = LU + kb * lda + kb;
-        launch_trsv_diag<false, true, false>(w, Lkk, lda, x + kb, ldx, nrhs, s);
-        HPLAI_HIP(hipGetLastError());
-        const int64_t m = n - kb - w;
-        if (m > 0) {
-            launch_gemv(false, m, w, Lkk + w, lda, x + kb, x + kb + w, ldx, nrhs, s);
-            HPLAI_HIP(hipGetLastError());
-        }
-    }
-    return HPLAI_OK;
-}
-
-// x := U^-1 x (upper U of LU)
-int launch_trsv_upper(int64_t n, int bs, const float *LU, int64_t lda, double *x, hipStream_t s, int nrhs,
-                      int64_t ldx)
-{
-    const int64_t nblk = ceil_div(n, bs);
-    for (int64_t q = nblk - 1; q >= 0; --q) {
-        const int64_t kb = q * bs;
-        const int w = n - kb < bs ? static_cast<int>(n - kb) : bs;
-        const float *Ukk = LU + kb * lda + kb;
-        launch_trsv_diag<true, false, false>(w, Ukk, lda, x + kb, ldx, nrhs, s);
-        HPLAI_HIP(hipGetLastError());
-        if (kb > 0) {
-            launch_gemv(false, kb, w, LU + kb * lda, lda, x + kb, x, ldx, nrhs, s);
-            HPLAI_HIP(hipGetLastError());
-        }
-    }
-    return HPLAI_OK;
-}
-
-// x := U^-T x: U^T is lower with U's diagonal; element (r, c) = LU[r*lda + c]
-int launch_trsv_upper_t(int64_t n, int bs, const float *LU, int64_t lda, double *x, hipStream_t s, int nrhs,
-                        int64_t ldx)
-{
-    for (int64_t kb = 0; kb < n; kb += bs) {
-        const int w = n - kb < bs ? static_cast<int>(n - kb) : bs;
-        const float *Tkk = LU + kb * lda + kb;
-        launch_trsv_diag<false, false, true>(w, Tkk, lda, x + kb, ldx, nrhs, s);
-        HPLAI_HIP(hipGetLastError());
-        const int64_t m = n - kb - w;
-        if (m > 0) {
-            // rows kb + w + r', columns kb + c: LU[(kb + w + r') * lda + kb + c]
-            launch_gemv(true, m, w, LU + (kb + w) * lda + kb, lda, x + kb, x + kb + w, ldx, nrhs, s);
-            HPLAI_HIP(hipGetLastError());
-        }
-    }
-    return HPLAI_OK;
-}
-
-// x := L^-T x: L^T is unit upper; element (r, c) = LU[r*lda + c]
-int launch_trsv_lower_t(int64_t n, int bs, const float *LU, int64_t lda, double *x, hipStream_t s, int nrhs,
-                        int64_t ldx)
-{
-    const int64_t nblk = ceil_div(n, bs);
-    for (int64_t q = nblk - 1; q >= 0; --q) {
-        const int64_t kb = q * bs;
-        const int w = n - kb < bs ? static_cast<int>(n - kb) : bs;
-        const float *Tkk = LU + kb * lda + kb;
-        launch_trsv_diag<true, true, true>(w, Tkk, lda, x + kb, ldx, nrhs, s);
-        HPLAI_HIP(hipGetLastError());
-        if (kb > 0) {
-            // rows r < kb, columns kb + c: LU[r * lda + kb + c]
-            launch_gemv(true, kb, w, LU + kb, lda, x + kb, x, ldx, nrhs, s);
-            HPLAI_HIP(hipGetLastError());
         }
     }
     return HPLAI_OK;

@@ -59,7 +59,7 @@ struct Buffers {
     int *info = nullptr;
     double *chk = nullptr;
     float *inv = nullptr;   // packed inverses of the diagonal blocks' triangles, one set per block
-    double *tsc = nullptr;  // one block of the IR's triangular solves (scratch)
+    double *tsc = nullptr;  // scratch of the IR's triangular solves
     uint16_t *P = nullptr;  // FP16 trailing storage (n x n, leading dimension n)
     uint16_t *Q = nullptr;  // its back buffer (n x n), when on
 
@@ -703,15 +703,9 @@ int hplai_lu_solve_f64(hplai_ctx ctx, int trans, int64_t n, int nrhs, int bs, co
     if (n == 0 || nrhs == 0) return HPLAI_OK;
     HPLAI_HIP(hipSetDevice(ctx->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    int rc;
-    if (trans == 0) {
-        rc = launch_trsv_lower(n, bs, LU, lda, X, s, nrhs, ldx);
-        if (rc == HPLAI_OK) rc = launch_trsv_upper(n, bs, LU, lda, X, s, nrhs, ldx);
-    } else {
-        rc = launch_trsv_upper_t(n, bs, LU, lda, X, s, nrhs, ldx);
-        if (rc == HPLAI_OK) rc = launch_trsv_lower_t(n, bs, LU, lda, X, s, nrhs, ldx);
-    }
-    return rc;
+    ScratchLease work(ctx, s, sizeof(double) * tri_solve_work_doubles(n, nrhs));
+    if (work.rc) return work.rc;
+    return launch_lu_solve(trans != 0, n, LU, lda, X, ldx, nrhs, work.as<double>(), s);
 }
 
 int hplai_release(hplai_ctx ctx)
@@ -827,7 +821,7 @@ int hplai_solve(hplai_ctx ctx, const hplai_params *p, hplai_result *res)
     alloc(B.rhs, sizeof(double) * n, "hplai_solve: hipMalloc rhs");
     alloc(B.x, sizeof(double) * n, "hplai_solve: hipMalloc x");
     alloc(B.r, sizeof(double) * n, "hplai_solve: hipMalloc r");
-    alloc(B.tsc, sizeof(double) * b, "hplai_solve: hipMalloc tsc");
+    alloc(B.tsc, sizeof(double) * (tri_inverse_ok(b) ? b : tri_solve_work_doubles(n, 1)), "hplai_solve: hipMalloc tsc");
     alloc(B.work, sizeof(double) * std::max(3 * n, std::max(otf_gemv_work_doubles(n), higham_gemv_work_doubles(n))),
           "hplai_solve: hipMalloc work");
     alloc(B.norms, sizeof(double) * 4, "hplai_solve: hipMalloc norms");
@@ -921,9 +915,7 @@ int hplai_solve(hplai_ctx ctx, const hplai_params *p, hplai_result *res)
                         if (r == HPLAI_OK) r = launch_trsv_upper_inv(n, b, B.A, lu.lda, B.r, B.inv, st, B.tsc, s);
                         return r;
                     }
-                    int r = launch_trsv_lower(n, b, B.A, lu.lda, B.r, s);
-                    if (r == HPLAI_OK) r = launch_trsv_upper(n, b, B.A, lu.lda, B.r, s);
-                    return r;
+                    return launch_lu_solve(false, n, B.A, lu.lda, B.r, n, 1, B.tsc, s);
                 });
                 if (rc == HPLAI_OK) rc = launch_vec_add(n, B.r, B.x, s);
             }

@@ -160,8 +160,8 @@ int hplai_otf_gemv_f64(hplai_ctx ctx, int64_t n, uint64_t seed, const double *d,
 int hplai_otf_gemv_f64_noalloc(hplai_ctx ctx, int64_t n, uint64_t seed, const double *d, double alpha,
                                const double *x, double *y, void *stream);
 /* Replaces panel_trsvL / tttrsvL (panel_trsv.hpp:115-124, 310-535):
- * x := L^-1 x, L the unit lower triangle of LU (FP32), x FP64.  bs is the
- * blocking (<= 1024; use the LU block size). */
+ * x := L^-1 x, L the unit lower triangle of LU (FP32), x FP64.  bs (1 ..
+ * 1024) is checked, the blocking is the library's own. */
 int hplai_trsv_lower_f32(hplai_ctx ctx, int64_t n, int bs, const float *LU, int64_t lda,
                          double *x, void *stream);
 /* Replaces panel_trsvU / tttrsvU (panel_trsv.hpp:142-153, 537-758). */
@@ -185,7 +185,8 @@ int hplai_factor_f32(hplai_ctx ctx, int64_t n, int b, int fmt, int outer, int lo
  * trans = 0: X := (L U)^-1 X;  trans = 1: X := (L U)^-T X = L^-T U^-T X,
  * the transposed solve for A^T lambda = g (no reference counterpart: it serves
  * the gradient of x = A^-1 b).  X (device, FP64) holds nrhs columns with
- * leading dimension ldx; bs (<= 1024) is the blocking, normally the LU's b. */
+ * leading dimension ldx; bs (1 .. 1024) is checked, the blocking is the
+ * library's own. */
 int hplai_lu_solve_f64(hplai_ctx ctx, int trans, int64_t n, int nrhs, int bs, const float *LU,
                        int64_t lda, double *X, int64_t ldx, void *stream);
 
