@@ -10,17 +10,25 @@
 //                     workgroups update the rest of the trailing matrix;
 //   lu_strip_kernel   L21 := A21 U11^-1 and U12 := L11^-1 A12 as products
 //                     with those inverses, 32 rows or columns per workgroup.
-// Then tri_merge_kernel joins the inverses of neighbouring sub-blocks (128 ->
-// 256 -> 512 -> 1024):
-//   [A 0; C B]^-1 = [A^-1 0; -B^-1 C A^-1, B^-1].
+// The inverses of the whole block grow by a sub-block q at a time,
+//   Linv(q, J) = -Linv_qq T,   T  = sum_K L(q, K) Linv(K, J)
+//   Uinv(J, q) = -T' Uinv_qq,  T' = sum_K Uinv(J, K) U(K, q)     (K < q),
+// T by more workgroups of the launch that factors sub-block q, which leaves
+// the device idle, and the products with Linv_qq and Uinv_qq by more
+// workgroups of the next launch.  A block that is factored already joins the
+// inverses of neighbouring sub-blocks (128 -> 256 -> 512 -> 1024) with the same
+// two products, all pairs of a size at once.
 //
 // What bounds it: the chain of 32 x 32 LUs, inverses and strips (17k clocks a
 // link, one or two waves working) and, between sub-blocks, a launch and the
 // 128^3 update of the next diagonal sub-block.  One workgroup for the whole
 // 512 block spent half its time on trailing updates through a single CU's
 // path to the L2, and the inverses were two more kernels after it: 511 + 73
-// us, now 200 us and about 25 us for the joins (b = 512, alone); b = 60: 94 ->
-// 15 us; n = 1000: 645 us with v_readlane steps, 427 us as here.
+// us, now 215 us with the inverses (b = 512, alone); b = 60: 94 -> 15 us; n =
+// 1000: 645 us with v_readlane steps, 423 us as here.  Joining by one
+// workgroup per 32 columns took 39 us a size (product by product, each behind
+// its loads) after the factorization.
+#include <cstddef>
 #include <type_traits>
 #include <utility>
 
@@ -34,7 +42,7 @@ typedef float floatx16g_t __attribute__((ext_vector_type(16)));
 constexpr int kLuNB = 128;            // columns per sub-block
 constexpr int kLuThreads = 512;
 constexpr int kLuS = kLuNB + 1;       // LDS column stride: odd, so that walks along rows and columns both spread
-constexpr int kMergeMax = 512;        // largest half joined by tri_merge_kernel
+constexpr int kJoinMax = 512;         // largest half joined by tri_join_kernel
 
 __device__ __forceinline__ floatx16g_t zero16()
 {
@@ -393,13 +401,136 @@ __device__ __forceinline__ void write_inverse_row(const float *V, float *tri, in
     for (int e = 0; e < 4; ++e) o[e] = float4{v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]};
 }
 
+// The inverses' packed blocks hold 16 floats per lane: a left operand's (L
+// side: row lane % 32, column 2 kk + lane / 32) or a right operand's (U side:
+// row 2 kk + lane / 32, column lane % 32).  Position of an entry:
+__device__ __forceinline__ int left_pos(int r, int c) { return (r + 32 * (c & 1)) * 16 + (c >> 1); }
+__device__ __forceinline__ int right_pos(int r, int c) { return (c + 32 * (r & 1)) * 16 + (r >> 1); }
+
+__device__ __forceinline__ void packed16(const float *blk, int lane, float (&v)[16])
+{
+    const float4 *p = reinterpret_cast<const float4 *>(blk) + lane * 4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float4 q = p[e];
+        v[4 * e] = q.x;
+        v[4 * e + 1] = q.y;
+        v[4 * e + 2] = q.z;
+        v[4 * e + 3] = q.w;
+    }
+}
+
+// First product, 512 threads: for the four 32-blocks X = R .. R + 3 (< Rend)
+//   L side:  T(X, J)  = sum_{J <= K < K1} L(X, K) Linv(K, J), as a right operand to Linv's slot (X, J)
+//   U side:  T'(J, X) = sum_{J <= K < K1} Uinv(J, K) U(K, X), as a left operand to Uinv's slot (J, X)
+// The inverse's strip comes out of its order through W (33 floats per k, the
+// K1 - J blocks' 32 k each); two waves per X take every other K.
+template <bool UP>
+__device__ __forceinline__ void tri_mid(int n, int nb, const float *A, int64_t lda, float *tri, int J, int K1, int R,
+                                        int Rend, float *W)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, lh = lane >> 5, X = R + (wave & 3), half = wave >> 2;
+#pragma unroll 4
+    for (int e = tid; e < (K1 - J) * 1024; e += kLuThreads) {
+        const int K = J + (e >> 10), ln = (e >> 4) & 63, kk = e & 15;
+        const float *blk = UP ? tri_block_u(tri, nb, J, K) : tri_block_l(tri, nb, K, J);
+        W[(32 * (K - J) + (ln & 31)) * 33 + 2 * kk + (ln >> 5)] = blk[e & 1023];
+    }
+    __syncthreads();
+    floatx16g_t acc = zero16();
+    const bool on = X < Rend;
+    if (on) {
+        const int x = 32 * X + l32;             // row of L, column of U
+        const int64_t xo = min(x, n - 1);
+        for (int K = J + half; K < K1; K += 8) {
+            float av[4][16];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (K + 2 * u < K1)
+#pragma unroll
+                    for (int kk = 0; kk < 16; ++kk) {
+                        const int64_t k = 32 * (K + 2 * u) + 2 * kk + lh;   // below n: the blocks before X are whole
+                        av[u][kk] = UP ? A[xo * lda + k] : A[k * lda + xo];
+                    }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (K + 2 * u < K1) {
+                    float wv[16];
+#pragma unroll
+                    for (int kk = 0; kk < 16; ++kk) {
+                        wv[kk] = W[(32 * (K + 2 * u - J) + 2 * kk + lh) * 33 + l32];
+                        if (x >= n) av[u][kk] = 0.0f;
+                    }
+                    acc = UP ? mfma16(wv, av[u], acc) : mfma16(av[u], wv, acc);
+                }
+        }
+    }
+    __syncthreads();
+    if (on && half == 1)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) W[((wave & 3) * 16 + e) * 64 + lane] = acc[e];
+    __syncthreads();
+    if (on && half == 0) {
+        float *o = UP ? tri_block_u(tri, nb, J, X) : tri_block_l(tri, nb, X, J);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int r = acc_row(e, lh);
+            o[UP ? left_pos(r, l32) : right_pos(r, l32)] = acc[e] + W[(wave * 16 + e) * 64 + lane];
+        }
+    }
+}
+
+// Second product, in place, NW waves, at most PER * NW blocks X = R0 .. R1 - 1:
+//   Linv(X, J) = -sum_{R0 <= K <= X} Linv(X, K) T(K, J),  Uinv(J, X) = -sum_{R0 <= K <= X} T'(J, K) Uinv(K, X)
+template <bool UP, int NW, int PER>
+__device__ __forceinline__ void tri_fin(int nb, float *tri, int J, int R0, int R1)
+{
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, lh = lane >> 5;
+    floatx16g_t acc[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int X = R0 + wave + NW * i;
+        acc[i] = zero16();
+        if (X >= R1) continue;
+        for (int K = R0; K <= X; K += 4) {
+            float av[4][16], bv[4][16];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (K + u <= X) {
+                    packed16(UP ? tri_block_u(tri, nb, J, K + u) : tri_block_l(tri, nb, X, K + u), lane, av[u]);
+                    packed16(UP ? tri_block_u(tri, nb, K + u, X) : tri_block_l(tri, nb, K + u, J), lane, bv[u]);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (K + u <= X) acc[i] = mfma16(av[u], bv[u], acc[i]);
+        }
+    }
+    __syncthreads();   // every T of column (row) J is read
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int X = R0 + wave + NW * i;
+        if (X >= R1) continue;
+        float *o = UP ? tri_block_u(tri, nb, J, X) : tri_block_l(tri, nb, X, J);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int r = acc_row(e, lh);
+            o[UP ? right_pos(r, l32) : left_pos(r, l32)] = -acc[i][e];
+        }
+    }
+}
+
 // Sub-block k0 of the n x n block A.  FACTOR: the update with sub-block
-// k0 - 128 (when there is one), LU, inverses; workgroups 1.. update the rest
-// of the trailing matrix.  Without FACTOR: A is already factored and
+// k0 - 128 (when there is one), LU, inverses; the next workgroups update the
+// rest of the trailing matrix and the last form the first products of the
+// whole block's inverses.  Without FACTOR: A is already factored and
 // workgroup q inverts the triangles of sub-block q.
 template <bool FACTOR>
 __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, float *__restrict__ A, int64_t lda,
-                                                               float *__restrict__ tri, int sides,
+                                                               float *tri, int sides,
                                                                int *__restrict__ info)
 {
     __shared__ LuLds sm;
@@ -417,6 +548,16 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
         // tiles in row-major order without the two of the diagonal sub-block
         const int two = ct < 2 ? ct : 2;
         const int t = static_cast<int>(blockIdx.x) - 1 + two;
+        if (t >= (rest + 127) / 128 * ct) {
+            static_assert(offsetof(LuLds, V) == sizeof(float) * kLuNB * kLuS && (1024 - kLuNB) * 33 <= 2 * kLuNB * kLuS,
+                          "the strip of an inverse spans S and V");
+            const int z = t - (rest + 127) / 128 * ct, q0 = k0 / 32;
+            if (z & 1)
+                tri_mid<true>(n, nb, A, lda, tri, z >> 1, q0, q0, nb < q0 + 4 ? nb : q0 + 4, S);
+            else
+                tri_mid<false>(n, nb, A, lda, tri, z >> 1, q0, q0, nb < q0 + 4 ? nb : q0 + 4, S);
+            return;
+        }
         const int r0 = (t / ct) * 128 + (wave & 3) * 32, c0 = (t % ct) * 64, cw = c0 + (wave >> 2) * 32;
         // U12 (128 x 64) through LDS: its MFMA operand walks along columns
         {
@@ -638,14 +779,23 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
 
 // L21 := A21 Uinv and U12 := Linv A12 for the rows and columns past the
 // sub-block at p0 (128 wide).  A workgroup owns 32 rows of L21 (blockIdx.x <
-// strips) or 32 columns of U12; wave j computes its 32-wide block j.
-__global__ __launch_bounds__(256) void lu_strip_kernel(int n, int p0, float *__restrict__ A, int64_t lda,
-                                                       const float *__restrict__ tri, int strips)
+// strips) or 32 columns of U12; wave j computes its 32-wide block j.  The
+// workgroups past those finish the whole block's inverses of this sub-block.
+__global__ __launch_bounds__(256) void lu_strip_kernel(int n, int p0, float *__restrict__ A, int64_t lda, float *tri,
+                                                       int strips)
 {
     __shared__ float X[kLuNB * 33];
     const int tid = threadIdx.x, lane = tid & 63, J = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
     const int nb = (n + 31) / 32, q0 = p0 / 32, k1 = p0 + kLuNB;
+    if (static_cast<int>(blockIdx.x) >= 2 * strips) {
+        const int z = static_cast<int>(blockIdx.x) - 2 * strips;
+        if (z & 1)
+            tri_fin<true, 4, 1>(nb, tri, z >> 1, q0, nb < q0 + 4 ? nb : q0 + 4);
+        else
+            tri_fin<false, 4, 1>(nb, tri, z >> 1, q0, nb < q0 + 4 ? nb : q0 + 4);
+        return;
+    }
     const bool up = static_cast<int>(blockIdx.x) >= strips;
     const int o = k1 + 32 * (static_cast<int>(blockIdx.x) - (up ? strips : 0));   // first row / column
     const int cnt = n - o < 32 ? n - o : 32;
@@ -697,99 +847,31 @@ __global__ __launch_bounds__(256) void lu_strip_kernel(int n, int p0, float *__r
 }
 
 // Joins the inverses of the halves [I0, I0 + H) and [I0 + H, I1) (32-blocks)
-// of every pair.  blockIdx.x: a 32-column strip J; blockIdx.y + side0: 0 the
-// L side (J in the first half), 1 the U side (J in the second):
-//   T(I, J) = sum_K L(I, K) Linv(K, J),   Linv(I, J) = -sum_K Linv(I, K) T(K, J)
-//   T(I, J) = sum_K U(I, K) Uinv(K, J),   Uinv(I, J) = -sum_K Uinv(I, K) T(K, J)
-__global__ __launch_bounds__(kLuThreads) void tri_merge_kernel(int n, int H, const float *__restrict__ A, int64_t lda,
-                                                               float *__restrict__ tri, int side0)
+// of every pair: blockIdx.x the pair and J of its first half, blockIdx.z +
+// side0 the L or the U side.  MID: the first product for four blocks of the
+// second half (blockIdx.y); else the second product.
+template <bool MID>
+__global__ __launch_bounds__(kLuThreads) void tri_join_kernel(int n, int H, const float *__restrict__ A, int64_t lda,
+                                                              float *tri, int side0)
 {
-    __shared__ float T[kMergeMax * 33];   // T[row * 33 + c], rows from the half's first
-    __shared__ float W[kMergeMax * 33];   // the strip of the L side's first factor, Linv(:, J)
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31, lh = lane >> 5;
     const int nb = (n + 31) / 32;
-    const bool up = static_cast<int>(blockIdx.y) + side0 != 0;
-    const int I0 = static_cast<int>(blockIdx.x) / H * 2 * H;
-    const int I1 = I0 + 2 * H < nb ? I0 + 2 * H : nb;
-    const int J = I0 + (up ? H : 0) + static_cast<int>(blockIdx.x) % H;
-    if (I0 + H >= I1 || J >= I1) return;
-    const int R0 = up ? I0 : I0 + H, R1 = up ? I0 + H : I1;   // output rows
-    if (!up) {
-        for (int K = J; K < I0 + H; ++K)
-            for (int e = tid; e < 1024; e += kLuThreads) {
-                const int ln = e >> 4, kk = e & 15;   // lane ln holds row ln % 32, column 2 kk + ln / 32
-                W[((K - I0) * 32 + (ln & 31)) * 33 + 2 * kk + (ln >> 5)] = tri_block_l(tri, nb, K, J)[e];
-            }
-        __syncthreads();
-    }
-    for (int I = R0 + wave; I < R1; I += kLuThreads / 64) {
-        floatx16g_t acc = zero16();
-        const int row = 32 * I + l32;
-        const int K0 = up ? I0 + H : J, K1 = up ? J + 1 : I0 + H;
-        for (int K = K0; K < K1; ++K) {
-            float av[16], bv[16];
-#pragma unroll
-            for (int kk = 0; kk < 16; ++kk) {
-                const int col = 32 * K + 2 * kk + lh;
-                const float v = A[static_cast<int64_t>(min(col, n - 1)) * lda + min(row, n - 1)];
-                av[kk] = (row < n && col < n) ? v : 0.0f;
-            }
-            if (up) {
-                const float4 *b4 = reinterpret_cast<const float4 *>(tri_block_u(tri, nb, K, J)) + lane * 4;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float4 q = b4[e];
-                    bv[4 * e] = q.x;
-                    bv[4 * e + 1] = q.y;
-                    bv[4 * e + 2] = q.z;
-                    bv[4 * e + 3] = q.w;
-                }
-            } else {
-#pragma unroll
-                for (int kk = 0; kk < 16; ++kk) bv[kk] = W[((K - I0) * 32 + 2 * kk + lh) * 33 + l32];
-            }
-            acc = mfma16(av, bv, acc);
-        }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) T[((I - R0) * 32 + acc_row(e, lh)) * 33 + l32] = acc[e];
-    }
-    __syncthreads();
-    // rows with the most products first: I from the end (L) or from the start (U)
-    for (int p = wave; p < R1 - R0; p += kLuThreads / 64) {
-        const int I = up ? R0 + p : R1 - 1 - p;
-        floatx16g_t acc = zero16();
-        const int K0 = up ? I : R0, K1 = up ? R1 : I + 1;
-        for (int K = K0; K < K1; ++K) {
-            float av[16], bv[16];
-            if (up) {
-                // Uinv(I, K) as the left operand (row l32, k = 2 kk + lh) out of the right-operand order
-                const float *blk = tri_block_u(tri, nb, I, K) + 512 * (l32 & 1) + (l32 >> 1);
-#pragma unroll
-                for (int kk = 0; kk < 16; ++kk) av[kk] = blk[(2 * kk + lh) * 16];
-            } else {
-                const float4 *a4 = reinterpret_cast<const float4 *>(tri_block_l(tri, nb, I, K)) + lane * 4;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float4 q = a4[e];
-                    av[4 * e] = q.x;
-                    av[4 * e + 1] = q.y;
-                    av[4 * e + 2] = q.z;
-                    av[4 * e + 3] = q.w;
-                }
-            }
-#pragma unroll
-            for (int kk = 0; kk < 16; ++kk) bv[kk] = T[((K - R0) * 32 + 2 * kk + lh) * 33 + l32];
-            acc = mfma16(av, bv, acc);
-        }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int rho = acc_row(e, lh);
-            if (up)
-                tri_block_u(tri, nb, I, J)[(l32 + 32 * (rho & 1)) * 16 + (rho >> 1)] = -acc[e];
-            else
-                tri_block_l(tri, nb, I, J)[(rho + 32 * (l32 & 1)) * 16 + (l32 >> 1)] = -acc[e];
-        }
+    const bool up = static_cast<int>(blockIdx.z) + side0 != 0;
+    const int J = static_cast<int>(blockIdx.x) / H * 2 * H + static_cast<int>(blockIdx.x) % H;
+    const int R0 = static_cast<int>(blockIdx.x) / H * 2 * H + H, R1 = R0 + H < nb ? R0 + H : nb;
+    if constexpr (MID) {
+        __shared__ float W[kJoinMax * 33];
+        const int R = R0 + 4 * static_cast<int>(blockIdx.y), Rend = R + 4 < R1 ? R + 4 : R1;
+        if (R >= Rend) return;
+        if (up)
+            tri_mid<true>(n, nb, A, lda, tri, J, R0, R, Rend, W);
+        else
+            tri_mid<false>(n, nb, A, lda, tri, J, R0, R, Rend, W);
+    } else {
+        if (R0 >= R1) return;
+        if (up)
+            tri_fin<true, 8, kJoinMax / 32 / 8>(nb, tri, J, R0, R1);
+        else
+            tri_fin<false, 8, kJoinMax / 32 / 8>(nb, tri, J, R0, R1);
     }
 }
 
@@ -797,18 +879,6 @@ int64_t tri_floats(int b)
 {
     const int64_t nb = ceil_div(b, 32);
     return 2 * nb * nb * 1024;
-}
-
-static int merge_inverses(int n, const float *A, int64_t lda, float *tri, int sides, hipStream_t s)
-{
-    const int nb = static_cast<int>(ceil_div(n, 32));
-    for (int H = kLuNB / 32; H < nb; H *= 2) {
-        const unsigned strips = static_cast<unsigned>(ceil_div(nb, 2 * H)) * H;
-        hipLaunchKernelGGL(tri_merge_kernel, dim3(strips, sides == 3 ? 2 : 1), dim3(kLuThreads), 0, s, n, H, A, lda,
-                           tri, sides == 2 ? 1 : 0);
-        HPLAI_HIP(hipGetLastError());
-    }
-    return HPLAI_OK;
 }
 
 int64_t getrf_scratch_floats(int n) { return n > kLuNB ? tri_floats(n) : 0; }
@@ -820,18 +890,19 @@ int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, bool full,
         const int rest = n - k;
         const int rt = (rest + 127) / 128, ct = (rest + 63) / 64;
         const int tiles = k == 0 ? 0 : rt * ct - (ct < 2 ? ct : 2);
-        // the last sub-block's inverses serve only a caller who asked for them
-        hipLaunchKernelGGL((lu_update_kernel<true>), dim3(static_cast<unsigned>(1 + tiles)), dim3(kLuThreads), 0, s,
-                           n, k, A, lda, !full && rest <= kLuNB ? nullptr : tri, 3, info);
+        // the whole block's inverses, and the last sub-block's, serve only a caller who asked for them
+        const unsigned join = full ? 2 * (k / 32) : 0;
+        hipLaunchKernelGGL((lu_update_kernel<true>), dim3(static_cast<unsigned>(1 + tiles) + join), dim3(kLuThreads),
+                           0, s, n, k, A, lda, !full && rest <= kLuNB ? nullptr : tri, 3, info);
         HPLAI_HIP(hipGetLastError());
-        if (rest > kLuNB) {
-            const int strips = (rest - kLuNB + 31) / 32;
-            hipLaunchKernelGGL(lu_strip_kernel, dim3(static_cast<unsigned>(2 * strips)), dim3(256), 0, s, n, k, A,
-                               lda, tri, strips);
+        const int strips = rest > kLuNB ? (rest - kLuNB + 31) / 32 : 0;
+        if (2 * strips + join > 0) {
+            hipLaunchKernelGGL(lu_strip_kernel, dim3(static_cast<unsigned>(2 * strips) + join), dim3(256), 0, s, n, k,
+                               A, lda, tri, strips);
             HPLAI_HIP(hipGetLastError());
         }
     }
-    return full ? merge_inverses(n, A, lda, tri, 3, s) : HPLAI_OK;
+    return HPLAI_OK;
 }
 
 int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, hipStream_t s)
@@ -840,7 +911,16 @@ int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int side
     hipLaunchKernelGGL((lu_update_kernel<false>), dim3(static_cast<unsigned>(ceil_div(b, kLuNB))), dim3(kLuThreads), 0,
                        s, b, 0, const_cast<float *>(LU), lda, tri, sides, nullptr);
     HPLAI_HIP(hipGetLastError());
-    return merge_inverses(b, LU, lda, tri, sides, s);
+    const int nb = static_cast<int>(ceil_div(b, 32));
+    for (int H = kLuNB / 32; H < nb; H *= 2) {
+        const unsigned cols = static_cast<unsigned>(ceil_div(nb, 2 * H)) * H, z = sides == 3 ? 2 : 1;
+        hipLaunchKernelGGL((tri_join_kernel<true>), dim3(cols, H / 4, z), dim3(kLuThreads), 0, s, b, H, LU, lda, tri,
+                           sides == 2 ? 1 : 0);
+        hipLaunchKernelGGL((tri_join_kernel<false>), dim3(cols, 1, z), dim3(kLuThreads), 0, s, b, H, LU, lda, tri,
+                           sides == 2 ? 1 : 0);
+        HPLAI_HIP(hipGetLastError());
+    }
+    return HPLAI_OK;
 }
 
 }  // namespace hplai

@@ -107,3 +107,20 @@ def test_getrf_captured(ctx, oracle):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(buf, want)
+
+
+@pytest.mark.parametrize("b", [160, 257, 384, 500, 650, 1000])
+def test_inverses_grown_with_the_factorization(ctx, oracle, b):
+    """Two diagonal blocks: the panels beside the first are products with the
+    inverses that grow by a 128-column sub-block at a time.  L21 U11 = A21 and
+    L11 U12 = A12 in FP64, within the 2e-5 of the TRSM tests."""
+    import torch
+    n = 2 * b
+    A = oracle.gen_block(2 * n, 0, 0, n, n, SEED)             # A[col, row]
+    F = _dev(A)
+    ctx.factor(n, b, F, n, fmt="f16")
+    A, F = torch.from_numpy(A).t().double(), F.cpu().t().double()
+    L = F[:b, :b].tril(-1) + torch.eye(b, dtype=torch.float64)
+    U = F[:b, :b].triu()
+    for got, want in ((F[b:, :b] @ U, A[b:, :b]), (L @ F[:b, b:], A[:b, b:])):
+        assert ((got - want).abs().max() / want.abs().max()).item() < 2e-5
