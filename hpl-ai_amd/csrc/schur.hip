@@ -76,8 +76,12 @@ __device__ __forceinline__ void store_c_nt(float *p, const float4 &c)
 // column lrow of block (i, j).  The MFMA layout gives each lane 4 rows of one
 // column, so a direct access touches 32 columns with 32 bytes each; through
 // the LDS scratch T (32 columns x kEpiAnyS(IB) floats, private to the wave)
-// every instruction covers 64 consecutive rows of one column.  (A column-major
-// C with an odd leading dimension, 4001 x 3003 x 60: the kernel 89 -> 31 us.)
+// every instruction covers 64 consecutive rows of one column.  All of a part's
+// loads are in flight together: past an edge they repeat the last row or
+// column, since a condition on each would make the compiler wait for each
+// (4001 x 3003 x 60, odd leading dimension: 89 us with direct accesses, 48 with
+// conditional loads, 22 as here, about what C's 96 MB take; 1140 x 1140 x 60:
+// 20 -> 8 us).
 constexpr int kEpiAnyS(int IB) { return 32 * IB + 1; }   // odd: both walks spread over the banks
 
 template <int IB, int JB>
@@ -96,21 +100,24 @@ __device__ __forceinline__ void epilogue_any(float *__restrict__ C, int64_t ldc,
                 for (int r = 0; r < 4; ++r) T[lrow * S + i * 32 + 8 * q + 4 * lgrp + r] = acc[i][j][4 * q + r];
 #pragma unroll
         for (int h = 0; h < IB / 2; ++h) {
-            const int64_t gr = row0 + 64 * h + lane;
-            float *cp = C + (col0 + j * 32) * ldc + gr;
-            const int64_t left = N - (col0 + j * 32);
-            const int nc = left < 32 ? static_cast<int>(left) : 32;   // may be negative: nothing to do
-            if (gr < M) {
+            const int64_t nr = M - (row0 + 64 * h), left = N - (col0 + j * 32);
+            if (nr <= 0 || left <= 0) continue;
+            const int nc = left < 32 ? static_cast<int>(left) : 32;
+            const int r = nr < 64 ? min(lane, static_cast<int>(nr) - 1) : lane;
+            float *cp = C + (col0 + j * 32) * ldc + row0 + 64 * h;
+            float v[32];
 #pragma unroll
-                for (int c0 = 0; c0 < 32; c0 += 16) {
-                    float v[16];
+            for (int c = 0; c < 32; ++c) v[c] = (cp + min(c, nc - 1) * ldc)[r];
 #pragma unroll
-                    for (int c = 0; c < 16; ++c)
-                        if (c0 + c < nc) v[c] = cp[(c0 + c) * ldc];
+            for (int c = 0; c < 32; ++c) v[c] -= T[c * S + 64 * h + lane];
+            if (r != lane) continue;
+            if (nc == 32) {
 #pragma unroll
-                    for (int c = 0; c < 16; ++c)
-                        if (c0 + c < nc) cp[(c0 + c) * ldc] = v[c] - T[(c0 + c) * S + 64 * h + lane];
-                }
+                for (int c = 0; c < 32; ++c) (cp + c * ldc)[lane] = v[c];
+            } else {
+#pragma unroll
+                for (int c = 0; c < 32; ++c)
+                    if (c < nc) (cp + c * ldc)[lane] = v[c];
             }
         }
     }

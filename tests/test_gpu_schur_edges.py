@@ -1,0 +1,29 @@
+"""Schur update of a C that is no whole number of tiles: one row, one column
+and the neighbours of 32, 64 and 128, an odd leading dimension, nothing written
+outside.  K = 64 products of FP16 values below 1/2, so every sum of magnitudes
+is at most 16 and 64 FP32 roundings differ from the exact sum by at most
+64 * 16 * 2^-24 = 6.2e-5."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m", [1, 31, 63, 64, 65, 129])
+@pytest.mark.parametrize("n", [1, 31, 33, 64, 127, 130])
+def test_schur_f16_edges(ctx, m, n):
+    import torch
+    rng = np.random.default_rng(m * 1000 + n)
+    L = (rng.random((m, 64)) - 0.5).astype(np.float16)
+    U = (rng.random((n, 64)) - 0.5).astype(np.float16)
+    C = rng.random((n + 2, m + 5)).astype(np.float32)          # C[col, row]
+    g = torch.from_numpy(C).cuda()
+    ctx.schur_update(0, m, n, 1, 64, torch.from_numpy(L).cuda(), 64, None, 0, torch.from_numpy(U).cuda(), 64, None, 0,
+                     0, g[1, 2:], m + 5)
+    got = g.cpu().numpy()
+    want = C.astype(np.float64)
+    want[1:n + 1, 2:m + 2] -= U.astype(np.float64) @ L.astype(np.float64).T
+    assert np.max(np.abs(got - want)) < 6.2e-5
+    inside = np.zeros(C.shape, dtype=bool)
+    inside[1:n + 1, 2:m + 2] = True
+    assert np.array_equal(got[~inside], C[~inside])
