@@ -381,14 +381,17 @@ struct LU {
         int rc = HPLAI_OK;
         const int64_t Bw = static_cast<int64_t>(sw) * b;
         const int64_t rb0 = c0 + Bw, mb = n - rb0;   // rows below the outer block
-        hipStream_t q = bulk;
+        // with one inner block there is no chain beside the rows below, and the
+        // hops to the bulk stream and back would lie on the panel's path
+        hipStream_t q = sw > 1 ? bulk : s;
+        const bool fork = mb > 0 && q != s;
         hipEvent_t ev_fork = ev[3], ev_inv = ev[4], ev_u = ev[5], ev_join = ev[6];
         if (tiled()) {
             rc = launch_fill_f32(B->amaxL[buf], static_cast<int64_t>(outer) * ntiles, 0.0f, s);
             if (rc == HPLAI_OK) rc = launch_fill_f32(B->amaxU[buf], static_cast<int64_t>(outer) * ntiles, 0.0f, s);
             if (rc) return rc;
         }
-        if (mb > 0) {
+        if (fork) {
             HPLAI_HIP(hipEventRecord(ev_fork, s));
             HPLAI_HIP(hipStreamWaitEvent(q, ev_fork, 0));
         }
@@ -406,7 +409,7 @@ struct LU {
             // t - 1 (the wait refers to the record of the previous iteration)
             if (mb > 0) {
                 if (t > 0) {
-                    HPLAI_HIP(hipStreamWaitEvent(q, ev_u, 0));
+                    if (fork) HPLAI_HIP(hipStreamWaitEvent(q, ev_u, 0));
                     if (mid) rc = gemm(buf, 0, split, rb0, c, mb, rb0 - c, q, kBulk);
                     if (rc == HPLAI_OK && nsl > 0) rc = gemm(buf, base, nsl, rb0, c, mb, b, q, kBulk);
                 }
@@ -427,8 +430,10 @@ struct LU {
             if (rc) break;
             // bulk: L := A U^-1 and quantization of the rows below
             if (mb > 0) {
-                HPLAI_HIP(hipEventRecord(ev_inv, s));
-                HPLAI_HIP(hipStreamWaitEvent(q, ev_inv, 0));
+                if (fork) {
+                    HPLAI_HIP(hipEventRecord(ev_inv, s));
+                    HPLAI_HIP(hipStreamWaitEvent(q, ev_inv, 0));
+                }
                 rc = timed(HPLAI_PHASE_TRSM_L, static_cast<double>(mb) * bd * bd, q, [&] {
                     return launch_trsm_l(mb, b, dinv(c), a(rb0, c), lda, aml(buf, t, rb0), b, q);
                 });
@@ -465,9 +470,9 @@ struct LU {
                                            amu(buf, t, c + b), eu(buf, t, c + b), s, packed);
                 });
             if (rc) break;
-            if (mb > 0) HPLAI_HIP(hipEventRecord(ev_u, s));
+            if (fork) HPLAI_HIP(hipEventRecord(ev_u, s));
         }
-        if (mb > 0) {
+        if (fork) {
             HPLAI_HIP(hipEventRecord(ev_join, q));
             if (join) HPLAI_HIP(hipStreamWaitEvent(s, ev_join, 0));
         }
@@ -505,9 +510,21 @@ struct LU {
         return rc;
     }
 
+    // Whether to overlap a step's trailing update with the next panel: the hops
+    // between streams, 10-25 us each on the chain from panel to panel, cost
+    // more than an update of less than about 100 us hides (C at 3 TB/s or the
+    // products at 600 TF/s).  LU alone, overlapped always / below 100 us not:
+    // 1200 blocks of 60 1347 / 924 us, 2400 2716 / 1846, 7200 9886 / 8328 (200
+    // us: 8543), 8192 blocks of 512 (e4m3) 5488 / 5205 (200 us: 5308).
+    bool overlap_pays(int64_t rest, int sw) const
+    {
+        const double m2 = static_cast<double>(rest) * static_cast<double>(rest);
+        return m2 * std::max(8.0 / 3e12, 2.0 * sw * b / 600e12) > 100e-6;
+    }
+
     // lookahead 0: update, then the next panel, all on the main stream.
     // lookahead 1: the next outer panel's columns first, then the panel on the
-    // side stream while the main stream updates the rest.
+    // side stream while the main stream updates the rest, where that pays.
     // lookahead 2: as 1, and the rest is updated in two parts: the rows of
     // the next block row first, so that the side stream computes that block
     // row (after the panel chain) while the main stream updates the rows below.
@@ -534,7 +551,7 @@ struct LU {
             const int64_t c1 = r0;
             const int sw1 = rest > 0 ? static_cast<int>(std::min<int64_t>(outer, rest / b)) : 0;
             if (rest > 0) {
-                if (lookahead) {
+                if (lookahead && overlap_pays(rest, sw)) {
                     // next panel's columns first, then hand them to the side stream
                     const int64_t B1 = static_cast<int64_t>(sw1) * b;
                     const bool ahead = lookahead > 1 && rest > B1;
@@ -556,7 +573,7 @@ struct LU {
                         HPLAI_HIP(hipEventRecord(ev[1], side));
                         rc = gemm(buf, 0, sw, r0 + B1, r0 + B1, rest - B1, rest - B1, main, kTrailing);
                         if (rc) break;
-                        HPLAI_HIP(hipStreamWaitEvent(main, ev[6], 0));   // the panel's bulk stream
+                        if (sw1 > 1) HPLAI_HIP(hipStreamWaitEvent(main, ev[6], 0));   // the panel's bulk stream
                         row_done = true;
                     } else {
                         HPLAI_HIP(hipEventRecord(ev[1], side));

@@ -248,7 +248,8 @@ typedef struct hplai_params {
     uint64_t seed;       /* 42 in the reference (main.cpp:174)                     */
     int      fmt;        /* HPLAI_FMT_*                                            */
     int      outer;      /* panels per trailing update (1 = reference schedule)    */
-    int      lookahead;  /* 1: factor panel k+1 on a second stream during update k;
+    int      lookahead;  /* 1: factor panel k+1 on a second stream during update k
+                            (updates too short to hide a panel stay on one stream);
                             2: also block row k+1 there (the update's rows of block
                             row k+1 first, then the rows below)                      */
     int      lazy;       /* 1: -d lazy initialisation (lazy_init.hpp:92-227): the trailing
