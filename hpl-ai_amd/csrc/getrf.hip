@@ -5,11 +5,12 @@
 // sub-blocks of 128 columns; per sub-block three kinds of work, all FP32 on
 // v_mfma_f32_32x32x2_f32:
 //   lu_update_kernel  workgroup 0 takes the 128 x 128 diagonal sub-block: its
-//                     update with the sub-block before it, its LU and the
-//                     inverses of both triangles, all in LDS; the other
-//                     workgroups update the rest of the trailing matrix;
+//                     LU and the inverses of both triangles, all in LDS; the
+//                     other workgroups update the rest of the trailing matrix;
 //   lu_strip_kernel   L21 := A21 U11^-1 and U12 := L11^-1 A12 as products
-//                     with those inverses, 32 rows or columns per workgroup.
+//                     with those inverses, 32 rows or columns per workgroup,
+//                     and in more workgroups, which form the strips that they
+//                     need again, the update of the next diagonal sub-block.
 // The inverses of the whole block grow by a sub-block q at a time,
 //   Linv(q, J) = -Linv_qq T,   T  = sum_K L(q, K) Linv(K, J)
 //   Uinv(J, q) = -T' Uinv_qq,  T' = sum_K Uinv(J, K) U(K, q)     (K < q),
@@ -20,14 +21,16 @@
 // two products, all pairs of a size at once.
 //
 // What bounds it: the chain of 32 x 32 LUs, inverses and strips (17k clocks a
-// link, one or two waves working) and, between sub-blocks, a launch and the
-// 128^3 update of the next diagonal sub-block.  One workgroup for the whole
-// 512 block spent half its time on trailing updates through a single CU's
-// path to the L2, and the inverses were two more kernels after it: 511 + 73
-// us, now 215 us with the inverses (b = 512, alone); b = 60: 94 -> 15 us; n =
-// 1000: 645 us with v_readlane steps, 423 us as here.  Joining by one
-// workgroup per 32 columns took 39 us a size (product by product, each behind
-// its loads) after the factorization.
+// link, one or two waves working) and, between sub-blocks, two launches (9 us
+// with the strips and the next sub-block's update).  One workgroup for the
+// whole 512 block spent half its time on trailing updates through a single
+// CU's path to the L2, and the inverses were two more kernels after it: 511 +
+// 73 us, now 172 us with the inverses and 157 without (b = 512, alone); b = 60:
+// 94 -> 14 us; n = 1000: 645 us with v_readlane steps, 329 us as here.  The
+// next sub-block's update in the workgroup that factors it took 11 us of each
+// sub-block (its operands, 192 KB, again through one CU): 198 us at b = 512.
+// Joining the inverses by one workgroup per 32 columns took 39 us a size
+// (product by product, each behind its loads) after the factorization.
 #include <cstddef>
 #include <type_traits>
 #include <utility>
@@ -407,6 +410,12 @@ __device__ __forceinline__ void write_inverse_row(const float *V, float *tri, in
 __device__ __forceinline__ int left_pos(int r, int c) { return (r + 32 * (c & 1)) * 16 + (c >> 1); }
 __device__ __forceinline__ int right_pos(int r, int c) { return (c + 32 * (r & 1)) * 16 + (r >> 1); }
 
+// Copies of A21's and A12's blocks (I, J) beside a diagonal sub-block, [32 k +
+// row or column], in the slots of the other triangle that the inverses leave
+// free: the strips overwrite the blocks in A while others still need them.
+__device__ __forceinline__ float *copy_l(float *tri, int nb, int I, int J) { return tri_block_u(tri, nb, I, J); }
+__device__ __forceinline__ float *copy_u(float *tri, int nb, int I, int J) { return tri_block_l(tri, nb, I, J); }
+
 __device__ __forceinline__ void packed16(const float *blk, int lane, float (&v)[16])
 {
     const float4 *p = reinterpret_cast<const float4 *>(blk) + lane * 4;
@@ -523,9 +532,9 @@ __device__ __forceinline__ void tri_fin(int nb, float *tri, int J, int R0, int R
     }
 }
 
-// Sub-block k0 of the n x n block A.  FACTOR: the update with sub-block
-// k0 - 128 (when there is one), LU, inverses; the next workgroups update the
-// rest of the trailing matrix and the last form the first products of the
+// Sub-block k0 of the n x n block A.  FACTOR: LU, inverses; the next workgroups
+// update the rest of the trailing matrix with sub-block k0 - 128 (when there is
+// one) and copy the blocks beside the diagonal one, and the last form the first products of the
 // whole block's inverses.  Without FACTOR: A is already factored and
 // workgroup q inverts the triangles of sub-block q.
 template <bool FACTOR>
@@ -544,23 +553,24 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
 
     if (FACTOR && blockIdx.x > 0) {
         // ---- a 128 x 64 tile of the trailing matrix, one 32 x 32 block per wave ----
-        const int rest = n - k0, ct = (rest + 63) / 64;
-        // tiles in row-major order without the two of the diagonal sub-block
-        const int two = ct < 2 ? ct : 2;
-        const int t = static_cast<int>(blockIdx.x) - 1 + two;
-        if (t >= (rest + 127) / 128 * ct) {
+        const int rest = n - k0, ct = (rest + 63) / 64, rt = (rest + 127) / 128;
+        // tiles in row-major order without the two of the diagonal sub-block;
+        // of the first sub-block only the four that are copied
+        const int two = ct < 2 ? ct : 2, z = static_cast<int>(blockIdx.x) - 1;
+        const int t = p0 >= 0 ? z + two : z < 2 ? ct + z : z;
+        if (p0 >= 0 && t >= rt * ct) {
             static_assert(offsetof(LuLds, V) == sizeof(float) * kLuNB * kLuS && (1024 - kLuNB) * 33 <= 2 * kLuNB * kLuS,
                           "the strip of an inverse spans S and V");
-            const int z = t - (rest + 127) / 128 * ct, q0 = k0 / 32;
-            if (z & 1)
-                tri_mid<true>(n, nb, A, lda, tri, z >> 1, q0, q0, nb < q0 + 4 ? nb : q0 + 4, S);
+            const int y = t - rt * ct, q0 = k0 / 32;
+            if (y & 1)
+                tri_mid<true>(n, nb, A, lda, tri, y >> 1, q0, q0, nb < q0 + 4 ? nb : q0 + 4, S);
             else
-                tri_mid<false>(n, nb, A, lda, tri, z >> 1, q0, q0, nb < q0 + 4 ? nb : q0 + 4, S);
+                tri_mid<false>(n, nb, A, lda, tri, y >> 1, q0, q0, nb < q0 + 4 ? nb : q0 + 4, S);
             return;
         }
         const int r0 = (t / ct) * 128 + (wave & 3) * 32, c0 = (t % ct) * 64, cw = c0 + (wave >> 2) * 32;
         // U12 (128 x 64) through LDS: its MFMA operand walks along columns
-        {
+        if (p0 >= 0) {
             float v[16];
 #pragma unroll
             for (int u = 0; u < 16; ++u) {
@@ -572,31 +582,45 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
         }
         __syncthreads();
         if (r0 >= rest || cw >= rest) return;
-        const float *lp = A + static_cast<int64_t>(p0 + lh) * lda + k0 + min(r0 + l32, rest - 1);
         float cv[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e)
             cv[e] = Ak[static_cast<int64_t>(min(cw + l32, rest - 1)) * lda + min(r0 + acc_row(e, lh), rest - 1)];
-        floatx16g_t acc = zero16();
-        float av[64];
+        if (p0 >= 0) {
+            const float *lp = A + static_cast<int64_t>(p0 + lh) * lda + k0 + min(r0 + l32, rest - 1);
+            floatx16g_t acc = zero16();
+            float av[64];
 #pragma unroll
-        for (int kk = 0; kk < 64; ++kk) av[kk] = lp[static_cast<int64_t>(2 * kk) * lda];
+            for (int kk = 0; kk < 64; ++kk) av[kk] = lp[static_cast<int64_t>(2 * kk) * lda];
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-            float bv[16];
+            for (int h = 0; h < 4; ++h) {
+                float bv[16];
 #pragma unroll
-            for (int kk = 0; kk < 16; ++kk) bv[kk] = S[(cw - c0 + l32) * kLuS + 32 * h + 2 * kk + lh];
+                for (int kk = 0; kk < 16; ++kk) bv[kk] = S[(cw - c0 + l32) * kLuS + 32 * h + 2 * kk + lh];
 #pragma unroll
-            for (int kk = 0; kk < 16; ++kk)
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[16 * h + kk], bv[kk], acc, 0, 0, 0);
-        }
-        if (cw + l32 < rest) {
-            float *cp = Ak + static_cast<int64_t>(cw + l32) * lda + r0;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int r = acc_row(e, lh);
-                if (r0 + r < rest) cp[r] = cv[e] - acc[e];
+                for (int kk = 0; kk < 16; ++kk)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[16 * h + kk], bv[kk], acc, 0, 0, 0);
             }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) cv[e] -= acc[e];
+            if (cw + l32 < rest) {
+                float *cp = Ak + static_cast<int64_t>(cw + l32) * lda + r0;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int r = acc_row(e, lh);
+                    if (r0 + r < rest) cp[r] = cv[e];
+                }
+            }
+        }
+        // the blocks right of and below the diagonal sub-block once more, k by k
+        if (r0 >= kLuNB && r0 < 2 * kLuNB && cw < kLuNB) {
+            float4 *o = reinterpret_cast<float4 *>(copy_l(tri, nb, (k0 + r0) / 32, (k0 + cw) / 32) + l32 * 32 + 4 * lh);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) o[2 * q] = float4{cv[4 * q], cv[4 * q + 1], cv[4 * q + 2], cv[4 * q + 3]};
+        } else if (r0 < kLuNB && cw >= kLuNB && cw < 2 * kLuNB) {
+            float *o = copy_u(tri, nb, (k0 + r0) / 32, (k0 + cw) / 32);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[acc_row(e, lh) * 32 + l32] = cv[e];
         }
         return;
     }
@@ -604,23 +628,18 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
     // ---- the diagonal sub-block, padded to 128 with the identity ----
     const int w = n - k0 < kLuNB ? n - k0 : kLuNB;
     const int steps = (w + 31) / 32, q0 = k0 / 32;
-    const bool pre = FACTOR && k0 > 0;   // the update with the sub-block before: U12 of it goes to V
     {
         const int r = tid & 127;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            float v[16], u[16];
+            float v[16];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int c = (tid >> 7) + 4 * (16 * h + e);
-                v[e] = Ak[static_cast<int64_t>(min(c, w - 1)) * lda + min(r, w - 1)];
-                if (pre) u[e] = A[static_cast<int64_t>(k0 + min(c, w - 1)) * lda + p0 + r];
-            }
+            for (int e = 0; e < 16; ++e)
+                v[e] = Ak[static_cast<int64_t>(min((tid >> 7) + 4 * (16 * h + e), w - 1)) * lda + min(r, w - 1)];
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int c = (tid >> 7) + 4 * (16 * h + e);
                 S[c * kLuS + r] = (r < w && c < w) ? v[e] : (r == c ? 1.0f : 0.0f);
-                if (pre) V[c * kLuS + r] = u[e];
             }
         }
     }
@@ -646,35 +665,6 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
         return;
     }
 
-    // blocks (rb, cb .. cb + nc - 1) of S take L21 U12 of the sub-block before (K = 128)
-    auto pre_update = [&](int ln, int rb, int cb, int nc) {
-        const int l32 = ln & 31, lh = ln >> 5;
-        const float *lp = A + static_cast<int64_t>(p0 + lh) * lda + k0 + min(32 * rb + l32, w - 1);
-        float av[4][16];
-#pragma unroll
-        for (int h = 0; h < 4; ++h)
-#pragma unroll
-            for (int kk = 0; kk < 16; ++kk) av[h][kk] = lp[static_cast<int64_t>(32 * h + 2 * kk) * lda];
-        for (int y = 0; y < nc; ++y, ++cb) {
-            floatx16g_t acc = zero16();
-            float bv[2][16];
-            auto read = [&](int h) {
-#pragma unroll
-                for (int kk = 0; kk < 16; ++kk) bv[h & 1][kk] = V[(32 * cb + l32) * kLuS + 32 * h + 2 * kk + lh];
-            };
-            read(0);
-#pragma unroll
-            for (int h = 0; h < 4; ++h) {
-                if (h < 3) read(h + 1);
-                acc = mfma16(av[h], bv[h & 1], acc);
-            }
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int r = 32 * rb + acc_row(e, lh), c = 32 * cb + l32;
-                if (r < w && c < w) S[c * kLuS + r] -= acc[e];
-            }
-        }
-    };
     // 32 x 32 block (r0, cc) of S takes the strips of the 32 columns at c0
     auto update = [&](int ln, int c0, int r0, int cc) {
         const int l32 = ln & 31, lh = ln >> 5;
@@ -705,9 +695,6 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
             if (q > 0) {
                 update(ln, c0 - 32, c0, c0);
                 wave_lds_sync();
-            } else if (pre) {
-                pre_update(ln, 0, 0, 1);
-                wave_lds_sync();
             }
             const int z = lu32(S, c0, ln);
             if (bad == 0 && z != 0) bad = k0 + c0 + z;
@@ -717,10 +704,6 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
             write_inverse_row(V, tri, nb, q0, q - 1, wave - 1, sides, ln);
             if (tri != nullptr && t < 2 * q)
                 T = t & 1 ? inverse_row_product<true>(S, V, q, t >> 1, ln) : inverse_row_product<false>(S, V, q, t >> 1, ln);
-        } else if (pre) {
-            // row block wave % 4: columns 0, 1 or 2, 3; wave 4 also wave 0's second
-            const int cb = wave < 4 ? 0 : wave == 4 ? 1 : 2, ce = wave < 4 ? 2 : 4;
-            if ((wave & 3) < steps) pre_update(ln, wave & 3, cb, (ce < steps ? ce : steps) - cb);
         }
         __syncthreads();
         if (wave == 0) {
@@ -777,20 +760,95 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
     if (tid == 0 && info != nullptr && (k0 == 0 || (bad != 0 && *info == 0))) *info = bad;
 }
 
+// Block (r, c) of the next diagonal sub-block -= L21(r, :) U12(:, c), with its
+// strips formed from the copies: wave J forms L21(r, J)^T and U12(J, c), whose
+// accumulators are the operands of their product (k = acc_row either way).
+__device__ __forceinline__ void next_diagonal(int n, int nb, int q0, int r, int c, float *A, int64_t lda, float *tri,
+                                              float *XL, float *XU)
+{
+    const int tid = threadIdx.x, lane = tid & 63, J = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, lh = lane >> 5;
+    const int R = q0 + 4 + r, C = q0 + 4 + c;
+    float il[4][16], iu[4][16];   // the inverses' blocks, clamped to the last that is used
+    float4 xl[4], xu[4];
+#pragma unroll
+    for (int K = 0; K < 4; ++K) {
+        xl[K] = reinterpret_cast<const float4 *>(copy_l(tri, nb, R, q0 + K))[tid];
+        xu[K] = reinterpret_cast<const float4 *>(copy_u(tri, nb, q0 + K, C))[tid];
+    }
+#pragma unroll
+    for (int K = 0; K < 4; ++K) {
+        packed16(tri_block_u(tri, nb, q0 + min(K, J), q0 + J), lane, il[K]);
+        packed16(tri_block_l(tri, nb, q0 + J, q0 + min(K, J)), lane, iu[K]);
+    }
+    const int64_t col = min(32 * C + l32, n - 1);
+    float d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = A[col * lda + min(32 * R + 8 * J + 4 * lh + i, n - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int K = 0; K < 4; ++K) {
+        float *x = XL + (32 * K + (tid >> 3)) * 33 + 4 * (tid & 7), *y = XU + (32 * K + (tid >> 3)) * 33 + 4 * (tid & 7);
+        x[0] = xl[K].x;
+        x[1] = xl[K].y;
+        x[2] = xl[K].z;
+        x[3] = xl[K].w;
+        y[0] = xu[K].x;
+        y[1] = xu[K].y;
+        y[2] = xu[K].z;
+        y[3] = xu[K].w;
+    }
+    __syncthreads();
+    floatx16g_t al = zero16(), au = zero16();
+#pragma unroll
+    for (int K = 0; K < 4; ++K) {
+        if (K > J) break;
+        float xv[16], yv[16];
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk) {
+            xv[kk] = XL[(32 * K + 2 * kk + lh) * 33 + l32];
+            yv[kk] = XU[(32 * K + 2 * kk + lh) * 33 + l32];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk) {
+            al = __builtin_amdgcn_mfma_f32_32x32x2f32(il[K][kk], xv[kk], al, 0, 0, 0);
+            au = __builtin_amdgcn_mfma_f32_32x32x2f32(iu[K][kk], yv[kk], au, 0, 0, 0);
+        }
+    }
+    floatx16g_t acc = zero16();
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(al[kk], au[kk], acc, 0, 0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 16; ++e) XL[(J * 16 + e) * 64 + lane] = acc[e];
+    __syncthreads();
+    // wave J: rows 8 J + 4 lh + i, the waves' sums in order
+    if (32 * C + l32 < n)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float *p = XL + (4 * J + i) * 64 + lane;
+            const int row = 32 * R + 8 * J + 4 * lh + i;
+            if (row < n) A[col * lda + row] = d[i] - (((p[0] + p[1024]) + p[2048]) + p[3072]);
+        }
+}
+
 // L21 := A21 Uinv and U12 := Linv A12 for the rows and columns past the
 // sub-block at p0 (128 wide).  A workgroup owns 32 rows of L21 (blockIdx.x <
-// strips) or 32 columns of U12; wave j computes its 32-wide block j.  The
-// workgroups past those finish the whole block's inverses of this sub-block.
-__global__ __launch_bounds__(256) void lu_strip_kernel(int n, int p0, float *__restrict__ A, int64_t lda, float *tri,
-                                                       int strips)
+// strips) or 32 columns of U12; wave j computes its 32-wide block j.  The next
+// workgroups update a block each of the next diagonal sub-block, the last ones
+// finish the whole block's inverses of this one.
+__global__ __launch_bounds__(256) void lu_strip_kernel(int n, int p0, float *A, int64_t lda, float *tri, int strips)
 {
-    __shared__ float X[kLuNB * 33];
+    __shared__ float X[kLuNB * 33], X2[kLuNB * 33];
     const int tid = threadIdx.x, lane = tid & 63, J = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
     const int nb = (n + 31) / 32, q0 = p0 / 32, k1 = p0 + kLuNB;
     if (static_cast<int>(blockIdx.x) >= 2 * strips) {
-        const int z = static_cast<int>(blockIdx.x) - 2 * strips;
-        if (z & 1)
+        const int nd = strips < 4 ? strips : 4, y = static_cast<int>(blockIdx.x) - 2 * strips, z = y - nd * nd;
+        if (z < 0)
+            next_diagonal(n, nb, q0, y % nd, y / nd, A, lda, tri, X, X2);
+        else if (z & 1)
             tri_fin<true, 4, 1>(nb, tri, z >> 1, q0, nb < q0 + 4 ? nb : q0 + 4);
         else
             tri_fin<false, 4, 1>(nb, tri, z >> 1, q0, nb < q0 + 4 ? nb : q0 + 4);
@@ -799,13 +857,23 @@ __global__ __launch_bounds__(256) void lu_strip_kernel(int n, int p0, float *__r
     const bool up = static_cast<int>(blockIdx.x) >= strips;
     const int o = k1 + 32 * (static_cast<int>(blockIdx.x) - (up ? strips : 0));   // first row / column
     const int cnt = n - o < 32 ? n - o : 32;
+    float iv[4][16];   // the inverse's blocks, clamped to the last that is used
     {
         float v[16];
+        auto inverse = [&] {
+#pragma unroll
+            for (int K = 0; K < 4; ++K) {
+                const int k = q0 + min(K, J);
+                packed16(up ? tri_block_l(tri, nb, q0 + J, k) : tri_block_u(tri, nb, k, q0 + J), lane, iv[K]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
         if (up) {
             // X[k * 33 + c]: row p0 + k, column o + c
 #pragma unroll
             for (int u = 0; u < 16; ++u)
                 v[u] = A[static_cast<int64_t>(o + min((tid >> 7) + 2 * u, cnt - 1)) * lda + p0 + (tid & 127)];
+            inverse();
 #pragma unroll
             for (int u = 0; u < 16; ++u) X[(tid & 127) * 33 + (tid >> 7) + 2 * u] = v[u];
         } else {
@@ -813,24 +881,20 @@ __global__ __launch_bounds__(256) void lu_strip_kernel(int n, int p0, float *__r
 #pragma unroll
             for (int u = 0; u < 16; ++u)
                 v[u] = A[static_cast<int64_t>(p0 + (tid >> 5) + 8 * u) * lda + o + min(tid & 31, cnt - 1)];
+            inverse();
 #pragma unroll
             for (int u = 0; u < 16; ++u) X[((tid >> 5) + 8 * u) * 33 + (tid & 31)] = v[u];
         }
     }
     __syncthreads();
     floatx16g_t acc = zero16();
-    for (int K = 0; K <= J; ++K) {
-        const float *blk = up ? tri_block_l(tri, nb, q0 + J, q0 + K) : tri_block_u(tri, nb, q0 + K, q0 + J);
-        const float4 *b4 = reinterpret_cast<const float4 *>(blk) + lane * 4;
-        const float4 t0 = b4[0], t1 = b4[1], t2 = b4[2], t3 = b4[3];
-        const float iv[16] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w,
-                              t2.x, t2.y, t2.z, t2.w, t3.x, t3.y, t3.z, t3.w};
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            const float x = X[(32 * K + 2 * kk + lh) * 33 + l32];
-            acc = up ? __builtin_amdgcn_mfma_f32_32x32x2f32(iv[kk], x, acc, 0, 0, 0)
-                     : __builtin_amdgcn_mfma_f32_32x32x2f32(x, iv[kk], acc, 0, 0, 0);
-        }
+    for (int K = 0; K < 4; ++K) {
+        if (K > J) break;
+        float xv[16];
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk) xv[kk] = X[(32 * K + 2 * kk + lh) * 33 + l32];
+        acc = up ? mfma16(iv[K], xv, acc) : mfma16(xv, iv[K], acc);
     }
     if (up) {
         if (l32 < cnt) {
@@ -889,15 +953,16 @@ int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, bool full,
     for (int k = 0; k < n; k += kLuNB) {
         const int rest = n - k;
         const int rt = (rest + 127) / 128, ct = (rest + 63) / 64;
-        const int tiles = k == 0 ? 0 : rt * ct - (ct < 2 ? ct : 2);
+        const int tiles = k == 0 ? (rest > kLuNB ? 4 : 0) : rt * ct - (ct < 2 ? ct : 2);
         // the whole block's inverses, and the last sub-block's, serve only a caller who asked for them
         const unsigned join = full ? 2 * (k / 32) : 0;
         hipLaunchKernelGGL((lu_update_kernel<true>), dim3(static_cast<unsigned>(1 + tiles) + join), dim3(kLuThreads),
                            0, s, n, k, A, lda, !full && rest <= kLuNB ? nullptr : tri, 3, info);
         HPLAI_HIP(hipGetLastError());
         const int strips = rest > kLuNB ? (rest - kLuNB + 31) / 32 : 0;
-        if (2 * strips + join > 0) {
-            hipLaunchKernelGGL(lu_strip_kernel, dim3(static_cast<unsigned>(2 * strips) + join), dim3(256), 0, s, n, k,
+        const int nd = strips < 4 ? strips : 4;
+        if (strips + join > 0) {
+            hipLaunchKernelGGL(lu_strip_kernel, dim3(static_cast<unsigned>(2 * strips + nd * nd) + join), dim3(256), 0, s, n, k,
                                A, lda, tri, strips);
             HPLAI_HIP(hipGetLastError());
         }
