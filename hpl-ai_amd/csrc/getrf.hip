@@ -380,7 +380,7 @@ __device__ __forceinline__ void inverse_row_finish(float *V, int q, int b, int l
 }
 
 // One wave: block t of row q of Linv (t <= q) or column q of Uinv (t - q - 1)
-// into the packed arrays, 16 consecutive floats per MFMA lane.  sides: 1
+// into the packed arrays, 16 floats per MFMA lane.  sides: 1
 // Linv, 2 Uinv, 3 both.
 __device__ __forceinline__ void write_inverse_row(const float *V, float *tri, int nb, int q0, int q, int t, int sides,
                                                   int lane)
@@ -399,16 +399,14 @@ __device__ __forceinline__ void write_inverse_row(const float *V, float *tri, in
         for (int kk = 0; kk < 16; ++kk)
             v[kk] = up ? upper_entry(v[kk], 2 * kk + lh, l32) : lower_entry(v[kk], l32, 2 * kk + lh);
     float4 *o = reinterpret_cast<float4 *>(up ? tri_block_u(tri, nb, q0 + b, q0 + q)
-                                              : tri_block_l(tri, nb, q0 + q, q0 + b)) + lane * 4;
+                                              : tri_block_l(tri, nb, q0 + q, q0 + b)) + lane;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = float4{v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]};
+    for (int e = 0; e < 4; ++e) o[e * 64] = float4{v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]};
 }
 
-// The inverses' packed blocks hold 16 floats per lane: a left operand's (L
-// side: row lane % 32, column 2 kk + lane / 32) or a right operand's (U side:
-// row 2 kk + lane / 32, column lane % 32).  Position of an entry:
-__device__ __forceinline__ int left_pos(int r, int c) { return (r + 32 * (c & 1)) * 16 + (c >> 1); }
-__device__ __forceinline__ int right_pos(int r, int c) { return (c + 32 * (r & 1)) * 16 + (r >> 1); }
+// Position of entry (r, c) in a packed block, as a left or a right operand
+__device__ __forceinline__ int left_pos(int r, int c) { return tri_pos(r + 32 * (c & 1), c >> 1); }
+__device__ __forceinline__ int right_pos(int r, int c) { return tri_pos(c + 32 * (r & 1), r >> 1); }
 
 // Copies of A21's and A12's blocks (I, J) beside a diagonal sub-block, [32 k +
 // row or column], in the slots of the other triangle that the inverses leave
@@ -418,10 +416,10 @@ __device__ __forceinline__ float *copy_u(float *tri, int nb, int I, int J) { ret
 
 __device__ __forceinline__ void packed16(const float *blk, int lane, float (&v)[16])
 {
-    const float4 *p = reinterpret_cast<const float4 *>(blk) + lane * 4;
+    const float4 *p = reinterpret_cast<const float4 *>(blk) + lane;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        const float4 q = p[e];
+        const float4 q = p[e * 64];
         v[4 * e] = q.x;
         v[4 * e + 1] = q.y;
         v[4 * e + 2] = q.z;
@@ -442,7 +440,7 @@ __device__ __forceinline__ void tri_mid(int n, int nb, const float *A, int64_t l
     const int l32 = lane & 31, lh = lane >> 5, X = R + (wave & 3), half = wave >> 2;
 #pragma unroll 4
     for (int e = tid; e < (K1 - J) * 1024; e += kLuThreads) {
-        const int K = J + (e >> 10), ln = (e >> 4) & 63, kk = e & 15;
+        const int K = J + (e >> 10), ln = (e >> 2) & 63, kk = ((e >> 8) & 3) * 4 + (e & 3);   // as tri_pos
         const float *blk = UP ? tri_block_u(tri, nb, J, K) : tri_block_l(tri, nb, K, J);
         W[(32 * (K - J) + (ln & 31)) * 33 + 2 * kk + (ln >> 5)] = blk[e & 1023];
     }

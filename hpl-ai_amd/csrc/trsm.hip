@@ -6,9 +6,12 @@
 // output blocks are independent, so the eight waves run without barriers
 // between them instead of walking a substitution chain.  Products run on
 // v_mfma_f32_32x32x2_f32 (FP32 inputs and accumulation); the inverse is read
-// from global memory (L2-resident) in MFMA operand order, 16 consecutive
-// floats per lane.  b need not be a multiple of 32: the strip is padded with
-// zeros and the packed inverse with the identity.
+// from global memory (L2-resident) in MFMA operand order (tri_pos).  b need not
+// be a multiple of 32: the strip is padded with zeros and the packed inverse
+// with the identity.  What bounds it: the FP32 matrix cores, 14.5 us of the 20
+// a strip takes at b = 512 with two workgroups per CU.  (One workgroup per CU
+// that walks over its strips and loads ahead, in the same or in two more waves,
+// was slower: 512 x 98304 L 253 -> 274 us, U 237 -> 262.)
 // MFMA layout: A operand lane -> (row lane % 32, k 2 kk + lane / 32), B
 // operand lane -> (k 2 kk + lane / 32, column lane % 32); output acc[4 q + r]
 // is row 8 q + 4 (lane / 32) + r, column lane % 32.
@@ -132,21 +135,21 @@ template <bool INV_LEFT>
 __device__ __forceinline__ floatx16t_t tri_product(const float *X, const float *__restrict__ inv, int last, int lane)
 {
     const int l32 = lane & 31, lh = lane >> 5;
-    const float4 *ip = reinterpret_cast<const float4 *>(inv) + lane * 4;
+    const float4 *ip = reinterpret_cast<const float4 *>(inv) + lane;
     floatx16t_t acc;
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
     // the inverse two blocks ahead (L2 latency under a full GPU)
     float4 cur[4], nxt[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) cur[e] = ip[e];
+    for (int e = 0; e < 4; ++e) cur[e] = ip[e * 64];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) nxt[e] = ip[min(1, last) * 256 + e];
+    for (int e = 0; e < 4; ++e) nxt[e] = ip[min(1, last) * 256 + e * 64];
     for (int kb = 0; kb <= last; ++kb) {
         float4 nx2[4];
         const float4 *in = ip + min(kb + 2, last) * 256;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) nx2[e] = in[e];
+        for (int e = 0; e < 4; ++e) nx2[e] = in[e * 64];
         float xv[16];
 #pragma unroll
         for (int kk = 0; kk < 16; ++kk) xv[kk] = X[(32 * kb + 2 * kk + lh) * kXS + l32];
@@ -167,6 +170,58 @@ __device__ __forceinline__ floatx16t_t tri_product(const float *X, const float *
         }
     }
     return acc;
+}
+
+// The same for a strip of 16 rows or columns, on v_mfma_f32_16x16x4_f32: a
+// lane's K of step t is 2 (8 (lane / 32) + t) + (lane / 16) % 2, which makes its
+// part of a packed block whole quarters.  acc[h]: the
+// block's columns (INV_LEFT: rows) 16 h .. + 15; acc[h][r] is row 4 (lane / 16)
+// + r, column lane % 16.
+typedef float floatx4t_t __attribute__((ext_vector_type(4)));
+constexpr int kStrip16 = 16, kXS16 = kStrip16 + 1;
+
+template <bool INV_LEFT>
+__device__ __forceinline__ void tri_product16(const float *X, const float *__restrict__ inv, int last, int lane,
+                                              floatx4t_t (&acc)[2])
+{
+    const int l16 = lane & 15, odd = (lane >> 4) & 1, hi = lane >> 5;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) acc[h] = floatx4t_t{0.0f, 0.0f, 0.0f, 0.0f};
+    // packed lane 32 odd + 16 h + l16, quarters 2 hi and 2 hi + 1
+    const float4 *ip = reinterpret_cast<const float4 *>(inv) + 128 * hi + 32 * odd + l16;
+    float4 cur[4], nxt[4];
+    auto fetch = [&](float4 (&v)[4], int kb) {
+        const float4 *p = ip + min(kb, last) * 256;
+        v[0] = p[0];
+        v[1] = p[64];
+        v[2] = p[16];
+        v[3] = p[80];
+    };
+    fetch(cur, 0);
+    fetch(nxt, 1);
+    for (int kb = 0; kb <= last; ++kb) {
+        float4 nx2[4];
+        fetch(nx2, kb + 2);
+        float xv[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) xv[t] = X[(32 * kb + 2 * (8 * hi + t) + odd) * kXS16 + l16];
+        asm volatile("" ::: "memory");   // as in tri_product
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float4 &q = cur[2 * h + (t >> 2)];
+                const float iv = (t & 3) == 0 ? q.x : (t & 3) == 1 ? q.y : (t & 3) == 2 ? q.z : q.w;
+                acc[h] = INV_LEFT ? __builtin_amdgcn_mfma_f32_16x16x4f32(iv, xv[t], acc[h], 0, 0, 0)
+                                  : __builtin_amdgcn_mfma_f32_16x16x4f32(xv[t], iv, acc[h], 0, 0, 0);
+            }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            cur[e] = nxt[e];
+            nxt[e] = nx2[e];
+        }
+    }
 }
 
 // L(m x b) := L Ukk^-1 (update_left_panels, panel_trf.hpp:143-157) as
@@ -258,6 +313,103 @@ __global__ __launch_bounds__(kTriThreads) void trsm_u_tri_kernel(int b, int64_t 
     tile_max_reduce(amax, j0 / tb, vmax, true);
 }
 
+// Panels that 32-wide strips leave CUs idle with: 16-wide ones, b <= 512, any
+// alignment.  A strip's time is its products on one CU, the same for one strip
+// as for a device full, so half the strip is half the time: 512 x 2048, L 27 ->
+// 22 us, U 25 -> 19 us (the inverse's 0.5 MB through one CU are the other part).
+__global__ __launch_bounds__(kTriThreads) void trsm_l_tri16_kernel(int64_t m, int b, const float *__restrict__ tri,
+                                                                   float *__restrict__ L, int64_t ldl,
+                                                                   float *__restrict__ amax, int tb)
+{
+    __shared__ float X[512 * kXS16];   // X[c * kXS16 + r]: column c, row i0 + r
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kStrip16;
+    const int nr = m - i0 < kStrip16 ? static_cast<int>(m - i0) : kStrip16;
+    const int nb = (b + 31) / 32;
+    {
+        const int r = tid & 15;
+        const float *src = L + i0 + min(r, nr - 1);
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = src[static_cast<int64_t>(min((tid >> 4) + 32 * u, b - 1)) * ldl];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int c = (tid >> 4) + 32 * u;
+            if (u < nb) X[c * kXS16 + r] = (r < nr && c < b) ? v[u] : 0.0f;
+        }
+    }
+    __syncthreads();
+    float vmax = 0.0f;
+    for (int p = 0; p < nb; ++p) {
+        if (tri_snake(p) != wave) continue;
+        const int jb = nb - 1 - p;
+        floatx4t_t acc[2];
+        tri_product16<false>(X, tri_block_u(tri, nb, 0, jb), jb, lane, acc);
+        const int r0 = 4 * (lane >> 4);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int c = 32 * jb + 16 * h + (lane & 15);
+            if (c >= b) continue;
+            float *dst = L + static_cast<int64_t>(c) * ldl + i0 + r0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (r0 + r < nr) {
+                    dst[r] = acc[h][r];
+                    vmax = fmaxf(vmax, fabsf(acc[h][r]));
+                }
+        }
+    }
+    tile_max_reduce(amax, i0 / tb, vmax, true);
+}
+
+__global__ __launch_bounds__(kTriThreads) void trsm_u_tri16_kernel(int b, int64_t n, const float *__restrict__ tri,
+                                                                   float *__restrict__ U, int64_t ldu,
+                                                                   float *__restrict__ amax, int tb)
+{
+    __shared__ float X[512 * kXS16];   // X[r * kXS16 + c]: row r of column j0 + c
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t j0 = static_cast<int64_t>(blockIdx.x) * kStrip16;
+    const int nc = n - j0 < kStrip16 ? static_cast<int>(n - j0) : kStrip16;
+    const int nb = (b + 31) / 32;
+    {   // wave w: columns 2 w, 2 w + 1, 64 rows an access
+        float v[2][8];
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                v[q][u] = U[(j0 + min(2 * wave + q, nc - 1)) * ldu + min(64 * u + lane, b - 1)];
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int c = 2 * wave + q, r = 64 * u + lane;
+                if (r < nb * 32) X[r * kXS16 + c] = (c < nc && r < b) ? v[q][u] : 0.0f;
+            }
+    }
+    __syncthreads();
+    float vmax = 0.0f;
+    for (int p = 0; p < nb; ++p) {
+        if (tri_snake(p) != wave) continue;
+        const int rb = nb - 1 - p;
+        floatx4t_t acc[2];
+        tri_product16<true>(X, tri_block_l(tri, nb, rb, 0), rb, lane, acc);
+        const int c = lane & 15;
+        if (c >= nc) continue;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int r0 = 32 * rb + 16 * h + 4 * (lane >> 4);
+            float *dst = U + (j0 + c) * ldu + r0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (r0 + r < b) {
+                    dst[r] = acc[h][r];
+                    vmax = fmaxf(vmax, fabsf(acc[h][r]));
+                }
+        }
+    }
+    tile_max_reduce(amax, j0 / tb, vmax, true);
+}
+
 // x_out := Tinv x_in for one factored diagonal block (the IR's diagonal-block
 // solve as a product with the stored inverse): Linv (UPPER = false, the unit
 // lower solve) or Uinv (UPPER = true).  Workgroup I computes rows
@@ -279,11 +431,11 @@ __global__ __launch_bounds__(256) void tri_trsv_kernel(int b, const float *__res
     if (!UPPER) {
         for (int J = p; J <= I; J += 8) {
             const float *blk = tri_block_l(tri, nb, I, J);
-            const float4 *ev = reinterpret_cast<const float4 *>(blk + rho * 16);          // gamma = 2 kk
-            const float4 *od = reinterpret_cast<const float4 *>(blk + (rho + 32) * 16);   // gamma = 2 kk + 1
+            const float4 *ev = reinterpret_cast<const float4 *>(blk) + rho;   // gamma = 2 kk
+            const float4 *od = ev + 32;                                       // gamma = 2 kk + 1
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float4 a = ev[e], c = od[e];
+                const float4 a = ev[e * 64], c = od[e * 64];
                 const double *xj = xs + 32 * J + 8 * e;
                 acc = fma(static_cast<double>(a.x), xj[0], acc);
                 acc = fma(static_cast<double>(c.x), xj[1], acc);
@@ -297,10 +449,10 @@ __global__ __launch_bounds__(256) void tri_trsv_kernel(int b, const float *__res
         }
     } else {
         for (int J = I + p; J < nb; J += 8) {
-            const float *blk = tri_block_u(tri, nb, I, J) + 32 * 16 * (rho & 1) + (rho >> 1);
+            const float *blk = tri_block_u(tri, nb, I, J) + tri_pos(32 * (rho & 1), rho >> 1);
             const double *xj = xs + 32 * J;
 #pragma unroll
-            for (int g = 0; g < 32; ++g) acc = fma(static_cast<double>(blk[g * 16]), xj[g], acc);
+            for (int g = 0; g < 32; ++g) acc = fma(static_cast<double>(blk[g * 4]), xj[g], acc);
         }
     }
     part[p][rho] = acc;
@@ -338,11 +490,21 @@ static int tri_variant(int b, const float *P, int64_t ld)
     return b > 512 ? 2 : (b % 64 == 0 && aligned16(P, ld)) ? 0 : 1;
 }
 
+// Largest number of 32-wide strips that is split into 16-wide ones instead:
+// half the CUs.  Both measured at b = 512, L / U: 4001 wide 36 / 25 against 29 /
+// 20 us, 6000 wide 31 / 26 against 37 / 31.
+constexpr int64_t kStrips16 = 128;
+
 int launch_trsm_l(int64_t m, int b, const float *tri, float *L, int64_t ldl, float *amax, int tb, hipStream_t s)
 {
     if (m <= 0 || b <= 0) return HPLAI_OK;
     HPLAI_CHECK(amax == nullptr || tb % kStrip == 0, "trsm: tile %d not a multiple of %d", tb, kStrip);
     const dim3 g(static_cast<unsigned>(ceil_div(m, kStrip))), th(kTriThreads);
+    if (b <= 512 && g.x <= kStrips16) {
+        hipLaunchKernelGGL(trsm_l_tri16_kernel, dim3(static_cast<unsigned>(ceil_div(m, kStrip16))), th, 0, s, m, b, tri, L, ldl, amax, tb);
+        HPLAI_HIP(hipGetLastError());
+        return HPLAI_OK;
+    }
     switch (tri_variant(b, L, ldl)) {
     case 0: hipLaunchKernelGGL((trsm_l_tri_kernel<512, true>), g, th, 0, s, m, b, tri, L, ldl, amax, tb); break;
     case 1: hipLaunchKernelGGL((trsm_l_tri_kernel<512, false>), g, th, 0, s, m, b, tri, L, ldl, amax, tb); break;
@@ -357,6 +519,11 @@ int launch_trsm_u(int b, int64_t n, const float *tri, float *U, int64_t ldu, flo
     if (n <= 0 || b <= 0) return HPLAI_OK;
     HPLAI_CHECK(amax == nullptr || tb % kStrip == 0, "trsm: tile %d not a multiple of %d", tb, kStrip);
     const dim3 g(static_cast<unsigned>(ceil_div(n, kStrip))), th(kTriThreads);
+    if (b <= 512 && g.x <= kStrips16) {
+        hipLaunchKernelGGL(trsm_u_tri16_kernel, dim3(static_cast<unsigned>(ceil_div(n, kStrip16))), th, 0, s, b, n, tri, U, ldu, amax, tb);
+        HPLAI_HIP(hipGetLastError());
+        return HPLAI_OK;
+    }
     switch (tri_variant(b, U, ldu)) {
     case 0: hipLaunchKernelGGL((trsm_u_tri_kernel<512, true>), g, th, 0, s, b, n, tri, U, ldu, amax, tb); break;
     case 1: hipLaunchKernelGGL((trsm_u_tri_kernel<512, false>), g, th, 0, s, b, n, tri, U, ldu, amax, tb); break;

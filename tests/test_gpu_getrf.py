@@ -124,3 +124,25 @@ def test_inverses_grown_with_the_factorization(ctx, oracle, b):
     U = F[:b, :b].triu()
     for got, want in ((F[b:, :b] @ U, A[b:, :b]), (L @ F[:b, b:], A[:b, b:])):
         assert ((got - want).abs().max() / want.abs().max()).item() < 2e-5
+
+
+@pytest.mark.parametrize("b", [1, 31, 60, 128, 200, 512])
+@pytest.mark.parametrize("m", [1, 15, 17, 4096, 4097])
+def test_trsm_strip_widths(ctx, oracle, b, m):
+    """16-wide strips up to 4096, 32-wide ones past it, unaligned panels;
+    L U11 = A21 and L11 U = A12 in FP64, within the 2e-5 above."""
+    import torch
+    D, ref = _factored(oracle, b, 4 * b + 4)
+    F = _dev(ref)                                             # F[col, row]
+    g = torch.Generator(device="cuda").manual_seed(m)
+    L = torch.rand(b, m + 1, generator=g, device="cuda") - 0.5
+    U = torch.rand(m, b + 1, generator=g, device="cuda") - 0.5
+    L0, U0 = L.clone(), U.clone()
+    ctx.trsm_lpanel(m, b, F, b, L, m + 1)
+    ctx.trsm_upanel(b, m, F, b, U, b + 1)
+    assert torch.equal(L[:, m:], L0[:, m:]) and torch.equal(U[:, b:], U0[:, b:])
+    T = F.t().double()
+    low = T.tril(-1) + torch.eye(b, device="cuda", dtype=torch.float64)
+    for got, want in ((L[:, :m].t().double() @ T.triu(), L0[:, :m].t().double()),
+                      (low @ U[:, :b].t().double(), U0[:, :b].t().double())):
+        assert ((got - want).abs().max() / want.abs().max()).item() < 2e-5
