@@ -223,10 +223,11 @@ typedef struct hplai_batch_stats {
 int hplai_batch_create(hplai_ctx ctx, int count, const int32_t *n, const int32_t *nrhs,
                        const uint64_t *seed, hplai_batch *out);
 int hplai_batch_destroy(hplai_batch b);
-/* panel width (16, 32 or 64) per size bucket */
+/* panel width (16, 32 or 64) per size bucket; 16 runs as 32, whose wider FP32
+ * panel is the more accurate one */
 int hplai_batch_set_nb(hplai_batch b, const int32_t nb[4]);
 int hplai_batch_get_nb(hplai_batch b, int32_t nb[4]);
-/* times every feasible panel width on up to 2 systems per CU of each bucket
+/* times the panel widths 32 and 64 on up to 2 systems per CU of each bucket
  * and keeps the fastest; nb_out (may be NULL) receives the table */
 int hplai_batch_autotune(hplai_batch b, int maxit, int32_t nb_out[4]);
 /* mode 0: one persistent launch; 1: the same launch captured once in a
