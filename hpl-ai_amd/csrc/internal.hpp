@@ -155,7 +155,7 @@ int launch_schur_c16(int fmt, int64_t m, int64_t n, int nslices, int kslice, con
                      const int32_t *eU, int64_t ldeu, int tb, uint16_t *C, int64_t ldc, float cscale,
                      int num_cu, hipStream_t s, bool packed = false);
 // true when launch_schur runs the streamed 256 x 256 kernel for this shape
-bool schur_large_tiles(int fmt, int64_t m, int64_t n, int tb, int num_cu);
+bool schur_large_tiles(int fmt, int64_t m, int64_t n, int64_t K, int tb, int num_cu);
 
 // the reference's column-major gemmschur seam (gemmschur.hip): both operands
 // staged K-contiguous with K padded to 64 in `scratch`

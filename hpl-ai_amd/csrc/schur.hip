@@ -753,17 +753,26 @@ static int schur_launch(int64_t m, int64_t n, int nslices, int kslice, const voi
     return HPLAI_OK;
 }
 
-// The streamed 256 x 256 kernel for updates with at least two tiles per CU;
-// the 128 x 128 kernel for thin ones.  With per-tile exponents every
-// workgroup tile must lie inside one tb x tb tile, so the large tiles also
-// need tb % 256 == 0.  The per-tile FP16 form rescales its accumulators
-// between slices and keeps the 128 x 128 tile.
-bool schur_large_tiles(int fmt, int64_t m, int64_t n, int tb, int num_cu)
+// The streamed 256 x 256 kernel for updates with at least two tiles per CU; the
+// 128 x 128 one, which starts faster and runs two workgroups per CU, for thin
+// ones.  Between, the 256 x 256 kernel takes an update whose K is 2 KB or more
+// (at 1 KB it is 0.9 times as fast, at 2 KB 1.02, 4 KB 1.15, 8 KB 1.23) unless
+// the last round of its tiles is emptier than that of the 128 x 128 kernel's:
+// T tiles fill ceil(T / CUs) rounds, their 4 T quarters ceil(2 T / CUs) rounds of
+// two per CU, so the rounds are as full when the latter is even (28672 x 512 x
+// 4096 FP16, 224 tiles: 162 -> 132 us; 36864, 288 tiles: 236 against 233; LU of
+// 61440 with blocks of 512, outer 16: FP16 201.8 -> 195.6 ms, FP8 122.3 -> 119.3).
+// With per-tile exponents every workgroup tile must lie inside one tb x tb tile,
+// so the large tiles also need tb % 256 == 0.  The per-tile FP16 form rescales
+// its accumulators between slices and keeps the 128 x 128 tile.
+bool schur_large_tiles(int fmt, int64_t m, int64_t n, int64_t K, int tb, int num_cu)
 {
     if (fmt == HPLAI_FMT_F16_TILE) return false;
     if (fmt == HPLAI_FMT_E4M3 && tb % kDmaTile != 0) return false;
     if (num_cu <= 0) num_cu = 256;
-    return ceil_div(m, kDmaTile) * ceil_div(n, kDmaTile) >= 2 * num_cu;
+    const int64_t tiles = ceil_div(m, kDmaTile) * ceil_div(n, kDmaTile);
+    if (tiles >= 2 * num_cu) return true;
+    return K * (fmt == HPLAI_FMT_E4M3 ? 1 : 2) >= 2048 && ceil_div(2 * tiles, num_cu) % 2 == 0;
 }
 
 template <int FMT, bool PACKED>
@@ -774,7 +783,7 @@ static int schur_dispatch(int64_t m, int64_t n, int nslices, int kslice, const v
 {
     if constexpr (FMT != HPLAI_FMT_F16_TILE) {
         // the FP16 trailing storage takes the streamed kernel only for whole 256 x 256 tiles
-        if (schur_large_tiles(FMT, m, n, tb, num_cu) && (!c16 || (m % kDmaTile == 0 && n % kDmaTile == 0)) &&
+        if (schur_large_tiles(FMT, m, n, static_cast<int64_t>(nslices) * kslice, tb, num_cu) && (!c16 || (m % kDmaTile == 0 && n % kDmaTile == 0)) &&
             (FMT != HPLAI_FMT_E4M3 || nslices <= kDmaMaxSlices))
             return schur_dma_launch<FMT, PACKED>(m, n, nslices, kslice, Lq, ldl, eL, ldel, Uq, ldu, eU, ldeu,
                                          tb, C, ldc, s, c16, cscale);

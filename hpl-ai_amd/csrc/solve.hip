@@ -327,7 +327,7 @@ struct LU {
             const double K = static_cast<double>(nsl) * b;
             timer->begin(s, 2.0 * static_cast<double>(m) * static_cast<double>(nn) * K,
                          static_cast<double>(m + nn) * K * es + 4.0 * static_cast<double>(m) * nn,
-                         schur_large_tiles(fmt, m, nn, b, num_cu), false, cls);
+                         schur_large_tiles(fmt, m, nn, static_cast<int64_t>(nsl) * kpad, b, num_cu), false, cls);
             const int rc = launch_schur_c16(fmt, m, nn, nsl, kpad, lq(buf, row0, t0), ldq, el(buf, t0, row0),
                                             ntiles, uq(buf, col0, t0), ldq, eu(buf, t0, col0), ntiles, b,
                                             B->P + col0 * n + row0, n, pscale, num_cu, s, packed);
@@ -337,7 +337,7 @@ struct LU {
         const double K = static_cast<double>(nsl) * b;
         timer->begin(s, 2.0 * static_cast<double>(m) * static_cast<double>(nn) * K,
                      static_cast<double>(m + nn) * K * es + 8.0 * static_cast<double>(m) * nn,
-                     schur_large_tiles(fmt, m, nn, b, num_cu), in_block, cls);
+                     schur_large_tiles(fmt, m, nn, static_cast<int64_t>(nsl) * kpad, b, num_cu), in_block, cls);
         const int rc = launch_schur(fmt, m, nn, nsl, kpad, lq(buf, row0, t0), ldq, el(buf, t0, row0),
                                     ntiles, uq(buf, col0, t0), ldq, eu(buf, t0, col0), ntiles, b,
                                     a(row0, col0), lda, num_cu, s, packed);

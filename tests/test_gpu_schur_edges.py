@@ -27,3 +27,28 @@ def test_schur_f16_edges(ctx, m, n):
     inside = np.zeros(C.shape, dtype=bool)
     inside[1:n + 1, 2:m + 2] = True
     assert np.array_equal(got[~inside], C[~inside])
+
+
+@pytest.mark.parametrize("fmt", [0, 2])
+@pytest.mark.parametrize("m,n", [(8192, 1024), (8391, 1000), (8448, 1024), (16384, 1024), (16640, 1024)])
+def test_schur_tile_choice(ctx, fmt, m, n):
+    """128, 132 and 256, 260 tiles of 256 x 256: the edges of the range below two
+    tiles per CU that the larger tile takes, with ragged edges, K of 2 KB.  An
+    FP32 sum of K products in any order is within K 2^-24 of the sum of their
+    magnitudes."""
+    import torch
+    K = 1024 if fmt == 0 else 2048
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    dt = torch.float16 if fmt == 0 else torch.float8_e4m3fn
+    L = (torch.rand(m, K, generator=g, device="cuda") - 0.5).to(dt)
+    U = (torch.rand(n, K, generator=g, device="cuda") - 0.5).to(dt)
+    ns = K // 512
+    eL = torch.zeros(ns, (m + 511) // 512, dtype=torch.int32, device="cuda")
+    eU = torch.zeros(ns, (n + 511) // 512, dtype=torch.int32, device="cuda")
+    C = torch.rand(n, m, generator=g, device="cuda")
+    C0 = C.clone()
+    ctx.schur_update(fmt, m, n, ns, 512, L, K, eL, eL.shape[1], U, K, eU, eU.shape[1], 512, C, m)
+    Ld, Ud = L.double(), U.double()
+    want = C0.double() - Ud @ Ld.t()
+    bound = (Ud.abs() @ Ld.abs().t() + C0.double()) * (K * 2.0 ** -24)
+    assert ((C.double() - want).abs() <= bound).all()
