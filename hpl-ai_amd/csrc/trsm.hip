@@ -207,15 +207,30 @@ __device__ __forceinline__ void tri_product16(const float *X, const float *__res
         for (int t = 0; t < 8; ++t) xv[t] = X[(32 * kb + 2 * (8 * hi + t) + odd) * kXS16 + l16];
         asm volatile("" ::: "memory");   // as in tri_product
         __builtin_amdgcn_sched_barrier(0);
+        auto step = [&](int h, int t, bool on) {
+            const float4 &q = cur[2 * h + (t >> 2)];
+            const float e = (t & 3) == 0 ? q.x : (t & 3) == 1 ? q.y : (t & 3) == 2 ? q.z : q.w;
+            const float iv = on ? e : 0.0f;
+            acc[h] = INV_LEFT ? __builtin_amdgcn_mfma_f32_16x16x4f32(iv, xv[t], acc[h], 0, 0, 0)
+                              : __builtin_amdgcn_mfma_f32_16x16x4f32(xv[t], iv, acc[h], 0, 0, 0);
+        };
+        if (kb < last) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
+            for (int t = 0; t < 8; ++t)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const float4 &q = cur[2 * h + (t >> 2)];
-                const float iv = (t & 3) == 0 ? q.x : (t & 3) == 1 ? q.y : (t & 3) == 2 ? q.z : q.w;
-                acc[h] = INV_LEFT ? __builtin_amdgcn_mfma_f32_16x16x4f32(iv, xv[t], acc[h], 0, 0, 0)
-                                  : __builtin_amdgcn_mfma_f32_16x16x4f32(xv[t], iv, acc[h], 0, 0, 0);
+                for (int h = 0; h < 2; ++h) step(h, t, true);
+        } else {
+            // the triangle's own block: K in ascending order, so that the
+            // diagonal's term, the largest, is the last one added (in the order
+            // above the result has twice the error: 4.8e-8 against 2.3e-8)
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                step(0, t, true);
+                step(1, t, hi == 0);
             }
+#pragma unroll
+            for (int t = 0; t < 8; ++t) step(1, t, hi == 1);
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             cur[e] = nxt[e];

@@ -146,3 +146,23 @@ def test_trsm_strip_widths(ctx, oracle, b, m):
     for got, want in ((L[:, :m].t().double() @ T.triu(), L0[:, :m].t().double()),
                       (low @ U[:, :b].t().double(), U0[:, :b].t().double())):
         assert ((got - want).abs().max() / want.abs().max()).item() < 2e-5
+
+
+@pytest.mark.parametrize("b", [60, 128, 512])
+def test_narrow_strips_add_the_diagonal_last(ctx, oracle, b):
+    """U12 of a diagonally dominant block is A12 minus sums of small products:
+    one rounding of the large term (rms 2^-25 of it) when the unit diagonal's
+    term is the last one added, and two or more otherwise.  Both strip widths
+    on the same columns, each within 1.5 of that one rounding."""
+    import torch
+    D, ref = _factored(oracle, b, 4 * b + 4)
+    F = _dev(ref)
+    g = torch.Generator(device="cuda").manual_seed(b)
+    wide = torch.rand(6000, b, generator=g, device="cuda") - 0.5      # U[col, row]
+    narrow = wide[:2000].clone()
+    low = F.t().double().tril(-1) + torch.eye(b, device="cuda", dtype=torch.float64)
+    want = torch.linalg.solve_triangular(low, wide.t().double(), upper=False, unitriangular=True).t()
+    ctx.trsm_upanel(b, 6000, F, b, wide, b)
+    ctx.trsm_upanel(b, 2000, F, b, narrow, b)
+    for got, w in ((wide, want), (narrow, want[:2000])):
+        assert ((got.double() - w).norm() / w.norm()).item() < 1.5 * 2.0 ** -25
