@@ -29,9 +29,18 @@ __global__ __launch_bounds__(256) void seam_pack_a_kernel(int64_t n, int64_t k, 
     const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kSeamTile;
     const int64_t k0 = static_cast<int64_t>(blockIdx.y) * kSeamTile;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    for (int kk = ty; kk < kSeamTile; kk += 4) {
-        const int64_t gk = k0 + kk, gi = i0 + tx;
-        t[kk][tx] = (gk < k && gi < n) ? a[gk * lda + gi] : uint16_t(0);
+    {   // all loads in flight; past an edge they repeat the last entry
+        const int64_t gi = i0 + tx;
+        const uint16_t *row = a + (gi < n ? gi : n - 1);
+        uint16_t v[kSeamTile / 4];
+#pragma unroll
+        for (int u = 0; u < kSeamTile / 4; ++u) {
+            const int64_t gk = k0 + ty + 4 * u;
+            v[u] = row[(gk < k ? gk : k - 1) * lda];
+        }
+#pragma unroll
+        for (int u = 0; u < kSeamTile / 4; ++u)
+            t[ty + 4 * u][tx] = (gi < n && k0 + ty + 4 * u < k) ? v[u] : uint16_t(0);
     }
     __syncthreads();
     for (int r = ty; r < kSeamTile; r += 4) {

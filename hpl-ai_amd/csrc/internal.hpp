@@ -129,8 +129,17 @@ int64_t tri_floats(int b);
 // the same inverses of a block that is already factored; sides: 1 L, 2 U, 3 both
 int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, hipStream_t s);
 // tri: the packed inverses of the factored diagonal block
-int launch_trsm_l(int64_t m, int b, const float *tri, float *L, int64_t ldl, float *amax, int tb, hipStream_t s);
-int launch_trsm_u(int b, int64_t n, const float *tri, float *U, int64_t ldu, float *amax, int tb, hipStream_t s);
+// half: where the results also go as FP16 (dst NULL: nowhere), operand rows ld
+// bytes apart, each slice padded to whole 32-blocks; packed as for launch_quantize
+struct TrsmHalf {
+    void *dst = nullptr;
+    int64_t ld = 0;
+    int packed = 0;
+};
+int launch_trsm_l(int64_t m, int b, const float *tri, float *L, int64_t ldl, float *amax, int tb, hipStream_t s,
+                  TrsmHalf half = {});
+int launch_trsm_u(int b, int64_t n, const float *tri, float *U, int64_t ldu, float *amax, int tb, hipStream_t s,
+                  TrsmHalf half = {});
 // amax: per-tile maxima of |src|; NULL: the exponents are in exps (FMT_F16: 0).
 // packed: dst in the panel-packed layout (packed_off), rows a multiple of 256 from its base.
 int launch_quantize(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds,

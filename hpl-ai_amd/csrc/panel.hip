@@ -108,9 +108,17 @@ __global__ __launch_bounds__(256) void quant_l_kernel(int64_t m, int64_t k, int 
     const int64_t r0 = static_cast<int64_t>(blockIdx.x) * 64;
     const int64_t c0 = static_cast<int64_t>(blockIdx.y) * 64;
     const int tx = threadIdx.x % 64, ty = threadIdx.x / 64;
-    for (int c = ty; c < 64; c += 4) {
-        const int64_t gr = r0 + tx, gc = c0 + c;
-        T[c][tx] = (gr < m && gc < k) ? src[gc * lds + gr] : 0.0f;
+    {
+        const int64_t gr = r0 + tx;
+        const float *col = src + (gr < m ? gr : m - 1);
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int64_t gc = c0 + ty + 4 * u;
+            v[u] = col[(gc < k ? gc : k - 1) * lds];
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) T[ty + 4 * u][tx] = (gr < m && c0 + ty + 4 * u < k) ? v[u] : 0.0f;
     }
     __syncthreads();
     // each thread writes 4 consecutive k values of one row (16 rows x 16 chunks per pass)

@@ -313,6 +313,14 @@ struct LU {
     }
     float *dinv(int64_t c) const { return B->inv + (c / b) * tri_floats(b); }
 
+    // Plain FP16 panels are converted by the TRSM that forms them: no pass over
+    // the panel and no launch of its own.  The profile keeps the phases apart.
+    bool half_fused() const { return fmt == HPLAI_FMT_F16 && !timer->on; }
+    TrsmHalf half(uint8_t *q) const
+    {
+        return half_fused() ? TrsmHalf{q, ldq * es, packed ? 1 : 0} : TrsmHalf{};
+    }
+
     // cls: kTrailing, an outer step's update of blocks that have not joined a
     // panel yet (to the FP16 trailing storage when it is on); kBulk, the rows
     // below the outer block taking the earlier panels of the block; kInBlock,
@@ -435,9 +443,10 @@ struct LU {
                     HPLAI_HIP(hipStreamWaitEvent(q, ev_inv, 0));
                 }
                 rc = timed(HPLAI_PHASE_TRSM_L, static_cast<double>(mb) * bd * bd, q, [&] {
-                    return launch_trsm_l(mb, b, dinv(c), a(rb0, c), lda, aml(buf, t, rb0), b, q);
+                    return launch_trsm_l(mb, b, dinv(c), a(rb0, c), lda, aml(buf, t, rb0), b, q,
+                                         half(lq(buf, rb0, t)));
                 });
-                if (rc == HPLAI_OK)
+                if (rc == HPLAI_OK && !half_fused())
                     rc = timed(HPLAI_PHASE_CONV_L, static_cast<double>(mb) * bd, q, [&] {
                         return launch_quantize(fmt, 0, mb, b, b, a(rb0, c), lda, lq(buf, rb0, t), ldq,
                                                aml(buf, t, rb0), el(buf, t, rb0), q, packed);
@@ -448,9 +457,10 @@ struct LU {
             const int64_t mrow = rb0 - c - b;
             if (mrow <= 0) continue;
             rc = timed(HPLAI_PHASE_TRSM_L, static_cast<double>(mrow) * bd * bd, s, [&] {
-                return launch_trsm_l(mrow, b, dinv(c), a(c + b, c), lda, aml(buf, t, c + b), b, s);
+                return launch_trsm_l(mrow, b, dinv(c), a(c + b, c), lda, aml(buf, t, c + b), b, s,
+                                     half(lq(buf, c + b, t)));
             });
-            if (rc == HPLAI_OK)
+            if (rc == HPLAI_OK && !half_fused())
                 rc = timed(HPLAI_PHASE_CONV_L, static_cast<double>(mrow) * bd, s, [&] {
                     return launch_quantize(fmt, 0, mrow, b, b, a(c + b, c), lda, lq(buf, c + b, t), ldq,
                                            aml(buf, t, c + b), el(buf, t, c + b), s, packed);
@@ -462,9 +472,10 @@ struct LU {
             if (rc == HPLAI_OK) rc = lazy_init(c, c + b, b, ncols, s);
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_TRSM_R, static_cast<double>(ncols) * bd * bd, s, [&] {
-                    return launch_trsm_u(b, ncols, dinv(c), a(c, c + b), lda, amu(buf, t, c + b), b, s);
+                    return launch_trsm_u(b, ncols, dinv(c), a(c, c + b), lda, amu(buf, t, c + b), b, s,
+                                         half(uq(buf, c + b, t)));
                 });
-            if (rc == HPLAI_OK)
+            if (rc == HPLAI_OK && !half_fused())
                 rc = timed(HPLAI_PHASE_CONV_R, static_cast<double>(ncols) * bd, s, [&] {
                     return launch_quantize(fmt, 1, ncols, b, b, a(c, c + b), lda, uq(buf, c + b, t), ldq,
                                            amu(buf, t, c + b), eu(buf, t, c + b), s, packed);
@@ -499,9 +510,10 @@ struct LU {
             if (rc == HPLAI_OK) rc = lazy_init(c, col0, b, ncols, s);   // block row right of the outer panel
             if (rc == HPLAI_OK)
                 rc = timed(HPLAI_PHASE_TRSM_R, static_cast<double>(ncols) * bd * bd, s, [&] {
-                    return launch_trsm_u(b, ncols, dinv(c), a(c, col0), lda, amu(buf, t, col0), b, s);
+                    return launch_trsm_u(b, ncols, dinv(c), a(c, col0), lda, amu(buf, t, col0), b, s,
+                                         half(uq(buf, col0, t)));
                 });
-            if (rc == HPLAI_OK)
+            if (rc == HPLAI_OK && !half_fused())
                 rc = timed(HPLAI_PHASE_CONV_R, static_cast<double>(ncols) * bd, s, [&] {
                     return launch_quantize(fmt, 1, ncols, b, b, a(c, col0), lda, uq(buf, col0, t), ldq,
                                            amu(buf, t, col0), eu(buf, t, col0), s, packed);

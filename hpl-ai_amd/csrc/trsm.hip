@@ -239,13 +239,47 @@ __device__ __forceinline__ void tri_product16(const float *X, const float *__res
     }
 }
 
+// The FP16 copies of a panel's results for the Schur update (the quantizer's
+// plain FP16 form, the same bits), straight from the accumulators instead of a
+// pass over the panel (7 + 3 of the 47 us of a panel of 1140 x 60): operand
+// row i (a row of L, a column of U), K along the bytes.  Columns past b are the
+// padding's zeros.
+__device__ __forceinline__ uint8_t *half_at(const TrsmHalf &o, int64_t i, int kbyte)
+{
+    return static_cast<uint8_t *>(o.dst) + (o.packed ? packed_off(i, kbyte, o.ld) : i * o.ld + kbyte);
+}
+// Four consecutive rows (v) of one column per lane, columns along the lanes:
+// neighbouring lanes swap, the even one then holds both columns of rows 0 and 1,
+// the odd one of rows 2 and 3.
+__device__ __forceinline__ void store_half_rows(const TrsmHalf &o, int64_t i0, int left, int k, int lane, const float (&v)[4])
+{
+    const bool odd = lane & 1;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const float give = odd ? v[r] : v[r + 2], keep = odd ? v[r + 2] : v[r];
+        const float got = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(give), 0xB1, 0xF, 0xF, true));
+        const uint32_t w = f32_to_f16_bits(odd ? got : keep) |
+                           (static_cast<uint32_t>(f32_to_f16_bits(odd ? keep : got)) << 16);
+        const int row = odd ? r + 2 : r;
+        if (row < left) *reinterpret_cast<uint32_t *>(half_at(o, i0 + row, 2 * (k & ~1))) = w;
+    }
+}
+// Four consecutive K of one column of U
+__device__ __forceinline__ void store_half_ks(const TrsmHalf &o, int64_t j, int k, const float (&v)[4])
+{
+    uint2 w;
+    w.x = f32_to_f16_bits(v[0]) | (static_cast<uint32_t>(f32_to_f16_bits(v[1])) << 16);
+    w.y = f32_to_f16_bits(v[2]) | (static_cast<uint32_t>(f32_to_f16_bits(v[3])) << 16);
+    *reinterpret_cast<uint2 *>(half_at(o, j, 2 * k)) = w;
+}
+
 // L(m x b) := L Ukk^-1 (update_left_panels, panel_trf.hpp:143-157) as
 // L := L Uinv: output block jb = sum_{kb <= jb} X(:, kb) Uinv(kb, jb).
 // PMAX: the LDS strip's height; VEC: aligned16, b a multiple of 64, b <= 512.
 template <int PMAX, bool VEC>
 __global__ __launch_bounds__(kTriThreads) void trsm_l_tri_kernel(int64_t m, int b, const float *__restrict__ tri,
                                                                  float *__restrict__ L, int64_t ldl,
-                                                                 float *__restrict__ amax, int tb)
+                                                                 float *__restrict__ amax, int tb, TrsmHalf half)
 {
     __shared__ float X[PMAX * kXS];   // X[c * kXS + r]: column c, row i0 + r
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -264,6 +298,12 @@ __global__ __launch_bounds__(kTriThreads) void trsm_l_tri_kernel(int64_t m, int 
         const int jb = nb - 1 - p;
         const floatx16t_t acc = tri_product<false>(X, tri_block_u(tri, nb, 0, jb), jb, lane);
         const int c = 32 * jb + l32;
+        if (half.dst != nullptr)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float o[4] = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+                store_half_rows(half, i0 + 8 * q + 4 * lh, nr - (8 * q + 4 * lh), c, lane, o);
+            }
         float *dst = L + static_cast<int64_t>(c) * ldl + i0 + 4 * lh;
         if (VEC && nr == kStrip) {
 #pragma unroll
@@ -291,7 +331,7 @@ __global__ __launch_bounds__(kTriThreads) void trsm_l_tri_kernel(int64_t m, int 
 template <int PMAX, bool VEC>
 __global__ __launch_bounds__(kTriThreads) void trsm_u_tri_kernel(int b, int64_t n, const float *__restrict__ tri,
                                                                  float *__restrict__ U, int64_t ldu,
-                                                                 float *__restrict__ amax, int tb)
+                                                                 float *__restrict__ amax, int tb, TrsmHalf half)
 {
     __shared__ float X[PMAX * kXS];   // X[r * kXS + c]: row r of column j0 + c
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -310,6 +350,12 @@ __global__ __launch_bounds__(kTriThreads) void trsm_u_tri_kernel(int b, int64_t 
         const int rb = nb - 1 - p;
         const floatx16t_t acc = tri_product<true>(X, tri_block_l(tri, nb, rb, 0), rb, lane);
         if (l32 >= nc) continue;
+        if (half.dst != nullptr)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float o[4] = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+                store_half_ks(half, j0 + l32, 32 * rb + 8 * q + 4 * lh, o);
+            }
         float *dst = U + (j0 + l32) * ldu + 32 * rb + 4 * lh;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -334,7 +380,7 @@ __global__ __launch_bounds__(kTriThreads) void trsm_u_tri_kernel(int b, int64_t 
 // 22 us, U 25 -> 19 us (the inverse's 0.5 MB through one CU are the other part).
 __global__ __launch_bounds__(kTriThreads) void trsm_l_tri16_kernel(int64_t m, int b, const float *__restrict__ tri,
                                                                    float *__restrict__ L, int64_t ldl,
-                                                                   float *__restrict__ amax, int tb)
+                                                                   float *__restrict__ amax, int tb, TrsmHalf half)
 {
     __shared__ float X[512 * kXS16];   // X[c * kXS16 + r]: column c, row i0 + r
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -364,6 +410,10 @@ __global__ __launch_bounds__(kTriThreads) void trsm_l_tri16_kernel(int64_t m, in
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int c = 32 * jb + 16 * h + (lane & 15);
+            if (half.dst != nullptr) {
+                const float o[4] = {acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
+                store_half_rows(half, i0 + r0, nr - r0, c, lane, o);
+            }
             if (c >= b) continue;
             float *dst = L + static_cast<int64_t>(c) * ldl + i0 + r0;
 #pragma unroll
@@ -379,7 +429,7 @@ __global__ __launch_bounds__(kTriThreads) void trsm_l_tri16_kernel(int64_t m, in
 
 __global__ __launch_bounds__(kTriThreads) void trsm_u_tri16_kernel(int b, int64_t n, const float *__restrict__ tri,
                                                                    float *__restrict__ U, int64_t ldu,
-                                                                   float *__restrict__ amax, int tb)
+                                                                   float *__restrict__ amax, int tb, TrsmHalf half)
 {
     __shared__ float X[512 * kXS16];   // X[r * kXS16 + c]: row r of column j0 + c
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -413,6 +463,10 @@ __global__ __launch_bounds__(kTriThreads) void trsm_u_tri16_kernel(int b, int64_
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int r0 = 32 * rb + 16 * h + 4 * (lane >> 4);
+            if (half.dst != nullptr) {
+                const float o[4] = {acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
+                store_half_ks(half, j0 + c, r0, o);
+            }
             float *dst = U + (j0 + c) * ldu + r0;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -510,39 +564,41 @@ static int tri_variant(int b, const float *P, int64_t ld)
 // 20 us, 6000 wide 31 / 26 against 37 / 31.
 constexpr int64_t kStrips16 = 128;
 
-int launch_trsm_l(int64_t m, int b, const float *tri, float *L, int64_t ldl, float *amax, int tb, hipStream_t s)
+int launch_trsm_l(int64_t m, int b, const float *tri, float *L, int64_t ldl, float *amax, int tb, hipStream_t s,
+                  TrsmHalf half)
 {
     if (m <= 0 || b <= 0) return HPLAI_OK;
     HPLAI_CHECK(amax == nullptr || tb % kStrip == 0, "trsm: tile %d not a multiple of %d", tb, kStrip);
     const dim3 g(static_cast<unsigned>(ceil_div(m, kStrip))), th(kTriThreads);
     if (b <= 512 && g.x <= kStrips16) {
-        hipLaunchKernelGGL(trsm_l_tri16_kernel, dim3(static_cast<unsigned>(ceil_div(m, kStrip16))), th, 0, s, m, b, tri, L, ldl, amax, tb);
+        hipLaunchKernelGGL(trsm_l_tri16_kernel, dim3(static_cast<unsigned>(ceil_div(m, kStrip16))), th, 0, s, m, b, tri, L, ldl, amax, tb, half);
         HPLAI_HIP(hipGetLastError());
         return HPLAI_OK;
     }
     switch (tri_variant(b, L, ldl)) {
-    case 0: hipLaunchKernelGGL((trsm_l_tri_kernel<512, true>), g, th, 0, s, m, b, tri, L, ldl, amax, tb); break;
-    case 1: hipLaunchKernelGGL((trsm_l_tri_kernel<512, false>), g, th, 0, s, m, b, tri, L, ldl, amax, tb); break;
-    default: hipLaunchKernelGGL((trsm_l_tri_kernel<1024, false>), g, th, 0, s, m, b, tri, L, ldl, amax, tb); break;
+    case 0: hipLaunchKernelGGL((trsm_l_tri_kernel<512, true>), g, th, 0, s, m, b, tri, L, ldl, amax, tb, half); break;
+    case 1: hipLaunchKernelGGL((trsm_l_tri_kernel<512, false>), g, th, 0, s, m, b, tri, L, ldl, amax, tb, half); break;
+    default: hipLaunchKernelGGL((trsm_l_tri_kernel<1024, false>), g, th, 0, s, m, b, tri, L, ldl, amax, tb, half); break;
     }
     HPLAI_HIP(hipGetLastError());
     return HPLAI_OK;
 }
 
-int launch_trsm_u(int b, int64_t n, const float *tri, float *U, int64_t ldu, float *amax, int tb, hipStream_t s)
+int launch_trsm_u(int b, int64_t n, const float *tri, float *U, int64_t ldu, float *amax, int tb, hipStream_t s,
+                  TrsmHalf half)
 {
     if (n <= 0 || b <= 0) return HPLAI_OK;
     HPLAI_CHECK(amax == nullptr || tb % kStrip == 0, "trsm: tile %d not a multiple of %d", tb, kStrip);
     const dim3 g(static_cast<unsigned>(ceil_div(n, kStrip))), th(kTriThreads);
     if (b <= 512 && g.x <= kStrips16) {
-        hipLaunchKernelGGL(trsm_u_tri16_kernel, dim3(static_cast<unsigned>(ceil_div(n, kStrip16))), th, 0, s, b, n, tri, U, ldu, amax, tb);
+        hipLaunchKernelGGL(trsm_u_tri16_kernel, dim3(static_cast<unsigned>(ceil_div(n, kStrip16))), th, 0, s, b, n, tri, U, ldu, amax, tb, half);
         HPLAI_HIP(hipGetLastError());
         return HPLAI_OK;
     }
     switch (tri_variant(b, U, ldu)) {
-    case 0: hipLaunchKernelGGL((trsm_u_tri_kernel<512, true>), g, th, 0, s, b, n, tri, U, ldu, amax, tb); break;
-    case 1: hipLaunchKernelGGL((trsm_u_tri_kernel<512, false>), g, th, 0, s, b, n, tri, U, ldu, amax, tb); break;
-    default: hipLaunchKernelGGL((trsm_u_tri_kernel<1024, false>), g, th, 0, s, b, n, tri, U, ldu, amax, tb); break;
+    case 0: hipLaunchKernelGGL((trsm_u_tri_kernel<512, true>), g, th, 0, s, b, n, tri, U, ldu, amax, tb, half); break;
+    case 1: hipLaunchKernelGGL((trsm_u_tri_kernel<512, false>), g, th, 0, s, b, n, tri, U, ldu, amax, tb, half); break;
+    default: hipLaunchKernelGGL((trsm_u_tri_kernel<1024, false>), g, th, 0, s, b, n, tri, U, ldu, amax, tb, half); break;
     }
     HPLAI_HIP(hipGetLastError());
     return HPLAI_OK;
