@@ -126,51 +126,54 @@ int launch_otf_gemv(int64_t n, uint64_t seed, const double *d, double alpha, con
 constexpr int kTrsvMax = 512;
 
 // y(0:m) -= P(m x w) * xb(0:w), P column-major (ttgemv, panel_trsv.hpp:10-45).
-// Workgroup = 64 rows x 4 column groups; the 4 partial sums of a row are added
-// in a fixed order through LDS.  Workgroup 0 also stores xb into xcopy(0:w):
-// the solved segment goes from its scratch copy to x while the update runs.
-constexpr int kGemvRowsT = 64;
+// Workgroup = 64 rows x 16 column groups; the partial sums of a row are added
+// in a fixed order through LDS.  A thread's 32 loads are all in flight: with 4
+// groups of 128 columns, 8 loads at a time, the latencies one after the other
+// were 12 us of a 7680 x 512 update, now 7.  Workgroup 0 also stores xb into
+// xcopy(0:w): the solved segment goes from its scratch copy to x while the
+// update runs.
+constexpr int kGemvRowsT = 64, kGemvGroups = 16, kGemvCols = kTrsvMax / kGemvGroups;
 
-__global__ __launch_bounds__(256) void trsv_gemv_kernel(int64_t m, int w, const float *__restrict__ P,
-                                                        int64_t lda, const double *__restrict__ xb,
-                                                        double *__restrict__ y, double *__restrict__ xcopy)
+__global__ __launch_bounds__(kGemvRowsT * kGemvGroups) void trsv_gemv_kernel(
+    int64_t m, int w, const float *__restrict__ P, int64_t lda, const double *__restrict__ xb, double *__restrict__ y,
+    double *__restrict__ xcopy)
 {
     __shared__ double xs[kTrsvMax];
-    __shared__ double part[4][kGemvRowsT];
-    for (int c = threadIdx.x; c < w; c += 256) {
+    __shared__ double part[kGemvGroups][kGemvRowsT];
+    const int lr = threadIdx.x % kGemvRowsT, g = __builtin_amdgcn_readfirstlane(threadIdx.x / kGemvRowsT);
+    const int64_t r = static_cast<int64_t>(blockIdx.x) * kGemvRowsT + lr;
+    const int cw = (w + kGemvGroups - 1) / kGemvGroups, c0 = g * cw;
+    const float *pr = P + (r < m ? r : m - 1);
+    float v[kGemvCols];
+#pragma unroll
+    for (int q = 0; q < kGemvCols; ++q) v[q] = pr[static_cast<int64_t>(min(c0 + q, w - 1)) * lda];
+    const int c = threadIdx.x;
+    if (c < w) {
         xs[c] = xb[c];
-        if (blockIdx.x == 0) xcopy[c] = xb[c];
+        if (blockIdx.x == 0) xcopy[c] = xs[c];
     }
     __syncthreads();
-    const int lr = threadIdx.x % kGemvRowsT, g = threadIdx.x / kGemvRowsT;
-    const int64_t r = static_cast<int64_t>(blockIdx.x) * kGemvRowsT + lr;
-    const int cw = (w + 3) / 4, c0 = g * cw, c1 = c0 + cw < w ? c0 + cw : w;
     double acc0 = 0.0, acc1 = 0.0;
-    if (r < m) {
-        const float *pr = P + r;
-        int c = c0;
-        for (; c + 7 < c1; c += 8) {
-            float v[8];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) v[q] = pr[static_cast<int64_t>(c + q) * lda];
-#pragma unroll
-            for (int q = 0; q < 8; q += 2) {
-                acc0 = fma(static_cast<double>(v[q]), xs[c + q], acc0);
-                acc1 = fma(static_cast<double>(v[q + 1]), xs[c + q + 1], acc1);
-            }
-        }
-        for (; c < c1; ++c) acc0 = fma(static_cast<double>(pr[static_cast<int64_t>(c) * lda]), xs[c], acc0);
+    for (int q = 0; q < kGemvCols; q += 2) {
+        if (q < cw && c0 + q < w) acc0 = fma(static_cast<double>(v[q]), xs[c0 + q], acc0);
+        if (q + 1 < cw && c0 + q + 1 < w) acc1 = fma(static_cast<double>(v[q + 1]), xs[c0 + q + 1], acc1);
     }
     part[g][lr] = acc0 + acc1;
     __syncthreads();
-    if (g == 0 && r < m) y[r] -= ((part[0][lr] + part[1][lr]) + part[2][lr]) + part[3][lr];
+    if (g == 0 && r < m) {
+        double sum = part[0][lr];
+#pragma unroll
+        for (int q = 1; q < kGemvGroups; ++q) sum += part[q][lr];
+        y[r] -= sum;
+    }
 }
 
 static void launch_gemv(int64_t m, int w, const float *P, int64_t lda, const double *xb, double *y, double *xcopy,
                         hipStream_t s)
 {
-    hipLaunchKernelGGL(trsv_gemv_kernel, dim3(static_cast<unsigned>(ceil_div(m, kGemvRowsT))), dim3(256), 0, s, m, w,
-                       P, lda, xb, y, xcopy);
+    hipLaunchKernelGGL(trsv_gemv_kernel, dim3(static_cast<unsigned>(ceil_div(m, kGemvRowsT))),
+                       dim3(kGemvRowsT * kGemvGroups), 0, s, m, w, P, lda, xb, y, xcopy);
 }
 
 // The block solves with the diagonal blocks applied through the inverses the
