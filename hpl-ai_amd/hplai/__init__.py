@@ -95,6 +95,8 @@ _SIGS = [
     ("hplai_norm_inf_f64", _int, [_vp, _i64, _vp, _vp, _vp]),
     ("hplai_factor_f32", _int, [_vp, _i64, _int, _int, _int, _int, _vp, _i64]),
     ("hplai_lu_solve_f64", _int, [_vp, _int, _i64, _int, _int, _vp, _i64, _vp, _i64, _vp]),
+    ("hplai_narrow_transpose_f32", _int, [_vp, _i64, _vp, _i64, _vp, _i64, _vp]),
+    ("hplai_norm_abs_f64", _int, [_vp, _int, _i64, _vp, _i64, _vp, _vp]),
     ("hplai_gemm_f64", _int, [_vp, _int, _int, _i64, _i64, _i64, _dbl, _vp, _i64, _vp, _i64, _dbl, _vp, _i64,
                               _vp]),
     ("hplai_batch_create", _int, [_vp, _int, _vp, _vp, _vp, ctypes.POINTER(_vp)]),
@@ -272,6 +274,14 @@ class Context:
         """LU of the n x n FP32 column-major device matrix A in place."""
         code = FMTS[fmt] if isinstance(fmt, str) else fmt
         check(lib().hplai_factor_f32(self.handle, n, b, code, outer, int(lookahead), ptr(A), lda))
+
+    def narrow_transpose(self, n, A, lda, F, ldf, stream=None):
+        """F (FP32, column-major) := the row-major FP64 A."""
+        check(lib().hplai_narrow_transpose_f32(self.handle, n, ptr(A), lda, ptr(F), ldf, stream_ptr(stream)))
+
+    def norm_abs(self, n, A, lda, out, trans=False, stream=None):
+        """out[0] := infinity norm of the row-major FP64 A, or of A^T with trans."""
+        check(lib().hplai_norm_abs_f64(self.handle, 1 if trans else 0, n, ptr(A), lda, ptr(out), stream_ptr(stream)))
 
     def gemm_f64(self, transa, transb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, stream=None):
         """C := alpha op(A) op(B) + beta C in FP64 (column-major, op = transpose when trans*)."""

@@ -15,8 +15,8 @@ FP64 GEMM) and dB = Lambda.  The factorization is not repeated.
 The factorization, the triangular solves and the FP64 products (the
 residuals B - A X and W - A^T Lambda and the gradient -Lambda X^T, on the
 FP64 matrix cores: `hplai_gemm_f64`) are the library's HIP kernels; torch
-does the elementwise work around them (transposed copies, x += d, the norms
-of the harness).
+does the elementwise work around them (transposed copies of X and B, x += d,
+the norms of the harness); the FP32 copy and the norm of A are kernels too.
 """
 import torch
 
@@ -63,7 +63,8 @@ def refine(hctx, A, F, bs, B, trans=False, tol=16.0, maxit=50, min_steps=0):
     n, k = B.shape
     A = A.contiguous()
     B = B.contiguous()
-    norma = (A.abs().sum(0) if trans else A.abs().sum(1)).amax()
+    norma = torch.empty((), dtype=torch.float64, device=A.device)
+    hctx.norm_abs(n, A, n, norma, trans=trans)
     Xc = B.t().contiguous()                 # column j of X at Xc[j]: leading dimension n
     hctx.lu_solve(n, k, bs, F, n, Xc, n, trans=trans)
     h = None
@@ -93,9 +94,11 @@ class LUSolve(torch.autograd.Function):
         if A.shape != (n, n) or B.shape[0] != n:
             raise ValueError("hplai.autograd.solve: A must be n x n and B n x k")
         hctx = opts["ctx"]
-        F = A.detach().t().contiguous().float()        # FP32 column-major copy, factored in place
+        Ac = A.detach().contiguous()
+        F = torch.empty((n, n), dtype=torch.float32, device=A.device)   # column-major copy, factored in place
+        hctx.narrow_transpose(n, Ac, n, F, n)
         hctx.factor(n, opts["b"], F, n, fmt=opts["fmt"], outer=opts["outer"])
-        X, steps, h = refine(hctx, A.detach(), F, opts["b"], B.detach(), False, opts["tol"],
+        X, steps, h = refine(hctx, Ac, F, opts["b"], B.detach(), False, opts["tol"],
                              opts["maxit"], opts["min_steps"])
         fctx.save_for_backward(A, X)
         fctx.F = F

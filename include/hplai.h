@@ -200,6 +200,14 @@ int hplai_gemm_f64(hplai_ctx ctx, int transa, int transb, int64_t m, int64_t n, 
                    const double *A, int64_t lda, const double *B, int64_t ldb, double beta, double *C,
                    int64_t ldc, void *stream);
 
+/* Its passes over a row-major FP64 A (n x n, rows lda apart):
+ * F(i, j) := (float)A(i, j), column-major, the copy that is factored, and
+ * *out_dev := the infinity norm of A (trans = 0) or A^T, NaN if A holds one. */
+int hplai_narrow_transpose_f32(hplai_ctx ctx, int64_t n, const double *A, int64_t lda, float *F,
+                               int64_t ldf, void *stream);
+int hplai_norm_abs_f64(hplai_ctx ctx, int trans, int64_t n, const double *A, int64_t lda,
+                       double *out_dev, void *stream);
+
 /* ---------------- batched solver (no reference counterpart) ----------------
  * Many independent HPL-AI systems (order 1..1024, 1..4 FP64 right-hand
  * sides, each built by the reference generator from its own seed: element
