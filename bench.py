@@ -217,17 +217,16 @@ def bench_batch(args):
     t = sum(r["seconds"] for r in runs) / len(runs)
     last = runs[-1]
     # roofline of batch_kernel: HBM-bound.  Algorithmic bytes per system: the
-    # LU's trailing FP32 matrix read and written at every panel step,
-    # sum_k 8 (n - k nb)^2 ~ 8 n^3 / (3 nb); the generation's FP64 and FP32
-    # copies, 12 n^2; one pass over the FP64 matrix per refinement residual,
-    # 8 n^2 per step.  The kernel is the whole timed launch.
-    bounds = (128, 256, 512)
+    # FP32 matrix written by the generation and read and written once by the
+    # LU, 12 n^2; its FP16 L written once, n^2, and read by every later block of
+    # 32 columns, sum_p 64 (n - 32 p) (n / 32 - p) ~ n^3 / 48; both triangles
+    # per correction, 4 n^2.  The kernel is the whole timed launch.
     nbytes = 0.0
     for q in range(args.batch_count):
         nq = float(n[q])
-        nb = table[sum(1 for x in bounds if n[q] >= x)]
-        trail = sum(8.0 * (nq - k * nb) ** 2 for k in range(int(n[q]) // nb + 1) if nq - k * nb > 0)
-        nbytes += trail + 12.0 * nq * nq + 8.0 * nq * nq * max(int(v) for v in steps[q][:int(nrhs[q])])
+        later = sum(64.0 * (nq - 32 * p) * ((nq - 32 * p) / 32.0) for p in range(1, int(n[q]) // 32 + 1)
+                    if nq > 32 * p)
+        nbytes += 13.0 * nq * nq + later + 4.0 * nq * nq * (max(int(v) for v in steps[q][:int(nrhs[q])]) - 1)
     achieved = nbytes / t * 1e-9
     line = {
         "metric": "batched HPL-AI solves: systems/s, one persistent hipGraph launch, 1 GPU",
