@@ -32,3 +32,26 @@ def test_otf_gemv_edges(ctx, oracle, n):
     ref = oracle.otf_gemv(n, d, -1.0, x, y, SEED)
     scale = np.max(np.abs(y)) + np.max(np.abs(d)) * 2 * np.max(np.abs(x))
     assert np.max(np.abs(gy.cpu().numpy() - ref)) / scale < 1e-13
+
+
+@pytest.mark.parametrize("n,i0,j0,m,k", [(1, 0, 0, 1, 1), (300, 0, 0, 300, 300), (700, 250, 200, 13, 71),
+                                         (700, 0, 255, 257, 65), (700, 256, 64, 256, 64), (2000, 1999, 0, 1, 2000),
+                                         (2000, 0, 1999, 2000, 1), (900, 100, 107, 600, 9)])
+@pytest.mark.parametrize("diag", [False, True])
+def test_gen_matrix_blocks(ctx, oracle, n, i0, j0, m, k, diag):
+    """Bit-exact blocks at the edges of 256 rows, 64 columns and groups of 8,
+    with and without the diagonal, nothing written outside."""
+    import torch
+    d = oracle.gen_diag(n, SEED)
+    A = torch.full((k + 1, m + 3), 7.0, device="cuda")
+    ctx.gen_matrix(n, SEED, i0, j0, m, k, torch.from_numpy(d).cuda() if diag else None, A, m + 3)
+    got = A.cpu().numpy()
+    want = oracle.gen_block(n, i0, j0, m, k, SEED)           # [col, row], diagonal entries d
+    if not diag:
+        for c in range(k):
+            r = j0 + c - i0
+            if 0 <= r < m:
+                want[c, r] = got[c, r]
+                assert abs(got[c, r]) <= 0.5
+    assert np.array_equal(got[:k, :m].view(np.uint32), want.view(np.uint32))
+    assert (got[k:] == 7.0).all() and (got[:, m:] == 7.0).all()
