@@ -212,7 +212,7 @@ int hplai_schur_update(hplai_ctx ctx, int fmt, int64_t m, int64_t n, int nslices
     HPLAI_CHECK(m >= 0 && n >= 0 && nslices >= 0 && Lq != nullptr && Uq != nullptr && C != nullptr,
                 "schur_update: bad shape/pointers");
     return launch_schur(fmt, m, n, nslices, kslice, Lq, ldl, eL, ldel, Uq, ldu, eU, ldeu, tb, C, ldc,
-                        ctx->num_cu, as_stream(stream));
+                        ctx->num_cu, as_stream(stream), false, ctx);
 }
 
 int hplai_gemmschur_f16(hplai_ctx ctx, int64_t n, int64_t m, int64_t k, const uint16_t *a, int64_t lda,

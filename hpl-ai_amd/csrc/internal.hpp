@@ -72,6 +72,7 @@ void block_free(int device, void *p, size_t bytes);
 
 // `bytes` of scratch for one call's kernels on `stream`, from construction to
 // the end of the scope that enqueues them.
+constexpr size_t kScratchMax = size_t(512) << 20;   // larger leases are allocated and freed in stream order
 class ScratchLease {
 public:
     ScratchLease(hplai_ctx ctx, hipStream_t stream, size_t bytes);
@@ -156,7 +157,7 @@ int launch_fill_f32(float *p, int64_t cnt, float v, hipStream_t s);
 int launch_schur(int fmt, int64_t m, int64_t n, int nslices, int kslice, const void *Lq,
                  int64_t ldl, const int32_t *eL, int64_t ldel, const void *Uq, int64_t ldu,
                  const int32_t *eU, int64_t ldeu, int tb, float *C, int64_t ldc, int num_cu,
-                 hipStream_t s, bool packed = false);
+                 hipStream_t s, bool packed = false, hplai_ctx ctx = nullptr);
 // The same update of the FP16 trailing storage: C := fp16(C - cscale * L U),
 // C holding cscale times the partial sums (m, n multiples of 128).
 int launch_schur_c16(int fmt, int64_t m, int64_t n, int nslices, int kslice, const void *Lq,

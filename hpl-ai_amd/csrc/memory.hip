@@ -135,7 +135,7 @@ void block_free(int device, void *p, size_t bytes)
 
 namespace {
 // per context: kept in all, and the largest buffer kept
-constexpr size_t kScratchTotal = size_t(1) << 30, kScratchMax = size_t(256) << 20;
+constexpr size_t kScratchTotal = size_t(1) << 30;
 }  // namespace
 
 ScratchLease::ScratchLease(hplai_ctx ctx, hipStream_t stream, size_t bytes) : stream_(stream)

@@ -792,8 +792,50 @@ static int schur_dispatch(int64_t m, int64_t n, int nslices, int kslice, const v
                                        C, ldc, s, c16, cscale);
 }
 
+// Operand rows to the panel-packed layout: a wave takes 8 rows, 128 bytes of
+// each at a time (whole lines), which go to two stage blocks.
+__global__ __launch_bounds__(256) void schur_repack_kernel(int64_t rows, int64_t kbytes, const uint8_t *__restrict__ src,
+                                                           int64_t ld_b, uint8_t *__restrict__ dst)
+{
+    const int lane = threadIdx.x & 63, part = lane & 7;
+    const int64_t r = (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * 8 + (lane >> 3);
+    const int64_t row = r < rows ? r : rows - 1;
+    for (int64_t k0 = static_cast<int64_t>(blockIdx.y) * 1024; k0 < kbytes && k0 < (blockIdx.y + 1) * int64_t(1024);
+         k0 += 512) {
+        intx4_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t k = k0 + 128 * u;
+            v[u] = *reinterpret_cast<const intx4_t *>(src + row * ld_b + (k < kbytes ? k : kbytes - 128) + part * 16);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (r < rows && k0 + 128 * u < kbytes)
+                *reinterpret_cast<intx4_t *>(dst + packed_off(row, k0 + 128 * u + part * 16, kbytes)) = v[u];
+    }
+}
+
+static int schur_repack(int64_t rows, int64_t kbytes, const void *src, int64_t ld_b, uint8_t *dst, hipStream_t s)
+{
+    hipLaunchKernelGGL(schur_repack_kernel,
+                       dim3(static_cast<unsigned>(ceil_div(rows, 32)), static_cast<unsigned>(ceil_div(kbytes, 1024))),
+                       dim3(256), 0, s, rows, kbytes, static_cast<const uint8_t *>(src), ld_b, dst);
+    HPLAI_HIP(hipGetLastError());
+    return HPLAI_OK;
+}
+
+// Whether a row-layout update is packed first: the pass over the operands, 2 (m
+// + n) K bytes, against 8-10 % of the update's 2 m n K operations.  Row layout /
+// packed with the pass, e4m3, K = 8192: 16384 x 16384 1856 / 1846 us, 24000 x 24000
+// 4811 / 4333, 32768 x 32768 8056 / 7339; K = 4096: 12000 x 12000 674 / 675, 24000 x
+// 24000 2772 / 2551; K <= 1024 within 3 % either way; FP16 alike.
+static bool schur_repack_pays(int64_t m, int64_t n, int64_t kbytes)
+{
+    return kbytes >= 2048 && static_cast<double>(m) * static_cast<double>(n) >= 11000.0 * static_cast<double>(m + n);
+}
+
 // Validation lives here so the C ABI and the solver share it.
-static int schur_update(int fmt, int64_t m, int64_t n, int nslices, int kslice, const void *Lq,
+static int schur_update(hplai_ctx ctx, int fmt, int64_t m, int64_t n, int nslices, int kslice, const void *Lq,
                         int64_t ldl, const int32_t *eL, int64_t ldel, const void *Uq, int64_t ldu,
                         const int32_t *eU, int64_t ldeu, int tb, void *C, int64_t ldc, int num_cu,
                         hipStream_t s, bool packed, bool c16, float cscale)
@@ -826,6 +868,24 @@ static int schur_update(int fmt, int64_t m, int64_t n, int nslices, int kslice, 
                         fmt != HPLAI_FMT_F16_TILE,
                     "schur_update: FP16 trailing storage needs whole 128 x 128 tiles, ldc %% 4 == 0, an "
                     "8-byte aligned C and the FP16 or e4m3 format");
+    const int64_t K = static_cast<int64_t>(nslices) * kslice, kbytes = K * es;
+    if (ctx != nullptr && !packed && !c16 && schur_repack_pays(m, n, kbytes) && schur_large_tiles(fmt, m, n, K, tb, num_cu) &&
+        (fmt != HPLAI_FMT_E4M3 || nslices <= kDmaMaxSlices)) {
+        const int64_t lbytes = ceil_div(m, 256) * 256 * kbytes, ubytes = ceil_div(n, 256) * 256 * kbytes;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (lbytes + ubytes <= kScratchMax && hipStreamIsCapturing(s, &cap) == hipSuccess &&
+            cap == hipStreamCaptureStatusNone) {
+            ScratchLease work(ctx, s, static_cast<size_t>(lbytes + ubytes));
+            if (work.rc == HPLAI_OK) {
+                uint8_t *Lp = work.as<uint8_t>(), *Up = Lp + lbytes;
+                int rc = schur_repack(m, kbytes, Lq, ldl * es, Lp, s);
+                if (rc == HPLAI_OK) rc = schur_repack(n, kbytes, Uq, ldu * es, Up, s);
+                if (rc) return rc;
+                return schur_update(nullptr, fmt, m, n, nslices, kslice, Lp, K, eL, ldel, Up, K, eU, ldeu, tb, C, ldc,
+                                    num_cu, s, true, false, cscale);
+            }
+        }
+    }
     switch (fmt) {
     case HPLAI_FMT_F16:
         return packed ? schur_dispatch<HPLAI_FMT_F16, true>(m, n, nslices, kslice, Lq, ldl, nullptr, 0, Uq, ldu,
@@ -849,9 +909,9 @@ static int schur_update(int fmt, int64_t m, int64_t n, int nslices, int kslice, 
 int launch_schur(int fmt, int64_t m, int64_t n, int nslices, int kslice, const void *Lq,
                  int64_t ldl, const int32_t *eL, int64_t ldel, const void *Uq, int64_t ldu,
                  const int32_t *eU, int64_t ldeu, int tb, float *C, int64_t ldc, int num_cu,
-                 hipStream_t s, bool packed)
+                 hipStream_t s, bool packed, hplai_ctx ctx)
 {
-    return schur_update(fmt, m, n, nslices, kslice, Lq, ldl, eL, ldel, Uq, ldu, eU, ldeu, tb, C, ldc, num_cu, s,
+    return schur_update(ctx, fmt, m, n, nslices, kslice, Lq, ldl, eL, ldel, Uq, ldu, eU, ldeu, tb, C, ldc, num_cu, s,
                         packed, false, 1.0f);
 }
 
@@ -860,8 +920,8 @@ int launch_schur_c16(int fmt, int64_t m, int64_t n, int nslices, int kslice, con
                      const int32_t *eU, int64_t ldeu, int tb, uint16_t *C, int64_t ldc, float cscale,
                      int num_cu, hipStream_t s, bool packed)
 {
-    return schur_update(fmt, m, n, nslices, kslice, Lq, ldl, eL, ldel, Uq, ldu, eU, ldeu, tb, C, ldc, num_cu, s,
-                        packed, true, cscale);
+    return schur_update(nullptr, fmt, m, n, nslices, kslice, Lq, ldl, eL, ldel, Uq, ldu, eU, ldeu, tb, C, ldc, num_cu,
+                        s, packed, true, cscale);
 }
 
 }  // namespace hplai

@@ -98,7 +98,10 @@ int hplai_quantize(hplai_ctx ctx, int fmt, int side, int64_t m, int64_t k, int t
  * K = nslices * kslice; FP32 accumulation, C FP32.  eL/eU are
  * [nslices][ntiles] int32 with row strides ldel/ldeu (NULL for HPLAI_FMT_F16);
  * i and j count from the first row / column of C and tb must be a multiple
- * of the kernel tile (128) when exponents are used. */
+ * of the kernel tile (128) when exponents are used.  Large updates (m n past
+ * 11000 (m + n)) pack the operands into the context's scratch for the stream
+ * first, (m + n) K elements up to 512 MiB; without it, under capture or past
+ * that they read them as they are.  The results are the same bits. */
 int hplai_schur_update(hplai_ctx ctx, int fmt, int64_t m, int64_t n, int nslices, int kslice,
                        const void *Lq, int64_t ldl, const int32_t *eL, int64_t ldel,
                        const void *Uq, int64_t ldu, const int32_t *eU, int64_t ldeu, int tb,
@@ -112,7 +115,7 @@ int hplai_schur_update(hplai_ctx ctx, int fmt, int64_t m, int64_t n, int nslices
  * (device).  Any k >= 0 (the reference's C1 has k = b = 60).  The operands are
  * staged K-contiguous in scratch memory ((n + m) * roundup(k, 64) * 2 bytes):
  * the context's buffer for the stream, or a stream-ordered allocation past
- * 256 MiB and under capture. */
+ * 512 MiB and under capture. */
 int hplai_gemmschur_f16(hplai_ctx ctx, int64_t n, int64_t m, int64_t k, const uint16_t *a, int64_t lda,
                         const uint16_t *b, int64_t ldb, float *c, int64_t ldc, void *stream);
 /* Replaces the FP16-C overload gemmschur(fp16 a, fp16 b, fp16 c) (schur_updator.hpp:24-27,

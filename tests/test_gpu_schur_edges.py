@@ -52,3 +52,26 @@ def test_schur_tile_choice(ctx, fmt, m, n):
     want = C0.double() - Ud @ Ld.t()
     bound = (Ud.abs() @ Ld.abs().t() + C0.double()) * (K * 2.0 ** -24)
     assert ((C.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("fmt,pad", [(0, 0), (2, 0), (2, 128)])
+def test_schur_packed_first(ctx, fmt, pad):
+    """A row-layout update large enough to be packed first, ragged in rows,
+    columns and leading dimension, against the same update as two row blocks,
+    which are not: the same sums in the same order, so the same bits."""
+    import torch
+    m, n, K, cut = 22311, 21903, 1024 if fmt == 0 else 2048, 11264
+    g = torch.Generator(device="cuda").manual_seed(7)
+    dt = torch.float16 if fmt == 0 else torch.float8_e4m3fn
+    L = (torch.rand(m, K + pad, generator=g, device="cuda") - 0.5).to(dt)
+    U = (torch.rand(n, K + pad, generator=g, device="cuda") - 0.5).to(dt)
+    ns, tl, tu = K // 512, (m + 511) // 512, (n + 511) // 512
+    eL = torch.randint(-2, 3, (ns, tl), generator=g, device="cuda", dtype=torch.int32)
+    eU = torch.randint(-2, 3, (ns, tu), generator=g, device="cuda", dtype=torch.int32)
+    C = torch.rand(n, m, generator=g, device="cuda")
+    D = C.clone()
+    ctx.schur_update(fmt, m, n, ns, 512, L, K + pad, eL, tl, U, K + pad, eU, tu, 512, C, m)
+    for r0, r1 in ((0, cut), (cut, m)):
+        ctx.schur_update(fmt, r1 - r0, n, ns, 512, L[r0:], K + pad, eL[0, r0 // 512:], tl, U, K + pad, eU, tu, 512,
+                         D[0, r0:], m)
+    assert torch.equal(C, D)
