@@ -192,12 +192,13 @@ int hplai_quantize(hplai_ctx ctx, int fmt, int side, int64_t m, int64_t k, int t
             return rc ? rc : launch_quantize(fmt, side, m, k, tb, src, lds, dst, ldd, nullptr, exps, s);
         }
         const int64_t ntiles = ceil_div(m, tb);
-        ScratchLease amax(ctx, s, sizeof(float) * ntiles);
+        const int slots = tile_amax_slots(m, k, tb);
+        ScratchLease amax(ctx, s, sizeof(float) * ntiles * slots);
         if (amax.rc) return amax.rc;
-        int rc = launch_fill_f32(amax.as<float>(), ntiles, 0.0f, s);
+        int rc = slots > 1 ? HPLAI_OK : launch_fill_f32(amax.as<float>(), ntiles, 0.0f, s);
         if (rc == HPLAI_OK) rc = launch_tile_amax(fmt, side, m, k, tb, src, lds, amax.as<float>(), exps, s);
         if (rc == HPLAI_OK)
-            rc = launch_quantize(fmt, side, m, k, tb, src, lds, dst, ldd, amax.as<float>(), exps, s);
+            rc = launch_quantize(fmt, side, m, k, tb, src, lds, dst, ldd, amax.as<float>(), exps, s, false, slots);
         return rc;
     }
     return launch_quantize(fmt, side, m, k, tb > 0 ? tb : 1, src, lds, dst, ldd, nullptr, nullptr, s);

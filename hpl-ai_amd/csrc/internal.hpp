@@ -145,11 +145,14 @@ int launch_trsm_u(int b, int64_t n, const float *tri, float *U, int64_t ldu, flo
 // packed: dst in the panel-packed layout (packed_off), rows a multiple of 256 from its base.
 int launch_quantize(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds,
                     void *dst, int64_t ldd, const float *amax, int32_t *exps, hipStream_t s,
-                    bool packed = false);
+                    bool packed = false, int slots = 1);
 // Exponents of a panel's tiles for launch_quantize without amax: written to
 // exps when one workgroup serves a tile (tile_amax_splits 1, amax NULL), else
-// the maxima to amax (zeroed by the caller).
+// the maxima to amax: tile_amax_slots a tile, one slot a part, or one where all
+// parts meet (zeroed by the caller).
+constexpr int kAmaxSlots = 4;
 int tile_amax_splits(int64_t m, int64_t k, int tb);
+int tile_amax_slots(int64_t m, int64_t k, int tb);
 int launch_tile_amax(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds, float *amax,
                      int32_t *exps, hipStream_t s);
 int launch_fill_f32(float *p, int64_t cnt, float v, hipStream_t s);

@@ -15,16 +15,19 @@ __device__ __forceinline__ int amax_exponent(float a)
 // per-tile max|x| of a panel (side 0: m x k L panel, tiles by row / tb;
 // side 1: k x m U panel, tiles by column / tb).  blockIdx.x is the tile: `in`
 // contiguous entries of `out` columns.  One workgroup per tile writes the
-// tile's exponent itself; with blockIdx.y splitting the columns the maxima
-// meet in amax.  HBM-bound: 512 x 32768 in 9 us (151 us with a thread per row
-// or column, whose loads of a U panel were 2 KB apart).
+// tile's exponent itself; with blockIdx.y splitting the columns its maximum
+// goes to the tile's slot of that part (slots 4), or they meet in amax
+// (slots 1).  HBM-bound: 512 x 32768 in 18 us (26 with a workgroup per tile,
+// which keeps 64 of the 256 CUs busy; 151 with a thread per row or column,
+// whose loads of a U panel were 2 KB apart).
 // ---------------------------------------------------------------------------
 constexpr int kAmaxThreads = 1024;
 
 template <int FMT>
 __global__ __launch_bounds__(kAmaxThreads) void tile_amax_kernel(int side, int64_t m, int64_t k, int tb,
                                                                  const float *__restrict__ src, int64_t lds,
-                                                                 float *__restrict__ amax, int32_t *__restrict__ exps)
+                                                                 float *__restrict__ amax, int slots,
+                                                                 int32_t *__restrict__ exps)
 {
     __shared__ float red[kAmaxThreads / 64];
     const int64_t t0 = static_cast<int64_t>(blockIdx.x) * tb;
@@ -70,7 +73,9 @@ __global__ __launch_bounds__(kAmaxThreads) void tile_amax_kernel(int side, int64
     if (tid == 0) {
 #pragma unroll
         for (int q = 1; q < kAmaxThreads / 64; ++q) v = fmaxf(v, red[q]);
-        if (amax != nullptr)
+        if (amax != nullptr && slots > 1)
+            amax[static_cast<int64_t>(blockIdx.x) * kAmaxSlots + blockIdx.y] = v;
+        else if (amax != nullptr)
             atomic_max_pos(amax + blockIdx.x, v);
         else
             exps[blockIdx.x] = amax_exponent<FMT>(v);
@@ -85,15 +90,21 @@ __global__ void fill_f32_kernel(float *p, int64_t cnt, float v)
 
 // ---------------------------------------------------------------------------
 // Quantizer (convert_left_panels / convert_right_panels, panel_trf.hpp:173-233)
-// q = round(x * 2^e) with e from the tile's max (0 for plain FP16); without
-// amax the exponents are in exps already.
+// q = round(x * 2^e) with e from the tile's max (0 for plain FP16), the largest
+// of its kAmaxSlots where slots > 1; without amax the exponents are in exps
+// already.
 // side 0: L panel m x k col-major -> dst[i*ldd + kk] (transposed through LDS)
 // side 1: U panel k x m col-major -> dst[j*ldd + kk]
 // ---------------------------------------------------------------------------
 template <int FMT>
-__device__ __forceinline__ int fmt_exponent(const float *amax, const int32_t *exps, int64_t tile)
+__device__ __forceinline__ int fmt_exponent(const float *amax, int slots, const int32_t *exps, int64_t tile)
 {
     if (FMT == HPLAI_FMT_F16) return 0;
+    if (amax != nullptr && slots > 1) {
+        static_assert(kAmaxSlots == 4, "one float4 a tile");
+        const float4 a = reinterpret_cast<const float4 *>(amax)[tile];
+        return amax_exponent<FMT>(fmaxf(fmaxf(a.x, a.y), fmaxf(a.z, a.w)));
+    }
     return amax != nullptr ? amax_exponent<FMT>(amax[tile]) : exps[tile];
 }
 
@@ -101,7 +112,7 @@ template <int FMT, bool PACKED>
 __global__ __launch_bounds__(256) void quant_l_kernel(int64_t m, int64_t k, int tb,
                                                       const float *__restrict__ src, int64_t lds,
                                                       void *__restrict__ dst, int64_t ldd,
-                                                      const float *__restrict__ amax,
+                                                      const float *__restrict__ amax, int slots,
                                                       int32_t *__restrict__ exps)
 {
     __shared__ float T[64][65];
@@ -126,7 +137,7 @@ __global__ __launch_bounds__(256) void quant_l_kernel(int64_t m, int64_t k, int 
         const int r = p / 16, kc = (p % 16) * 4;
         const int64_t gr = r0 + r;
         if (gr >= m || c0 + kc >= k) continue;
-        const int e = fmt_exponent<FMT>(amax, exps, gr / tb);
+        const int e = fmt_exponent<FMT>(amax, slots, exps, gr / tb);
         if (amax != nullptr && (gr % tb) == 0 && c0 == 0 && kc == 0) exps[gr / tb] = e;
         float v[4];
 #pragma unroll
@@ -159,7 +170,7 @@ template <int FMT, bool PACKED>
 __global__ __launch_bounds__(256) void quant_u_kernel(int64_t m, int64_t k, int tb,
                                                       const float *__restrict__ src, int64_t lds,
                                                       void *__restrict__ dst, int64_t ldd,
-                                                      const float *__restrict__ amax,
+                                                      const float *__restrict__ amax, int slots,
                                                       int32_t *__restrict__ exps)
 {
     // thread handles 4 consecutive rows (k index) of one column j
@@ -167,7 +178,7 @@ __global__ __launch_bounds__(256) void quant_u_kernel(int64_t m, int64_t k, int 
     const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     const int64_t j = t / kq, r = (t % kq) * 4;
     if (j >= m) return;
-    const int e = fmt_exponent<FMT>(amax, exps, j / tb);
+    const int e = fmt_exponent<FMT>(amax, slots, exps, j / tb);
     if (amax != nullptr && r == 0 && (j % tb) == 0) exps[j / tb] = e;
     const int nk = k - r < 4 ? static_cast<int>(k - r) : 4;
     float v[4];
@@ -228,7 +239,7 @@ template <int FMT, bool PACKED>
 __global__ __launch_bounds__(256) void quant_l16_kernel(int64_t m, int64_t k, int tb,
                                                         const float *__restrict__ src, int64_t lds,
                                                         void *__restrict__ dst, int64_t ldd,
-                                                        const float *__restrict__ amax,
+                                                        const float *__restrict__ amax, int slots,
                                                         int32_t *__restrict__ exps)
 {
     __shared__ float T[64][65];
@@ -269,7 +280,7 @@ __global__ __launch_bounds__(256) void quant_l16_kernel(int64_t m, int64_t k, in
     const int r = tid & 63, kc = (tid >> 6) * 16;
     const int64_t gr = r0 + r;
     if (gr >= m || c0 + kc >= k) return;
-    const int e = fmt_exponent<FMT>(amax, exps, gr / tb);
+    const int e = fmt_exponent<FMT>(amax, slots, exps, gr / tb);
     if (amax != nullptr && (gr % tb) == 0 && c0 == 0 && kc == 0) exps[gr / tb] = e;
     float v[16];
 #pragma unroll
@@ -284,7 +295,7 @@ template <int FMT, bool PACKED>
 __global__ __launch_bounds__(256) void quant_u16_kernel(int64_t m, int64_t k, int tb,
                                                         const float *__restrict__ src, int64_t lds,
                                                         void *__restrict__ dst, int64_t ldd,
-                                                        const float *__restrict__ amax,
+                                                        const float *__restrict__ amax, int slots,
                                                         int32_t *__restrict__ exps)
 {
     constexpr int es = FMT == HPLAI_FMT_E4M3 ? 1 : 2;
@@ -292,7 +303,7 @@ __global__ __launch_bounds__(256) void quant_u16_kernel(int64_t m, int64_t k, in
     const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     const int64_t j = t / kq, r = (t % kq) * 16;
     if (j >= m) return;
-    const int e = fmt_exponent<FMT>(amax, exps, j / tb);
+    const int e = fmt_exponent<FMT>(amax, slots, exps, j / tb);
     if (amax != nullptr && r == 0 && (j % tb) == 0) exps[j / tb] = e;
     const float4 *s4 = reinterpret_cast<const float4 *>(src + j * lds + r);
     float v[16];
@@ -311,14 +322,25 @@ __global__ __launch_bounds__(256) void quant_u16_kernel(int64_t m, int64_t k, in
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-// tiles with more entries than this are split over several workgroups, which
-// then need amax (zeroed) to meet in
-constexpr int64_t kAmaxTile = int64_t(1) << 19;
+// Tiles with more entries than kAmaxTile are split over up to 64 workgroups.
+// Up to kAmaxSlots parts have a slot each; more meet in amax (zeroed).  Smaller
+// tiles of at least kAmaxPart entries are split in kAmaxSlots as well where
+// there are no more parts than CUs: 64 tiles of 512 x 512 take 18 us instead of
+// 26 from HBM (with the conversion, panels that are in the cache: 16 tiles of
+// 512 x 1024 21 for 32, 8 of 512 x 512 12 for 14, 64 of them 31 for 30; 120 of
+// them were 49 for 43, hence the line).
+constexpr int64_t kAmaxTile = int64_t(1) << 19, kAmaxPart = int64_t(1) << 18;
 
 int tile_amax_splits(int64_t m, int64_t k, int tb)
 {
-    const int64_t s = ceil_div((m < tb ? m : tb) * k, kAmaxTile);
-    return static_cast<int>(s < 64 ? s : 64);
+    const int64_t entries = (m < tb ? m : tb) * k, s = ceil_div(entries, kAmaxTile);
+    if (s > kAmaxSlots) return static_cast<int>(s < 64 ? s : 64);
+    return s > 1 || (entries >= kAmaxPart && ceil_div(m, tb) * kAmaxSlots <= 256) ? kAmaxSlots : 1;
+}
+
+int tile_amax_slots(int64_t m, int64_t k, int tb)
+{
+    return tile_amax_splits(m, k, tb) == kAmaxSlots ? kAmaxSlots : 1;
 }
 
 int launch_tile_amax(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds, float *amax,
@@ -328,12 +350,13 @@ int launch_tile_amax(int fmt, int side, int64_t m, int64_t k, int tb, const floa
     HPLAI_CHECK(ceil_div(m, tb) < (int64_t(1) << 31), "quantize: %lld tiles", (long long)ceil_div(m, tb));
     const dim3 g(static_cast<unsigned>(ceil_div(m, tb)),
                  amax != nullptr ? static_cast<unsigned>(tile_amax_splits(m, k, tb)) : 1u);
+    const int slots = tile_amax_slots(m, k, tb);
     if (fmt == HPLAI_FMT_E4M3)
         hipLaunchKernelGGL(tile_amax_kernel<HPLAI_FMT_E4M3>, g, dim3(kAmaxThreads), 0, s, side, m, k, tb, src, lds,
-                           amax, exps);
+                           amax, slots, exps);
     else
         hipLaunchKernelGGL(tile_amax_kernel<HPLAI_FMT_F16_TILE>, g, dim3(kAmaxThreads), 0, s, side, m, k, tb, src,
-                           lds, amax, exps);
+                           lds, amax, slots, exps);
     HPLAI_HIP(hipGetLastError());
     return HPLAI_OK;
 }
@@ -349,7 +372,7 @@ int launch_fill_f32(float *p, int64_t cnt, float v, hipStream_t s)
 
 template <int FMT, bool PACKED>
 static int quant_dispatch(int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds,
-                          void *dst, int64_t ldd, const float *amax, int32_t *exps, hipStream_t s)
+                          void *dst, int64_t ldd, const float *amax, int slots, int32_t *exps, hipStream_t s)
 {
     constexpr int es = FMT == HPLAI_FMT_E4M3 ? 1 : 2;
     const bool v16 = k % 16 == 0 && lds % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
@@ -357,19 +380,19 @@ static int quant_dispatch(int side, int64_t m, int64_t k, int tb, const float *s
     if (side == 0 && v16) {
         dim3 grid(static_cast<unsigned>(ceil_div(m, 64)), static_cast<unsigned>(ceil_div(k, 64)));
         hipLaunchKernelGGL((quant_l16_kernel<FMT, PACKED>), grid, dim3(256), 0, s, m, k, tb, src, lds, dst, ldd,
-                           amax, exps);
+                           amax, slots, exps);
     } else if (side == 0) {
         dim3 grid(static_cast<unsigned>(ceil_div(m, 64)), static_cast<unsigned>(ceil_div(k, 64)));
         hipLaunchKernelGGL((quant_l_kernel<FMT, PACKED>), grid, dim3(256), 0, s, m, k, tb, src, lds, dst, ldd,
-                           amax, exps);
+                           amax, slots, exps);
     } else if (v16) {
         const int64_t thr = m * (k / 16);
         hipLaunchKernelGGL((quant_u16_kernel<FMT, PACKED>), dim3(static_cast<unsigned>(ceil_div(thr, 256))),
-                           dim3(256), 0, s, m, k, tb, src, lds, dst, ldd, amax, exps);
+                           dim3(256), 0, s, m, k, tb, src, lds, dst, ldd, amax, slots, exps);
     } else {
         const int64_t thr = m * ceil_div(k, 4);
         hipLaunchKernelGGL((quant_u_kernel<FMT, PACKED>), dim3(static_cast<unsigned>(ceil_div(thr, 256))),
-                           dim3(256), 0, s, m, k, tb, src, lds, dst, ldd, amax, exps);
+                           dim3(256), 0, s, m, k, tb, src, lds, dst, ldd, amax, slots, exps);
     }
     HPLAI_HIP(hipGetLastError());
     return HPLAI_OK;
@@ -377,23 +400,23 @@ static int quant_dispatch(int side, int64_t m, int64_t k, int tb, const float *s
 
 template <int FMT>
 static int quant_dispatch(bool packed, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds,
-                          void *dst, int64_t ldd, const float *amax, int32_t *exps, hipStream_t s)
+                          void *dst, int64_t ldd, const float *amax, int slots, int32_t *exps, hipStream_t s)
 {
-    return packed ? quant_dispatch<FMT, true>(side, m, k, tb, src, lds, dst, ldd, amax, exps, s)
-                  : quant_dispatch<FMT, false>(side, m, k, tb, src, lds, dst, ldd, amax, exps, s);
+    return packed ? quant_dispatch<FMT, true>(side, m, k, tb, src, lds, dst, ldd, amax, slots, exps, s)
+                  : quant_dispatch<FMT, false>(side, m, k, tb, src, lds, dst, ldd, amax, slots, exps, s);
 }
 
 int launch_quantize(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds,
-                    void *dst, int64_t ldd, const float *amax, int32_t *exps, hipStream_t s, bool packed)
+                    void *dst, int64_t ldd, const float *amax, int32_t *exps, hipStream_t s, bool packed, int slots)
 {
     if (m <= 0 || k <= 0) return HPLAI_OK;
     switch (fmt) {
     case HPLAI_FMT_F16:
-        return quant_dispatch<HPLAI_FMT_F16>(packed, side, m, k, tb, src, lds, dst, ldd, amax, exps, s);
+        return quant_dispatch<HPLAI_FMT_F16>(packed, side, m, k, tb, src, lds, dst, ldd, amax, slots, exps, s);
     case HPLAI_FMT_F16_TILE:
-        return quant_dispatch<HPLAI_FMT_F16_TILE>(packed, side, m, k, tb, src, lds, dst, ldd, amax, exps, s);
+        return quant_dispatch<HPLAI_FMT_F16_TILE>(packed, side, m, k, tb, src, lds, dst, ldd, amax, slots, exps, s);
     case HPLAI_FMT_E4M3:
-        return quant_dispatch<HPLAI_FMT_E4M3>(packed, side, m, k, tb, src, lds, dst, ldd, amax, exps, s);
+        return quant_dispatch<HPLAI_FMT_E4M3>(packed, side, m, k, tb, src, lds, dst, ldd, amax, slots, exps, s);
     default:
         set_error("quantize: unknown format %d", fmt);
         return HPLAI_EINVAL;
