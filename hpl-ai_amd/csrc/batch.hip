@@ -26,9 +26,13 @@
 // 1431, panels 1646 / 328, U 1545 / in the update, generation 978 / 148,
 // residuals 1493 / 358, triangular solves 1153 / 460), 512 3045 / 1060, 200 672 /
 // 370, 64 258 / 180; 1024 systems of 32 .. 1024: 20.7 -> 5.9 ms.
+// Joining a step's norms and leaving out waves without rows (batch_norms) took
+// that to 5.7 ms, and 256 systems with 1 to 4 right-hand sides of order 64 from
+// 181 to 141 us, 200 513 to 445, 512 1415 to 1312 (1024: 4060, the same).
 #include <algorithm>
 #include <cfloat>
 #include <chrono>
+#include <type_traits>
 #include <vector>
 
 #include "device_common.hpp"
@@ -545,6 +549,52 @@ __device__ __forceinline__ void batch_residual(const BatchSys &S, const double *
     }
 }
 
+// |b - A x| and |x| of NR right-hand sides, their maxima over the rows at once:
+// one barrier, and only the waves that own rows: latency-bound at small orders,
+// where a reduction for each of the eight maxima over all 16 waves took longer
+// than the residual (150 systems of order 4 to 16: 97 -> 71 us, of order 100:
+// 369 -> 305 us).  red is free again after the caller's next barrier.
+template <int NR>
+__device__ __forceinline__ void batch_norms(int n, const double (&acc)[4], const double *xl, double *R, double *red,
+                                            double (&rm)[4], double (&xm)[4])
+{
+    constexpr int NV = 2 * NR;
+    const int tid = own_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nw = (n + 63) / 64;
+    if (wave < nw) {
+        double v[NV];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            v[2 * r] = v[2 * r + 1] = 0.0;
+            if (tid < n) {
+                R[static_cast<int64_t>(r) * n + tid] = acc[r];
+                v[2 * r] = fabs(acc[r]);
+                v[2 * r + 1] = fabs(xl[r * n + tid]);
+            }
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+            for (int q = 0; q < NV; ++q) v[q] = fmax(v[q], __shfl_xor(v[q], off));
+        if (lane == 0)
+#pragma unroll
+            for (int q = 0; q < NV; ++q) red[wave * NV + q] = v[q];
+    }
+    __syncthreads();
+    double m[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) m[q] = red[q];
+    for (int w = 1; w < nw; ++w)
+#pragma unroll
+        for (int q = 0; q < NV; ++q) m[q] = fmax(m[q], red[w * NV + q]);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+        // rows past the end count as zeros, also beside NaNs
+        rm[r] = nw < kBT / 64 ? fmax(m[2 * r], 0.0) : m[2 * r];
+        xm[r] = nw < kBT / 64 ? fmax(m[2 * r + 1], 0.0) : m[2 * r + 1];
+    }
+}
+
 // ---- FP64 refinement of every right-hand side (iterative_refinement.hpp:18-57) ----
 __device__ __forceinline__ void batch_refine(const BatchSys &S, const float *LU, const double *d,
                              const double *B, double *X, double *R, double *xl, double *xs, double *red,
@@ -578,29 +628,22 @@ __device__ __forceinline__ void batch_refine(const BatchSys &S, const float *LU,
                 for (int i = tid; i < n; i += kBT) xl[rr * n + i] = X[static_cast<int64_t>(rr) * n + i];
         __syncthreads();
         double xm[4] = {0.0, 0.0, 0.0, 0.0}, rm[4] = {0.0, 0.0, 0.0, 0.0};
-        double acc[4];
+        auto residual = [&](auto nrhs) {
+            constexpr int NR = decltype(nrhs)::value;
+            double acc[4];
+            if ((tid & ~63) < n) batch_residual<NR>(S, d, B, xl, acc);   // waves that own rows
+            batch_norms<NR>(n, acc, xl, R, red, rm, xm);
+        };
         switch (nr) {
-        case 1: batch_residual<1>(S, d, B, xl, acc); break;
-        case 2: batch_residual<2>(S, d, B, xl, acc); break;
-        case 3: batch_residual<3>(S, d, B, xl, acc); break;
-        default: batch_residual<4>(S, d, B, xl, acc); break;
-        }
-        if (tid < n) {
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-                if (rr < nr && !done[rr]) {
-                    R[static_cast<int64_t>(rr) * n + tid] = acc[rr];
-                    rm[rr] = fabs(acc[rr]);
-                    xm[rr] = fabs(xl[rr * n + tid]);
-                }
-            }
+        case 1: residual(std::integral_constant<int, 1>{}); break;
+        case 2: residual(std::integral_constant<int, 2>{}); break;
+        case 3: residual(std::integral_constant<int, 3>{}); break;
+        default: residual(std::integral_constant<int, 4>{}); break;
         }
         bool all = true;
         for (int rr = 0; rr < nr; ++rr) {
             if (done[rr]) continue;
-            const double normr = block_max(rm[rr], red);
-            const double normx = block_max(xm[rr], red);
-            h[rr] = normr / (norma * normx + normb[rr]) * 1. / (static_cast<double>(n) * DBL_EPSILON / 2);
+            h[rr] = rm[rr] / (norma * xm[rr] + normb[rr]) * 1. / (static_cast<double>(n) * DBL_EPSILON / 2);
             steps[rr] = it + 1;
             done[rr] = h[rr] < 16.0;
             all = all && done[rr];
@@ -637,7 +680,7 @@ __global__ __launch_bounds__(kBT) void batch_kernel(const BatchSys *__restrict__
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ double xs[2 * 4 * 32];
-    __shared__ double red[kBT / 64];
+    __shared__ double red[kBT / 64 * 8];
     __shared__ int32_t next;
     for (;;) {
         if (threadIdx.x == 0) next = atomicAdd(counter, 1);
