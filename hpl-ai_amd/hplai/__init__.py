@@ -164,6 +164,17 @@ def stream_ptr(stream=None):
     return stream.cuda_stream
 
 
+def _default_after_current(device):
+    """Puts the default (NULL) stream after torch's current stream on `device`,
+    for the entry points that take no stream and start on the NULL stream:
+    torch's other streams are non-blocking, so nothing else orders the two."""
+    import torch
+    if torch.cuda.is_available():
+        current = torch.cuda.current_stream(device)
+        if current.cuda_stream != 0:
+            torch.cuda.default_stream(device).wait_stream(current)
+
+
 class Context:
     """An hplai_ctx bound to one device (default: torch's current device)."""
 
@@ -271,7 +282,9 @@ class Context:
 
     # ---- dense factor and multi-RHS solves ----
     def factor(self, n, b, A, lda, fmt="f16", outer=1, lookahead=True):
-        """LU of the n x n FP32 column-major device matrix A in place."""
+        """LU of the n x n FP32 column-major device matrix A in place, after the
+        work of torch's current stream; complete on return."""
+        _default_after_current(self.device)
         code = FMTS[fmt] if isinstance(fmt, str) else fmt
         check(lib().hplai_factor_f32(self.handle, n, b, code, outer, int(lookahead), ptr(A), lda))
 

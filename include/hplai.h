@@ -180,7 +180,11 @@ int hplai_norm_inf_f64(hplai_ctx ctx, int64_t n, const double *x, double *out_de
  * lda >= n) in place, with the same kernels and schedule as hplai_solve
  * (FP32 panel, Schur update in `fmt`, `outer` panels per trailing update,
  * look-ahead on a second stream).  n % b == 0; b % 128 == 0 for the
- * tile-scaled formats.  Synchronous; HPLAI_EPIVOT on a zero pivot. */
+ * tile-scaled formats.  Synchronous; HPLAI_EPIVOT on a zero pivot.  It takes
+ * no stream and starts on the NULL stream: work on a stream that does not
+ * synchronise with that one (hipStreamNonBlocking) and writes A has to be
+ * complete, or the NULL stream made to wait for it, before the call.  The
+ * Python binding does so for torch's current stream. */
 int hplai_factor_f32(hplai_ctx ctx, int64_t n, int b, int fmt, int outer, int lookahead, float *A,
                      int64_t lda);
 /* Solves with the factors of hplai_factor_f32 / hplai_solve (FP32 entries

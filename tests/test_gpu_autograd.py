@@ -171,3 +171,35 @@ def test_autograd_solve_n8192(ctx):
     rel_fd = np.max(np.abs(fd - an)) / np.max(np.abs(an))
     print("vs central differences (32 entries): %.3g" % rel_fd)
     assert rel_fd < 1e-6
+
+
+@pytest.mark.parametrize("n,b", [(1200, 60), (2048, 512)])
+def test_solve_on_a_side_stream(ctx, n, b):
+    """The inputs come late on a non-blocking stream: the factorization, which
+    takes no stream, has to wait for them.  Same kernels, same bits."""
+    import torch
+    from hplai import autograd
+    A = _gen_A64(ctx, n)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    B = torch.rand(n, 3, generator=g, device="cuda", dtype=torch.float64) - 0.5
+
+    def run(A, B):
+        A, B = A.requires_grad_(), B.requires_grad_()
+        X = autograd.solve(A, B, ctx=ctx, b=b)
+        X.square().sum().backward()
+        return X.detach(), A.grad, B.grad
+
+    want = run(A.clone(), B.clone())
+    M = torch.rand(4096, 4096, generator=g, device="cuda") / 4096
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        late = torch.full_like(A, float("nan"))
+        P = M
+        for _ in range(20):            # some ms of work ahead of the inputs
+            P = P @ M
+        late.copy_(A).add_(P[0, 0].double() * 0.0)
+        got = run(late, B.clone())
+    torch.cuda.synchronize()
+    for a, w in zip(got, want):
+        assert torch.equal(a, w)
