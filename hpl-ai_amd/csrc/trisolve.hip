@@ -14,13 +14,15 @@
 // What bounds it: that chain, 6 + 13 us a block with 64 columns and 5 + 5 us
 // with one (the inverses of both triangles together: 40 + 28 + 23 us at 8192).
 // Substitution in one workgroup per block and reading the factors once per
-// column took, both triangles, 2728 us at 8192 x 64 (6330 us transposed), now
-// 753 (719); 2060 us at 8192 x 1, now 525; 288 us at 1200 x 3, now 118; 9.5 ms
+// column took, both triangles, 2707 us at 8192 x 64 (6320 us transposed), now
+// 764 (744); 2060 us at 8192 x 1, now 540; 285 us at 1200 x 3, now 127; 9.5 ms
 // at 30000 x 1, now 2.8.
 // A product with an inverse has the error of substitution times the condition
-// of the 512 x 512 block: nothing measurable for factors of matrices that
-// admit elimination without pivoting in FP32 (1e-16 .. 6e-16 of the solution
-// for both, orders 1 .. 3000), more for triangles that are nearly singular.
+// of the 512 x 512 block.  So each block's condition, the largest row sum of
+// |T_kk^-1| |T_kk|, is formed with its inverse (9 us at 1200, 22 at 8192), and a
+// block past kTsCond is solved by substitution instead (tri64_substitute): all
+// blocks so, 2.6 ms at 8192 x 64 (3.5 transposed), 2.3 at 8192 x 1, 0.38 at
+// 1200 x 3, bound by the triangle's way into one CU.
 //
 // An upper triangle is a lower one with rows and columns taken from the end;
 // TriView numbers entries that way, so the kernels only know lower ones.
@@ -36,6 +38,12 @@ constexpr int kTsInv = 32 * 32 * 256;     // doubles of one block's inverse, 16 
 constexpr int kTsMid = 16 * 16 * 256;     // doubles of one block's intermediate product
 constexpr int kTsGroup = 32;              // blocks inverted at a time (96 MiB a triangle)
 constexpr int kTsCols = 1024;             // right-hand sides at a time
+constexpr int kTsRow = kTsBlock + 16;     // doubles of one block's row sums of |T| and, at kTsBlock, its mark
+// Largest condition that is solved through the inverse.  Errors of inverse /
+// substitution (FP64, order 512, b = T x): condition 3.6 (factors of HPL-AI
+// matrices) 1.2e-16 / 1.2e-16 of the solution, 18 1.5e-16 / 1.3e-16, 54 3.5e-16
+// / 1.4e-16, 3e2 2.7e-15 / 4.8e-16, 6e5 2.6e-8 / 1.1e-12.
+constexpr double kTsCond = 16.0;
 
 // MFMA layout: left operand lane -> (row lane % 16, k lane / 16), right operand
 // lane -> (k lane / 16, column lane % 16), result q -> (row lane / 16 + 4 q,
@@ -186,20 +194,117 @@ __device__ __forceinline__ void tri64_inv(const TriView<UPPER, TRANS> &E, int64_
     }
 }
 
+// Row sums of |T| over the 512-block for 64 rows of the 256-block blockIdx.x
+// (blockIdx.y - 4), zeros past the matrix.  The lanes run along the factor's
+// contiguous direction.
+template <bool UPPER, bool TRANS>
+__device__ __forceinline__ void tri64_rows(const TriView<UPPER, TRANS> &E, int64_t first, double *__restrict__ rows,
+                                           double *red)
+{
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t h = static_cast<int64_t>(blockIdx.x), b0 = first + (h >> 1) * kTsBlock;
+    const int c0 = static_cast<int>(h & 1) * kTsHalf + 64 * (static_cast<int>(blockIdx.y) - 4);   // first row in the block
+    double *out = rows + (h >> 1) * kTsRow;
+    auto term = [&](int r, int k, float v) {
+        const double a = k == r && TriView<UPPER, TRANS>::kUnit ? 1.0 : fabs(static_cast<double>(v));
+        return k <= r && b0 + r < E.n ? a : 0.0;
+    };
+    if constexpr (TRANS) {
+        double acc[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) acc[u] = 0.0;
+        for (int k0 = 0; k0 < c0 + 64; k0 += 64) {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+                v[u] = *E.ptr(min(b0 + c0 + 16 * wave + u, E.n - 1), min(b0 + k0 + lane, E.n - 1));
+#pragma unroll
+            for (int u = 0; u < 16; ++u) acc[u] += term(c0 + 16 * wave + u, k0 + lane, v[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            double s = acc[u];
+            for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+            if (lane == u) out[c0 + 16 * wave + u] = s;
+        }
+    } else {
+        double acc = 0.0;
+        for (int k0 = 0; k0 < c0 + 64; k0 += 64) {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+                v[u] = *E.ptr(min(b0 + c0 + lane, E.n - 1), min(b0 + k0 + 16 * wave + u, E.n - 1));
+#pragma unroll
+            for (int u = 0; u < 16; ++u) acc += term(c0 + lane, k0 + 16 * wave + u, v[u]);
+        }
+        red[wave * 64 + lane] = acc;
+        __syncthreads();
+        if (wave == 0) out[c0 + lane] = ((red[lane] + red[64 + lane]) + red[128 + lane]) + red[192 + lane];
+    }
+    if (c0 == 0 && threadIdx.x == 0) out[kTsBlock] = 0.0;
+}
+
 // blockIdx.z (+ upper0): the lower or the upper triangle of the pair that one
-// lu_solve needs; z2: doubles from the first's scratch to the second's
+// lu_solve needs; z2: doubles from the first's scratch to the second's.
+// blockIdx.y < 4: the inverses; 4 .. 7: the row sums
 template <bool TRANS>
 __global__ __launch_bounds__(256) void tri64_inv_kernel(const float *__restrict__ LU, int64_t lda, int64_t n,
                                                         int64_t first, int upper0, double *__restrict__ inv,
-                                                        double *__restrict__ bop, int64_t z2)
+                                                        double *__restrict__ bop, double *__restrict__ rows, int64_t z2)
 {
     __shared__ TsInvLds sm;
     inv += blockIdx.z * z2;
     bop += blockIdx.z * z2;
-    if ((upper0 + static_cast<int>(blockIdx.z)) & 1)
-        tri64_inv(TriView<true, TRANS>{LU, lda, n}, first, inv, bop, sm);
-    else
-        tri64_inv(TriView<false, TRANS>{LU, lda, n}, first, inv, bop, sm);
+    rows += blockIdx.z * z2;
+    const TriView<true, TRANS> U{LU, lda, n};
+    const TriView<false, TRANS> L{LU, lda, n};
+    const bool upper = (upper0 + static_cast<int>(blockIdx.z)) & 1;
+    if (blockIdx.y >= 4) {
+        if (upper)
+            tri64_rows(U, first, rows, &sm.rd[0][0]);
+        else
+            tri64_rows(L, first, rows, &sm.rd[0][0]);
+    } else if (upper) {
+        tri64_inv(U, first, inv, bop, sm);
+    } else {
+        tri64_inv(L, first, inv, bop, sm);
+    }
+}
+
+// Marks the 512-block blockIdx.x when a row sum of |T^-1| |T| is past kTsCond
+// or no number.  A wave takes the 16 rows of tile 4 blockIdx.y + wave.
+__global__ __launch_bounds__(256) void tri64_cond_kernel(int64_t left, const double *__restrict__ inv, double *rows,
+                                                         int64_t z2)
+{
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, lk = lane >> 4;
+    const double *bi = inv + blockIdx.z * z2 + static_cast<int64_t>(blockIdx.x) * kTsInv;
+    double *row = rows + blockIdx.z * z2 + static_cast<int64_t>(blockIdx.x) * kTsRow;
+    const int64_t over = left - static_cast<int64_t>(blockIdx.x) * kTsBlock;
+    const int w = over < kTsBlock ? static_cast<int>(over) : kTsBlock;
+    const int I = 4 * static_cast<int>(blockIdx.y) + wave;
+    if (16 * I >= w) return;
+    double s = 0.0;
+    for (int K0 = 0; K0 <= I; K0 += 4) {
+        double a[4][4], r[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int K = min(K0 + u, I);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                a[u][t] = bi[(I * 32 + K) * 256 + lane * 4 + t];
+                r[u][t] = row[16 * K + 4 * t + lk];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (K0 + u <= I)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) s = fma(fabs(a[u][t]), r[u][t], s);
+    }
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    if (__any(16 * I + l16 < w && !(s <= kTsCond)) && lane == 0) row[kTsBlock] = 1.0;
 }
 
 // 256 -> 512: the lower left quarter -B^-1 C A^-1.  MID: tile (I, J) of
@@ -280,14 +385,98 @@ __device__ __forceinline__ int64_t solved_pos(int k, int c)
     return (static_cast<int64_t>(c >> 4) * 32 + (k >> 4)) * 256 + lane * 4 + t;
 }
 
+__device__ __forceinline__ double readlane64(double v, int lane)
+{
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+    return __hiloint2double(hi, lo);
+}
+
+// One column of T_kk^-1 x_k by substitution, 256 threads, rows tid and tid + 256
+// in registers.  The 16 rows of a tile are solved in the wave that owns them
+// (x_c by v_readlane, diagonals as reciprocals), the rows further on subtract
+// the tile's 16 columns, loaded a tile ahead.  A barrier a tile: the parts of xs take turns.
+template <bool UPPER, bool TRANS>
+__device__ __forceinline__ void tri64_substitute(const TriView<UPPER, TRANS> &E, int64_t kb, const double *x, double *xt,
+                                                 int col, double (&xs)[2][16])
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int w = E.n - kb < kTsBlock ? static_cast<int>(E.n - kb) : kTsBlock;
+    double xr[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) xr[q] = x[E.index(min(kb + tid + 256 * q, E.n - 1))];
+    __syncthreads();   // xs: the column before
+    float t[2][16], next[2][16];
+    auto load = [&](float (&v)[2][16], int c0) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            if (256 * q + 64 * wave + 63 >= c0)   // rows that the tile reaches
+#pragma unroll
+                for (int c = 0; c < 16; ++c)
+                    v[q][c] = *E.ptr(min(kb + tid + 256 * q, E.n - 1), min(kb + c0 + c, E.n - 1));
+    };
+    load(t, 0);
+    for (int s0 = 0; s0 < w; s0 += 16) {
+        double *part = xs[(s0 >> 4) & 1];
+        if (s0 + 16 < w) load(next, s0 + 16);
+        auto diagonal = [&](const float (&a)[16], double &x) {
+            const int i = lane - (s0 & 63);   // row s0 + i for 0 <= i < 16
+            double v = x, rinv = 1.0;
+            if (!TriView<UPPER, TRANS>::kUnit) {
+                float d = 1.0f;
+#pragma unroll
+                for (int c = 0; c < 16; ++c) d = c == i ? a[c] : d;
+                rinv = 1.0 / static_cast<double>(d);
+            }
+#pragma unroll
+            for (int c = 0; c < 16; ++c) {
+                if (s0 + c >= w) break;
+                if (!TriView<UPPER, TRANS>::kUnit && i == c) v *= rinv;
+                const double xc = readlane64(v, (s0 & 63) + c);
+                if (i > c && i < 16) v = fma(-static_cast<double>(a[c]), xc, v);
+            }
+            if (i >= 0 && i < 16) {
+                part[i] = v;
+                x = v;
+            }
+        };
+        if (wave == (s0 & 255) >> 6) {
+            if (s0 < 256)
+                diagonal(t[0], xr[0]);
+            else
+                diagonal(t[1], xr[1]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            if (tid + 256 * q >= s0 + 16) {
+                double acc = 0.0;
+#pragma unroll
+                for (int c = 0; c < 16; ++c) acc = fma(static_cast<double>(t[q][c]), part[c], acc);
+                xr[q] -= acc;
+            }
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int c = 0; c < 16; ++c) t[q][c] = next[q][c];
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        if (tid + 256 * q < w) xt[solved_pos<TRANS>(tid + 256 * q, col)] = xr[q];
+}
+
 // Rows 16 I .. + 15 (blockIdx.x) of T_kk^-1 x_k for 16 columns (blockIdx.y) to
-// xt.  The four waves split K and are added in order.
+// xt.  The four waves split K and are added in order.  A marked block: the
+// workgroups take a column each instead.
 template <bool UPPER, bool TRANS>
 __global__ __launch_bounds__(256) void tri64_solve_kernel(TriView<UPPER, TRANS> E, int64_t kb,
-                                                          const double *__restrict__ inv, const double *__restrict__ X,
-                                                          int64_t ldx, int nrhs, double *__restrict__ xt)
+                                                          const double *__restrict__ inv, const double *__restrict__ mark,
+                                                          const double *__restrict__ X, int64_t ldx, int nrhs,
+                                                          double *__restrict__ xt)
 {
     __shared__ double red[3][4][64];
+    __shared__ double xs[2][16];
+    const double marked = *mark;   // asked for after the product's loads
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, lk = lane >> 4;
     const int I = static_cast<int>(blockIdx.x), c0 = static_cast<int>(blockIdx.y) * 16;
@@ -330,6 +519,11 @@ __global__ __launch_bounds__(256) void tri64_solve_kernel(TriView<UPPER, TRANS> 
 #pragma unroll
                 for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][t], b[u][t], acc, 0, 0, 0);
             }
+    }
+    if (marked != 0.0) {
+        for (int c = static_cast<int>(blockIdx.x); c < 16 && c0 + c < nrhs; c += static_cast<int>(gridDim.x))
+            tri64_substitute(E, kb, X + static_cast<int64_t>(c0 + c) * ldx, xt, c0 + c, xs);
+        return;
     }
     if (wave > 0)
 #pragma unroll
@@ -430,7 +624,8 @@ static int64_t tri_group(int64_t n)
     const int64_t blocks = ceil_div(n, kTsBlock);
     return blocks < kTsGroup ? blocks : kTsGroup;
 }
-static int64_t tri_inv_doubles(int64_t n) { return tri_group(n) * (kTsInv + 2 * kTsMid); }
+static int64_t tri_inv_doubles(int64_t n) { return tri_group(n) * (kTsInv + 2 * kTsMid + kTsRow); }
+static double *tri_rows(int64_t n, double *inv) { return inv + tri_group(n) * (kTsInv + 2 * kTsMid); }
 
 // both triangles' inverses fit beside each other where one group holds all
 int64_t tri_solve_work_doubles(int64_t n, int nrhs)
@@ -446,16 +641,17 @@ static int tri_invert(bool upper, bool both, int64_t n, int64_t first, const flo
 {
     const int64_t g = tri_group(n), left = ceil_div(n - first, kTsBlock);
     const unsigned gc = static_cast<unsigned>(left < g ? left : g), z = both ? 2 : 1;
-    double *mid = inv + g * kTsInv, *bop = mid + g * kTsMid;
+    double *mid = inv + g * kTsInv, *bop = mid + g * kTsMid, *rows = tri_rows(n, inv);
     const int64_t z2 = tri_inv_doubles(n);
-    hipLaunchKernelGGL((tri64_inv_kernel<TRANS>), dim3(2 * gc, 4, z), dim3(256), 0, s, LU, lda, n, first,
-                       upper ? 1 : 0, inv, bop, z2);
+    hipLaunchKernelGGL((tri64_inv_kernel<TRANS>), dim3(2 * gc, 8, z), dim3(256), 0, s, LU, lda, n, first,
+                       upper ? 1 : 0, inv, bop, rows, z2);
     if (n - first > kTsHalf) {
         hipLaunchKernelGGL((tri64_merge_kernel<TRANS, true>), dim3(gc, 64, z), dim3(256), 0, s, LU, lda, n, first,
                            upper ? 1 : 0, inv, bop, mid, z2);
         hipLaunchKernelGGL((tri64_merge_kernel<TRANS, false>), dim3(gc, 64, z), dim3(256), 0, s, LU, lda, n, first,
                            upper ? 1 : 0, inv, bop, mid, z2);
     }
+    hipLaunchKernelGGL(tri64_cond_kernel, dim3(gc, 8, z), dim3(256), 0, s, n - first, inv, rows, z2);
     HPLAI_HIP(hipGetLastError());
     return HPLAI_OK;
 }
@@ -480,7 +676,8 @@ static int tri_solve(int64_t n, const float *LU, int64_t lda, double *X, int64_t
             double *Xc = X + static_cast<int64_t>(c) * ldx;
             hipLaunchKernelGGL((tri64_solve_kernel<UPPER, TRANS>),
                                dim3(static_cast<unsigned>((w + 15) / 16), static_cast<unsigned>((nc + 15) / 16)),
-                               dim3(256), 0, s, E, kb, inv + (q % group) * kTsInv, Xc, ldx, nc, xt);
+                               dim3(256), 0, s, E, kb, inv + (q % group) * kTsInv,
+                               tri_rows(n, inv) + (q % group) * kTsRow + kTsBlock, Xc, ldx, nc, xt);
             if (nc <= 16)
                 hipLaunchKernelGGL((tri64_update_kernel<UPPER, TRANS, 1, 2>), dim3(16 + rows, 1), dim3(512), 0, s, E, kb,
                                    w, xt, Xc, ldx, nc);

@@ -193,7 +193,9 @@ int hplai_factor_f32(hplai_ctx ctx, int64_t n, int b, int fmt, int outer, int lo
  * the transposed solve for A^T lambda = g (no reference counterpart: it serves
  * the gradient of x = A^-1 b).  X (device, FP64) holds nrhs columns with
  * leading dimension ldx; bs (1 .. 1024) is checked, the blocking is the
- * library's own. */
+ * library's own.  Diagonal blocks are applied through their FP64 inverses
+ * where they are well conditioned, by substitution elsewhere: the accuracy is
+ * substitution's, for hplai_trsv_lower_f32 and hplai_trsv_upper_f32 as well. */
 int hplai_lu_solve_f64(hplai_ctx ctx, int trans, int64_t n, int nrhs, int bs, const float *LU,
                        int64_t lda, double *X, int64_t ldx, void *stream);
 

@@ -94,3 +94,50 @@ def test_captured_and_replayed(ctx):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(X, want[k])
+
+
+def _hard(n, kind, rng):
+    """Triangles far from the identity: T (lower, unit) in FP32 values."""
+    T = np.tril(rng.standard_normal((n, n)) * 0.3, -1) if kind == "normal" else np.tril(np.full((n, n), -0.02), -1)
+    if kind == "first":
+        T = np.tril(rng.uniform(-0.5, 0.5, (n, n)) / n, -1)
+        T[:400, :400] = np.tril(rng.standard_normal((400, 400)) * 0.3, -1)
+    return (T + np.eye(n)).astype(np.float32).astype(np.float64)
+
+
+@pytest.mark.parametrize("n", [120, 512, 900, 1600])
+@pytest.mark.parametrize("kind", ["normal", "constant", "first"])
+@pytest.mark.parametrize("upper,trans", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("nrhs", [1, 18])
+def test_ill_conditioned_triangles(ctx, n, kind, upper, trans, nrhs):
+    """Blocks whose inverse would cost accuracy.  Substitution in any order has
+    |b - T x| <= gamma |T| |x| entry by entry with gamma = (n + 2) u / (1 - (n +
+    2) u), u = 2^-53 (one more rounding for the reciprocal diagonal); b = T x0
+    with a small x0, the right-hand side for which a product with the inverse is
+    1e3 and more above that."""
+    import torch
+    if kind == "first" and n < 400:
+        pytest.skip("smaller than its hard block")
+    rng = np.random.default_rng(n)
+    T = _hard(n, kind, rng)
+    if upper:
+        T = np.ascontiguousarray(T[::-1, ::-1])          # unit upper
+        T = (T * rng.uniform(0.5, 2.0, n)[:, None]).astype(np.float32).astype(np.float64)
+    M = T + 0.0
+    opT = T.T if trans else T
+    X0 = rng.standard_normal((n, nrhs))
+    B = (opT.astype(np.longdouble) @ X0.astype(np.longdouble)).astype(np.float64)
+    # the other triangle is the identity's: L = I has no stored diagonal, U = I does
+    LU = np.triu(M) if upper else np.tril(M, -1) + np.eye(n)
+    F = torch.from_numpy(np.ascontiguousarray(LU.T.astype(np.float32))).cuda()
+    Xc = torch.from_numpy(np.ascontiguousarray(B.T)).cuda()
+    if nrhs == 1 and not trans:
+        (ctx.trsv_upper if upper else ctx.trsv_lower)(n, 512, F, n, Xc)
+    else:
+        ctx.lu_solve(n, nrhs, 512, F, n, Xc, n, trans=trans)
+    X = Xc.cpu().numpy().T.astype(np.longdouble)
+    R = np.abs(B.astype(np.longdouble) - opT.astype(np.longdouble) @ X)
+    u = 2.0 ** -53
+    gamma = (n + 2) * u / (1 - (n + 2) * u)
+    assert np.isfinite(X).all()
+    assert (R <= gamma * (np.abs(opT) @ np.abs(X))).all(), float((R / (np.abs(opT) @ np.abs(X))).max() / gamma)
