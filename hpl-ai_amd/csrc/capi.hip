@@ -155,8 +155,7 @@ int hplai_trsm_lpanel_f32(hplai_ctx ctx, int64_t m, int b, const float *Ukk, int
     hipStream_t s = as_stream(stream);
     ScratchLease tri(ctx, s, sizeof(float) * tri_floats(b));
     if (tri.rc) return tri.rc;
-    const int rc = launch_tri_inverse(b, Ukk, ldu, tri.as<float>(), 2, s);
-    return rc ? rc : launch_trsm_l(m, b, tri.as<float>(), L, ldl, nullptr, 1, s);
+    return launch_trsm_panel(false, m, b, Ukk, ldu, tri.as<float>(), L, ldl, s);
 }
 
 int hplai_trsm_upanel_f32(hplai_ctx ctx, int b, int64_t n, const float *Lkk, int64_t ldl, float *U,
@@ -169,8 +168,7 @@ int hplai_trsm_upanel_f32(hplai_ctx ctx, int b, int64_t n, const float *Lkk, int
     hipStream_t s = as_stream(stream);
     ScratchLease tri(ctx, s, sizeof(float) * tri_floats(b));
     if (tri.rc) return tri.rc;
-    const int rc = launch_tri_inverse(b, Lkk, ldl, tri.as<float>(), 1, s);
-    return rc ? rc : launch_trsm_u(b, n, tri.as<float>(), U, ldu, nullptr, 1, s);
+    return launch_trsm_panel(true, n, b, Lkk, ldl, tri.as<float>(), U, ldu, s);
 }
 
 int hplai_quantize(hplai_ctx ctx, int fmt, int side, int64_t m, int64_t k, int tb, const float *src,

@@ -725,14 +725,14 @@ int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, bool full,
     return HPLAI_OK;
 }
 
-int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, hipStream_t s)
+int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, bool join, hipStream_t s)
 {
     if (b <= 0) return HPLAI_OK;
     hipLaunchKernelGGL((lu_update_kernel<false>), dim3(static_cast<unsigned>(ceil_div(b, kLuNB))), dim3(kLuThreads), 0,
                        s, b, 0, const_cast<float *>(LU), lda, tri, sides, nullptr);
     HPLAI_HIP(hipGetLastError());
     const int nb = static_cast<int>(ceil_div(b, 32));
-    for (int H = kLuNB / 32; H < nb; H *= 2) {
+    for (int H = kLuNB / 32; join && H < nb; H *= 2) {
         const unsigned cols = static_cast<unsigned>(ceil_div(nb, 2 * H)) * H, z = sides == 3 ? 2 : 1;
         hipLaunchKernelGGL((tri_join_kernel<true>), dim3(cols, H / 4, z), dim3(kLuThreads), 0, s, b, H, LU, lda, tri,
                            sides == 2 ? 1 : 0);

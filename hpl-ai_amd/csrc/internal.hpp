@@ -127,8 +127,9 @@ int launch_gen_rhs(int64_t n, uint64_t seed, int64_t i0, int64_t cnt, double *b,
 int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, bool full, hipStream_t s);
 int64_t getrf_scratch_floats(int n);
 int64_t tri_floats(int b);
-// the same inverses of a block that is already factored; sides: 1 L, 2 U, 3 both
-int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, hipStream_t s);
+// the same inverses of a block that is already factored, without join those of
+// its 128-blocks only; sides: 1 L, 2 U, 3 both
+int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, bool join, hipStream_t s);
 // tri: the packed inverses of the factored diagonal block
 // half: where the results also go as FP16 (dst NULL: nowhere), operand rows ld
 // bytes apart, each slice padded to whole 32-blocks; packed as for launch_quantize
@@ -141,6 +142,10 @@ int launch_trsm_l(int64_t m, int b, const float *tri, float *L, int64_t ldl, flo
                   TrsmHalf half = {});
 int launch_trsm_u(int b, int64_t n, const float *tri, float *U, int64_t ldu, float *amax, int tb, hipStream_t s,
                   TrsmHalf half = {});
+// A panel of m columns (up: P := L^-1 P) or rows (P := P U^-1) with the caller's
+// triangle in T; tri: tri_floats(b) of scratch
+int launch_trsm_panel(bool up, int64_t m, int b, const float *T, int64_t ldt, float *tri, float *P, int64_t ldp,
+                      hipStream_t s);
 // amax: per-tile maxima of |src|; NULL: the exponents are in exps (FMT_F16: 0).
 // packed: dst in the panel-packed layout (packed_off), rows a multiple of 256 from its base.
 int launch_quantize(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds,

@@ -1,6 +1,7 @@
 // trsm.hip — panel TRSMs of the blocked LU as products with the inverse of
 // the diagonal block's triangle (getrf.hip), b <= 1024:
-//   L := A Uinv,  U := Linv A.
+//   L := A Uinv,  U := Linv A,
+// and for a caller's own triangle block by block (trsm_walk_kernel, at the end).
 // One workgroup owns a strip of 32 rows (L panel) or 32 columns (U panel)
 // with all b entries of its other dimension in LDS.  The strip's 32 x 32
 // output blocks are independent, so the eight waves run without barriers
@@ -17,6 +18,7 @@
 // is row 8 q + 4 (lane / 32) + r, column lane % 32.
 #include "device_common.hpp"
 #include "internal.hpp"
+#include "lu32.hpp"
 
 namespace hplai {
 
@@ -479,6 +481,170 @@ __global__ __launch_bounds__(kTriThreads) void trsm_u_tri16_kernel(int b, int64_
     tile_max_reduce(amax, j0 / tb, vmax, true);
 }
 
+// The caller's own triangle (hplai_trsm_*) where b > 512 or b % 32 != 0: the
+// strip is solved 32 rows (U panel) or columns (L panel) at a time through the
+// inverses of the 32 x 32 diagonal blocks only.  A product with the whole
+// inverse has the error of that walk times the triangle's condition: 31 u
+// against 2.7 u of |T| |X| for order 777 and condition 1e4, 6e5 u against 3.2 u
+// for 4e8.  (b <= 512 in whole 32-blocks takes the whole inverse, and so does
+// the LU, whose triangles are its own factors.)
+// The strip lives in accumulators, transposed for the L panel, so that a block
+// of the result is the right operand of the next products as it is (k =
+// acc_row); wave w holds blocks w, w + 8, ..  Step K: X_K is in LDS; the wave of
+// block K + 1 updates that block, solves it and stores it before its other
+// blocks, so a step is two products of the chain or the updates, whichever is
+// longer.  A wave's operands of the next step are loaded as soon as the
+// registers are free.  What bounds it: those two products a step up to a strip
+// per CU, then the FP32 matrix cores at one workgroup per CU (245 registers).  b
+// = 777, L / U, with the inverses: 4000 wide 109 / 126 us, 40000 wide 483 / 534
+// (with the whole inverse 167 / 143 and 419 / 387, by substitution on one row or
+// column per thread 2784 / 11500 and 4267 / 15062); b = 60, 40000 wide 33 / 32
+// (28.6 / 27.9; 50 / 63 with the walk in LDS).
+template <bool UP, int PER, bool VEC>
+__global__ __launch_bounds__(kTriThreads) void trsm_walk_kernel(int64_t m, int b, const float *__restrict__ tri,
+                                                                const float *__restrict__ T, int64_t ldt,
+                                                                float *__restrict__ P, int64_t ldp)
+{
+    __shared__ float xl[2][1024];   // -X_K, [kk 64 + lane]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, lh = lane >> 5, nb = (b + 31) / 32;
+    const int64_t p0 = static_cast<int64_t>(blockIdx.x) * kStrip;
+    const int cnt = m - p0 < kStrip ? static_cast<int>(m - p0) : kStrip;
+    // row (U panel) or column (L panel) `index` of the strip's lane
+    const int64_t step = UP ? 1 : ldp;
+    float *strip = P + (UP ? (p0 + min(l32, cnt - 1)) * ldp : p0 + min(l32, cnt - 1));
+    // left operand of block J's product with X_K: T(J, K), for the L panel U(K, J)^T
+    auto load_left = [&](float (&v)[16], int J, int K) {
+        const int64_t j = min(32 * J + l32, b - 1);
+        if constexpr (UP) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) v[e] = T[static_cast<int64_t>(32 * K + acc_row(e, lh)) * ldt + j];
+        } else {
+            const float *col = T + j * ldt + 32 * K + 4 * lh;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (VEC) {
+                    const float4 x = *reinterpret_cast<const float4 *>(col + 8 * q);
+                    v[4 * q] = x.x;
+                    v[4 * q + 1] = x.y;
+                    v[4 * q + 2] = x.z;
+                    v[4 * q + 3] = x.w;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[4 * q + r] = col[8 * q + r];
+                }
+            }
+        }
+    };
+    // the inverse of diagonal block J: entry (l32, acc_row), for the L panel (acc_row, l32)
+    auto inverse = [&](int J) { return UP ? tri_block_l(tri, nb, J, J) : tri_block_u(tri, nb, J, J); };
+    float iv[16];
+    auto load_inverse = [&](int J) {
+        const float *o = inverse(J) + l32 * 4 + 2 * lh;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float2 even = *reinterpret_cast<const float2 *>(o + 256 * q);
+            const float2 odd = *reinterpret_cast<const float2 *>(o + 256 * q + 128);
+            iv[4 * q] = even.x;
+            iv[4 * q + 1] = odd.x;
+            iv[4 * q + 2] = even.y;
+            iv[4 * q + 3] = odd.y;
+        }
+    };
+    floatx16t_t acc[PER];
+    float left[PER][16];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int J = wave + 8 * i;
+        if (J >= nb) continue;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][e] = strip[min(32 * J + acc_row(e, lh), b - 1) * step];
+    }
+    if (wave < nb) load_inverse(wave);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int J = wave + 8 * i;
+        if (J >= nb) continue;
+        if (J > 0) load_left(left[i], J, 0);
+        if (32 * J + 32 > b)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][e] = 32 * J + acc_row(e, lh) < b ? acc[i][e] : 0.0f;
+    }
+    // X_J := inverse of block J times D
+    auto solve = [&](int J, const floatx16t_t &D) {
+        int ln = lane;   // addresses that are not kept through the walk
+        asm volatile("" : "+v"(ln));
+        const int h = ln >> 5;
+        float *out = &xl[J & 1][ln];
+        floatx16t_t x;
+        bool fine = true;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            x[e] = 0.0f;
+            fine = fine && isfinite(D[e]);
+        }
+        if (__all(fine)) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) x = __builtin_amdgcn_mfma_f32_32x32x2f32(iv[e], D[e], x, 0, 0, 0);
+        } else {
+            // the zeros of the inverse would carry it to the entries before
+#pragma unroll
+            for (int e = 0; e < 16; ++e) out[64 * e] = D[e];
+            wave_lds_sync();
+            const float *o = inverse(J);
+#pragma clang loop unroll(disable)
+            for (int k = 0; k < 32; ++k) {
+                const float d = xl[J & 1][((k >> 3) * 4 + (k & 3)) * 64 + ((k >> 2) & 1) * 32 + (ln & 31)];
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int j = acc_row(e, h);
+                    if (k <= j) x[e] = fmaf(o[tri_pos(j + 32 * (k & 1), k >> 1)], d, x[e]);
+                }
+            }
+            wave_lds_sync();
+        }
+        float *dst = strip + static_cast<int64_t>(32 * J + 4 * h) * step;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            out[64 * e] = -x[e];
+            if ((ln & 31) < cnt && 32 * J + acc_row(e, h) < b) dst[static_cast<int64_t>(acc_row(e, 0)) * step] = x[e];
+        }
+        if (J + 8 < nb) load_inverse(J + 8);
+    };
+    auto update = [&](int i, int J, int K, const float (&xv)[16]) {
+        if (32 * J + 32 > b)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) left[i][e] = 32 * J + l32 < b ? left[i][e] : 0.0f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(left[i][e], xv[e], acc[i], 0, 0, 0);
+        if (J > K + 1) load_left(left[i], J, K + 1);
+    };
+    for (int K = -1; K + 1 < nb; ++K) {
+        __syncthreads();   // X_K is there, X_(K-1) no longer read
+        float xv[16];
+        if (K >= 0)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) xv[e] = xl[K & 1][e * 64 + lane];
+        __builtin_amdgcn_sched_barrier(0);
+        floatx16t_t D;
+        bool mine = false;
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (wave + 8 * i == K + 1) {
+                if (K >= 0) update(i, K + 1, K, xv);
+                D = acc[i];
+                mine = true;
+            }
+        if (mine) solve(K + 1, D);
+        if (K < 0) continue;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int J = wave + 8 * i;
+            if (J > K + 1 && J < nb) update(i, J, K, xv);
+        }
+    }
+}
+
 // x_out := Tinv x_in for one factored diagonal block (the IR's diagonal-block
 // solve as a product with the stored inverse): Linv (UPPER = false, the unit
 // lower solve) or Uinv (UPPER = true).  Workgroup I computes rows
@@ -602,6 +768,40 @@ int launch_trsm_u(int b, int64_t n, const float *tri, float *U, int64_t ldu, flo
     }
     HPLAI_HIP(hipGetLastError());
     return HPLAI_OK;
+}
+
+template <bool UP>
+static int trsm_walk(int64_t m, int b, const float *tri, const float *T, int64_t ldt, float *P, int64_t ldp,
+                     hipStream_t s)
+{
+    const dim3 g(static_cast<unsigned>(ceil_div(m, kStrip))), th(kTriThreads);
+    const int nb = (b + 31) / 32;
+    auto launch = [&](auto per) {
+        constexpr int PER = decltype(per)::value;
+        if (!UP && aligned16(T, ldt))   // L's columns are read along the lanes
+            hipLaunchKernelGGL((trsm_walk_kernel<UP, PER, !UP>), g, th, 0, s, m, b, tri, T, ldt, P, ldp);
+        else
+            hipLaunchKernelGGL((trsm_walk_kernel<UP, PER, false>), g, th, 0, s, m, b, tri, T, ldt, P, ldp);
+    };
+    if (nb <= 8)
+        launch(std::integral_constant<int, 1>{});
+    else if (nb <= 16)
+        launch(std::integral_constant<int, 2>{});
+    else
+        launch(std::integral_constant<int, 4>{});
+    HPLAI_HIP(hipGetLastError());
+    return HPLAI_OK;
+}
+
+int launch_trsm_panel(bool up, int64_t m, int b, const float *T, int64_t ldt, float *tri, float *P, int64_t ldp,
+                      hipStream_t s)
+{
+    if (m <= 0 || b <= 0) return HPLAI_OK;
+    const bool whole = b <= 512 && b % 32 == 0;
+    const int rc = launch_tri_inverse(b, T, ldt, tri, up ? 1 : 2, whole, s);
+    if (rc) return rc;
+    if (!whole) return up ? trsm_walk<true>(m, b, tri, T, ldt, P, ldp, s) : trsm_walk<false>(m, b, tri, T, ldt, P, ldp, s);
+    return up ? launch_trsm_u(b, m, tri, P, ldp, nullptr, 1, s) : launch_trsm_l(m, b, tri, P, ldp, nullptr, 1, s);
 }
 
 }  // namespace hplai

@@ -166,3 +166,73 @@ def test_narrow_strips_add_the_diagonal_last(ctx, oracle, b):
     ctx.trsm_upanel(b, 2000, F, b, narrow, b)
     for got, w in ((wide, want), (narrow, want[:2000])):
         assert ((got.double() - w).norm() / w.norm()).item() < 1.5 * 2.0 ** -25
+
+
+def _hard_triangle(b, rng):
+    """Unit lower, 32 x 32 diagonal blocks near the identity, condition 1e6 and more as a whole."""
+    T = rng.standard_normal((b, b)) * (0.2 if b > 500 else 1.0)
+    for i in range(0, b, 32):
+        T[i:i + 32, i:i + 32] = rng.uniform(-0.5, 0.5, T[i:i + 32, i:i + 32].shape) / 32
+    return (np.tril(T, -1) + np.eye(b)).astype(np.float32)
+
+
+@pytest.mark.parametrize("b", [60, 100, 257, 500, 513, 640, 777, 1000, 1024])
+@pytest.mark.parametrize("m,pad", [(1, 0), (33, 1), (700, 4)])
+def test_trsm_ill_conditioned(ctx, b, m, pad):
+    """The entrywise bound of substitution in 32-blocks: |B - T X| <= g |T| |X|
+    with g = 2 (b + 64) u, u = 2^-24.  b + 32 roundings of the products and the
+    subtractions; 32 more and the factor 2 for the 32 x 32 inverses, whose
+    |D^-1| |D| is below 2."""
+    import torch
+    rng = np.random.default_rng(b + m)
+    L = _hard_triangle(b, rng)
+    D = rng.uniform(0.5, 2.0, b).astype(np.float32)
+    U = (np.ascontiguousarray(L.T) * D[None, :]).astype(np.float32)          # upper, columns scaled
+    u = 2.0 ** -24
+    X0 = rng.standard_normal((b, m))
+    for up in (True, False):
+        T = L.astype(np.float64) if up else U.T.astype(np.float64)           # op on a b x m panel of columns
+        B = (T @ X0).astype(np.float32)
+        M = L if up else U
+        F = torch.from_numpy(np.ascontiguousarray(np.pad(M.T, ((0, 0), (0, pad))))).cuda()
+        # U panel: column j at P[j]; L panel: row i of the panel is column i here, P[k, i]
+        P = torch.from_numpy(np.ascontiguousarray(np.pad(B.T if up else B, ((0, 0), (0, pad))))).cuda()
+        before = P.clone()
+        if up:
+            ctx.trsm_upanel(b, m, F, b + pad, P, b + pad)
+            X = P.cpu().numpy()[:, :b].T.astype(np.float64)
+            assert torch.equal(P[:, b:], before[:, b:])
+        else:
+            ctx.trsm_lpanel(m, b, F, b + pad, P, m + pad)
+            X = P.cpu().numpy()[:, :m].astype(np.float64)
+            assert torch.equal(P[:, m:], before[:, m:])
+        R = np.abs(B.astype(np.float64) - T @ X)
+        bound = 2 * (b + 64) * u * (np.abs(T) @ np.abs(X))
+        assert np.isfinite(X).all()
+        assert (R <= bound).all(), (up, float((R / bound).max()))
+
+
+@pytest.mark.parametrize("b", [100, 600])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_trsm_entries_before_a_nonfinite_one_stay(ctx, b, bad):
+    """Entry k of one row or column: what the triangle solves before it, and the
+    other rows or columns, are not touched."""
+    import torch
+    rng = np.random.default_rng(b)
+    m, k, j = 40, b - 45, 7
+    T = torch.from_numpy((rng.uniform(-0.5, 0.5, (b, b)) / b + 2 * np.eye(b)).astype(np.float32)).cuda()
+    P = torch.from_numpy(rng.uniform(-0.5, 0.5, (m, b)).astype(np.float32)).cuda()
+    for up in (True, False):
+        good = P.clone() if up else P.t().contiguous()
+        got = good.clone()
+        (got if up else got.t())[j, k] = bad
+        for Q in (good, got):
+            if up:
+                ctx.trsm_upanel(b, m, T, b, Q, b)
+            else:
+                ctx.trsm_lpanel(m, b, T, b, Q, m)
+        a, w = (got, good) if up else (got.t(), good.t())
+        keep = torch.ones_like(w, dtype=torch.bool)
+        keep[j, k:] = False
+        assert not torch.isfinite(a[j, k])
+        assert ((a - w)[keep].abs().max() / w.abs().max()).item() < 1e-6
