@@ -1017,7 +1017,7 @@ int hplai_batch_autotune(hplai_batch b, int maxit, int32_t nb_out[4])
     int32_t best[kBuckets];
     for (int k = 0; k < kBuckets; ++k) best[k] = b->nb_table[k];
     int32_t *d_sub = nullptr;
-    HPLAI_HIP(hipMalloc(&d_sub, sizeof(int32_t) * b->count));
+    HPLAI_HIP(device_malloc(b->ctx->device, reinterpret_cast<void **>(&d_sub), sizeof(int32_t) * b->count));
     int rc = HPLAI_OK;
     for (int k = 0; k < kBuckets && rc == HPLAI_OK; ++k) {
         // up to 2 systems per CU of this bucket, largest first

@@ -66,6 +66,7 @@ int hip_fail(hipError_t e, const char *what);
 // ---- device memory (memory.hip) ----
 int block_cache_open(int device, size_t device_bytes);
 void block_cache_close(int device);
+bool block_cache_empty(int device);
 hipError_t device_malloc(int device, void **p, size_t bytes);
 hipError_t block_alloc(int device, void **p, size_t *bytes);
 void block_free(int device, void *p, size_t bytes);

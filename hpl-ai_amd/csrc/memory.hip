@@ -71,21 +71,33 @@ void block_cache_close(int device)
     if (--c.contexts == 0) trim_locked(c, 0);
 }
 
-// hipMalloc that empties the device's cache before it gives up.
-hipError_t device_malloc(int device, void **p, size_t bytes)
+// Every idle block back to the device; false if there was none.
+bool block_cache_empty(int device)
 {
-    hipError_t e = hipMalloc(p, bytes);
+    BlockCache &c = g_cache[device];
+    std::lock_guard<std::mutex> lock(c.mu);
+    const bool some = c.count > 0;
+    trim_locked(c, 0);
+    return some;
+}
+
+namespace {
+// an allocation that empties the device's cache before it gives up
+template <typename F>
+hipError_t or_empty_cache(int device, F &&alloc)
+{
+    hipError_t e = alloc();
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        BlockCache &c = g_cache[device];
-        {
-            std::lock_guard<std::mutex> lock(c.mu);
-            if (c.total == 0) return e;
-            trim_locked(c, 0);
-        }
-        e = hipMalloc(p, bytes);
+        if (block_cache_empty(device)) e = alloc();
     }
     return e;
+}
+}  // namespace
+
+hipError_t device_malloc(int device, void **p, size_t bytes)
+{
+    return or_empty_cache(device, [&] { return hipMalloc(p, bytes); });
 }
 
 // The smallest idle block of the size asked for or up to an eighth more, else
@@ -145,8 +157,8 @@ ScratchLease::ScratchLease(hplai_ctx ctx, hipStream_t stream, size_t bytes) : st
     // a captured call needs memory of its own: its graph may run beside later
     // calls on this stream
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (bytes <= kScratchMax && hipStreamIsCapturing(stream, &cap) == hipSuccess &&
-        cap == hipStreamCaptureStatusNone) {
+    const bool eager = hipStreamIsCapturing(stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+    if (eager && bytes <= kScratchMax) {
         // held until the call's kernels are enqueued: no other call on this
         // context can put its own between them
         lock_ = std::unique_lock<std::mutex>(sc.mu);
@@ -182,7 +194,8 @@ ScratchLease::ScratchLease(hplai_ctx ctx, hipStream_t stream, size_t bytes) : st
         return;
     }
     (void)hipGetLastError();
-    const hipError_t err = hipMallocAsync(&ptr, bytes, stream);
+    auto alloc = [&] { return hipMallocAsync(&ptr, bytes, stream); };
+    const hipError_t err = eager ? or_empty_cache(ctx->device, alloc) : alloc();
     if (err != hipSuccess) {
         ptr = nullptr;
         rc = hip_fail(err, "hipMallocAsync scratch");

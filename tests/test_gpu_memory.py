@@ -102,3 +102,24 @@ def test_what_stays_allocated_is_bounded(ctx):
         ctx.release()
         assert torch.cuda.mem_get_info()[0] >= min(free0, total) - total // 6 - (1 << 30)
     assert total - torch.cuda.mem_get_info()[0] <= total // 6 + (8 << 30)
+
+
+def test_large_scratch_takes_what_the_cache_holds(ctx):
+    """A call whose scratch is allocated in stream order (3.2 GB of partial
+    sums), with the device full but for 2 GB and the solve's idle buffers."""
+    import torch
+    n = 900000
+    torch.cuda.empty_cache()
+    d, x, want = _residual_case(ctx, n, 5)
+    ctx.solve(65536, 512, fmt="e4m3", outer=16)            # 18 GB of buffers, kept idle
+    torch.cuda.synchronize()
+    y = torch.zeros_like(want)
+    hog = torch.empty(torch.cuda.mem_get_info()[0] - (2 << 30), dtype=torch.uint8, device="cuda")
+    try:
+        assert torch.cuda.mem_get_info()[0] < 3 << 30
+        ctx.otf_gemv(n, 5, d, 1.0, x, y)
+        torch.cuda.synchronize()
+    finally:
+        del hog
+        torch.cuda.empty_cache()
+    assert torch.equal(y, want)
