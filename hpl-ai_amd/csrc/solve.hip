@@ -749,6 +749,18 @@ int hplai_release(hplai_ctx ctx)
     return HPLAI_OK;
 }
 
+int hplai_trim(hplai_ctx ctx)
+{
+    HPLAI_CHECK(ctx != nullptr, "null hplai_ctx");
+    HPLAI_HIP(hipSetDevice(ctx->device));
+    {
+        std::lock_guard<std::mutex> lock(ctx->pool.mu);
+        ctx->pool.clear(ctx->device);
+    }
+    (void)block_cache_empty(ctx->device);
+    return HPLAI_OK;
+}
+
 int hplai_solution_x(hplai_ctx ctx, double *x_host)
 {
     HPLAI_CHECK(ctx != nullptr && ctx->x != nullptr && x_host != nullptr,

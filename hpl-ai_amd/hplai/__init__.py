@@ -112,6 +112,7 @@ _SIGS = [
     ("hplai_solution_factors", _int, [_vp, _vp, _i64]),
     ("hplai_solution_block", _int, [_vp, _i64, _i64, _i64, _i64, _vp, _i64]),
     ("hplai_release", _int, [_vp]),
+    ("hplai_trim", _int, [_vp]),
 ]
 
 _lib = None
@@ -360,7 +361,12 @@ class Context:
         return blk
 
     def release(self):
+        """Drops the kept factors and solution; their memory stays for the next solve."""
         check(lib().hplai_release(self.handle))
+
+    def trim(self):
+        """Gives the memory that is kept for later calls back to the device."""
+        check(lib().hplai_trim(self.handle))
 
 
 def exported_symbols():

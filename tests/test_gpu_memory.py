@@ -123,3 +123,27 @@ def test_large_scratch_takes_what_the_cache_holds(ctx):
         del hog
         torch.cuda.empty_cache()
     assert torch.equal(y, want)
+
+
+def test_trim_gives_everything_back(ctx):
+    """After a trim the device has what it had before: for another allocator
+    (torch's here) that cannot reach the library's idle memory."""
+    import torch
+    n = 20000
+    d, x, want = _residual_case(ctx, n, 6)
+    torch.cuda.empty_cache()
+    ctx.trim()
+    free0 = torch.cuda.mem_get_info()[0]
+    r = ctx.solve(65536, 512, fmt="e4m3", outer=16, keep_factors=True)
+    sol = ctx.solution_x(65536)
+    y = torch.zeros_like(want)
+    ctx.otf_gemv(n, 6, d, 1.0, x, y)
+    ctx.trim()
+    assert torch.equal(y, want)
+    assert np.array_equal(ctx.solution_x(65536), sol)      # kept until they are released
+    ctx.release()
+    assert torch.cuda.mem_get_info()[0] < free0 - (15 << 30)   # A, 16 GiB, is idle now
+    ctx.trim()
+    torch.cuda.empty_cache()
+    assert torch.cuda.mem_get_info()[0] >= free0 - (64 << 20)
+    assert ctx.solve(65536, 512, fmt="e4m3", outer=16)["checksum"] == r["checksum"]
