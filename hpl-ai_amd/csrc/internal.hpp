@@ -16,13 +16,16 @@ struct StreamScratch {
         void *p;
         hipEvent_t done;   // end of the last use
         size_t bytes;
+        bool owned;        // its stream's buffer, not an outgrown one
     };
     static constexpr int kMax = 32;
+    static constexpr size_t kTotal = size_t(1) << 30;   // kept in all
     std::mutex mu;
     Entry entries[kMax];
     int count = 0;
     size_t total = 0;
-    void drop(int device, Entry *e);
+    Entry *find(hipStream_t stream);
+    Entry *replace(int device, Entry *old, hipStream_t stream, size_t bytes, hipError_t *err);
     void clear(int device);
 };
 }  // namespace hplai
@@ -70,6 +73,7 @@ bool block_cache_empty(int device);
 hipError_t device_malloc(int device, void **p, size_t bytes);
 hipError_t block_alloc(int device, void **p, size_t *bytes);
 void block_free(int device, void *p, size_t bytes);
+bool block_put(int device, void *p, size_t bytes);
 
 // `bytes` of scratch for one call's kernels on `stream`, from construction to
 // the end of the scope that enqueues them.

@@ -5,7 +5,9 @@
 //    points, one buffer per stream.  An event marks the end of each use; the
 //    next call waits for it on its own stream, which costs nothing where the
 //    stream is the same (a destroyed stream's handle may come back as another
-//    stream, so the handle alone proves no order).  A stream-ordered
+//    stream, so the handle alone proves no order).  No call waits on the host,
+//    also where its buffer has to grow; a call that finds no room allocates in
+//    stream order.  A stream-ordered
 //    allocation per call instead stalls: on this runtime hipFreeAsync of
 //    memory that an earlier call had freed waits for the device, which made
 //    every second such call synchronous (18 us a call at least, 4 us as here).
@@ -124,31 +126,39 @@ hipError_t block_alloc(int device, void **p, size_t *bytes)
     return device_malloc(device, p, *bytes);
 }
 
-// p must be idle on the device.
+namespace {
+// into the cache if it has room for the block; the caller holds c.mu
+bool put_locked(BlockCache &c, void *p, size_t bytes)
+{
+    if (c.contexts == 0 || c.count == kMaxIdle || c.total + bytes > c.bound) return false;
+    c.idle[c.count++] = Block{p, bytes};
+    c.total += bytes;
+    return true;
+}
+}  // namespace
+
+// p must be idle on the device.  Older blocks make room; freeing one waits for the device.
 void block_free(int device, void *p, size_t bytes)
 {
     if (p == nullptr) return;
     BlockCache &c = g_cache[device];
     {
         std::lock_guard<std::mutex> lock(c.mu);
-        if (c.contexts > 0 && bytes <= c.bound) {
-            trim_locked(c, c.bound - bytes);
-            if (c.count < kMaxIdle) {
-                c.idle[c.count++] = Block{p, bytes};
-                c.total += bytes;
-                return;
-            }
-        }
+        if (c.contexts > 0 && bytes <= c.bound) trim_locked(c, c.bound - bytes);
+        if (put_locked(c, p, bytes)) return;
     }
     (void)hipFree(p);
 }
 
-// ---------------------------------------------------------------------------
+// The same without a wait: false, and p still the caller's, if there is no room.
+bool block_put(int device, void *p, size_t bytes)
+{
+    BlockCache &c = g_cache[device];
+    std::lock_guard<std::mutex> lock(c.mu);
+    return put_locked(c, p, bytes);
+}
 
-namespace {
-// per context: kept in all, and the largest buffer kept
-constexpr size_t kScratchTotal = size_t(1) << 30;
-}  // namespace
+// ---------------------------------------------------------------------------
 
 ScratchLease::ScratchLease(hplai_ctx ctx, hipStream_t stream, size_t bytes) : stream_(stream)
 {
@@ -162,36 +172,22 @@ ScratchLease::ScratchLease(hplai_ctx ctx, hipStream_t stream, size_t bytes) : st
         // held until the call's kernels are enqueued: no other call on this
         // context can put its own between them
         lock_ = std::unique_lock<std::mutex>(sc.mu);
-        StreamScratch::Entry *e = nullptr;
-        for (int k = 0; k < sc.count; ++k)
-            if (sc.entries[k].stream == stream) e = &sc.entries[k];
-        if (e == nullptr || e->bytes < bytes) {
-            size_t want = size_t(1) << 20;
-            while (want < bytes) want *= 2;
-            if (e != nullptr) sc.drop(ctx->device, e);   // outgrown
-            // buffers of many streams, some of them gone
-            if (sc.total + want > kScratchTotal || sc.count == StreamScratch::kMax) sc.clear(ctx->device);
-            StreamScratch::Entry n{stream, nullptr, nullptr, want};
-            hipError_t err = hipEventCreateWithFlags(&n.done, hipEventDisableTiming);
-            if (err == hipSuccess) err = block_alloc(ctx->device, &n.p, &n.bytes);
-            if (err != hipSuccess) {
-                if (n.done != nullptr) (void)hipEventDestroy(n.done);
-                rc = hip_fail(err, "scratch memory");
-                return;
-            }
-            e = &sc.entries[sc.count++];
-            *e = n;
-            sc.total += n.bytes;
-        } else {
-            const hipError_t err = hipStreamWaitEvent(stream, e->done, 0);
-            if (err != hipSuccess) {
-                rc = hip_fail(err, "hipStreamWaitEvent scratch");
-                return;
-            }
+        StreamScratch::Entry *e = sc.find(stream);
+        hipError_t err = hipSuccess;
+        if (e != nullptr && e->bytes >= bytes)
+            err = hipStreamWaitEvent(stream, e->done, 0);
+        else
+            e = sc.replace(ctx->device, e, stream, bytes, &err);
+        if (err != hipSuccess) {
+            rc = hip_fail(err, "scratch memory");
+            return;
         }
-        ptr = e->p;
-        done_ = e->done;
-        return;
+        if (e != nullptr) {
+            ptr = e->p;
+            done_ = e->done;
+            return;
+        }
+        lock_.unlock();   // no room: this call's own
     }
     (void)hipGetLastError();
     auto alloc = [&] { return hipMallocAsync(&ptr, bytes, stream); };
@@ -210,18 +206,73 @@ ScratchLease::~ScratchLease()
     if (done_ != nullptr) (void)hipEventRecord(done_, stream_);
 }
 
-void StreamScratch::drop(int device, Entry *e)
+StreamScratch::Entry *StreamScratch::find(hipStream_t stream)
 {
-    (void)hipEventSynchronize(e->done);
-    (void)hipEventDestroy(e->done);
-    block_free(device, e->p, e->bytes);
-    total -= e->bytes;
-    *e = entries[--count];
+    for (int k = 0; k < count; ++k)
+        if (entries[k].owned && entries[k].stream == stream) return &entries[k];
+    return nullptr;
 }
 
+// A buffer of at least `bytes` for `stream` in place of `old` (may be NULL),
+// which is outgrown: its memory may be in use until its event has passed.  No
+// work is waited for: buffers that are done with go back to the block cache
+// where it has room, or to the call if they fit; NULL without an error if all
+// others are in use.
+StreamScratch::Entry *StreamScratch::replace(int device, Entry *old, hipStream_t stream, size_t bytes, hipError_t *err)
+{
+    // allocating and asking for events is legal beside another stream's capture only so
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    Entry *fit = nullptr;
+    if (old != nullptr) old->owned = false;
+    size_t want = size_t(1) << 20;
+    while (want < bytes) want *= 2;
+    // twice: buffers without a stream, then, if there is no room yet, other streams' as well
+    for (int pass = 0; pass < 2 && fit == nullptr; ++pass) {
+        if (pass == 1 && total + want <= kTotal && count < kMax) break;
+        for (int k = count - 1; k >= 0 && fit == nullptr; --k) {
+            Entry &e = entries[k];
+            if ((pass == 0 && e.owned) || hipEventQuery(e.done) != hipSuccess) continue;
+            if (e.bytes >= want) {
+                fit = &e;
+            } else if (block_put(device, e.p, e.bytes)) {
+                (void)hipEventDestroy(e.done);
+                total -= e.bytes;
+                e = entries[--count];
+            }
+        }
+    }
+    (void)hipGetLastError();   // hipErrorNotReady
+    if (fit == nullptr && total + want <= kTotal && count < kMax) {
+        Entry n{stream, nullptr, nullptr, want, true};
+        *err = hipEventCreateWithFlags(&n.done, hipEventDisableTiming);
+        if (*err == hipSuccess) *err = block_alloc(device, &n.p, &n.bytes);
+        if (*err == hipSuccess) {
+            fit = &entries[count++];
+            *fit = n;
+            total += n.bytes;
+        } else if (n.done != nullptr) {
+            (void)hipEventDestroy(n.done);
+        }
+    }
+    if (fit != nullptr) {
+        fit->stream = stream;
+        fit->owned = true;
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return fit;
+}
+
+// Everything back, after the work enqueued on it.
 void StreamScratch::clear(int device)
 {
-    while (count > 0) drop(device, &entries[count - 1]);
+    for (; count > 0; --count) {
+        Entry &e = entries[count - 1];
+        (void)hipEventSynchronize(e.done);
+        (void)hipEventDestroy(e.done);
+        block_free(device, e.p, e.bytes);
+    }
+    total = 0;
 }
 
 }  // namespace hplai

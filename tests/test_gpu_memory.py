@@ -147,3 +147,92 @@ def test_trim_gives_everything_back(ctx):
     torch.cuda.empty_cache()
     assert torch.cuda.mem_get_info()[0] >= free0 - (64 << 20)
     assert ctx.solve(65536, 512, fmt="e4m3", outer=16)["checksum"] == r["checksum"]
+
+
+def _busy(stream, ms=300):
+    """A spinning kernel of about `ms` on the stream, and an event behind it."""
+    import torch
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(1000)                              # loaded before it is timed
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        torch.cuda._sleep(1 << 20)
+        b.record()
+    stream.synchronize()
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(int((1 << 20) * ms / max(a.elapsed_time(b), 1e-3)))
+        done = torch.cuda.Event()
+        done.record()
+    return done
+
+
+def test_a_growing_buffer_does_not_wait_for_its_stream():
+    import hplai
+    import torch
+    cases = [(n, 7) + _residual_case(hplai.Context(0), n, 7) for n in (500, 3000, 9000, 30000)]
+    c = hplai.Context(0)
+    for first in (1, 0):                                     # once with the kernels loaded
+        st = torch.cuda.Stream()
+        outs = []
+        done = _busy(st)
+        with torch.cuda.stream(st):
+            for n, s, d, x, _ in cases:
+                y = torch.zeros(n, dtype=torch.float64, device="cuda")
+                c.otf_gemv(n, s, d, 1.0, x, y)
+                outs.append(y)
+        waited = done.query()
+        st.synchronize()
+        for y, case in zip(outs, cases):
+            assert torch.equal(y, case[4])
+        assert first or not waited
+    c.close()
+
+
+def test_streams_past_the_bound_do_not_wait():
+    """Three streams with buffers of 512 MiB: the third's call does not wait for
+    the other two, whose buffers stay theirs."""
+    import hplai
+    import torch
+    c = hplai.Context(0)
+    n, m, k = 4096, 4096, 1 << 15                            # (n + m) k 2 bytes: 512 MiB
+    g = torch.Generator(device="cuda").manual_seed(1)
+    a = torch.rand(k, n, generator=g, device="cuda").half()
+    b = torch.rand(m, k, generator=g, device="cuda").half()
+    want = torch.zeros(m, n, device="cuda")
+    c.gemmschur_f16(n, m, k, a, n, b, k, want, n)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    outs = [torch.zeros(m, n, device="cuda") for _ in range(3)]
+    torch.cuda.synchronize()
+    done = [_busy(st, 500) for st in streams]
+    for st, out in zip(streams, outs):
+        c.gemmschur_f16(n, m, k, a, n, b, k, out, n, stream=st)
+    assert not any(e.query() for e in done)
+    torch.cuda.synchronize()
+    for out in outs:
+        assert torch.equal(out, want)
+    c.close()
+
+
+def test_first_call_on_a_stream_beside_another_streams_capture():
+    """While a stream of the thread is captured (global mode), a call on another
+    stream may not use what such a capture forbids."""
+    import hplai
+    import torch
+    c = hplai.Context(0)
+    n = 3000
+    d, x, want = _residual_case(c, n, 3)
+    y, z = torch.zeros_like(want), torch.zeros_like(want)
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, capture_error_mode="global"):
+        z.add_(1.0)
+        c.otf_gemv(n, 3, d, 1.0, x, y, stream=other)
+    other.synchronize()
+    assert torch.equal(y, want)
+    for k in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (z == k + 1).all()
+    c.close()
