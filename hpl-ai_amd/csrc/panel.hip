@@ -82,6 +82,60 @@ __global__ __launch_bounds__(kAmaxThreads) void tile_amax_kernel(int side, int64
     }
 }
 
+// The same for tiles of fewer than kAmaxShort lines: a workgroup takes the whole
+// tiles of up to 64 lines, rows along the lanes (side 0) or a column per wave
+// (side 1), and the lines' maxima meet in LDS.
+template <int FMT>
+__global__ __launch_bounds__(kAmaxThreads) void tile_amax_short_kernel(int side, int64_t m, int64_t k, int tb, int group,
+                                                                       const float *__restrict__ src, int64_t lds,
+                                                                       int32_t *__restrict__ exps)
+{
+    constexpr int W = kAmaxThreads / 64, UN = 8;
+    __shared__ float part[W][64], line[64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t l0 = static_cast<int64_t>(blockIdx.x) * group;
+    const int cnt = m - l0 < group ? static_cast<int>(m - l0) : group;
+    if (side == 0) {
+        const float *row = src + l0 + min(lane, cnt - 1);
+        float v = 0.0f;
+        for (int64_t c = wave; c < k; c += W * UN) {
+            float x[UN];
+#pragma unroll
+            for (int u = 0; u < UN; ++u) x[u] = row[(c + W * u < k ? c + W * u : c) * lds];
+#pragma unroll
+            for (int u = 0; u < UN; ++u) v = fmaxf(v, fabsf(x[u]));
+        }
+        part[wave][lane] = v;
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int q = 1; q < W; ++q) v = fmaxf(v, part[q][lane]);
+            line[lane] = v;
+        }
+    } else {
+        for (int j = wave; j < cnt; j += W) {
+            const float *col = src + (l0 + j) * lds;
+            float v = 0.0f;
+            for (int64_t r = lane; r < k; r += 64 * UN) {
+                float x[UN];
+#pragma unroll
+                for (int u = 0; u < UN; ++u) x[u] = col[r + 64 * u < k ? r + 64 * u : r];
+#pragma unroll
+                for (int u = 0; u < UN; ++u) v = fmaxf(v, fabsf(x[u]));
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
+            if (lane == 0) line[j] = v;
+        }
+    }
+    __syncthreads();
+    if (tid * tb < cnt) {
+        float v = line[tid * tb];
+        for (int q = tid * tb + 1; q < min(tid * tb + tb, cnt); ++q) v = fmaxf(v, line[q]);
+        exps[l0 / tb + tid] = amax_exponent<FMT>(v);
+    }
+}
+
 __global__ void fill_f32_kernel(float *p, int64_t cnt, float v)
 {
     const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -329,10 +383,13 @@ __global__ __launch_bounds__(256) void quant_u16_kernel(int64_t m, int64_t k, in
 // 26 from HBM (with the conversion, panels that are in the cache: 16 tiles of
 // 512 x 1024 21 for 32, 8 of 512 x 512 12 for 14, 64 of them 31 for 30; 120 of
 // them were 49 for 43, hence the line).
+// Tiles of fewer than kAmaxShort lines share a workgroup.
 constexpr int64_t kAmaxTile = int64_t(1) << 19, kAmaxPart = int64_t(1) << 18;
+constexpr int kAmaxShort = 16;
 
 int tile_amax_splits(int64_t m, int64_t k, int tb)
 {
+    if (tb < kAmaxShort) return 1;
     const int64_t entries = (m < tb ? m : tb) * k, s = ceil_div(entries, kAmaxTile);
     if (s > kAmaxSlots) return static_cast<int>(s < 64 ? s : 64);
     return s > 1 || (entries >= kAmaxPart && ceil_div(m, tb) * kAmaxSlots <= 256) ? kAmaxSlots : 1;
@@ -347,17 +404,30 @@ int launch_tile_amax(int fmt, int side, int64_t m, int64_t k, int tb, const floa
                      int32_t *exps, hipStream_t s)
 {
     if (m <= 0 || k <= 0) return HPLAI_OK;
-    HPLAI_CHECK(ceil_div(m, tb) < (int64_t(1) << 31), "quantize: %lld tiles", (long long)ceil_div(m, tb));
-    const dim3 g(static_cast<unsigned>(ceil_div(m, tb)),
-                 amax != nullptr ? static_cast<unsigned>(tile_amax_splits(m, k, tb)) : 1u);
+    const unsigned parts = amax != nullptr ? static_cast<unsigned>(tile_amax_splits(m, k, tb)) : 1u;
     const int slots = tile_amax_slots(m, k, tb);
-    if (fmt == HPLAI_FMT_E4M3)
-        hipLaunchKernelGGL(tile_amax_kernel<HPLAI_FMT_E4M3>, g, dim3(kAmaxThreads), 0, s, side, m, k, tb, src, lds,
-                           amax, slots, exps);
-    else
-        hipLaunchKernelGGL(tile_amax_kernel<HPLAI_FMT_F16_TILE>, g, dim3(kAmaxThreads), 0, s, side, m, k, tb, src,
-                           lds, amax, slots, exps);
-    HPLAI_HIP(hipGetLastError());
+    const bool e4m3 = fmt == HPLAI_FMT_E4M3, together = tb < kAmaxShort && amax == nullptr;
+    const int group = together ? 64 / tb * tb : tb;
+    // a launch has at most 2^32 threads
+    const int64_t most = (int64_t(1) << 21) * group;
+    for (int64_t l0 = 0; l0 < m; l0 += most) {
+        const int64_t lines = m - l0 < most ? m - l0 : most;
+        const float *from = src + (side == 0 ? l0 : l0 * lds);
+        int32_t *ex = exps + l0 / tb;
+        float *am = amax != nullptr ? amax + l0 / tb * slots : nullptr;
+        const dim3 g(static_cast<unsigned>(ceil_div(lines, group)), parts), th(kAmaxThreads);
+        if (together && e4m3)
+            hipLaunchKernelGGL(tile_amax_short_kernel<HPLAI_FMT_E4M3>, g, th, 0, s, side, lines, k, tb, group, from, lds, ex);
+        else if (together)
+            hipLaunchKernelGGL(tile_amax_short_kernel<HPLAI_FMT_F16_TILE>, g, th, 0, s, side, lines, k, tb, group, from, lds,
+                               ex);
+        else if (e4m3)
+            hipLaunchKernelGGL(tile_amax_kernel<HPLAI_FMT_E4M3>, g, th, 0, s, side, lines, k, tb, from, lds, am, slots, ex);
+        else
+            hipLaunchKernelGGL(tile_amax_kernel<HPLAI_FMT_F16_TILE>, g, th, 0, s, side, lines, k, tb, from, lds, am, slots,
+                               ex);
+        HPLAI_HIP(hipGetLastError());
+    }
     return HPLAI_OK;
 }
 

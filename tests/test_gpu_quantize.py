@@ -40,3 +40,35 @@ def test_tile_exponents(ctx, oracle, m, k, tb, pad, side, fmt):
         assert np.array_equal(got.reshape(m, k), oracle.f32_to_e4m3_bits(scaled))
     else:
         assert np.array_equal(got.view(np.uint16).reshape(m, k), oracle.f32_to_f16_bits(scaled))
+
+
+@pytest.mark.parametrize("m,k,tb,pad", [(300, 70, 1, 0), (301, 33, 3, 1), (64, 64, 15, 0), (1000, 600, 5, 2),
+                                        (1, 1, 1, 0), (200, 17, 16, 0)])
+@pytest.mark.parametrize("side", [0, 1])
+@pytest.mark.parametrize("fmt", ["e4m3", "f16t"])
+def test_short_tiles(ctx, oracle, m, k, tb, pad, side, fmt):
+    """Tiles of a few lines, several of them in a workgroup's 64."""
+    test_tile_exponents(ctx, oracle, m, k, tb, pad, side, fmt)
+
+
+@pytest.mark.parametrize("tb", [1, 16])
+@pytest.mark.parametrize("side", [0, 1])
+def test_more_tiles_than_one_launch_takes(ctx, oracle, tb, side):
+    import hplai
+    import torch
+    tiles, k = (1 << 22) + 5, 1
+    m = tiles * tb
+    values = (2.0 ** np.arange(-20, 12)).astype(np.float32) * np.float32(1.37)
+    want = np.array([oracle.tile_exp(2, v) for v in values], dtype=np.int32)
+    pick = torch.randint(0, len(values), (tiles,), generator=torch.Generator().manual_seed(1))
+    # one line of a tile holds its maximum
+    src = torch.zeros(m, device="cuda")
+    src[torch.arange(tiles, device="cuda") * tb + tb // 2] = torch.from_numpy(values).cuda()[pick.cuda()]
+    dst = torch.zeros(m, dtype=torch.uint8, device="cuda")
+    exps = torch.full((tiles,), 99, dtype=torch.int32, device="cuda")
+    ctx.quantize(hplai.FMT_E4M3, side, m, k, tb, src, m if side == 0 else k, dst, k, exps)
+    assert np.array_equal(exps.cpu().numpy(), want[pick.numpy()])
+    q = oracle.f32_to_e4m3_bits(np.ldexp(values, want).astype(np.float32))
+    got = dst.cpu().numpy().reshape(tiles, tb)
+    assert np.array_equal(got[:, tb // 2], q[pick.numpy()])
+    assert (np.delete(got, tb // 2, axis=1) == 0).all()
