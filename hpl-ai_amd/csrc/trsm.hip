@@ -490,22 +490,27 @@ __global__ __launch_bounds__(kTriThreads) void trsm_u_tri16_kernel(int b, int64_
 // the LU, whose triangles are its own factors.)
 // The strip lives in accumulators, transposed for the L panel, so that a block
 // of the result is the right operand of the next products as it is (k =
-// acc_row); wave w holds blocks w, w + 8, ..  Step K: X_K is in LDS; the wave of
+// acc_row); wave w of W holds blocks w, w + W, ..  An accumulator sums the
+// products of a block; its entries (in LDS, [kk 64 + lane]) with the diagonal's
+// term, the largest, are added last, in one rounding.  Step K: X_K is in LDS; the wave of
 // block K + 1 updates that block, solves it and stores it before its other
 // blocks, so a step is two products of the chain or the updates, whichever is
 // longer.  A wave's operands of the next step are loaded as soon as the
 // registers are free.  What bounds it: those two products a step up to a strip
-// per CU, then the FP32 matrix cores at one workgroup per CU (245 registers).  b
-// = 777, L / U, with the inverses: 4000 wide 109 / 126 us, 40000 wide 483 / 534
-// (with the whole inverse 167 / 143 and 419 / 387, by substitution on one row or
-// column per thread 2784 / 11500 and 4267 / 15062); b = 60, 40000 wide 33 / 32
-// (28.6 / 27.9; 50 / 63 with the walk in LDS).
-template <bool UP, int PER, bool VEC>
-__global__ __launch_bounds__(kTriThreads) void trsm_walk_kernel(int64_t m, int b, const float *__restrict__ tri,
+// per CU, then the FP32 matrix cores at one workgroup per CU (256 registers at b
+// > 512).  b = 777, L / U, with the inverses: 4000 wide 125 / 129 us, 40000 wide
+// 558 / 560 (with the whole inverse 167 / 143 and 419 / 387, by substitution on
+// one row or column per thread 2784 / 11500 and 4267 / 15062); b = 60, 40000 wide
+// 27 / 29 (28.6 / 27.9; 50 / 63 with the walk in LDS).  Error for factors of
+// HPL-AI matrices, b = 60 .. 1000: 2.4e-8 U, 4.1e-8 L, as with the whole inverse
+// (2.8e-8 / 4.4e-8 for 60, 4.5e-7 for 777 by substitution).
+template <bool UP, int W, int PER, bool VEC>
+__global__ __launch_bounds__(64 * W) void trsm_walk_kernel(int64_t m, int b, const float *__restrict__ tri,
                                                                 const float *__restrict__ T, int64_t ldt,
                                                                 float *__restrict__ P, int64_t ldp)
 {
     __shared__ float xl[2][1024];   // -X_K, [kk 64 + lane]
+    __shared__ float own[W * PER][1024], diag[32 * W * PER];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5, nb = (b + 31) / 32;
     const int64_t p0 = static_cast<int64_t>(blockIdx.x) * kStrip;
@@ -517,8 +522,9 @@ __global__ __launch_bounds__(kTriThreads) void trsm_walk_kernel(int64_t m, int b
     auto load_left = [&](float (&v)[16], int J, int K) {
         const int64_t j = min(32 * J + l32, b - 1);
         if constexpr (UP) {
+            const float *row = T + j + static_cast<int64_t>(32 * K + 4 * lh) * ldt;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) v[e] = T[static_cast<int64_t>(32 * K + acc_row(e, lh)) * ldt + j];
+            for (int e = 0; e < 16; ++e) v[e] = row[acc_row(e, 0) * ldt];
         } else {
             const float *col = T + j * ldt + 32 * K + 4 * lh;
 #pragma unroll
@@ -538,6 +544,7 @@ __global__ __launch_bounds__(kTriThreads) void trsm_walk_kernel(int64_t m, int b
     };
     // the inverse of diagonal block J: entry (l32, acc_row), for the L panel (acc_row, l32)
     auto inverse = [&](int J) { return UP ? tri_block_l(tri, nb, J, J) : tri_block_u(tri, nb, J, J); };
+    // without its diagonal
     float iv[16];
     auto load_inverse = [&](int J) {
         const float *o = inverse(J) + l32 * 4 + 2 * lh;
@@ -550,36 +557,45 @@ __global__ __launch_bounds__(kTriThreads) void trsm_walk_kernel(int64_t m, int b
             iv[4 * q + 2] = even.y;
             iv[4 * q + 3] = odd.y;
         }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) iv[e] = acc_row(e, lh) == l32 ? 0.0f : iv[e];
     };
     floatx16t_t acc[PER];
     float left[PER][16];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-        const int J = wave + 8 * i;
-        if (J >= nb) continue;
+        const int J = wave + W * i;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][e] = strip[min(32 * J + acc_row(e, lh), b - 1) * step];
+        for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+        if (J > 0 && J < nb) load_left(left[i], J, 0);
     }
     if (wave < nb) load_inverse(wave);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-        const int J = wave + 8 * i;
+        const int J = wave + W * i;
         if (J >= nb) continue;
-        if (J > 0) load_left(left[i], J, 0);
-        if (32 * J + 32 > b)
+        float v[16];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][e] = 32 * J + acc_row(e, lh) < b ? acc[i][e] : 0.0f;
+        for (int e = 0; e < 16; ++e) v[e] = strip[min(32 * J + acc_row(e, lh), b - 1) * step];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) own[J][e * 64 + lane] = 32 * J + acc_row(e, lh) < b ? v[e] : 0.0f;
     }
-    // X_J := inverse of block J times D
-    auto solve = [&](int J, const floatx16t_t &D) {
+    for (int j = tid; j < 32 * nb; j += 64 * W) {
+        const int r = j & 31;
+        diag[j] = UP ? 1.0f : inverse(j >> 5)[tri_pos(r + 32 * (r & 1), r >> 1)];
+    }
+    // X_J := inverse of block J times D, the block less its products (-S)
+    auto solve = [&](int J, const floatx16t_t &S) {
         int ln = lane;   // addresses that are not kept through the walk
         asm volatile("" : "+v"(ln));
         const int h = ln >> 5;
         float *out = &xl[J & 1][ln];
-        floatx16t_t x;
+        const float *a = &own[J][ln];
+        floatx16t_t D, x;
         bool fine = true;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
+            D[e] = a[64 * e] + S[e];
             x[e] = 0.0f;
             fine = fine && isfinite(D[e]);
         }
@@ -598,18 +614,20 @@ __global__ __launch_bounds__(kTriThreads) void trsm_walk_kernel(int64_t m, int b
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     const int j = acc_row(e, h);
-                    if (k <= j) x[e] = fmaf(o[tri_pos(j + 32 * (k & 1), k >> 1)], d, x[e]);
+                    if (k < j) x[e] = fmaf(o[tri_pos(j + 32 * (k & 1), k >> 1)], d, x[e]);
                 }
             }
             wave_lds_sync();
         }
-        float *dst = strip + static_cast<int64_t>(32 * J + 4 * h) * step;
+        float *dst = strip + (32 * J + 4 * h) * step;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
+            const float d = diag[32 * J + acc_row(e, h)];
+            x[e] = fmaf(d, a[64 * e], fmaf(d, S[e], x[e]));
             out[64 * e] = -x[e];
-            if ((ln & 31) < cnt && 32 * J + acc_row(e, h) < b) dst[static_cast<int64_t>(acc_row(e, 0)) * step] = x[e];
+            if ((ln & 31) < cnt && 32 * J + acc_row(e, h) < b) dst[acc_row(e, 0) * step] = x[e];
         }
-        if (J + 8 < nb) load_inverse(J + 8);
+        if (J + W < nb) load_inverse(J + W);
     };
     auto update = [&](int i, int J, int K, const float (&xv)[16]) {
         if (32 * J + 32 > b)
@@ -626,20 +644,20 @@ __global__ __launch_bounds__(kTriThreads) void trsm_walk_kernel(int64_t m, int b
 #pragma unroll
             for (int e = 0; e < 16; ++e) xv[e] = xl[K & 1][e * 64 + lane];
         __builtin_amdgcn_sched_barrier(0);
-        floatx16t_t D;
+        floatx16t_t S;
         bool mine = false;
 #pragma unroll
         for (int i = 0; i < PER; ++i)
-            if (wave + 8 * i == K + 1) {
+            if (wave + W * i == K + 1) {
                 if (K >= 0) update(i, K + 1, K, xv);
-                D = acc[i];
+                S = acc[i];
                 mine = true;
             }
-        if (mine) solve(K + 1, D);
+        if (mine) solve(K + 1, S);
         if (K < 0) continue;
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int J = wave + 8 * i;
+            const int J = wave + W * i;
             if (J > K + 1 && J < nb) update(i, J, K, xv);
         }
     }
@@ -774,21 +792,26 @@ template <bool UP>
 static int trsm_walk(int64_t m, int b, const float *tri, const float *T, int64_t ldt, float *P, int64_t ldp,
                      hipStream_t s)
 {
-    const dim3 g(static_cast<unsigned>(ceil_div(m, kStrip))), th(kTriThreads);
+    const dim3 g(static_cast<unsigned>(ceil_div(m, kStrip)));
     const int nb = (b + 31) / 32;
-    auto launch = [&](auto per) {
-        constexpr int PER = decltype(per)::value;
+    auto launch = [&](auto waves, auto per) {
+        constexpr int W = decltype(waves)::value, PER = decltype(per)::value;
         if (!UP && aligned16(T, ldt))   // L's columns are read along the lanes
-            hipLaunchKernelGGL((trsm_walk_kernel<UP, PER, !UP>), g, th, 0, s, m, b, tri, T, ldt, P, ldp);
+            hipLaunchKernelGGL((trsm_walk_kernel<UP, W, PER, !UP>), g, dim3(64 * W), 0, s, m, b, tri, T, ldt, P, ldp);
         else
-            hipLaunchKernelGGL((trsm_walk_kernel<UP, PER, false>), g, th, 0, s, m, b, tri, T, ldt, P, ldp);
+            hipLaunchKernelGGL((trsm_walk_kernel<UP, W, PER, false>), g, dim3(64 * W), 0, s, m, b, tri, T, ldt, P, ldp);
     };
-    if (nb <= 8)
-        launch(std::integral_constant<int, 1>{});
+    using std::integral_constant;
+    if (nb <= 2)   // more workgroups on a CU
+        launch(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+    else if (nb <= 4)
+        launch(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+    else if (nb <= 8)
+        launch(integral_constant<int, 8>{}, integral_constant<int, 1>{});
     else if (nb <= 16)
-        launch(std::integral_constant<int, 2>{});
+        launch(integral_constant<int, 8>{}, integral_constant<int, 2>{});
     else
-        launch(std::integral_constant<int, 4>{});
+        launch(integral_constant<int, 8>{}, integral_constant<int, 4>{});
     HPLAI_HIP(hipGetLastError());
     return HPLAI_OK;
 }
