@@ -816,6 +816,8 @@ static int trsm_walk(int64_t m, int b, const float *tri, const float *T, int64_t
     return HPLAI_OK;
 }
 
+constexpr int64_t kTrsmLines = int64_t(1) << 27;
+
 int launch_trsm_panel(bool up, int64_t m, int b, const float *T, int64_t ldt, float *tri, float *P, int64_t ldp,
                       hipStream_t s)
 {
@@ -823,8 +825,15 @@ int launch_trsm_panel(bool up, int64_t m, int b, const float *T, int64_t ldt, fl
     const bool whole = b <= 512 && b % 32 == 0;
     const int rc = launch_tri_inverse(b, T, ldt, tri, up ? 1 : 2, whole, s);
     if (rc) return rc;
-    if (!whole) return up ? trsm_walk<true>(m, b, tri, T, ldt, P, ldp, s) : trsm_walk<false>(m, b, tri, T, ldt, P, ldp, s);
-    return up ? launch_trsm_u(b, m, tri, P, ldp, nullptr, 1, s) : launch_trsm_l(m, b, tri, P, ldp, nullptr, 1, s);
+    // a launch has at most 2^32 threads: 2^28 lines
+    for (int64_t l0 = 0; l0 < m; l0 += kTrsmLines) {
+        const int64_t c = m - l0 < kTrsmLines ? m - l0 : kTrsmLines;
+        float *Q = P + (up ? l0 * ldp : l0);
+        const int r = up ? (whole ? launch_trsm_u(b, c, tri, Q, ldp, nullptr, 1, s) : trsm_walk<true>(c, b, tri, T, ldt, Q, ldp, s))
+                         : (whole ? launch_trsm_l(c, b, tri, Q, ldp, nullptr, 1, s) : trsm_walk<false>(c, b, tri, T, ldt, Q, ldp, s));
+        if (r) return r;
+    }
+    return HPLAI_OK;
 }
 
 }  // namespace hplai

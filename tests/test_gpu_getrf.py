@@ -236,3 +236,18 @@ def test_trsm_entries_before_a_nonfinite_one_stay(ctx, b, bad):
         keep[j, k:] = False
         assert not torch.isfinite(a[j, k])
         assert ((a - w)[keep].abs().max() / w.abs().max()).item() < 1e-6
+
+
+def test_trsm_of_more_lines_than_one_launch_takes(ctx):
+    """2^28 + 70 rows or columns of two entries: the launch would have 2^32
+    threads and more."""
+    import torch
+    m, b = (1 << 28) + 70, 2
+    T = torch.tensor([[2.0, 0.5], [0.25, 4.0]], device="cuda")        # column-major: L = [1, .5], U = [2 .25; 0 4]
+    P = torch.ones(m * b, device="cuda")
+    ctx.trsm_lpanel(m, b, T, b, P, m)
+    # x0 = 1 / 2, x1 = (1 - .25 x0) / 4, exact in FP32
+    assert bool((P[:m] == 0.5).all()) and bool((P[m:] == 0.21875).all())
+    P.fill_(1.0)
+    ctx.trsm_upanel(b, m, T, b, P, b)
+    assert bool((P[0::2] == 1.0).all()) and bool((P[1::2] == 0.5).all())
