@@ -5,6 +5,12 @@
 
 namespace hplai {
 
+// a workgroup's number in a grid of grid_x(blocks) by `rest` = grid_rest(blocks)
+__device__ __forceinline__ int64_t block_number(unsigned rest)
+{
+    return static_cast<int64_t>(rest) * gridDim.x + blockIdx.x;
+}
+
 // ---------------------------------------------------------------------------
 // LCG of hpl_rand.hpp:8-57: x <- a x + c mod 2^64.  A coefficient pair (a, c)
 // is an affine map; composition l*r = (l.a r.a, l.a r.c + l.c) applies r first.

@@ -14,6 +14,7 @@
 // workgroup, coalesced on both sides), B's columns are copied, and K is
 // padded with zeros to a multiple of 64; then the update runs with FP32
 // accumulation.  Any k >= 0 is accepted (the reference's C1 uses k = 60).
+#include "device_common.hpp"
 #include "internal.hpp"
 
 namespace hplai {
@@ -26,7 +27,7 @@ __global__ __launch_bounds__(256) void seam_pack_a_kernel(int64_t n, int64_t k, 
                                                           uint16_t *__restrict__ dst)
 {
     __shared__ uint16_t t[kSeamTile][kSeamTile + 2];
-    const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kSeamTile;
+    const int64_t i0 = block_number(blockIdx.z) * kSeamTile;
     const int64_t k0 = static_cast<int64_t>(blockIdx.y) * kSeamTile;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
     {   // all loads in flight; past an edge they repeat the last entry
@@ -54,7 +55,7 @@ __global__ __launch_bounds__(256) void seam_pack_b_kernel(int64_t m, int64_t k, 
                                                           const uint16_t *__restrict__ b, int64_t ldb,
                                                           uint16_t *__restrict__ dst)
 {
-    const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t idx = block_number(blockIdx.y) * 256 + threadIdx.x;
     if (idx >= m * kpad) return;
     const int64_t j = idx / kpad, kk = idx - j * kpad;
     dst[idx] = kk < k ? b[j * ldb + kk] : uint16_t(0);
@@ -75,14 +76,15 @@ int launch_gemmschur_f16(int64_t n, int64_t m, int64_t k, const uint16_t *a, int
     HPLAI_CHECK(ceil_div(n, kSeamTile) < (int64_t(1) << 31) && ceil_div(kpad, kSeamTile) <= 65535,
                 "gemmschur: n=%lld k=%lld too large", (long long)n, (long long)k);
     hipLaunchKernelGGL(seam_pack_a_kernel,
-                       dim3(static_cast<unsigned>(ceil_div(n, kSeamTile)), static_cast<unsigned>(kpad / kSeamTile)),
+                       dim3(grid_x(ceil_div(n, kSeamTile)), static_cast<unsigned>(kpad / kSeamTile),
+                            grid_rest(ceil_div(n, kSeamTile))),
                        dim3(256), 0, s, n, k, kpad, a, lda, ap);
     HPLAI_HIP(hipGetLastError());
     const int64_t nb = m * kpad;
     HPLAI_CHECK(ceil_div(nb, 256) < (int64_t(1) << 31), "gemmschur: m=%lld k=%lld too large", (long long)m,
                 (long long)k);
-    hipLaunchKernelGGL(seam_pack_b_kernel, dim3(static_cast<unsigned>(ceil_div(nb, 256))), dim3(256), 0, s, m, k,
-                       kpad, b, ldb, bp);
+    hipLaunchKernelGGL(seam_pack_b_kernel, dim3(grid_x(ceil_div(nb, 256)), grid_rest(ceil_div(nb, 256))), dim3(256), 0,
+                       s, m, k, kpad, b, ldb, bp);
     HPLAI_HIP(hipGetLastError());
     // kslice must be a multiple of 64 binary16 values; one slice covers K
     return launch_schur(HPLAI_FMT_F16, n, m, 1, static_cast<int>(kpad), ap, kpad, nullptr, 0, bp, kpad, nullptr,

@@ -168,8 +168,9 @@ __global__ __launch_bounds__(kHgRows) void higham_gemv_partial_kernel(int64_t n,
                                                                       double *__restrict__ work)
 {
     __shared__ double xs[kHgChunk];
-    const int64_t rb = blockIdx.x % row_blocks, cb = blockIdx.x / row_blocks;
+    const int64_t block = block_number(blockIdx.y), rb = block % row_blocks, cb = block / row_blocks;
     const int64_t j0 = cb * kHgChunk;
+    if (j0 >= n) return;
     const int64_t j1 = j0 + kHgChunk < n ? j0 + kHgChunk : n;
     for (int64_t c = threadIdx.x; c < j1 - j0; c += kHgRows) xs[c] = x[j0 + c];
     __syncthreads();
@@ -272,7 +273,7 @@ static int higham_gemv(bool abs_entries, int64_t n, double alpha, double beta, d
 {
     if (n <= 0) return HPLAI_OK;
     const int64_t row_blocks = ceil_div(n, kHgRows), nchunks = ceil_div(n, kHgChunk);
-    const dim3 grid(static_cast<unsigned>(row_blocks * nchunks));
+    const dim3 grid(grid_x(row_blocks * nchunks), grid_rest(row_blocks * nchunks));
     if (abs_entries)
         hipLaunchKernelGGL(higham_gemv_partial_kernel<true>, grid, dim3(kHgRows), 0, s, n, row_blocks, alpha,
                            beta, alpha * beta, x, work);

@@ -101,6 +101,11 @@ private:
 
 inline hipStream_t as_stream(void *s) { return static_cast<hipStream_t>(s); }
 __host__ __device__ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+// x and y (or z) of a grid of `blocks` workgroups and up to x - 1 more: a launch
+// has at most 2^32 threads along a dimension (block_number)
+constexpr int64_t kGridX = int64_t(1) << 22;
+inline unsigned grid_x(int64_t blocks) { return static_cast<unsigned>(blocks < kGridX ? blocks : kGridX); }
+inline unsigned grid_rest(int64_t blocks) { return static_cast<unsigned>(ceil_div(blocks, kGridX)); }
 
 // ---- kernel launchers (no argument validation; callers validate) ----
 // accumulate != 0: A += generated block (lazy initialisation); P (FP16,

@@ -40,9 +40,10 @@ __global__ __launch_bounds__(kGemvRows) void otf_gemv_partial_kernel(
     int64_t n, uint64_t x1, int chunk, int row_blocks, LcgCoeff jn, LcgCoeff jn2, const double *__restrict__ x,
     double *__restrict__ partial)
 {
-    const int rb = static_cast<int>(blockIdx.x) % row_blocks;
-    const int cb = static_cast<int>(blockIdx.x) / row_blocks;
+    const int block = static_cast<int>(block_number(blockIdx.y));
+    const int rb = block % row_blocks, cb = block / row_blocks;
     const int64_t r0 = static_cast<int64_t>(rb) * kGemvRows, j0 = static_cast<int64_t>(cb) * chunk;
+    if (j0 >= n) return;
     const int len = static_cast<int>(j0 + chunk < n ? chunk : n - j0);
     const int64_t i = r0 + threadIdx.x;
     uint64_t s0 = lcg_jump_lanes<8>(x1, static_cast<uint64_t>(r0) + static_cast<uint64_t>(n) * static_cast<uint64_t>(j0),
@@ -109,7 +110,7 @@ int launch_otf_gemv(int64_t n, uint64_t seed, const double *d, double alpha, con
     const int64_t nchunks = ceil_div(n, chunk);
     const LcgCoeff jn = lcg_pow_host(static_cast<uint64_t>(n));
     const LcgCoeff jn2 = lcg_mul(jn, jn);
-    hipLaunchKernelGGL(otf_gemv_partial_kernel, dim3(static_cast<unsigned>(row_blocks * nchunks)),
+    hipLaunchKernelGGL(otf_gemv_partial_kernel, dim3(grid_x(row_blocks * nchunks), grid_rest(row_blocks * nchunks)),
                        dim3(kGemvRows), 0, s, n, lcg_init(seed), chunk, static_cast<int>(row_blocks), jn, jn2, x, work);
     HPLAI_HIP(hipGetLastError());
     hipLaunchKernelGGL(otf_gemv_reduce_kernel, dim3(static_cast<unsigned>(ceil_div(n, 256))),

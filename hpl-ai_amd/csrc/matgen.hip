@@ -180,8 +180,8 @@ int launch_gen_matrix(int64_t n, uint64_t seed, int64_t i0, int64_t j0, int64_t 
     const int64_t row_blocks = ceil_div(m, kGenRows);
     const int64_t col_groups = ceil_div(k, kGenCols);
     const LcgCoeff jn = lcg_pow_host(static_cast<uint64_t>(n));
-    // split launches so the grid stays below 2^31 blocks
-    const int64_t max_groups = (int64_t(1) << 30) / row_blocks;
+    // split launches so the grid stays below 2^32 threads
+    const int64_t max_groups = row_blocks < kGridX ? kGridX / row_blocks : 1;
     for (int64_t g0 = 0; g0 < col_groups; g0 += max_groups) {
         int64_t g = col_groups - g0 < max_groups ? col_groups - g0 : max_groups;
         int64_t jj = g0 * kGenCols;

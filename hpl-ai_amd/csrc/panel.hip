@@ -170,7 +170,7 @@ __global__ __launch_bounds__(256) void quant_l_kernel(int64_t m, int64_t k, int 
                                                       int32_t *__restrict__ exps)
 {
     __shared__ float T[64][65];
-    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * 64;
+    const int64_t r0 = block_number(blockIdx.z) * 64;
     const int64_t c0 = static_cast<int64_t>(blockIdx.y) * 64;
     const int tx = threadIdx.x % 64, ty = threadIdx.x / 64;
     {
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void quant_u_kernel(int64_t m, int64_t k, int 
 {
     // thread handles 4 consecutive rows (k index) of one column j
     const int64_t kq = ceil_div(k, 4);
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t t = block_number(blockIdx.y) * 256 + threadIdx.x;
     const int64_t j = t / kq, r = (t % kq) * 4;
     if (j >= m) return;
     const int e = fmt_exponent<FMT>(amax, slots, exps, j / tb);
@@ -298,7 +298,7 @@ __global__ __launch_bounds__(256) void quant_l16_kernel(int64_t m, int64_t k, in
 {
     __shared__ float T[64][65];
     constexpr int es = FMT == HPLAI_FMT_E4M3 ? 1 : 2;
-    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * 64;
+    const int64_t r0 = block_number(blockIdx.z) * 64;
     const int64_t c0 = static_cast<int64_t>(blockIdx.y) * 64;
     const int tid = threadIdx.x;
     // loads: 64 columns x 16 float4; thread tid takes float4 i = tid % 16 of
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256) void quant_u16_kernel(int64_t m, int64_t k, in
 {
     constexpr int es = FMT == HPLAI_FMT_E4M3 ? 1 : 2;
     const int64_t kq = k / 16;
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t t = block_number(blockIdx.y) * 256 + threadIdx.x;
     const int64_t j = t / kq, r = (t % kq) * 16;
     if (j >= m) return;
     const int e = fmt_exponent<FMT>(amax, slots, exps, j / tb);
@@ -448,20 +448,20 @@ static int quant_dispatch(int side, int64_t m, int64_t k, int tb, const float *s
     const bool v16 = k % 16 == 0 && lds % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(dst) % 16 == 0 && (ldd * es) % 16 == 0;
     if (side == 0 && v16) {
-        dim3 grid(static_cast<unsigned>(ceil_div(m, 64)), static_cast<unsigned>(ceil_div(k, 64)));
+        dim3 grid(grid_x(ceil_div(m, 64)), static_cast<unsigned>(ceil_div(k, 64)), grid_rest(ceil_div(m, 64)));
         hipLaunchKernelGGL((quant_l16_kernel<FMT, PACKED>), grid, dim3(256), 0, s, m, k, tb, src, lds, dst, ldd,
                            amax, slots, exps);
     } else if (side == 0) {
-        dim3 grid(static_cast<unsigned>(ceil_div(m, 64)), static_cast<unsigned>(ceil_div(k, 64)));
+        dim3 grid(grid_x(ceil_div(m, 64)), static_cast<unsigned>(ceil_div(k, 64)), grid_rest(ceil_div(m, 64)));
         hipLaunchKernelGGL((quant_l_kernel<FMT, PACKED>), grid, dim3(256), 0, s, m, k, tb, src, lds, dst, ldd,
                            amax, slots, exps);
     } else if (v16) {
         const int64_t thr = m * (k / 16);
-        hipLaunchKernelGGL((quant_u16_kernel<FMT, PACKED>), dim3(static_cast<unsigned>(ceil_div(thr, 256))),
+        hipLaunchKernelGGL((quant_u16_kernel<FMT, PACKED>), dim3(grid_x(ceil_div(thr, 256)), grid_rest(ceil_div(thr, 256))),
                            dim3(256), 0, s, m, k, tb, src, lds, dst, ldd, amax, slots, exps);
     } else {
         const int64_t thr = m * ceil_div(k, 4);
-        hipLaunchKernelGGL((quant_u_kernel<FMT, PACKED>), dim3(static_cast<unsigned>(ceil_div(thr, 256))),
+        hipLaunchKernelGGL((quant_u_kernel<FMT, PACKED>), dim3(grid_x(ceil_div(thr, 256)), grid_rest(ceil_div(thr, 256))),
                            dim3(256), 0, s, m, k, tb, src, lds, dst, ldd, amax, slots, exps);
     }
     HPLAI_HIP(hipGetLastError());

@@ -72,3 +72,17 @@ def test_more_tiles_than_one_launch_takes(ctx, oracle, tb, side):
     got = dst.cpu().numpy().reshape(tiles, tb)
     assert np.array_equal(got[:, tb // 2], q[pick.numpy()])
     assert (np.delete(got, tb // 2, axis=1) == 0).all()
+
+
+@pytest.mark.parametrize("side", [0, 1])
+def test_more_entries_than_threads_of_one_launch(ctx, side):
+    """Side 0: 2^30 + 70 rows (64 of them a workgroup); side 1: 2^32 + 70 columns
+    of one entry (a thread each)."""
+    import hplai
+    import torch
+    m = (1 << 30) + 70 if side == 0 else (1 << 32) + 70
+    src = torch.full((m,), 1.5, device="cuda")
+    src[-1] = -2.0
+    dst = torch.zeros(m, dtype=torch.float16, device="cuda")
+    ctx.quantize(hplai.FMT_F16, side, m, 1, 1, src, m if side == 0 else 1, dst, 1)
+    assert torch.equal(dst[:-1].min(), dst[:-1].max()) and dst[0].item() == 1.5 and dst[-1].item() == -2.0

@@ -75,3 +75,16 @@ def test_schur_packed_first(ctx, fmt, pad):
         ctx.schur_update(fmt, r1 - r0, n, ns, 512, L[r0:], K + pad, eL[0, r0 // 512:], tl, U, K + pad, eU, tu, 512,
                          D[0, r0:], m)
     assert torch.equal(C, D)
+
+
+def test_gemmschur_of_more_entries_than_one_launch_takes(ctx):
+    """B of (2^18 + 3) x 2^14 entries, staged by a thread each: past 2^32."""
+    import torch
+    n, m, k = 3, (1 << 18) + 3, 1 << 14
+    a = torch.ones(k, n, dtype=torch.float16, device="cuda")
+    b = torch.zeros(m, k, dtype=torch.float16, device="cuda")
+    b[:, 0], b[:, -1] = 1.0, 0.5                       # two entries a column: exact
+    b[-1, 7] = 3.0
+    c = torch.full((m, n), 2.0, device="cuda")
+    ctx.gemmschur_f16(n, m, k, a, n, b, k, c, n)
+    assert bool((c[:-1] == 0.5).all()) and bool((c[-1] == -2.5).all())
