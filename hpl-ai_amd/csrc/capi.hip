@@ -185,16 +185,17 @@ int hplai_quantize(hplai_ctx ctx, int fmt, int side, int64_t m, int64_t k, int t
     hipStream_t s = as_stream(stream);
     if (fmt != HPLAI_FMT_F16) {
         HPLAI_CHECK(exps != nullptr && tb > 0, "quantize: exps and tb required for tile formats");
-        if (tile_amax_splits(m, k, tb) == 1) {
-            const int rc = launch_tile_amax(fmt, side, m, k, tb, src, lds, nullptr, exps, s);
+        const int cus = ctx->num_cu;
+        if (tile_amax_splits(m, k, tb, cus) == 1) {
+            const int rc = launch_tile_amax(fmt, side, m, k, tb, src, lds, nullptr, exps, cus, s);
             return rc ? rc : launch_quantize(fmt, side, m, k, tb, src, lds, dst, ldd, nullptr, exps, s);
         }
         const int64_t ntiles = ceil_div(m, tb);
-        const int slots = tile_amax_slots(m, k, tb);
+        const int slots = tile_amax_slots(m, k, tb, cus);
         ScratchLease amax(ctx, s, sizeof(float) * ntiles * slots);
         if (amax.rc) return amax.rc;
         int rc = slots > 1 ? HPLAI_OK : launch_fill_f32(amax.as<float>(), ntiles, 0.0f, s);
-        if (rc == HPLAI_OK) rc = launch_tile_amax(fmt, side, m, k, tb, src, lds, amax.as<float>(), exps, s);
+        if (rc == HPLAI_OK) rc = launch_tile_amax(fmt, side, m, k, tb, src, lds, amax.as<float>(), exps, cus, s);
         if (rc == HPLAI_OK)
             rc = launch_quantize(fmt, side, m, k, tb, src, lds, dst, ldd, amax.as<float>(), exps, s, false, slots);
         return rc;

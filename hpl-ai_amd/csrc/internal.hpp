@@ -166,10 +166,10 @@ int launch_quantize(int fmt, int side, int64_t m, int64_t k, int tb, const float
 // the maxima to amax: tile_amax_slots a tile, one slot a part, or one where all
 // parts meet (zeroed by the caller).
 constexpr int kAmaxSlots = 4;
-int tile_amax_splits(int64_t m, int64_t k, int tb);
-int tile_amax_slots(int64_t m, int64_t k, int tb);
+int tile_amax_splits(int64_t m, int64_t k, int tb, int num_cu);
+int tile_amax_slots(int64_t m, int64_t k, int tb, int num_cu);
 int launch_tile_amax(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds, float *amax,
-                     int32_t *exps, hipStream_t s);
+                     int32_t *exps, int num_cu, hipStream_t s);
 int launch_fill_f32(float *p, int64_t cnt, float v, hipStream_t s);
 // packed: Lq and Uq in the panel-packed layout (packed_off) from their bases.
 int launch_schur(int fmt, int64_t m, int64_t n, int nslices, int kslice, const void *Lq,

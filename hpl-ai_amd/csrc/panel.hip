@@ -387,25 +387,25 @@ __global__ __launch_bounds__(256) void quant_u16_kernel(int64_t m, int64_t k, in
 constexpr int64_t kAmaxTile = int64_t(1) << 19, kAmaxPart = int64_t(1) << 18;
 constexpr int kAmaxShort = 16;
 
-int tile_amax_splits(int64_t m, int64_t k, int tb)
+int tile_amax_splits(int64_t m, int64_t k, int tb, int num_cu)
 {
     if (tb < kAmaxShort) return 1;
     const int64_t entries = (m < tb ? m : tb) * k, s = ceil_div(entries, kAmaxTile);
     if (s > kAmaxSlots) return static_cast<int>(s < 64 ? s : 64);
-    return s > 1 || (entries >= kAmaxPart && ceil_div(m, tb) * kAmaxSlots <= 256) ? kAmaxSlots : 1;
+    return s > 1 || (entries >= kAmaxPart && ceil_div(m, tb) * kAmaxSlots <= num_cu) ? kAmaxSlots : 1;
 }
 
-int tile_amax_slots(int64_t m, int64_t k, int tb)
+int tile_amax_slots(int64_t m, int64_t k, int tb, int num_cu)
 {
-    return tile_amax_splits(m, k, tb) == kAmaxSlots ? kAmaxSlots : 1;
+    return tile_amax_splits(m, k, tb, num_cu) == kAmaxSlots ? kAmaxSlots : 1;
 }
 
 int launch_tile_amax(int fmt, int side, int64_t m, int64_t k, int tb, const float *src, int64_t lds, float *amax,
-                     int32_t *exps, hipStream_t s)
+                     int32_t *exps, int num_cu, hipStream_t s)
 {
     if (m <= 0 || k <= 0) return HPLAI_OK;
-    const unsigned parts = amax != nullptr ? static_cast<unsigned>(tile_amax_splits(m, k, tb)) : 1u;
-    const int slots = tile_amax_slots(m, k, tb);
+    const unsigned parts = amax != nullptr ? static_cast<unsigned>(tile_amax_splits(m, k, tb, num_cu)) : 1u;
+    const int slots = tile_amax_slots(m, k, tb, num_cu);
     const bool e4m3 = fmt == HPLAI_FMT_E4M3, together = tb < kAmaxShort && amax == nullptr;
     const int group = together ? 64 / tb * tb : tb;
     // a launch has at most 2^32 threads
