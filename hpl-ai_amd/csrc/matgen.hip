@@ -15,11 +15,12 @@ namespace hplai {
 constexpr int kGenRows = 256;   // rows per block (one per thread)
 constexpr int kGenCols = 64;    // columns per thread: amortises the jump-ahead
 
-// The same without partial sums, the plain generation: a thread's columns in
-// groups of kGenPlain from as many states, all their stores in flight, and the
-// diagonal looked for only where the workgroup's block meets it.  Bound by the
-// stores; one column per iteration, behind the conditions of the general form,
-// took 106 us for 10007 x 10007, now 97 (8.1 -> 7.1 ms at 98304).
+// fill_one_panel_with_rand (hpl_rand.hpp:59-106) for a block at (i0, j0) without
+// partial sums, the plain generation: a thread's columns in groups of kGenPlain
+// from as many states, all their stores in flight, and the diagonal looked for
+// only where the workgroup's block meets it.  Bound by the stores; one column per
+// iteration, behind the conditions of the general form, took 106 us for 10007 x
+// 10007, now 97 (8.1 -> 7.1 ms at 98304).
 constexpr int kGenPlain = 8;
 
 __global__ __launch_bounds__(kGenRows) void gen_plain_kernel(uint64_t n, uint64_t x1, int64_t i0, int64_t j0, int64_t m,
@@ -55,7 +56,7 @@ __global__ __launch_bounds__(kGenRows) void gen_plain_kernel(uint64_t n, uint64_
     }
 }
 
-// fill_one_panel_with_rand (hpl_rand.hpp:59-106) for a block at (i0, j0).
+// The general form: added to what is there, with the FP16 partial sums.
 __global__ __launch_bounds__(kGenRows) void gen_matrix_kernel(
     int64_t n, uint64_t x1, int64_t i0, int64_t j0, int64_t m, int64_t k, int64_t row_blocks,
     LcgCoeff jn, const double *__restrict__ d, float *__restrict__ A, int64_t lda, int accumulate,
