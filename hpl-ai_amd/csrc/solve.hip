@@ -525,13 +525,17 @@ struct LU {
     // Whether to overlap a step's trailing update with the next panel: the hops
     // between streams, 10-25 us each on the chain from panel to panel, cost
     // more than an update of less than about 100 us hides (C at 3 TB/s or the
-    // products at 600 TF/s).  LU alone, overlapped always / below 100 us not:
-    // 1200 blocks of 60 1347 / 924 us, 2400 2716 / 1846, 7200 9886 / 8328 (200
-    // us: 8543), 8192 blocks of 512 (e4m3) 5488 / 5205 (200 us: 5308).
+    // products at 600 TF/s, e4m3 2000 TF/s, of 256 CUs).  LU alone, overlapped
+    // always / below 100 us not: 1200 blocks of 60 1347 / 924 us, 2400 2716 / 1846,
+    // 7200 9886 / 8328 (200 us: 8543), 8192 blocks of 512 (e4m3) 5488 / 5205 (200
+    // us: 5308).  e4m3 taken for 600 / 2000 TF/s: 8192 in blocks of 512, outer 8,
+    // 5259 / 5102 us, of 256, outer 16, 6813 / 6618, 16384 of 512, outer 8, 12730 /
+    // 12600.
     bool overlap_pays(int64_t rest, int sw) const
     {
         const double m2 = static_cast<double>(rest) * static_cast<double>(rest);
-        return m2 * std::max(8.0 / 3e12, 2.0 * sw * b / 600e12) > 100e-6;
+        const double flops = (fmt == HPLAI_FMT_E4M3 ? 2000e12 : 600e12) * (num_cu > 0 ? num_cu : 256) / 256;
+        return m2 * std::max(8.0 / 3e12, 2.0 * sw * b / flops) > 100e-6;
     }
 
     // lookahead 0: update, then the next panel, all on the main stream.
