@@ -199,7 +199,8 @@ namespace hplai {
 // load touched all 32 lines of the block, 4 loads one after the other: getrf and
 // TRSMs 512 x 40000 567 -> 562 us.)
 // Blocks above the diagonal of Linv and below the diagonal of Uinv are never
-// written or read.
+// written or read.  Behind the blocks, 64 floats: [2 q + 1 for U] is 1 where the
+// triangle of diagonal block q is not well conditioned (poor32).
 __device__ __forceinline__ int tri_pos(int lane, int kk) { return (kk >> 2) * 256 + lane * 4 + (kk & 3); }
 template <typename T>
 __device__ __forceinline__ T *tri_block_l(T *tri, int nb, int I, int J)
@@ -210,6 +211,11 @@ template <typename T>
 __device__ __forceinline__ T *tri_block_u(T *tri, int nb, int I, int J)
 {
     return tri + (static_cast<int64_t>(nb) * nb + static_cast<int64_t>(J) * nb + I) * 1024;
+}
+template <typename T>
+__device__ __forceinline__ T *tri_poor(T *tri, int nb)
+{
+    return tri + 2 * static_cast<int64_t>(nb) * nb * 1024;
 }
 
 }  // namespace hplai

@@ -1,6 +1,12 @@
 // getrf.hip — LU of a diagonal block (n <= 1024) and the inverses of its
 // triangles, spread over the device.
 //
+// Two forms: the LU's own (FULL), with the inverses that its panels need, and a
+// caller's (hplai_getrf_nopiv_f32), whose strips take only inverses of 32 x 32
+// blocks, and those only where the block is well conditioned.  With the inverses
+// of 128-blocks |A - L U| was past the 2 (n + 80) u |L| |U| of elimination for
+// blocks far from dominance (3.4 times for diagonals of 3 at 512).
+//
 // Replaces getrf_nopiv (getrf_nopiv.hpp:124-160).  The block is walked in
 // sub-blocks of 128 columns; per sub-block three kinds of work, all FP32 on
 // v_mfma_f32_32x32x2_f32:
@@ -25,8 +31,8 @@
 // with the strips and the next sub-block's update).  One workgroup for the
 // whole 512 block spent half its time on trailing updates through a single
 // CU's path to the L2, and the inverses were two more kernels after it: 511 +
-// 73 us, now 172 us with the inverses and 157 without (b = 512, alone); b = 60:
-// 94 -> 14 us; n = 1000: 645 us with v_readlane steps, 329 us as here.  The
+// 73 us, now 172 us with the inverses and 162 without (b = 512, alone); b = 60:
+// 94 -> 14 us; n = 1000: 645 us with v_readlane steps, 342 us as here.  The
 // next sub-block's update in the workgroup that factors it took 11 us of each
 // sub-block (its operands, 192 KB, again through one CU): 198 us at b = 512.
 // Joining the inverses by one workgroup per 32 columns took 39 us a size
@@ -60,6 +66,8 @@ struct LuLds {
     float S[kLuNB * kLuS];            // the sub-block, S[c * kLuS + r]
     float V[kLuNB * kLuS];            // its inverses: Linv below the diagonal (unit diagonal implied), Uinv on and above
     float Li[32 * 33], Ui[32 * 33];   // inverses of the current 32 x 32 triangles, row-major
+    float w[2][32];                   // row sums of the current 32 x 32 triangles, L and U
+    int poor[2];                      // they are not well conditioned
 };
 
 // entry (i, j) of a unit-lower / an upper triangle whose block also holds the other one
@@ -291,8 +299,10 @@ __device__ __forceinline__ void tri_fin(int nb, float *tri, int J, int R0, int R
 // update the rest of the trailing matrix with sub-block k0 - 128 (when there is
 // one) and copy the blocks beside the diagonal one, and the last form the first products of the
 // whole block's inverses.  Without FACTOR: A is already factored and
-// workgroup q inverts the triangles of sub-block q.
-template <bool FACTOR>
+// workgroup q inverts the triangles of sub-block q.  Without FULL (a caller's
+// own LU) only the 32 x 32 inverses are formed and written, and blocks that are
+// not well conditioned are substituted with instead.
+template <bool FACTOR, bool FULL>
 __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, float *__restrict__ A, int64_t lda,
                                                                float *tri, int sides,
                                                                int *__restrict__ info)
@@ -313,7 +323,7 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
         // of the first sub-block only the four that are copied
         const int two = ct < 2 ? ct : 2, z = static_cast<int>(blockIdx.x) - 1;
         const int t = p0 >= 0 ? z + two : z < 2 ? ct + z : z;
-        if (p0 >= 0 && t >= rt * ct) {
+        if (FULL && p0 >= 0 && t >= rt * ct) {
             static_assert(offsetof(LuLds, V) == sizeof(float) * kLuNB * kLuS && (1024 - kLuNB) * 33 <= 2 * kLuNB * kLuS,
                           "the strip of an inverse spans S and V");
             const int y = t - rt * ct, q0 = k0 / 32;
@@ -401,21 +411,40 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
     __syncthreads();
     if (!FACTOR) {
         // waves 2 q, 2 q + 1 invert the triangles of 32-block q
+        const int at = 32 * (wave >> 1) * (kLuS + 1);
         if (wave & 1)
-            invert32<true>(S + 32 * (wave >> 1) * (kLuS + 1), LuStride{}, V + 32 * (wave >> 1) * (kLuS + 1), lane, nullptr);
+            invert32<true>(S + at, LuStride{}, V + at, lane, nullptr);
         else
-            invert32<false>(S + 32 * (wave >> 1) * (kLuS + 1), LuStride{}, V + 32 * (wave >> 1) * (kLuS + 1), lane, nullptr);
-        __syncthreads();
-        for (int q = 0; q < steps; ++q) {
-            if (wave < 2 * q) {
-                const int b = wave >> 1;
-                if (wave & 1)
-                    inverse_row_finish<true>(V, q, b, lane, inverse_row_product<true>(S, V, q, b, lane));
-                else
-                    inverse_row_finish<false>(V, q, b, lane, inverse_row_product<false>(S, V, q, b, lane));
+            invert32<false>(S + at, LuStride{}, V + at, lane, nullptr);
+        wave_lds_sync();
+        {
+            float *w = sm.Li + 32 * wave;   // row sums of this wave's triangle
+            if (wave & 1)
+                row_sums32<true>(S + at, LuStride{}, w, lane);
+            else
+                row_sums32<false>(S + at, LuStride{}, w, lane);
+            wave_lds_sync();
+            const bool poor = poor32([&](int r, int c) {
+                const float v = V[at + c * kLuS + r];
+                return wave & 1 ? upper_entry(v, r, c) : lower_entry(v, r, c);
+            }, w, lane);
+            if (lane == 0 && (wave >> 1) < steps) tri_poor(tri, nb)[2 * q0 + wave] = poor ? 1.0f : 0.0f;
+        }
+        if (FULL) {
+            for (int q = 0; q < steps; ++q) {
+                if (wave < 2 * q) {
+                    const int b = wave >> 1;
+                    if (wave & 1)
+                        inverse_row_finish<true>(V, q, b, lane, inverse_row_product<true>(S, V, q, b, lane));
+                    else
+                        inverse_row_finish<false>(V, q, b, lane, inverse_row_product<false>(S, V, q, b, lane));
+                }
+                __syncthreads();
+                write_inverse_row(V, tri, nb, q0, q, wave, sides, lane);
             }
-            __syncthreads();
-            write_inverse_row(V, tri, nb, q0, q, wave, sides, lane);
+        } else {
+            const int q = wave >> 1;
+            if (q < steps) write_inverse_row(V, tri, nb, q0, q, wave & 1 ? 2 * q + 1 : q, sides, lane);
         }
         return;
     }
@@ -456,8 +485,11 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
         } else if (q > 0) {
             const int R = steps - q;
             for (int i = wave; i < R * R; i += kLuThreads / 64 - 1) update(ln, c0 - 32, c0 + 32 * (i % R), c0 + 32 * (i / R));
-            write_inverse_row(V, tri, nb, q0, q - 1, wave - 1, sides, ln);
-            if (tri != nullptr && t < 2 * q)
+            if (FULL)
+                write_inverse_row(V, tri, nb, q0, q - 1, wave - 1, sides, ln);
+            else if (wave < 3)
+                write_inverse_row(V, tri, nb, q0, q - 1, wave == 1 ? q - 1 : 2 * q - 1, sides, ln);
+            if (FULL && tri != nullptr && t < 2 * q)
                 T = t & 1 ? inverse_row_product<true>(S, V, q, t >> 1, ln) : inverse_row_product<false>(S, V, q, t >> 1, ln);
         }
         __syncthreads();
@@ -465,19 +497,24 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
             invert32<false>(S + c0 * (kLuS + 1), LuStride{}, V + c0 * (kLuS + 1), ln, sm.Li);
         } else if (wave == 1) {
             invert32<true>(S + c0 * (kLuS + 1), LuStride{}, V + c0 * (kLuS + 1), ln, sm.Ui);
-        } else if (q + 1 == steps) {   // all of S is final: factors back to A
+        } else {
+            if (!FULL && wave == 6) row_sums32<false>(S + c0 * (kLuS + 1), LuStride{}, sm.w[0], ln);
+            if (!FULL && wave == 7) row_sums32<true>(S + c0 * (kLuS + 1), LuStride{}, sm.w[1], ln);
+            if (q + 1 == steps)   // all of S is final: factors back to A
 #pragma unroll 4
-            for (int c = (wave - 2) >> 1; c < w; c += 3) {
-                const int r = 64 * (wave & 1) + ln;
-                if (r < w) Ak[static_cast<int64_t>(c) * lda + r] = S[c * kLuS + r];
-            }
+                for (int c = (wave - 2) >> 1; c < w; c += 3) {
+                    const int r = 64 * (wave & 1) + ln;
+                    if (r < w) Ak[static_cast<int64_t>(c) * lda + r] = S[c * kLuS + r];
+                }
         }
         __syncthreads();
         // L21 := A21 U11^-1 and U12 := L11^-1 A12, one 32 x 32 block per wave
         const int R = steps - 1 - q;
-        if (wave < 2 * R) {
-            const bool up = wave >= R;
-            const int o = c0 + 32 * (1 + (up ? wave - R : wave)), l32 = ln & 31, lh = ln >> 5;
+        const bool mine = wave < 2 * R, up = wave >= R;
+        const int o = c0 + 32 * (1 + (up ? wave - R : wave));
+        floatx16g_t X = zero16();
+        if (mine) {
+            const int l32 = ln & 31, lh = ln >> 5;
             float av[16], bv[16];
             if (up) {
 #pragma unroll
@@ -492,18 +529,44 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
                     bv[kk] = sm.Ui[(2 * kk + lh) * 33 + l32];
                 }
             }
-            floatx16g_t acc = zero16();
-            acc = mfma16(av, bv, acc);
+            X = mfma16(av, bv, X);
+        } else if (!FULL && wave >= 6 && (R > 0 || tri != nullptr)) {
+            const float *M = wave == 6 ? sm.Li : sm.Ui;
+            const bool poor = poor32([&](int r, int c) { return M[r * 33 + c]; }, sm.w[wave - 6], ln);
+            if (ln == 0) {
+                sm.poor[wave - 6] = poor;
+                if (tri != nullptr) tri_poor(tri, nb)[2 * (q0 + q) + wave - 6] = poor ? 1.0f : 0.0f;
+            }
+        }
+        if (!FULL && R > 0) __syncthreads();
+        if (!FULL && mine && sm.poor[up ? 0 : 1]) {
+            // by substitution, a row or column per lane
+            float *x = up ? S + (o + (ln & 31)) * kLuS + c0 : S + c0 * kLuS + o + (ln & 31);
+            const int dx = up ? 1 : kLuS;
+            if (ln < 32)
+#pragma clang loop unroll(disable)
+                for (int k = 0; k < 32; ++k) {
+                    float v = x[k * dx];
+                    if (!up) {
+                        v *= 1.0f / S[(c0 + k) * kLuS + c0 + k];
+                        x[k * dx] = v;
+                    }
+#pragma clang loop unroll_count(4)
+                    for (int j = k + 1; j < 32; ++j)
+                        x[j * dx] = fmaf(-v, up ? S[(c0 + k) * kLuS + c0 + j] : S[(c0 + j) * kLuS + c0 + k], x[j * dx]);
+                }
+        } else if (mine) {
+            const int l32 = ln & 31, lh = ln >> 5;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int r = acc_row(e, lh);
                 if (up)
-                    S[(o + l32) * kLuS + c0 + r] = acc[e];
+                    S[(o + l32) * kLuS + c0 + r] = X[e];
                 else
-                    S[(c0 + l32) * kLuS + o + r] = acc[e];
+                    S[(c0 + l32) * kLuS + o + r] = X[e];
             }
         }
-        if (tri != nullptr && t < 2 * q) {
+        if (FULL && tri != nullptr && t < 2 * q) {
             if (t & 1)
                 inverse_row_finish<true>(V, q, t >> 1, ln, T);
             else
@@ -511,7 +574,10 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
         }
         __syncthreads();
     }
-    write_inverse_row(V, tri, nb, q0, steps - 1, wave, sides, lane);
+    if (FULL)
+        write_inverse_row(V, tri, nb, q0, steps - 1, wave, sides, lane);
+    else if (wave < 2)
+        write_inverse_row(V, tri, nb, q0, steps - 1, wave == 0 ? steps - 1 : 2 * steps - 1, sides, lane);
     if (tid == 0 && info != nullptr && (k0 == 0 || (bad != 0 && *info == 0))) *info = bad;
 }
 
@@ -585,6 +651,134 @@ __device__ __forceinline__ void next_diagonal(int n, int nb, int q0, int r, int 
             const float *p = XL + (4 * J + i) * 64 + lane;
             const int row = 32 * R + 8 * J + 4 * lh + i;
             if (row < n) A[col * lda + row] = d[i] - (((p[0] + p[1024]) + p[2048]) + p[3072]);
+        }
+}
+
+// The same for a caller's own LU, 32-block by 32-block (trsm.hip has the walk
+// for panels): workgroup z takes 32 rows of L21 with four waves and 32 columns of
+// U12 with four, or, past the strips, both that a block of the next diagonal
+// sub-block needs, from the copies, and then that block.  Wave J of a side holds
+// block J in its accumulators' order, transposed for L21; the sides' waves J are
+// on different SIMDs.  Four solves and three products one after the other instead
+// of four products: 512 154 -> 162 us (both sides in the same waves: 167).
+__global__ __launch_bounds__(512) void lu_strip_walk_kernel(int n, int p0, float *A, int64_t lda, float *tri, int strips)
+{
+    __shared__ float xl[2][4][1024];   // -X_K of both sides
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, lh = lane >> 5;
+    const bool up = wave >= 4;
+    const int J = up ? (wave + 2) & 3 : wave;
+    const int nb = (n + 31) / 32, q0 = p0 / 32, k1 = p0 + kLuNB;
+    const float *T = A + static_cast<int64_t>(p0) * (lda + 1);
+    const int nd = strips < 4 ? strips : 4, y = static_cast<int>(blockIdx.x) - strips;   // y >= 0: a block (r, c)
+    const int r = y % nd, c = y / nd;
+    const int o = k1 + 32 * static_cast<int>(blockIdx.x), cnt = n - o < 32 ? n - o : 32;   // a strip
+    // entry k = 32 J + acc_row of row (L21) or column (U12) l32
+    float own[16], left[3][16], iv[16], diag[16];
+    const int64_t step = up ? 1 : lda;
+    float *line = A + (up ? (o + min(l32, cnt - 1)) * lda + p0 + 32 * J + 4 * lh
+                          : (p0 + 32 * J + 4 * lh) * lda + o + min(l32, cnt - 1));
+    {
+        const float *copy = up ? copy_u(tri, nb, q0 + J, q0 + 4 + c) : copy_l(tri, nb, q0 + 4 + r, q0 + J);
+        const float *from = y >= 0 ? copy + 128 * lh + l32 : line;
+        const int64_t d = y >= 0 ? 32 : step;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) own[e] = from[acc_row(e, 0) * d];
+        const float *blk = up ? tri_block_l(tri, nb, q0 + J, q0 + J) : tri_block_u(tri, nb, q0 + J, q0 + J);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int k = acc_row(e, lh);
+            iv[e] = blk[tri_pos(l32 + 32 * (k & 1), k >> 1)];
+            diag[e] = up ? 1.0f : blk[tri_pos(k + 32 * (k & 1), k >> 1)];
+        }
+        const int64_t dk = up ? lda : 1;
+        const float *t = T + (up ? 32 * J + l32 + 4 * lh * lda : (32 * J + l32) * lda + 4 * lh);
+#pragma unroll
+        for (int K = 0; K < 3; ++K)
+            if (K < J)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) left[K][e] = t[(32 * K + acc_row(e, 0)) * dk];
+    }
+    // accumulators 2 wave and 2 wave + 1 of the next block
+    const int R = 32 * (q0 + 4 + r), C = 32 * (q0 + 4 + c) + l32;
+    float next[2] = {0.0f, 0.0f};
+    if (y >= 0)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            next[i] = A[min(C, n - 1) * lda + min(R + acc_row(2 * wave + i, lh), n - 1)];
+    const bool poor = tri_poor(tri, nb)[2 * (q0 + J) + (up ? 0 : 1)] != 0.0f;
+    floatx16g_t S = zero16(), x = zero16();
+#pragma unroll
+    for (int K = 0; K < 4; ++K) {
+        float *xk = xl[up][K];
+        if (J == K) {
+            floatx16g_t D;
+            bool fine = !poor;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                D[e] = own[e] + S[e];
+                fine = fine && isfinite(D[e]);
+            }
+            if (__all(fine)) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e)   // the diagonal's term last, in one rounding
+                    x = __builtin_amdgcn_mfma_f32_32x32x2f32(acc_row(e, lh) == l32 ? 0.0f : iv[e], D[e], x, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) x[e] = fmaf(diag[e], own[e], fmaf(diag[e], S[e], x[e]));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) xk[e * 64 + lane] = D[e];
+                const float *d = T + 32 * static_cast<int64_t>(K) * (lda + 1);
+                if (up)
+                    subst32<true>(xk, d, lda, 32, lane);
+                else
+                    subst32<false>(xk, d, lda, 32, lane);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) x[e] = xk[e * 64 + lane];
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) xk[e * 64 + lane] = -x[e];
+        }
+        if (K == 3 && y < 0) break;
+        __syncthreads();
+        if (J > K) {
+            float xv[16];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) xv[e] = xk[e * 64 + lane];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                S = __builtin_amdgcn_mfma_f32_32x32x2f32(K == 0 ? left[0][e] : K == 1 ? left[1][e] : left[2][e], xv[e], S, 0, 0, 0);
+        }
+    }
+    if (y < 0) {
+        if (l32 < cnt)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) line[acc_row(e, 0) * step] = x[e];
+        return;
+    }
+    // block (r, c) of the next diagonal sub-block: a product per wave of the first four, added in order
+    float av[16], bv[16];
+    if (!up)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            av[e] = xl[0][wave][e * 64 + lane];
+            bv[e] = xl[1][wave][e * 64 + lane];
+        }
+    __syncthreads();
+    float *part = xl[0][0];
+    if (!up) {
+        const floatx16g_t acc = mfma16(av, bv, zero16());
+#pragma unroll
+        for (int e = 0; e < 16; ++e) part[(wave * 16 + e) * 64 + lane] = acc[e];
+    }
+    __syncthreads();
+    if (C < n)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float *p = part + (2 * wave + i) * 64 + lane;
+            const int row = R + acc_row(2 * wave + i, lh);
+            if (row < n) A[C * lda + row] = next[i] - (((p[0] + p[1024]) + p[2048]) + p[3072]);
         }
 }
 
@@ -697,7 +891,7 @@ __global__ __launch_bounds__(kLuThreads) void tri_join_kernel(int n, int H, cons
 int64_t tri_floats(int b)
 {
     const int64_t nb = ceil_div(b, 32);
-    return 2 * nb * nb * 1024;
+    return 2 * nb * nb * 1024 + 64;
 }
 
 int64_t getrf_scratch_floats(int n) { return n > kLuNB ? tri_floats(n) : 0; }
@@ -711,14 +905,22 @@ int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, bool full,
         const int tiles = k == 0 ? (rest > kLuNB ? 4 : 0) : rt * ct - (ct < 2 ? ct : 2);
         // the whole block's inverses, and the last sub-block's, serve only a caller who asked for them
         const unsigned join = full ? 2 * (k / 32) : 0;
-        hipLaunchKernelGGL((lu_update_kernel<true>), dim3(static_cast<unsigned>(1 + tiles) + join), dim3(kLuThreads),
-                           0, s, n, k, A, lda, !full && rest <= kLuNB ? nullptr : tri, 3, info);
+        const dim3 g(static_cast<unsigned>(1 + tiles) + join);
+        if (full)
+            hipLaunchKernelGGL((lu_update_kernel<true, true>), g, dim3(kLuThreads), 0, s, n, k, A, lda, tri, 3, info);
+        else
+            hipLaunchKernelGGL((lu_update_kernel<true, false>), g, dim3(kLuThreads), 0, s, n, k, A, lda,
+                               rest <= kLuNB ? nullptr : tri, 3, info);
         HPLAI_HIP(hipGetLastError());
         const int strips = rest > kLuNB ? (rest - kLuNB + 31) / 32 : 0;
         const int nd = strips < 4 ? strips : 4;
         if (strips + join > 0) {
-            hipLaunchKernelGGL(lu_strip_kernel, dim3(static_cast<unsigned>(2 * strips + nd * nd) + join), dim3(256), 0, s, n, k,
-                               A, lda, tri, strips);
+            if (full)
+                hipLaunchKernelGGL(lu_strip_kernel, dim3(static_cast<unsigned>(2 * strips + nd * nd) + join), dim3(256), 0, s,
+                                   n, k, A, lda, tri, strips);
+            else
+                hipLaunchKernelGGL(lu_strip_walk_kernel, dim3(static_cast<unsigned>(strips + nd * nd)), dim3(512), 0, s, n, k,
+                                   A, lda, tri, strips);
             HPLAI_HIP(hipGetLastError());
         }
     }
@@ -728,8 +930,13 @@ int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, bool full,
 int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, bool join, hipStream_t s)
 {
     if (b <= 0) return HPLAI_OK;
-    hipLaunchKernelGGL((lu_update_kernel<false>), dim3(static_cast<unsigned>(ceil_div(b, kLuNB))), dim3(kLuThreads), 0,
-                       s, b, 0, const_cast<float *>(LU), lda, tri, sides, nullptr);
+    const dim3 g(static_cast<unsigned>(ceil_div(b, kLuNB)));
+    if (join)
+        hipLaunchKernelGGL((lu_update_kernel<false, true>), g, dim3(kLuThreads), 0, s, b, 0, const_cast<float *>(LU), lda,
+                           tri, sides, nullptr);
+    else
+        hipLaunchKernelGGL((lu_update_kernel<false, false>), g, dim3(kLuThreads), 0, s, b, 0, const_cast<float *>(LU), lda,
+                           tri, sides, nullptr);
     HPLAI_HIP(hipGetLastError());
     const int nb = static_cast<int>(ceil_div(b, 32));
     for (int H = kLuNB / 32; join && H < nb; H *= 2) {

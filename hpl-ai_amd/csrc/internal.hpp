@@ -138,7 +138,7 @@ int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, bool full,
 int64_t getrf_scratch_floats(int n);
 int64_t tri_floats(int b);
 // the same inverses of a block that is already factored, without join those of
-// its 128-blocks only; sides: 1 L, 2 U, 3 both
+// its 32-blocks only; sides: 1 L, 2 U, 3 both
 int launch_tri_inverse(int b, const float *LU, int64_t lda, float *tri, int sides, bool join, hipStream_t s);
 // tri: the packed inverses of the factored diagonal block
 // half: where the results also go as FP16 (dst NULL: nowhere), operand rows ld

@@ -252,4 +252,56 @@ __device__ __forceinline__ void invert32(const float *B, Ld ld, float *V, int la
     }
 }
 
+// Whether a triangle is not well conditioned: a row sum of |X| |T| past kCond32,
+// or no number, X its inverse.  A product with X then costs accuracy that
+// substitution (subst32) does not.  In two parts, one wave each: the row sums of
+// |T| (block at B, columns ld apart) to w, and the rest with X(r, c) from entry.
+constexpr float kCond32 = 16.0f;
+
+template <bool UP, typename Ld>
+__device__ __forceinline__ void row_sums32(const float *B, Ld ld, float *w, int lane)
+{
+    const int r = lane & 31;
+    float s = UP ? 0.0f : 1.0f;
+#pragma unroll
+    for (int c = 0; c < 32; ++c) {
+        const float v = fabsf(B[c * ld + r]);
+        s += (UP ? c >= r : c < r) ? v : 0.0f;
+    }
+    if (lane < 32) w[r] = s;
+}
+template <typename F>
+__device__ __forceinline__ bool poor32(F &&entry, const float *w, int lane)
+{
+    const int r = lane & 31, h = 16 * (lane >> 5);
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) s = fmaf(fabsf(entry(r, h + j)), w[h + j], s);
+    s += __shfl_xor(s, 32);
+    return __any(!(s <= kCond32));
+}
+
+// x := L^-1 x (UP) or U^-T x for the w x w triangle at T (columns ldt apart) by
+// substitution, one wave, one column per lane below 32: x in LDS, entry k of
+// column c at (index of k's accumulator) 64 + 32 (k / 4 % 2) + c (acc_row).
+template <bool UP>
+__device__ __forceinline__ void subst32(float *xb, const float *T, int64_t ldt, int w, int lane)
+{
+    wave_lds_sync();
+    if (lane < 32) {
+        auto at = [&](int k) -> float & { return xb[((k >> 3) * 4 + (k & 3)) * 64 + ((k >> 2) & 1) * 32 + lane]; };
+#pragma clang loop unroll(disable)
+        for (int k = 0; k < w; ++k) {
+            float x = at(k);
+            if (!UP) {
+                x *= 1.0f / T[k * ldt + k];
+                at(k) = x;
+            }
+#pragma clang loop unroll_count(4)
+            for (int j = k + 1; j < w; ++j) at(j) = fmaf(-x, UP ? T[k * ldt + j] : T[j * ldt + k], at(j));
+        }
+    }
+    wave_lds_sync();
+}
+
 }  // namespace hplai

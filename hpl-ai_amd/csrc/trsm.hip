@@ -483,7 +483,8 @@ __global__ __launch_bounds__(kTriThreads) void trsm_u_tri16_kernel(int b, int64_
 
 // The caller's own triangle (hplai_trsm_*) where b > 512 or b % 32 != 0: the
 // strip is solved 32 rows (U panel) or columns (L panel) at a time through the
-// inverses of the 32 x 32 diagonal blocks only.  A product with the whole
+// inverses of the 32 x 32 diagonal blocks only, or by substitution where such a
+// block is not well conditioned (poor32).  A product with the whole
 // inverse has the error of that walk times the triangle's condition: 31 u
 // against 2.7 u of |T| |X| for order 777 and condition 1e4, 6e5 u against 3.2 u
 // for 4e8.  (b <= 512 in whole 32-blocks takes the whole inverse, and so does
@@ -498,10 +499,10 @@ __global__ __launch_bounds__(kTriThreads) void trsm_u_tri16_kernel(int b, int64_
 // longer.  A wave's operands of the next step are loaded as soon as the
 // registers are free.  What bounds it: those two products a step up to a strip
 // per CU, then the FP32 matrix cores at one workgroup per CU (256 registers at b
-// > 512).  b = 777, L / U, with the inverses: 4000 wide 125 / 129 us, 40000 wide
-// 558 / 560 (with the whole inverse 167 / 143 and 419 / 387, by substitution on
+// > 512).  b = 777, L / U, with the inverses: 4000 wide 127 / 127 us, 40000 wide
+// 593 / 587 (with the whole inverse 167 / 143 and 419 / 387, by substitution on
 // one row or column per thread 2784 / 11500 and 4267 / 15062); b = 60, 40000 wide
-// 27 / 29 (28.6 / 27.9; 50 / 63 with the walk in LDS).  Error for factors of
+// 23 / 24 (28.6 / 27.9; 50 / 63 with the walk in LDS).  Error for factors of
 // HPL-AI matrices, b = 60 .. 1000: 2.4e-8 U, 4.1e-8 L, as with the whole inverse
 // (2.8e-8 / 4.4e-8 for 60, 4.5e-7 for 777 by substitution).
 template <bool UP, int W, int PER, bool VEC>
@@ -510,7 +511,7 @@ __global__ __launch_bounds__(64 * W) void trsm_walk_kernel(int64_t m, int b, con
                                                                 float *__restrict__ P, int64_t ldp)
 {
     __shared__ float xl[2][1024];   // -X_K, [kk 64 + lane]
-    __shared__ float own[W * PER][1024], diag[32 * W * PER];
+    __shared__ float own[W * PER][1024], diag[32 * W * PER], poor[W * PER];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5, nb = (b + 31) / 32;
     const int64_t p0 = static_cast<int64_t>(blockIdx.x) * kStrip;
@@ -580,6 +581,7 @@ __global__ __launch_bounds__(64 * W) void trsm_walk_kernel(int64_t m, int b, con
 #pragma unroll
         for (int e = 0; e < 16; ++e) own[J][e * 64 + lane] = 32 * J + acc_row(e, lh) < b ? v[e] : 0.0f;
     }
+    if (tid < nb) poor[tid] = tri_poor(tri, nb)[2 * tid + (UP ? 0 : 1)];
     for (int j = tid; j < 32 * nb; j += 64 * W) {
         const int r = j & 31;
         diag[j] = UP ? 1.0f : inverse(j >> 5)[tri_pos(r + 32 * (r & 1), r >> 1)];
@@ -599,31 +601,21 @@ __global__ __launch_bounds__(64 * W) void trsm_walk_kernel(int64_t m, int b, con
             x[e] = 0.0f;
             fine = fine && isfinite(D[e]);
         }
-        if (__all(fine)) {
+        fine = __all(fine && poor[J] == 0.0f);
+        if (fine) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) x = __builtin_amdgcn_mfma_f32_32x32x2f32(iv[e], D[e], x, 0, 0, 0);
         } else {
             // the zeros of the inverse would carry it to the entries before
 #pragma unroll
             for (int e = 0; e < 16; ++e) out[64 * e] = D[e];
-            wave_lds_sync();
-            const float *o = inverse(J);
-#pragma clang loop unroll(disable)
-            for (int k = 0; k < 32; ++k) {
-                const float d = xl[J & 1][((k >> 3) * 4 + (k & 3)) * 64 + ((k >> 2) & 1) * 32 + (ln & 31)];
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int j = acc_row(e, h);
-                    if (k < j) x[e] = fmaf(o[tri_pos(j + 32 * (k & 1), k >> 1)], d, x[e]);
-                }
-            }
-            wave_lds_sync();
+            subst32<UP>(xl[J & 1], T + 32 * static_cast<int64_t>(J) * (ldt + 1), ldt, min(32, b - 32 * J), ln);
         }
         float *dst = strip + (32 * J + 4 * h) * step;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const float d = diag[32 * J + acc_row(e, h)];
-            x[e] = fmaf(d, a[64 * e], fmaf(d, S[e], x[e]));
+            x[e] = fine ? fmaf(d, a[64 * e], fmaf(d, S[e], x[e])) : out[64 * e];
             out[64 * e] = -x[e];
             if ((ln & 31) < cnt && 32 * J + acc_row(e, h) < b) dst[acc_row(e, 0) * step] = x[e];
         }

@@ -251,3 +251,27 @@ def test_trsm_of_more_lines_than_one_launch_takes(ctx):
     P.fill_(1.0)
     ctx.trsm_upanel(b, m, T, b, P, b)
     assert bool((P[0::2] == 1.0).all()) and bool((P[1::2] == 0.5).all())
+
+
+@pytest.mark.parametrize("n,pad", [(33, 0), (60, 0), (64, 3), (128, 0), (129, 1), (200, 0), (300, 0), (512, 0), (515, 1),
+                                   (777, 0), (1024, 0)])
+@pytest.mark.parametrize("diag", [0.3, 1.0, 3.0])
+def test_getrf_far_from_dominance(ctx, n, pad, diag):
+    """Elimination has |A - L U| <= g |L| |U| entry by entry whatever the growth:
+    n roundings of the sums, 64 more and the factor 2 for the 32 x 32 inverses,
+    which are taken only where |D^-1| |D| is below 16 (their products add at most
+    16 roundings' worth of the 32-block's own |L| |U|): g = 2 (n + 64 + 16) u."""
+    import torch
+    rng = np.random.default_rng(n)
+    A = (rng.uniform(-0.5, 0.5, (n, n)) * (1.0 - np.eye(n)) + np.eye(n) * diag * rng.choice([-1.0, 1.0], n)).astype(np.float32)
+    F = torch.from_numpy(np.ascontiguousarray(np.pad(A.T, ((0, 0), (0, pad))))).cuda()
+    info = torch.full((1,), 7, dtype=torch.int32, device="cuda")
+    ctx.getrf(n, F, n + pad, info)
+    assert info.item() == 0
+    M = F[:, :n].t().cpu().numpy().astype(np.float64)
+    L, U = np.tril(M, -1) + np.eye(n), np.triu(M)
+    assert np.isfinite(M).all()
+    u = 2.0 ** -24
+    bound = 2 * (n + 80) * u * (np.abs(L) @ np.abs(U))
+    R = np.abs(A.astype(np.float64) - L @ U)
+    assert (R <= bound).all(), float((R / bound).max())
