@@ -15,14 +15,15 @@
 // with one (the inverses of both triangles together: 40 + 28 + 23 us at 8192).
 // Substitution in one workgroup per block and reading the factors once per
 // column took, both triangles, 2707 us at 8192 x 64 (6320 us transposed), now
-// 764 (744); 2060 us at 8192 x 1, now 540; 285 us at 1200 x 3, now 127; 9.5 ms
+// 751 (729); 2060 us at 8192 x 1, now 529; 285 us at 1200 x 3, now 120; 9.5 ms
 // at 30000 x 1, now 2.8.
 // A product with an inverse has the error of substitution times the condition
-// of the 512 x 512 block.  So each block's condition, the largest row sum of
-// |T_kk^-1| |T_kk|, is formed with its inverse (9 us at 1200, 22 at 8192), and a
-// block past kTsCond is solved by substitution instead (tri64_substitute): all
-// blocks so, 2.6 ms at 8192 x 64 (3.5 transposed), 2.3 at 8192 x 1, 0.38 at
-// 1200 x 3, bound by the triangle's way into one CU.
+// of the 512 x 512 block.  So each block's condition, a bound of the largest row
+// sum of |T_kk^-1| |T_kk|, is formed with its inverse, by workgroups and registers
+// that have the operands anyway (2 us at 1200, 9 at 8192; a kernel of its own took
+// 8 and 22), and a block past kTsCond is solved by substitution instead
+// (tri64_substitute): all blocks so, 2.5 ms at 8192 x 64 (3.4 transposed), 2.3 at
+// 8192 x 1, 0.37 at 1200 x 3, bound by the triangle's way into one CU.
 //
 // An upper triangle is a lower one with rows and columns taken from the end;
 // TriView numbers entries that way, so the kernels only know lower ones.
@@ -38,7 +39,9 @@ constexpr int kTsInv = 32 * 32 * 256;     // doubles of one block's inverse, 16 
 constexpr int kTsMid = 16 * 16 * 256;     // doubles of one block's intermediate product
 constexpr int kTsGroup = 32;              // blocks inverted at a time (96 MiB a triangle)
 constexpr int kTsCols = 1024;             // right-hand sides at a time
-constexpr int kTsRow = kTsBlock + 16;     // doubles of one block's row sums of |T| and, at kTsBlock, its mark
+// doubles of one block's condition: row sums of |A|, of |B|, its mark, and from
+// kTsPart the parts of |C A^-1| |A| and of |C| for row r of the second half at J 256 + r, J < 16 and 16
+constexpr int kTsPart = kTsBlock + 16, kTsRow = kTsPart + 17 * kTsHalf;
 // Largest condition that is solved through the inverse.  Errors of inverse /
 // substitution (FP64, order 512, b = T x): condition 3.6 (factors of HPL-AI
 // matrices) 1.2e-16 / 1.2e-16 of the solution, 18 1.5e-16 / 1.3e-16, 54 3.5e-16
@@ -80,11 +83,12 @@ struct TsInvLds {
     double rd[16][16];        // reciprocals of their diagonals
     double P[16][256];        // their inverses, packed
     float R[2][240 * 17];     // E(I, :) of two rows of tiles, R[col * 17 + row]
+    double sum[16][257];      // each thread's part of the row sums of |E(I, :)|
 };
 
 template <bool UPPER, bool TRANS>
 __device__ __forceinline__ void tri64_inv(const TriView<UPPER, TRANS> &E, int64_t first, double *__restrict__ inv,
-                                          double *__restrict__ bop, TsInvLds &sm)
+                                          double *__restrict__ bop, double *__restrict__ rows, TsInvLds &sm)
 {
     auto &D = sm.D;
     auto &P = sm.P;
@@ -104,12 +108,15 @@ __device__ __forceinline__ void tri64_inv(const TriView<UPPER, TRANS> &E, int64_
             }
     };
     auto stage = [&](int I) {
+        double part = 0.0;
 #pragma unroll
         for (int u = 0; u < 15; ++u)
             if (u < I) {
                 const int r = TRANS ? tid >> 4 : tid & 15, c = 16 * u + (TRANS ? tid & 15 : tid >> 4);
                 R[I & 1][c * 17 + r] = rv[u];
+                part += fabs(static_cast<double>(rv[u]));
             }
+        sm.sum[I][tid] = part;
     };
     fetch(1);
     {
@@ -192,61 +199,23 @@ __device__ __forceinline__ void tri64_inv(const TriView<UPPER, TRANS> &E, int64_
             }
         if (I > 0 && I < 15) stage(I + 1);
     }
-}
-
-// Row sums of |T| over the 512-block for 64 rows of the 256-block blockIdx.x
-// (blockIdx.y - 4), zeros past the matrix.  The lanes run along the factor's
-// contiguous direction.
-template <bool UPPER, bool TRANS>
-__device__ __forceinline__ void tri64_rows(const TriView<UPPER, TRANS> &E, int64_t first, double *__restrict__ rows,
-                                           double *red)
-{
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t h = static_cast<int64_t>(blockIdx.x), b0 = first + (h >> 1) * kTsBlock;
-    const int c0 = static_cast<int>(h & 1) * kTsHalf + 64 * (static_cast<int>(blockIdx.y) - 4);   // first row in the block
-    double *out = rows + (h >> 1) * kTsRow;
-    auto term = [&](int r, int k, float v) {
-        const double a = k == r && TriView<UPPER, TRANS>::kUnit ? 1.0 : fabs(static_cast<double>(v));
-        return k <= r && b0 + r < E.n ? a : 0.0;
-    };
-    if constexpr (TRANS) {
-        double acc[16];
+    if (blockIdx.y != 0) return;
+    // row sums of |E|, a row per thread, zeros past the end
+    __syncthreads();
+    const int I = tid >> 4, r = tid & 15;
+    double s = 0.0;
 #pragma unroll
-        for (int u = 0; u < 16; ++u) acc[u] = 0.0;
-        for (int k0 = 0; k0 < c0 + 64; k0 += 64) {
-            float v[16];
+    for (int c = 0; c < 16; ++c) s += fabs(D[I][r][c]);
+    if (I > 0)
 #pragma unroll
-            for (int u = 0; u < 16; ++u)
-                v[u] = *E.ptr(min(b0 + c0 + 16 * wave + u, E.n - 1), min(b0 + k0 + lane, E.n - 1));
-#pragma unroll
-            for (int u = 0; u < 16; ++u) acc[u] += term(c0 + 16 * wave + u, k0 + lane, v[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            double s = acc[u];
-            for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-            if (lane == u) out[c0 + 16 * wave + u] = s;
-        }
-    } else {
-        double acc = 0.0;
-        for (int k0 = 0; k0 < c0 + 64; k0 += 64) {
-            float v[16];
-#pragma unroll
-            for (int u = 0; u < 16; ++u)
-                v[u] = *E.ptr(min(b0 + c0 + lane, E.n - 1), min(b0 + k0 + 16 * wave + u, E.n - 1));
-#pragma unroll
-            for (int u = 0; u < 16; ++u) acc += term(c0 + lane, k0 + 16 * wave + u, v[u]);
-        }
-        red[wave * 64 + lane] = acc;
-        __syncthreads();
-        if (wave == 0) out[c0 + lane] = ((red[lane] + red[64 + lane]) + red[128 + lane]) + red[192 + lane];
-    }
-    if (c0 == 0 && threadIdx.x == 0) out[kTsBlock] = 0.0;
+        for (int c = 0; c < 16; ++c) s += sm.sum[I][TRANS ? 16 * r + c : 16 * c + r];
+    double *row = rows + (h >> 1) * kTsRow;
+    row[(h & 1) * kTsHalf + tid] = e0 + tid < E.n ? s : 0.0;
+    if ((h & 1) == 0 && tid == 0) row[kTsBlock] = 0.0;
 }
 
 // blockIdx.z (+ upper0): the lower or the upper triangle of the pair that one
-// lu_solve needs; z2: doubles from the first's scratch to the second's.
-// blockIdx.y < 4: the inverses; 4 .. 7: the row sums
+// lu_solve needs; z2: doubles from the first's scratch to the second's
 template <bool TRANS>
 __global__ __launch_bounds__(256) void tri64_inv_kernel(const float *__restrict__ LU, int64_t lda, int64_t n,
                                                         int64_t first, int upper0, double *__restrict__ inv,
@@ -256,62 +225,19 @@ __global__ __launch_bounds__(256) void tri64_inv_kernel(const float *__restrict_
     inv += blockIdx.z * z2;
     bop += blockIdx.z * z2;
     rows += blockIdx.z * z2;
-    const TriView<true, TRANS> U{LU, lda, n};
-    const TriView<false, TRANS> L{LU, lda, n};
-    const bool upper = (upper0 + static_cast<int>(blockIdx.z)) & 1;
-    if (blockIdx.y >= 4) {
-        if (upper)
-            tri64_rows(U, first, rows, &sm.rd[0][0]);
-        else
-            tri64_rows(L, first, rows, &sm.rd[0][0]);
-    } else if (upper) {
-        tri64_inv(U, first, inv, bop, sm);
-    } else {
-        tri64_inv(L, first, inv, bop, sm);
-    }
-}
-
-// Marks the 512-block blockIdx.x when a row sum of |T^-1| |T| is past kTsCond
-// or no number.  A wave takes the 16 rows of tile 4 blockIdx.y + wave.
-__global__ __launch_bounds__(256) void tri64_cond_kernel(int64_t left, const double *__restrict__ inv, double *rows,
-                                                         int64_t z2)
-{
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int l16 = lane & 15, lk = lane >> 4;
-    const double *bi = inv + blockIdx.z * z2 + static_cast<int64_t>(blockIdx.x) * kTsInv;
-    double *row = rows + blockIdx.z * z2 + static_cast<int64_t>(blockIdx.x) * kTsRow;
-    const int64_t over = left - static_cast<int64_t>(blockIdx.x) * kTsBlock;
-    const int w = over < kTsBlock ? static_cast<int>(over) : kTsBlock;
-    const int I = 4 * static_cast<int>(blockIdx.y) + wave;
-    if (16 * I >= w) return;
-    double s = 0.0;
-    for (int K0 = 0; K0 <= I; K0 += 4) {
-        double a[4][4], r[4][4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int K = min(K0 + u, I);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                a[u][t] = bi[(I * 32 + K) * 256 + lane * 4 + t];
-                r[u][t] = row[16 * K + 4 * t + lk];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (K0 + u <= I)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) s = fma(fabs(a[u][t]), r[u][t], s);
-    }
-    s += __shfl_xor(s, 16);
-    s += __shfl_xor(s, 32);
-    if (__any(16 * I + l16 < w && !(s <= kTsCond)) && lane == 0) row[kTsBlock] = 1.0;
+    if ((upper0 + static_cast<int>(blockIdx.z)) & 1)
+        tri64_inv(TriView<true, TRANS>{LU, lda, n}, first, inv, bop, rows, sm);
+    else
+        tri64_inv(TriView<false, TRANS>{LU, lda, n}, first, inv, bop, rows, sm);
 }
 
 // 256 -> 512: the lower left quarter -B^-1 C A^-1.  MID: tile (I, J) of
-// C A^-1 to mid in right-operand order [q 64 + lane]; else of -B^-1 mid.
+// M = C A^-1 to mid in right-operand order [q 64 + lane], and the tile's parts of
+// the row sums of |M| |A| and |C|; else of -B^-1 mid.
 template <bool UPPER, bool TRANS, bool MID>
 __device__ __forceinline__ void tri64_merge(const TriView<UPPER, TRANS> &E, int64_t first, double *__restrict__ inv,
-                                            const double *__restrict__ bop, double *__restrict__ mid)
+                                            const double *__restrict__ bop, double *__restrict__ mid,
+                                            double *__restrict__ rows)
 {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, lk = lane >> 4;
@@ -320,6 +246,9 @@ __device__ __forceinline__ void tri64_merge(const TriView<UPPER, TRANS> &E, int6
     const int tile = static_cast<int>(blockIdx.y) * 4 + wave, I = tile >> 4, J = tile & 15;
     double *bi = inv + static_cast<int64_t>(blockIdx.x) * kTsInv, *m = mid + static_cast<int64_t>(blockIdx.x) * kTsMid;
     const double *bo = bop + static_cast<int64_t>(blockIdx.x) * kTsMid;
+    double *row = rows + static_cast<int64_t>(blockIdx.x) * kTsRow;
+    double w = 0.0, cs = 0.0;
+    if (MID) w = row[16 * J + l16];
     // four tiles' operands in flight; steps past the end take zeros
     const int K0 = MID ? J : 0, K1 = MID ? 16 : I + 1;
     const int64_t i = min(e0 + kTsHalf + 16 * I + l16, E.n - 1);
@@ -346,7 +275,10 @@ __device__ __forceinline__ void tri64_merge(const TriView<UPPER, TRANS> &E, int6
         for (int u = 0; u < 4; ++u)
             if (K + u < K1)
 #pragma unroll
-                for (int t = 0; t < 4; ++t) T = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][t], b[u][t], T, 0, 0, 0);
+                for (int t = 0; t < 4; ++t) {
+                    T = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][t], b[u][t], T, 0, 0, 0);
+                    if (MID && J == 0) cs += fabs(a[u][t]);
+                }
     }
     // rows past the end hold copies of the last: dropped with the rows of the inverse below them
 #pragma unroll
@@ -356,21 +288,91 @@ __device__ __forceinline__ void tri64_merge(const TriView<UPPER, TRANS> &E, int6
         else
             bi[((16 + I) * 32 + J) * 256 + tile_pos(lk + 4 * q, l16)] = -T[q];
     }
+    if constexpr (MID) {
+        double v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = fabs(T[q]) * w;
+#pragma unroll
+        for (int off = 1; off < 16; off *= 2)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] += __shfl_xor(v[q], off);
+        if (l16 == 0)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) row[kTsPart + J * kTsHalf + 16 * I + lk + 4 * q] = v[q];
+        if (J == 0) {
+            cs += __shfl_xor(cs, 16);
+            cs += __shfl_xor(cs, 32);
+            if (lane < 16) row[kTsPart + 16 * kTsHalf + 16 * I + lane] = cs;
+        }
+    }
 }
 
+// Marks the 512-block where a row sum of |A^-1| |A|, or of |B^-1| (|C A^-1| |A| +
+// |B| + |C|), which bounds the second half's of |T^-1| |T|, is past kTsCond or no
+// number.  Row tile blockIdx.y - 64; the four waves split K.  left: rows of the
+// matrix from the group's first.
+__device__ __forceinline__ void tri64_mark(int64_t left, const double *__restrict__ inv, double *rows, double *u,
+                                           double (&red)[4][16])
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lk = lane >> 4;
+    const double *bi = inv + static_cast<int64_t>(blockIdx.x) * kTsInv;
+    double *row = rows + static_cast<int64_t>(blockIdx.x) * kTsRow;
+    const int tile = static_cast<int>(blockIdx.y) - 64, h = tile >> 4, I = tile & 15;
+    const int64_t over = left - static_cast<int64_t>(blockIdx.x) * kTsBlock;
+    const int w = over < kTsBlock ? static_cast<int>(over) : kTsBlock;
+    if (16 * tile >= w) return;
+    if (tid < 16 * (I + 1)) {
+        double s = row[kTsHalf * h + tid];
+        if (h != 0) {
+            double p[17];
+#pragma unroll
+            for (int J = 0; J < 17; ++J) p[J] = row[kTsPart + J * kTsHalf + tid];
+#pragma unroll
+            for (int J = 0; J < 17; ++J) s += p[J];
+        }
+        u[tid] = s;
+    }
+    double a[4][4];   // K = wave + 4 q
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) a[q][t] = bi[(tile * 32 + 16 * h + min(wave + 4 * q, I)) * 256 + lane * 4 + t];
+    __syncthreads();
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (wave + 4 * q <= I)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) s = fma(fabs(a[q][t]), u[16 * (wave + 4 * q) + 4 * t + lk], s);
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    if (lane < 16) red[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0) {
+        s = ((red[0][l16] + red[1][l16]) + red[2][l16]) + red[3][l16];
+        if (__any(16 * tile + l16 < w && !(s <= kTsCond)) && lane == 0) row[kTsBlock] = 1.0;
+    }
+}
+
+// without MID also the marks (blockIdx.y from 64 on)
 template <bool TRANS, bool MID>
 __global__ __launch_bounds__(256) void tri64_merge_kernel(const float *__restrict__ LU, int64_t lda, int64_t n,
                                                           int64_t first, int upper0, double *__restrict__ inv,
                                                           const double *__restrict__ bop, double *__restrict__ mid,
-                                                          int64_t z2)
+                                                          double *__restrict__ rows, int64_t z2)
 {
+    __shared__ double u[kTsHalf], red[4][16];
     inv += blockIdx.z * z2;
     bop += blockIdx.z * z2;
     mid += blockIdx.z * z2;
-    if ((upper0 + static_cast<int>(blockIdx.z)) & 1)
-        tri64_merge<true, TRANS, MID>(TriView<true, TRANS>{LU, lda, n}, first, inv, bop, mid);
+    rows += blockIdx.z * z2;
+    if (!MID && blockIdx.y >= 64)
+        tri64_mark(n - first, inv, rows, u, red);
+    else if ((upper0 + static_cast<int>(blockIdx.z)) & 1)
+        tri64_merge<true, TRANS, MID>(TriView<true, TRANS>{LU, lda, n}, first, inv, bop, mid, rows);
     else
-        tri64_merge<false, TRANS, MID>(TriView<false, TRANS>{LU, lda, n}, first, inv, bop, mid);
+        tri64_merge<false, TRANS, MID>(TriView<false, TRANS>{LU, lda, n}, first, inv, bop, mid, rows);
 }
 
 // Position of entry (k, column c) in the solved block's array: 16 x 16 tiles
@@ -643,15 +645,13 @@ static int tri_invert(bool upper, bool both, int64_t n, int64_t first, const flo
     const unsigned gc = static_cast<unsigned>(left < g ? left : g), z = both ? 2 : 1;
     double *mid = inv + g * kTsInv, *bop = mid + g * kTsMid, *rows = tri_rows(n, inv);
     const int64_t z2 = tri_inv_doubles(n);
-    hipLaunchKernelGGL((tri64_inv_kernel<TRANS>), dim3(2 * gc, 8, z), dim3(256), 0, s, LU, lda, n, first,
+    hipLaunchKernelGGL((tri64_inv_kernel<TRANS>), dim3(2 * gc, 4, z), dim3(256), 0, s, LU, lda, n, first,
                        upper ? 1 : 0, inv, bop, rows, z2);
-    if (n - first > kTsHalf) {
+    if (n - first > kTsHalf)
         hipLaunchKernelGGL((tri64_merge_kernel<TRANS, true>), dim3(gc, 64, z), dim3(256), 0, s, LU, lda, n, first,
-                           upper ? 1 : 0, inv, bop, mid, z2);
-        hipLaunchKernelGGL((tri64_merge_kernel<TRANS, false>), dim3(gc, 64, z), dim3(256), 0, s, LU, lda, n, first,
-                           upper ? 1 : 0, inv, bop, mid, z2);
-    }
-    hipLaunchKernelGGL(tri64_cond_kernel, dim3(gc, 8, z), dim3(256), 0, s, n - first, inv, rows, z2);
+                           upper ? 1 : 0, inv, bop, mid, rows, z2);
+    hipLaunchKernelGGL((tri64_merge_kernel<TRANS, false>), dim3(gc, 96, z), dim3(256), 0, s, LU, lda, n, first,
+                       upper ? 1 : 0, inv, bop, mid, rows, z2);
     HPLAI_HIP(hipGetLastError());
     return HPLAI_OK;
 }
