@@ -200,7 +200,8 @@ namespace hplai {
 // TRSMs 512 x 40000 567 -> 562 us.)
 // Blocks above the diagonal of Linv and below the diagonal of Uinv are never
 // written or read.  Behind the blocks, 64 floats: [2 q + 1 for U] is 1 where the
-// triangle of diagonal block q is not well conditioned (poor32).
+// triangle of diagonal block q is not well conditioned (poor32), and 64 more: [Q] is
+// 1 where that matters to the strips beside 128-block Q.
 __device__ __forceinline__ int tri_pos(int lane, int kk) { return (kk >> 2) * 256 + lane * 4 + (kk & 3); }
 template <typename T>
 __device__ __forceinline__ T *tri_block_l(T *tri, int nb, int I, int J)
@@ -216,6 +217,11 @@ template <typename T>
 __device__ __forceinline__ T *tri_poor(T *tri, int nb)
 {
     return tri + 2 * static_cast<int64_t>(nb) * nb * 1024;
+}
+template <typename T>
+__device__ __forceinline__ T *tri_careful(T *tri, int nb)
+{
+    return tri_poor(tri, nb) + 64;
 }
 
 }  // namespace hplai

@@ -1,11 +1,13 @@
 // getrf.hip — LU of a diagonal block (n <= 1024) and the inverses of its
 // triangles, spread over the device.
 //
-// Two forms: the LU's own (FULL), with the inverses that its panels need, and a
-// caller's (hplai_getrf_nopiv_f32), whose strips take only inverses of 32 x 32
-// blocks, and those only where the block is well conditioned.  With the inverses
-// of 128-blocks |A - L U| was past the 2 (n + 80) u |L| |U| of elimination for
-// blocks far from dominance (3.4 times for diagonals of 3 at 512).
+// Products with inverses of 128-blocks take |A - L U| past the 2 (n + 80) u |L| |U|
+// of elimination where the diagonal does not dominate (3.4 times for diagonals of
+// 3 at 512, and refinement from such factors of 1024 with diagonals of 5 needed
+// three times the steps or diverged).  So each sub-block's rows are looked at
+// first: where the diagonal dominates, those products lose nothing; elsewhere
+// strips of a sub-block whose triangles are not well conditioned are walked through
+// with inverses of 32 x 32 blocks, and by substitution where one of those is not.
 //
 // Replaces getrf_nopiv (getrf_nopiv.hpp:124-160).  The block is walked in
 // sub-blocks of 128 columns; per sub-block three kinds of work, all FP32 on
@@ -31,12 +33,13 @@
 // with the strips and the next sub-block's update).  One workgroup for the
 // whole 512 block spent half its time on trailing updates through a single
 // CU's path to the L2, and the inverses were two more kernels after it: 511 +
-// 73 us, now 172 us with the inverses and 162 without (b = 512, alone); b = 60:
-// 94 -> 14 us; n = 1000: 645 us with v_readlane steps, 342 us as here.  The
+// 73 us, now 176 us with the inverses and 156 without (b = 512, alone); b = 60:
+// 94 -> 14 us; n = 1000: 645 us with v_readlane steps, 327 us as here.  The
 // next sub-block's update in the workgroup that factors it took 11 us of each
 // sub-block (its operands, 192 KB, again through one CU): 198 us at b = 512.
 // Joining the inverses by one workgroup per 32 columns took 39 us a size
 // (product by product, each behind its loads) after the factorization.
+#include <cfloat>
 #include <cstddef>
 #include <type_traits>
 
@@ -53,6 +56,15 @@ constexpr int kLuThreads = 512;
 constexpr int kLuS = kLuNB + 1;       // LDS column stride: odd, so that walks along rows and columns both spread
 using LuStride = std::integral_constant<int, kLuS>;
 constexpr int kJoinMax = 512;         // largest half joined by tri_join_kernel
+// Off-diagonal row sums up to this part of the diagonal entries bound the condition
+// of a sub-block's triangles: with D its diagonal, |U^-1| |D|, |D^-1| |U| and so on
+// have row sums of at most (1 + p) / (1 - p), |U^-1| |U| 4 at 0.6 and, rows scaled
+// by D, |L^-1| |L| 16.  Those of HPL-AI matrices have about 128 / n (getrf of 512
+// 156 us, 154 without the look).  Other sub-blocks look at their
+// inverses (170 us), and strips go through those where no row sum of |X| |T| is past
+// kCond128, else through 32-blocks (200 us).
+constexpr float kCond128 = 16.0f;
+constexpr float kDominance = 0.6f;
 
 __device__ __forceinline__ floatx16g_t zero16()
 {
@@ -68,6 +80,8 @@ struct LuLds {
     float Li[32 * 33], Ui[32 * 33];   // inverses of the current 32 x 32 triangles, row-major
     float w[2][32];                   // row sums of the current 32 x 32 triangles, L and U
     int poor[2];                      // they are not well conditioned
+    float sums[2][4][kLuNB];          // row sums of the sub-block's magnitudes, later of its triangles', in parts
+    int careful;                      // the sub-block's diagonal does not dominate
 };
 
 // entry (i, j) of a unit-lower / an upper triangle whose block also holds the other one
@@ -295,13 +309,12 @@ __device__ __forceinline__ void tri_fin(int nb, float *tri, int J, int R0, int R
     }
 }
 
-// Sub-block k0 of the n x n block A.  FACTOR: LU, inverses; the next workgroups
-// update the rest of the trailing matrix with sub-block k0 - 128 (when there is
-// one) and copy the blocks beside the diagonal one, and the last form the first products of the
-// whole block's inverses.  Without FACTOR: A is already factored and
-// workgroup q inverts the triangles of sub-block q.  Without FULL (a caller's
-// own LU) only the 32 x 32 inverses are formed and written, and blocks that are
-// not well conditioned are substituted with instead.
+// Sub-block k0 of the n x n block A.  FACTOR: LU, inverses and whether the strips
+// may go through these; the next workgroups update the rest of the trailing matrix
+// with sub-block k0 - 128 (when there is one) and copy the blocks beside the
+// diagonal one, and the last form the first products of the whole block's inverses.
+// Without FACTOR: A is already factored and workgroup q inverts the triangles of
+// sub-block q, or, without FULL, of its 32 x 32 blocks alone.
 template <bool FACTOR, bool FULL>
 __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, float *__restrict__ A, int64_t lda,
                                                                float *tri, int sides,
@@ -323,7 +336,7 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
         // of the first sub-block only the four that are copied
         const int two = ct < 2 ? ct : 2, z = static_cast<int>(blockIdx.x) - 1;
         const int t = p0 >= 0 ? z + two : z < 2 ? ct + z : z;
-        if (FULL && p0 >= 0 && t >= rt * ct) {
+        if (p0 >= 0 && t >= rt * ct) {
             static_assert(offsetof(LuLds, V) == sizeof(float) * kLuNB * kLuS && (1024 - kLuNB) * 33 <= 2 * kLuNB * kLuS,
                           "the strip of an inverse spans S and V");
             const int y = t - rt * ct, q0 = k0 / 32;
@@ -395,6 +408,7 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
     const int steps = (w + 31) / 32, q0 = k0 / 32;
     {
         const int r = tid & 127;
+        float s = 0.0f;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             float v[16];
@@ -404,9 +418,13 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int c = (tid >> 7) + 4 * (16 * h + e);
-                S[c * kLuS + r] = (r < w && c < w) ? v[e] : (r == c ? 1.0f : 0.0f);
+                v[e] = (r < w && c < w) ? v[e] : (r == c ? 1.0f : 0.0f);
+                S[c * kLuS + r] = v[e];
+                if (FACTOR) s += fabsf(v[e]);
             }
         }
+        if (FACTOR) sm.sums[0][tid >> 7][r] = s;
+        if (FACTOR && tid == 0) sm.careful = 0;
     }
     __syncthreads();
     if (!FACTOR) {
@@ -465,6 +483,7 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
         for (int e = 0; e < 16; ++e) S[(cc + l32) * kLuS + r0 + acc_row(e, lh)] -= acc[e];
     };
     int bad = 0;
+    bool careful = false;   // strips by substitution where the inverses are not well conditioned
     for (int q = 0; q < steps; ++q) {
         const int c0 = 32 * q, t = 7 - wave;   // t: this wave's block of the inverses' row q
         // a lane number of the iteration's own: addresses and masks hoisted out
@@ -485,21 +504,24 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
         } else if (q > 0) {
             const int R = steps - q;
             for (int i = wave; i < R * R; i += kLuThreads / 64 - 1) update(ln, c0 - 32, c0 + 32 * (i % R), c0 + 32 * (i / R));
-            if (FULL)
-                write_inverse_row(V, tri, nb, q0, q - 1, wave - 1, sides, ln);
-            else if (wave < 3)
-                write_inverse_row(V, tri, nb, q0, q - 1, wave == 1 ? q - 1 : 2 * q - 1, sides, ln);
-            if (FULL && tri != nullptr && t < 2 * q)
+            write_inverse_row(V, tri, nb, q0, q - 1, wave - 1, sides, ln);
+            if (tri != nullptr && t < 2 * q)
                 T = t & 1 ? inverse_row_product<true>(S, V, q, t >> 1, ln) : inverse_row_product<false>(S, V, q, t >> 1, ln);
+        } else if (wave >= 6) {
+            const int r = 64 * (wave - 6) + ln;
+            const float d = r < w ? fabsf(Ak[r * (lda + 1)]) : 1.0f;
+            const float *p = &sm.sums[0][0][r], s = ((p[0] + p[kLuNB]) + p[2 * kLuNB]) + p[3 * kLuNB];
+            if (!__all(s <= fminf((1.0f + kDominance) * d, FLT_MAX))) sm.careful = 1;
         }
         __syncthreads();
+        if (q == 0) careful = __builtin_amdgcn_readfirstlane(sm.careful) != 0;
         if (wave == 0) {
             invert32<false>(S + c0 * (kLuS + 1), LuStride{}, V + c0 * (kLuS + 1), ln, sm.Li);
         } else if (wave == 1) {
             invert32<true>(S + c0 * (kLuS + 1), LuStride{}, V + c0 * (kLuS + 1), ln, sm.Ui);
         } else {
-            if (!FULL && wave == 6) row_sums32<false>(S + c0 * (kLuS + 1), LuStride{}, sm.w[0], ln);
-            if (!FULL && wave == 7) row_sums32<true>(S + c0 * (kLuS + 1), LuStride{}, sm.w[1], ln);
+            if (careful && wave == 6) row_sums32<false>(S + c0 * (kLuS + 1), LuStride{}, sm.w[0], ln);
+            if (careful && wave == 7) row_sums32<true>(S + c0 * (kLuS + 1), LuStride{}, sm.w[1], ln);
             if (q + 1 == steps)   // all of S is final: factors back to A
 #pragma unroll 4
                 for (int c = (wave - 2) >> 1; c < w; c += 3) {
@@ -530,7 +552,7 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
                 }
             }
             X = mfma16(av, bv, X);
-        } else if (!FULL && wave >= 6 && (R > 0 || tri != nullptr)) {
+        } else if (careful && wave >= 6 && (R > 0 || tri != nullptr)) {
             const float *M = wave == 6 ? sm.Li : sm.Ui;
             const bool poor = poor32([&](int r, int c) { return M[r * 33 + c]; }, sm.w[wave - 6], ln);
             if (ln == 0) {
@@ -538,8 +560,8 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
                 if (tri != nullptr) tri_poor(tri, nb)[2 * (q0 + q) + wave - 6] = poor ? 1.0f : 0.0f;
             }
         }
-        if (!FULL && R > 0) __syncthreads();
-        if (!FULL && mine && sm.poor[up ? 0 : 1]) {
+        if (careful && R > 0) __syncthreads();
+        if (careful && mine && sm.poor[up ? 0 : 1]) {
             // by substitution, a row or column per lane
             float *x = up ? S + (o + (ln & 31)) * kLuS + c0 : S + c0 * kLuS + o + (ln & 31);
             const int dx = up ? 1 : kLuS;
@@ -566,7 +588,7 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
                     S[(c0 + l32) * kLuS + o + r] = X[e];
             }
         }
-        if (FULL && tri != nullptr && t < 2 * q) {
+        if (tri != nullptr && t < 2 * q) {
             if (t & 1)
                 inverse_row_finish<true>(V, q, t >> 1, ln, T);
             else
@@ -574,18 +596,59 @@ __global__ __launch_bounds__(kLuThreads) void lu_update_kernel(int n, int k0, fl
         }
         __syncthreads();
     }
-    if (FULL)
-        write_inverse_row(V, tri, nb, q0, steps - 1, wave, sides, lane);
-    else if (wave < 2)
-        write_inverse_row(V, tri, nb, q0, steps - 1, wave == 0 ? steps - 1 : 2 * steps - 1, sides, lane);
+    write_inverse_row(V, tri, nb, q0, steps - 1, wave, sides, lane);
+    if (k0 + kLuNB < n) {
+        int poor = 0;
+        if (careful) {
+            // the largest row sum of |X| |T|: row sums of |T| first, a quarter of the
+            // columns per two waves, side 0 L and side 1 U
+            int i = tid;
+            asm volatile("" : "+v"(i));   // as ln
+            const int r = i & 127, g = wave >> 1;
+            float sl = r >> 5 == g ? 1.0f : 0.0f, su = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 32; ++k) {
+                const float v = fabsf(S[(32 * g + k) * kLuS + r]);
+                sl += 32 * g + k < r ? v : 0.0f;
+                su += 32 * g + k < r ? 0.0f : v;
+            }
+            sm.sums[0][g][r] = sl;
+            sm.sums[1][g][r] = su;
+            __syncthreads();
+            const float *p = &sm.sums[0][0][32 * g + (i & 31)];
+            const float wl = ((p[0] + p[kLuNB]) + p[2 * kLuNB]) + p[3 * kLuNB];
+            p += 4 * kLuNB;
+            const float wu = ((p[0] + p[kLuNB]) + p[2 * kLuNB]) + p[3 * kLuNB];
+            __syncthreads();
+            const float d = __shfl(wl, r & 31);
+            sl = r >> 5 == g ? d : 0.0f;   // the unit diagonal's term
+            su = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 32; ++k) {
+                const float v = fabsf(V[(32 * g + k) * kLuS + r]);
+                const float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wl), k));
+                const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wu), k));
+                sl = fmaf(32 * g + k < r ? v : 0.0f, a, sl);
+                su = fmaf(32 * g + k < r ? 0.0f : v, c, su);
+            }
+            sm.sums[0][g][r] = sl;
+            sm.sums[1][g][r] = su;
+            __syncthreads();
+            p = &sm.sums[wave < 2 ? 0 : 1][0][r];
+            poor = wave < 4 && !__all(((p[0] + p[kLuNB]) + p[2 * kLuNB]) + p[3 * kLuNB] <= kCond128);
+            poor = __syncthreads_or(poor);
+        }
+        if (tid == 0) tri_careful(tri, nb)[q0 / 4] = poor ? 1.0f : 0.0f;
+    }
     if (tid == 0 && info != nullptr && (k0 == 0 || (bad != 0 && *info == 0))) *info = bad;
 }
 
 // Block (r, c) of the next diagonal sub-block -= L21(r, :) U12(:, c), with its
 // strips formed from the copies: wave J forms L21(r, J)^T and U12(J, c), whose
-// accumulators are the operands of their product (k = acc_row either way).
-__device__ __forceinline__ void next_diagonal(int n, int nb, int q0, int r, int c, float *A, int64_t lda, float *tri,
-                                              float *XL, float *XU)
+// accumulators are the operands of their product (k = acc_row either way).  With
+// careful: nothing.
+__device__ __forceinline__ bool next_diagonal(int n, int nb, int q0, int r, int c, float *A, int64_t lda, float *tri,
+                                              float *XL, float *XU, int careful)
 {
     const int tid = threadIdx.x, lane = tid & 63, J = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
@@ -620,6 +683,7 @@ __device__ __forceinline__ void next_diagonal(int n, int nb, int q0, int r, int 
         y[3] = xu[K].w;
     }
     __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(careful) != 0) return false;
     floatx16g_t al = zero16(), au = zero16();
 #pragma unroll
     for (int K = 0; K < 4; ++K) {
@@ -652,132 +716,126 @@ __device__ __forceinline__ void next_diagonal(int n, int nb, int q0, int r, int 
             const int row = 32 * R + 8 * J + 4 * lh + i;
             if (row < n) A[col * lda + row] = d[i] - (((p[0] + p[1024]) + p[2048]) + p[3072]);
         }
+    return true;
 }
 
-// The same for a caller's own LU, 32-block by 32-block (trsm.hip has the walk
-// for panels): workgroup z takes 32 rows of L21 with four waves and 32 columns of
-// U12 with four, or, past the strips, both that a block of the next diagonal
-// sub-block needs, from the copies, and then that block.  Wave J of a side holds
-// block J in its accumulators' order, transposed for L21; the sides' waves J are
-// on different SIMDs.  Four solves and three products one after the other instead
-// of four products: 512 154 -> 162 us (both sides in the same waves: 167).
-__global__ __launch_bounds__(512) void lu_strip_walk_kernel(int n, int p0, float *A, int64_t lda, float *tri, int strips)
+// The same 32-block by 32-block (trsm.hip has the walk for panels), where a
+// sub-block is not well conditioned: y < 0: strip z, 32 rows of L21 or (up1)
+// columns of U12; else both strips that block (r, c) = y of the next diagonal
+// sub-block needs, from the copies, one after the other, and then that block.
+// Wave J holds block J in its accumulators' order, transposed for L21.  xl: -X_K of
+// both sides.
+__device__ __forceinline__ void strip_walk(int n, int p0, float *A, int64_t lda, float *tri, int z, bool up1, int y,
+                                           int nd, float (*xl)[4][1024])
 {
-    __shared__ float xl[2][4][1024];   // -X_K of both sides
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tid = threadIdx.x, lane = tid & 63, J = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
-    const bool up = wave >= 4;
-    const int J = up ? (wave + 2) & 3 : wave;
     const int nb = (n + 31) / 32, q0 = p0 / 32, k1 = p0 + kLuNB;
     const float *T = A + static_cast<int64_t>(p0) * (lda + 1);
-    const int nd = strips < 4 ? strips : 4, y = static_cast<int>(blockIdx.x) - strips;   // y >= 0: a block (r, c)
     const int r = y % nd, c = y / nd;
-    const int o = k1 + 32 * static_cast<int>(blockIdx.x), cnt = n - o < 32 ? n - o : 32;   // a strip
-    // entry k = 32 J + acc_row of row (L21) or column (U12) l32
-    float own[16], left[3][16], iv[16], diag[16];
-    const int64_t step = up ? 1 : lda;
-    float *line = A + (up ? (o + min(l32, cnt - 1)) * lda + p0 + 32 * J + 4 * lh
-                          : (p0 + 32 * J + 4 * lh) * lda + o + min(l32, cnt - 1));
-    {
-        const float *copy = up ? copy_u(tri, nb, q0 + J, q0 + 4 + c) : copy_l(tri, nb, q0 + 4 + r, q0 + J);
-        const float *from = y >= 0 ? copy + 128 * lh + l32 : line;
-        const int64_t d = y >= 0 ? 32 : step;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) own[e] = from[acc_row(e, 0) * d];
-        const float *blk = up ? tri_block_l(tri, nb, q0 + J, q0 + J) : tri_block_u(tri, nb, q0 + J, q0 + J);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int k = acc_row(e, lh);
-            iv[e] = blk[tri_pos(l32 + 32 * (k & 1), k >> 1)];
-            diag[e] = up ? 1.0f : blk[tri_pos(k + 32 * (k & 1), k >> 1)];
-        }
-        const int64_t dk = up ? lda : 1;
-        const float *t = T + (up ? 32 * J + l32 + 4 * lh * lda : (32 * J + l32) * lda + 4 * lh);
-#pragma unroll
-        for (int K = 0; K < 3; ++K)
-            if (K < J)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) left[K][e] = t[(32 * K + acc_row(e, 0)) * dk];
-    }
-    // accumulators 2 wave and 2 wave + 1 of the next block
+    const int o = k1 + 32 * z, cnt = n - o < 32 ? n - o : 32;   // a strip
     const int R = 32 * (q0 + 4 + r), C = 32 * (q0 + 4 + c) + l32;
-    float next[2] = {0.0f, 0.0f};
-    if (y >= 0)
+    float next[4];   // rows 8 J + 4 lh + i of the next block
+#pragma clang loop unroll(disable)
+    for (int side = 0; side < (y >= 0 ? 2 : 1); ++side) {
+        const bool up = y >= 0 ? side != 0 : up1;
+        // entry k = 32 J + acc_row of row (L21) or column (U12) l32
+        float own[16], left[3][16], iv[16], diag[16];
+        const int64_t step = up ? 1 : lda;
+        float *line = A + (up ? (o + min(l32, cnt - 1)) * lda + p0 + 32 * J + 4 * lh
+                              : (p0 + 32 * J + 4 * lh) * lda + o + min(l32, cnt - 1));
+        {
+            const float *copy = up ? copy_u(tri, nb, q0 + J, q0 + 4 + c) : copy_l(tri, nb, q0 + 4 + r, q0 + J);
+            const float *from = y >= 0 ? copy + 128 * lh + l32 : line;
+            const int64_t d = y >= 0 ? 32 : step;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-            next[i] = A[min(C, n - 1) * lda + min(R + acc_row(2 * wave + i, lh), n - 1)];
-    const bool poor = tri_poor(tri, nb)[2 * (q0 + J) + (up ? 0 : 1)] != 0.0f;
-    floatx16g_t S = zero16(), x = zero16();
-#pragma unroll
-    for (int K = 0; K < 4; ++K) {
-        float *xk = xl[up][K];
-        if (J == K) {
-            floatx16g_t D;
-            bool fine = !poor;
+            for (int e = 0; e < 16; ++e) own[e] = from[acc_row(e, 0) * d];
+            const float *blk = up ? tri_block_l(tri, nb, q0 + J, q0 + J) : tri_block_u(tri, nb, q0 + J, q0 + J);
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                D[e] = own[e] + S[e];
-                fine = fine && isfinite(D[e]);
+                const int k = acc_row(e, lh);
+                iv[e] = blk[tri_pos(l32 + 32 * (k & 1), k >> 1)];
+                diag[e] = up ? 1.0f : blk[tri_pos(k + 32 * (k & 1), k >> 1)];
             }
-            if (__all(fine)) {
+            const int64_t dk = up ? lda : 1;
+            const float *t = T + (up ? 32 * J + l32 + 4 * lh * lda : (32 * J + l32) * lda + 4 * lh);
 #pragma unroll
-                for (int e = 0; e < 16; ++e)   // the diagonal's term last, in one rounding
-                    x = __builtin_amdgcn_mfma_f32_32x32x2f32(acc_row(e, lh) == l32 ? 0.0f : iv[e], D[e], x, 0, 0, 0);
+            for (int K = 0; K < 3; ++K)
+                if (K < J)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) x[e] = fmaf(diag[e], own[e], fmaf(diag[e], S[e], x[e]));
-            } else {
+                    for (int e = 0; e < 16; ++e) left[K][e] = t[(32 * K + acc_row(e, 0)) * dk];
+        }
+        if (y >= 0 && side == 0)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) xk[e * 64 + lane] = D[e];
-                const float *d = T + 32 * static_cast<int64_t>(K) * (lda + 1);
-                if (up)
-                    subst32<true>(xk, d, lda, 32, lane);
-                else
-                    subst32<false>(xk, d, lda, 32, lane);
+            for (int i = 0; i < 4; ++i) next[i] = A[min(C, n - 1) * lda + min(R + 8 * J + 4 * lh + i, n - 1)];
+        const bool poor = tri_poor(tri, nb)[2 * (q0 + J) + (up ? 0 : 1)] != 0.0f;
+        floatx16g_t S = zero16(), x = zero16();
 #pragma unroll
-                for (int e = 0; e < 16; ++e) x[e] = xk[e * 64 + lane];
+        for (int K = 0; K < 4; ++K) {
+            float *xk = xl[up][K];
+            if (J == K) {
+                floatx16g_t D;
+                bool fine = !poor;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    D[e] = own[e] + S[e];
+                    fine = fine && isfinite(D[e]);
+                }
+                if (__all(fine)) {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)   // the diagonal's term last, in one rounding
+                        x = __builtin_amdgcn_mfma_f32_32x32x2f32(acc_row(e, lh) == l32 ? 0.0f : iv[e], D[e], x, 0, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) x[e] = fmaf(diag[e], own[e], fmaf(diag[e], S[e], x[e]));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) xk[e * 64 + lane] = D[e];
+                    const float *d = T + 32 * static_cast<int64_t>(K) * (lda + 1);
+                    if (up)
+                        subst32<true>(xk, d, lda, 32, lane);
+                    else
+                        subst32<false>(xk, d, lda, 32, lane);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) x[e] = xk[e * 64 + lane];
+                }
+#pragma unroll
+                for (int e = 0; e < 16; ++e) xk[e * 64 + lane] = -x[e];
             }
+            if (K == 3 && y < 0) break;
+            __syncthreads();
+            if (J > K) {
+                float xv[16];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) xk[e * 64 + lane] = -x[e];
+                for (int e = 0; e < 16; ++e) xv[e] = xk[e * 64 + lane];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    S = __builtin_amdgcn_mfma_f32_32x32x2f32(K == 0 ? left[0][e] : K == 1 ? left[1][e] : left[2][e], xv[e], S, 0, 0, 0);
+            }
         }
-        if (K == 3 && y < 0) break;
-        __syncthreads();
-        if (J > K) {
-            float xv[16];
-#pragma unroll
-            for (int e = 0; e < 16; ++e) xv[e] = xk[e * 64 + lane];
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                S = __builtin_amdgcn_mfma_f32_32x32x2f32(K == 0 ? left[0][e] : K == 1 ? left[1][e] : left[2][e], xv[e], S, 0, 0, 0);
-        }
-    }
-    if (y < 0) {
-        if (l32 < cnt)
+        if (y < 0 && l32 < cnt)
 #pragma unroll
             for (int e = 0; e < 16; ++e) line[acc_row(e, 0) * step] = x[e];
-        return;
     }
-    // block (r, c) of the next diagonal sub-block: a product per wave of the first four, added in order
+    if (y < 0) return;
+    // block (r, c) of the next diagonal sub-block: a product per wave, added in order
     float av[16], bv[16];
-    if (!up)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            av[e] = xl[0][wave][e * 64 + lane];
-            bv[e] = xl[1][wave][e * 64 + lane];
-        }
+    for (int e = 0; e < 16; ++e) {
+        av[e] = xl[0][J][e * 64 + lane];
+        bv[e] = xl[1][J][e * 64 + lane];
+    }
     __syncthreads();
     float *part = xl[0][0];
-    if (!up) {
-        const floatx16g_t acc = mfma16(av, bv, zero16());
+    const floatx16g_t acc = mfma16(av, bv, zero16());
 #pragma unroll
-        for (int e = 0; e < 16; ++e) part[(wave * 16 + e) * 64 + lane] = acc[e];
-    }
+    for (int e = 0; e < 16; ++e) part[(J * 16 + e) * 64 + lane] = acc[e];
     __syncthreads();
     if (C < n)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const float *p = part + (2 * wave + i) * 64 + lane;
-            const int row = R + acc_row(2 * wave + i, lh);
+        for (int i = 0; i < 4; ++i) {
+            const float *p = part + (4 * J + i) * 64 + lane;
+            const int row = R + 8 * J + 4 * lh + i;
             if (row < n) A[C * lda + row] = next[i] - (((p[0] + p[1024]) + p[2048]) + p[3072]);
         }
 }
@@ -786,18 +844,25 @@ __global__ __launch_bounds__(512) void lu_strip_walk_kernel(int n, int p0, float
 // sub-block at p0 (128 wide).  A workgroup owns 32 rows of L21 (blockIdx.x <
 // strips) or 32 columns of U12; wave j computes its 32-wide block j.  The next
 // workgroups update a block each of the next diagonal sub-block, the last ones
-// finish the whole block's inverses of this one.
+// finish the whole block's inverses of this one.  Where the sub-block is not well
+// conditioned, the walk above takes their place; whether it does is looked up
+// beside the operands' loads.
 __global__ __launch_bounds__(256) void lu_strip_kernel(int n, int p0, float *A, int64_t lda, float *tri, int strips)
 {
-    __shared__ float X[kLuNB * 33], X2[kLuNB * 33];
+    __shared__ float X[2 * kLuNB * 33];
+    static_assert(sizeof(X) >= sizeof(float[2][4][1024]), "the walk's blocks");
+    auto walk = reinterpret_cast<float (*)[4][1024]>(X);
     const int tid = threadIdx.x, lane = tid & 63, J = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
     const int nb = (n + 31) / 32, q0 = p0 / 32, k1 = p0 + kLuNB;
+    const int careful = __float_as_int(tri_careful(tri, nb)[q0 / 4]);
+    const int nd = strips < 4 ? strips : 4;
     if (static_cast<int>(blockIdx.x) >= 2 * strips) {
-        const int nd = strips < 4 ? strips : 4, y = static_cast<int>(blockIdx.x) - 2 * strips, z = y - nd * nd;
-        if (z < 0)
-            next_diagonal(n, nb, q0, y % nd, y / nd, A, lda, tri, X, X2);
-        else if (z & 1)
+        const int y = static_cast<int>(blockIdx.x) - 2 * strips, z = y - nd * nd;
+        if (z < 0) {
+            if (!next_diagonal(n, nb, q0, y % nd, y / nd, A, lda, tri, X, X + kLuNB * 33, careful))
+                strip_walk(n, p0, A, lda, tri, 0, false, y, nd, walk);
+        } else if (z & 1)
             tri_fin<true, 4, 1>(nb, tri, z >> 1, q0, nb < q0 + 4 ? nb : q0 + 4);
         else
             tri_fin<false, 4, 1>(nb, tri, z >> 1, q0, nb < q0 + 4 ? nb : q0 + 4);
@@ -836,6 +901,10 @@ __global__ __launch_bounds__(256) void lu_strip_kernel(int n, int p0, float *A, 
         }
     }
     __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(careful) != 0) {
+        strip_walk(n, p0, A, lda, tri, static_cast<int>(blockIdx.x) - (up ? strips : 0), up, -1, nd, walk);
+        return;
+    }
     floatx16g_t acc = zero16();
 #pragma unroll
     for (int K = 0; K < 4; ++K) {
@@ -891,7 +960,7 @@ __global__ __launch_bounds__(kLuThreads) void tri_join_kernel(int n, int H, cons
 int64_t tri_floats(int b)
 {
     const int64_t nb = ceil_div(b, 32);
-    return 2 * nb * nb * 1024 + 64;
+    return 2 * nb * nb * 1024 + 128;
 }
 
 int64_t getrf_scratch_floats(int n) { return n > kLuNB ? tri_floats(n) : 0; }
@@ -905,22 +974,14 @@ int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, bool full,
         const int tiles = k == 0 ? (rest > kLuNB ? 4 : 0) : rt * ct - (ct < 2 ? ct : 2);
         // the whole block's inverses, and the last sub-block's, serve only a caller who asked for them
         const unsigned join = full ? 2 * (k / 32) : 0;
-        const dim3 g(static_cast<unsigned>(1 + tiles) + join);
-        if (full)
-            hipLaunchKernelGGL((lu_update_kernel<true, true>), g, dim3(kLuThreads), 0, s, n, k, A, lda, tri, 3, info);
-        else
-            hipLaunchKernelGGL((lu_update_kernel<true, false>), g, dim3(kLuThreads), 0, s, n, k, A, lda,
-                               rest <= kLuNB ? nullptr : tri, 3, info);
+        hipLaunchKernelGGL((lu_update_kernel<true, true>), dim3(static_cast<unsigned>(1 + tiles) + join), dim3(kLuThreads),
+                           0, s, n, k, A, lda, !full && rest <= kLuNB ? nullptr : tri, 3, info);
         HPLAI_HIP(hipGetLastError());
         const int strips = rest > kLuNB ? (rest - kLuNB + 31) / 32 : 0;
         const int nd = strips < 4 ? strips : 4;
         if (strips + join > 0) {
-            if (full)
-                hipLaunchKernelGGL(lu_strip_kernel, dim3(static_cast<unsigned>(2 * strips + nd * nd) + join), dim3(256), 0, s,
-                                   n, k, A, lda, tri, strips);
-            else
-                hipLaunchKernelGGL(lu_strip_walk_kernel, dim3(static_cast<unsigned>(strips + nd * nd)), dim3(512), 0, s, n, k,
-                                   A, lda, tri, strips);
+            hipLaunchKernelGGL(lu_strip_kernel, dim3(static_cast<unsigned>(2 * strips + nd * nd) + join), dim3(256), 0, s,
+                               n, k, A, lda, tri, strips);
             HPLAI_HIP(hipGetLastError());
         }
     }

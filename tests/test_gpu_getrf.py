@@ -275,3 +275,22 @@ def test_getrf_far_from_dominance(ctx, n, pad, diag):
     bound = 2 * (n + 80) * u * (np.abs(L) @ np.abs(U))
     R = np.abs(A.astype(np.float64) - L @ U)
     assert (R <= bound).all(), float((R / bound).max())
+
+
+@pytest.mark.parametrize("n,pad", [(129, 0), (160, 4), (256, 0), (300, 0), (512, 0), (777, 3), (1024, 0)])
+@pytest.mark.parametrize("diag", [0.3, 1.0, 3.0, 6.0, 400.0])
+def test_factor_of_one_block_far_from_dominance(ctx, n, pad, diag):
+    """The solve's own LU of a single block, whose factors stay FP32: the bound
+    above with 16 more roundings for the strips through inverses of 128 x 128
+    sub-blocks, which too are taken only where |D^-1| |D| is below 16."""
+    import torch
+    rng = np.random.default_rng(n)
+    A = (rng.uniform(-0.5, 0.5, (n, n)) * (1.0 - np.eye(n)) + np.eye(n) * diag * rng.choice([-1.0, 1.0], n)).astype(np.float32)
+    F = torch.from_numpy(np.ascontiguousarray(np.pad(A.T, ((0, 0), (0, pad))))).cuda()
+    ctx.factor(n, n, F, n + pad)
+    M = F[:, :n].t().cpu().numpy().astype(np.float64)
+    L, U = np.tril(M, -1) + np.eye(n), np.triu(M)
+    assert np.isfinite(M).all()
+    bound = 2 * (n + 96) * 2.0 ** -24 * (np.abs(L) @ np.abs(U))
+    R = np.abs(A.astype(np.float64) - L @ U)
+    assert (R <= bound).all(), float((R / bound).max())
