@@ -216,7 +216,8 @@ def bench_batch(args):
     ctx.close()
     t = sum(r["seconds"] for r in runs) / len(runs)
     last = runs[-1]
-    # roofline of batch_kernel: HBM-bound.  Algorithmic bytes per system: the
+    # roofline of batch_kernel against the HBM rate (its workgroups' chains of
+    # blocks bind it before memory does).  Algorithmic bytes per system: the
     # FP32 matrix written by the generation and read and written once by the
     # LU, 12 n^2; its FP16 L written once, n^2, and read by every later block of
     # 32 columns, sum_p 64 (n - 32 p) (n / 32 - p) ~ n^3 / 48; both triangles

@@ -132,7 +132,7 @@ int launch_higham_norm(int64_t n, double alpha, double beta, double *ones, doubl
 int launch_gen_rhs(int64_t n, uint64_t seed, int64_t i0, int64_t cnt, double *b, hipStream_t s);
 
 // LU of an n x n block (n <= 1024) in place.  tri: tri_floats(n), packed
-// (device_common.hpp): the full inverses of the triangles (FULL), or scratch
+// (device_common.hpp): the full inverses of the triangles (full), or scratch
 // (may be NULL up to getrf_scratch_floats(n) == 0).
 int launch_getrf(int n, float *A, int64_t lda, int *info, float *tri, bool full, hipStream_t s);
 int64_t getrf_scratch_floats(int n);

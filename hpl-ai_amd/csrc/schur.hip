@@ -828,7 +828,10 @@ static int schur_repack(int64_t rows, int64_t kbytes, const void *src, int64_t l
 // + n) K bytes, against 8-10 % of the update's 2 m n K operations.  Row layout /
 // packed with the pass, e4m3, K = 8192: 16384 x 16384 1856 / 1846 us, 24000 x 24000
 // 4811 / 4333, 32768 x 32768 8056 / 7339; K = 4096: 12000 x 12000 674 / 675, 24000 x
-// 24000 2772 / 2551; K <= 1024 within 3 % either way; FP16 alike.
+// 24000 2772 / 2551; K <= 1024 within 3 % either way; FP16 alike.  The copy has to
+// fit a scratch buffer that is kept (kScratchMax, (m + n) K <= 512 MiB; the largest
+// e4m3 shape above fills it): past that, and under capture, the update runs on the
+// row layout.
 static bool schur_repack_pays(int64_t m, int64_t n, int64_t kbytes)
 {
     return kbytes >= 2048 && static_cast<double>(m) * static_cast<double>(n) >= 11000.0 * static_cast<double>(m + n);

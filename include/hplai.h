@@ -385,9 +385,10 @@ int hplai_solution_block(hplai_ctx ctx, int64_t i0, int64_t j0, int64_t m, int64
 /* Drop the factors and the solution kept by keep_factors.  Their memory, like
  * the other buffers of hplai_solve and hplai_factor_f32, goes to a cache from
  * which the next solve on the device allocates: at most a sixth of the
- * device's memory, shared by the process's contexts, given back by hplai_trim,
- * when the last context on the device is destroyed and when an allocation of
- * this library would fail. */
+ * device's memory (48 GB of 288: the matrices of orders up to about 100 000;
+ * larger buffers are allocated and freed by each call), shared by the process's
+ * contexts, given back by hplai_trim, when the last context on the device is
+ * destroyed and when an allocation of this library would fail. */
 int hplai_release(hplai_ctx ctx);
 /* Gives memory that is kept for later calls back to the device, for another
  * allocator in the process to use: the idle blocks of the cache above and this
